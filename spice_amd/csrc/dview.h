@@ -10,15 +10,17 @@
 //   acc[a]   receive accumulators of attribute a  [2][N] by step parity: fp32 / int64 (fixed
 //                        point) / int32
 //   sa[a]    attribute a of every synapse         CSR order (plastic models only)
-//   ring     int32[(D+2) * N], counts uint32[D+2] spike ids of the last D+2 steps (entry t mod
-//                        (D+2): step T's update clears step T+1's entry while step T's
-//                        delivery may still read step T-D's)
+//   ring     int32[rsize * N], counts uint32[rsize] spike ids of the last steps (entry t mod
+//                        rsize; rsize >= D + 2 wcap: the last step of a window of W <= wcap steps
+//                        clears the entries of the wcap steps after it, while step T - D's may
+//                        still be read; never-written entries are empty)
 //   hring    uint64[HWORDS * N]  spike-history ring: bit (t mod H) of word (t mod H)/64 of
 //                        neuron i set iff i spiked at step t (H = 256 steps, plastic models)
 //   hasp     uint8[N]    row s has at least one plastic synapse
 //   pl_lo/hi int32[N]    first / one-past-last plastic slot of row s (offsets in the row)
 //   pivots   int32[N * (ntiles+1)]  per row and target tile: offset of the tile's first target
-//   tile_ids int32[nact] the tiles that some row has targets in (at least one tile)
+//   tile_ids int32[ntiles] the tiles: first the nact ones that some row has targets in (at least
+//                        one), then the rest
 // lazy plasticity (per-synapse contract):
 //   last_spk int32[N]    latest spike step
 //   synced   int32[N]    row s is up to date through this step
@@ -56,7 +58,7 @@ struct ctl_t
 	std::int64_t step; // index of the step being executed
 	float sum;         // Kahan sum of dt over completed steps
 	float c;           // Kahan compensation
-	std::int32_t rslot; // spike ring entry of this step: step mod (D + 2)
+	std::int32_t rslot; // spike ring entry of this step: step mod rsize
 };
 
 // Device counters live in per-block slots: block b of any step kernel adds its block-reduced
@@ -103,8 +105,8 @@ struct dview
 	std::int32_t overlap; // 1: the update of step T runs beside the delivery of T + 1 (it writes
 	                      // the spike log's step offsets then; otherwise the delivery does)
 	std::int32_t upd_slot0; // first statistics slot of the update blocks of an overlapped kernel
-	std::int32_t fused;     // 1: one kernel per step, each tile updated by its delivery workgroup
-	                        // (the update then writes the spike log's step offsets)
+	std::int32_t rsize;     // entries of the spike ring
+	std::int32_t wcap;      // longest window of steps run by one kernel
 	std::uint32_t flags;
 	std::uint64_t seed;
 	float param[4]; // per-net model parameters (snn_info::param)
@@ -146,7 +148,7 @@ struct dview
 
 	std::int32_t * pivots; // [N][ntiles + 1]: offset in row r of its first target >= t * tile_w
 	std::int32_t ntiles, tile_w;
-	std::int32_t * tile_ids; // [nact]: the tiles with incoming synapses (the delivery's tiles)
+	std::int32_t * tile_ids; // [ntiles]: the tiles with incoming synapses (the delivery's), then the others
 	std::int32_t nact;
 
 	slog_t * slog; // nullptr: no spike log

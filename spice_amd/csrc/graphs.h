@@ -22,6 +22,46 @@
 
 namespace spice::hipx
 {
+// Bounds the kernels queued ahead of the GPU by a run of eager launches: every EVERY launches an
+// event is recorded, and the host waits for the one recorded DEPTH records before.
+class launch_queue
+{
+public:
+	static constexpr int EVERY = 32, DEPTH = 8;
+
+	launch_queue() = default;
+	launch_queue( launch_queue const & ) = delete;
+	launch_queue & operator=( launch_queue const & ) = delete;
+	~launch_queue() { clear(); }
+
+	// The caller has synchronized the stream.
+	void clear()
+	{
+		for( auto & e : _ev )
+		{
+			if( e ) (void)hipEventDestroy( e );
+			e = nullptr;
+		}
+		_n = 0;
+	}
+
+	// One more launch was enqueued on s.
+	void launched( hipStream_t s )
+	{
+		if( ++_n % EVERY ) return;
+		hipEvent_t & e = _ev[_n / EVERY % DEPTH];
+		if( !e )
+			SPICE_HIP( hipEventCreateWithFlags( &e, hipEventDisableTiming ) );
+		else
+			SPICE_HIP( hipEventSynchronize( e ) );
+		SPICE_HIP( hipEventRecord( e, s ) );
+	}
+
+private:
+	hipEvent_t _ev[DEPTH] = {};
+	std::uint64_t _n = 0;
+};
+
 class step_graphs
 {
 public:

@@ -197,14 +197,14 @@ __device__ inline snn_info info_of( dview const & v )
 }
 __device__ inline float step_dt( dview const & v ) { return v.DT - v.ctl->c; }
 
-// Spike ring entry of step t (t >= -D): D + 2 entries, so that the update of step T clears the
-// entry of step T + 1 (last read by the delivery of step T - 1) while step T's delivery may
-// still read the entry of step T - D.
-__device__ inline int ring_slot( dview const & v, std::int64_t t ) { return int( ( t + v.D + 2 ) % ( v.D + 2 ) ); }
-// The same for step ctl->step + k, -D <= k <= 1, from the clock's entry (no division).
+// Spike ring entry of step t (t >= -D): at least D + 2 wcap entries, so that the update of step T
+// clears the entries of the wcap steps after it (last read by deliveries of earlier steps) while
+// step T's delivery may still read the entry of step T - D.
+__device__ inline int ring_slot( dview const & v, std::int64_t t ) { return int( ( t + v.rsize ) % v.rsize ); }
+// The same for step ctl->step + k, -D <= k <= wcap, from the clock's entry (no division).
 __device__ inline int ring_at( dview const & v, int k )
 {
-	int const r = v.ctl->rslot + k, R = v.D + 2;
+	int const r = v.ctl->rslot + k, R = v.rsize;
 	return r < 0 ? r + R : r >= R ? r - R : r;
 }
 
@@ -694,10 +694,8 @@ __device__ inline void deliver_event( A &&... a )
 // LDS with LDS atomics; at the end the tile's sums go to the global accumulators with plain
 // stores: one workgroup owns each tile, so no global atomics are needed. AHEAD: the kernel's
 // clock is step T - 1's (the overlapped step kernel delivers the next step beside the update).
-// KEEP (the fused step, one work item per tile): the sums stay in LDS for the same workgroup's
-// update of the tile; the returned pointer addresses them ([attribute][TM], as stored below).
-template <typename Model, bool FIXED, int BS, bool AHEAD = false, int TM = TILE_MAX, bool KEEP = false>
-__device__ inline void const * receive_tile( dview const & v, std::int32_t work )
+template <typename Model, bool FIXED, int BS, bool AHEAD = false, int TM = TILE_MAX>
+__device__ inline void receive_tile( dview const & v, std::int32_t work )
 {
 	// work item = (active tile, part): the tile's spike list is split into v.rparts parts,
 	// each delivered by its own workgroup (more workgroups in flight for few, large tiles);
@@ -750,7 +748,7 @@ __device__ inline void const * receive_tile( dview const & v, std::int32_t work 
 	std::int32_t const nall = T < v.D ? 0 : std::int32_t( v.counts[slot] );
 	std::int32_t const s_beg = std::int32_t( std::int64_t( nall ) * part / v.rparts );
 	std::int32_t const nspk = std::int32_t( std::int64_t( nall ) * ( part + 1 ) / v.rparts ) - s_beg;
-	if( !v.overlap && !v.fused && v.slog && work == 0 && threadIdx.x == 0 )
+	if( !v.overlap && v.slog && work == 0 && threadIdx.x == 0 )
 	{
 		// spike log: step T's ids start where step T-1's (final by now) end
 		std::int64_t const k = T - v.slog->t0;
@@ -1029,7 +1027,7 @@ __device__ inline void const * receive_tile( dview const & v, std::int32_t work 
 		bool const owned = v.rparts == 1;
 		std::int64_t const apar = ( T & 1 ) * std::int64_t( v.N );
 		util::for_n<N::size>( [&]( auto I ) {
-			if constexpr( !KEEP && ( ( rmask >> I ) & 1u ) != 0 )
+			if constexpr( ( ( rmask >> I ) & 1u ) != 0 )
 			{
 				using A = acc_type<typename N::template type<I>, FIXED>;
 				constexpr int a = __builtin_popcount( rmask & ( ( 1u << I ) - 1u ) );
@@ -1050,7 +1048,6 @@ __device__ inline void const * receive_tile( dview const & v, std::int32_t work 
 		__syncthreads();
 	}
 	block_add_stats<2>( v, work, { ev, pev }, { ST_EVENTS, ST_PLASTIC } );
-	return acc;
 }
 
 template <typename Model, bool FIXED>
@@ -1173,11 +1170,8 @@ __global__ __launch_bounds__( BS ) void k_batch_step_overlap( dview const * view
 // Neuron update of neurons [first, first + min(count, blockDim.x)) (blockDim.x <= 1024) at step
 // T; statistics go to slot `slot`. The range that starts at neuron 0 also clears the next
 // step's counters and writes the next step's clock.
-// lds (the fused step): the inputs are the tile sums a KEEP delivery left in LDS for neurons
-// lds_t0 ..; [attribute][lds_stride words]) instead of the global accumulators, which stay zero.
 template <typename Model, bool FIXED>
-__device__ inline void update_range( dview const & v, std::int64_t first, std::int32_t count, std::int64_t slot, void const * lds = nullptr,
-                                     std::int32_t lds_t0 = 0, std::int32_t lds_stride = 0 )
+__device__ inline void update_range( dview const & v, std::int64_t first, std::int32_t count, std::int64_t slot )
 {
 	using N = typename Model::neuron;
 	using S = typename Model::synapse;
@@ -1187,9 +1181,10 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 
 	std::int64_t const T = v.ctl->step;
 	int const wslot = ring_at( v, 0 );
+	// the next wcap steps' counters (the entries were last delivered before this step)
+	if( first == 0 && std::int32_t( threadIdx.x ) < v.wcap ) v.counts[ring_at( v, 1 + std::int32_t( threadIdx.x ) )] = 0;
 	if( first == 0 && threadIdx.x == 0 )
 	{
-		v.counts[ring_at( v, 1 )] = 0; // step T - D - 1's entry (delivered at T - 1); refilled at T + 1
 		if constexpr( plastic ) v.fl_count[( T + 1 ) & 3] = 0; // step T - 1's flush may still read slot (T - 1) & 3
 		if constexpr( eager ) v.po_count[( T + 1 ) & 3] = 0;
 		// next step's clock: exactly kahan_sum::add on the host
@@ -1199,7 +1194,7 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 		v.ctl_next->c = ( t - c.sum ) - y;
 		v.ctl_next->sum = t;
 		v.ctl_next->step = c.step + 1;
-		v.ctl_next->rslot = c.rslot + 1 == v.D + 2 ? 0 : c.rslot + 1;
+		v.ctl_next->rslot = c.rslot + 1 == v.rsize ? 0 : c.rslot + 1;
 	}
 	float const dt = step_dt( v );
 	snn_info const info = info_of( v );
@@ -1251,17 +1246,8 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 			{
 				using A = typename N::template type<I>;
 				using AC = acc_type<A, FIXED>;
-				AC a;
-				if( lds )
-				{
-					constexpr int slotI = __builtin_popcount( rmask & ( ( 1u << I ) - 1u ) );
-					a = reinterpret_cast<AC const *>( static_cast<acc_word<N, FIXED> const *>( lds ) + slotI * lds_stride )[i - lds_t0];
-				}
-				else
-				{
-					a = ld<AC>( v.acc[I], ai );
-					st<AC>( v.acc[I], ai, AC( 0 ) );
-				}
+				AC const a = ld<AC>( v.acc[I], ai );
+				st<AC>( v.acc[I], ai, AC( 0 ) );
 				if constexpr( std::is_floating_point_v<A> && FIXED )
 				{
 					if( open ) std::get<I>( s ) = std::get<I>( s ) + float( a ) * __builtin_ldexpf( 1.0f, -v.shift );
@@ -1366,15 +1352,14 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 		if( v.slog )
 		{
 			// where step T's ids start in the log: written by this step's delivery kernel, or
-			// (the overlapped step, whose delivery of step T ran beside step T - 1's update; the
-			// fused step, whose delivery may not have written it yet) here, from step T - 1's
-			// offset and count, both final (written by an earlier kernel; this update clears
-			// the count of step T + 1, not of T - 1)
+			// (the overlapped step, whose delivery of step T ran beside step T - 1's update) here,
+			// from step T - 1's offset and count, both final (written by an earlier kernel; this
+			// update clears the counts of steps after T, not of T - 1)
 			std::int64_t const k = T - v.slog->t0;
 			std::uint64_t base = 0;
 			if( k >= 0 && k < v.slog->nsteps )
 			{
-				if( !v.overlap && !v.fused )
+				if( !v.overlap )
 					base = v.slog_off[k];
 				else
 				{
@@ -1445,31 +1430,6 @@ template <typename Model, bool FIXED, int BS = SPICE_UPDATE_BLOCK>
 __global__ __launch_bounds__( BS ) void k_update( dview v )
 {
 	update_block<Model, FIXED>( v, blockIdx.x, blockIdx.x );
-}
-
-// The fused step (static models whose steps do not overlap, one delivery work item per tile,
-// every tile a delivery tile, tiles of at most FUSE_CHUNKS workgroup widths): one kernel per
-// step. The workgroup that delivers step T's arrivals to a tile holds all of the tile's inputs
-// (its LDS sums, which never go to the global accumulators), so it goes on to update the
-// tile's neurons at step T from them. No workgroup waits for another, and no delivery reads what an
-// update of the same step writes (other tiles' neurons, the ring entry of step T, the counters
-// of steps T and T + 1). Several work items per tile would need a device-scope fence per item
-// to hand the sums to the tile's last one (with one L2 per XCD, such a fence writes back and
-// invalidates the XCD's L2): measured 4.5-7x slower per step than two kernels. Update
-// statistics go to slots from upd_slot0 (FUSE_CHUNKS per tile).
-constexpr int FUSE_CHUNKS = 4;
-template <typename Model, bool FIXED, int BS>
-__global__ __launch_bounds__( BS ) void k_step_fused( dview v, std::int32_t grecv, std::int32_t upd_slot0 )
-{
-	for( std::int32_t w = blockIdx.x; w < v.nact; w += grecv )
-	{
-		void const * sums = receive_tile<Model, FIXED, BS, false, TILE_MAX, true>( v, w );
-		std::int32_t const tile = v.tile_ids[w];
-		std::int32_t const t0 = tile * v.tile_w;
-		std::int32_t const tw = ( v.N - t0 ) < v.tile_w ? ( v.N - t0 ) : v.tile_w;
-		for( std::int32_t c = 0; c < tw; c += BS )
-			update_range<Model, FIXED>( v, t0 + c, tw - c, upd_slot0 + std::int64_t( tile ) * FUSE_CHUNKS + c / BS, sums, t0, TILE_MAX );
-	}
 }
 
 // Batched neuron update: workgroup b updates block block_local[b] of net block_net[b].

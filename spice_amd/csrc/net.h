@@ -8,6 +8,7 @@
 #include "graph.h"
 #include "graphs.h"
 #include "kernels.h"
+#include "window.h"
 
 #include <spice/models/model.h>
 #include <spice/util/graphgen.h>
@@ -101,6 +102,21 @@ inline int device_cu_count()
 	return cus;
 }
 
+// Longest window of steps one kernel may run (k_window): static models whose delivery may run
+// before its targets' update, up to the delay.
+template <typename Model>
+int window_cap( int delay )
+{
+	return !is_plastic_v<Model> && overlap_capable_v<Model> && delay >= 2 ? window_steps( delay ) : 1;
+}
+// Entries of the spike ring: the delay and two windows; four at least, so that with a delay of
+// one step the entry of a step is its clock slot, known without reading the clock.
+template <typename Model>
+int ring_entries( int delay )
+{
+	return std::max( 4, delay + 2 * window_cap<Model>( delay ) );
+}
+
 template <typename Model>
 class hip_net final : public net_iface
 {
@@ -133,6 +149,7 @@ public:
 	{
 		if( _s ) (void)hipStreamSynchronize( _s );
 		_graphs.clear();
+		_queue.clear();
 		if( _s ) (void)hipStreamDestroy( _s );
 	}
 
@@ -142,7 +159,7 @@ public:
 		std::int64_t const t = _step;
 		launch_steps( t, 1 );
 		tick();
-		int const slot = int( t % ( _p.delay + 2 ) );
+		int const slot = int( t % _v.rsize );
 		if( dspk ) *dspk = _ring.data() + std::int64_t( slot ) * _g.n;
 		if( dcnt ) *dcnt = _counts.data() + slot;
 	}
@@ -152,6 +169,19 @@ public:
 	{
 		if( n < 0 ) throw std::invalid_argument( "negative step count" );
 		if( n == 0 ) return;
+		if( _window > 1 )
+		{
+			// windows are long enough to be launched one by one (a launch costs the host a few us)
+			while( n > 0 )
+			{
+				int const w = window_steps( std::min<std::int64_t>( n, _window ) );
+				launch_window( _step, w, nullptr, nullptr );
+				_queue.launched( _s );
+				for( int i = 0; i < w; i++ ) tick();
+				n -= w;
+			}
+			return;
+		}
 		if( _graphs.empty() ) _graphs.capture( _s, [&]( int t, int len ) { launch_steps( t, len ); } );
 		_graphs.run( _s, _step, n, [&] { tick(); } );
 	}
@@ -160,16 +190,13 @@ public:
 	// stream, and adds the summed kernel durations (ms) to kernel_ms[0..2]: receive (delivery,
 	// with the previous step's plasticity), update, and 0; overlapped steps: the first delivery,
 	// the last update (with the passes of the step before it), and the n - 1 overlapped step
-	// kernels; fused steps: 0, 0 and the n step kernels.
+	// kernels; windows: 0, 0 and the window kernels.
 	void run_profiled( std::int64_t n, double * kernel_ms ) override
 	{
 		if( n < 0 ) throw std::invalid_argument( "negative step count" );
-		if( _fused )
+		if( _window )
 		{
-			if( fixed() )
-				run_profiled_fused<true>( n, kernel_ms );
-			else
-				run_profiled_fused<false>( n, kernel_ms );
+			run_profiled_windows( n, kernel_ms );
 			return;
 		}
 		if( _overlap )
@@ -228,7 +255,7 @@ public:
 			*count = 0;
 			return;
 		}
-		int const slot = int( ( _step - 1 ) % ( _p.delay + 2 ) );
+		int const slot = int( ( _step - 1 ) % _v.rsize );
 		std::uint32_t c = 0;
 		SPICE_HIP( hipMemcpyAsync( &c, _counts.data() + slot, 4, hipMemcpyDeviceToHost, _s ) );
 		SPICE_HIP( hipStreamSynchronize( _s ) );
@@ -262,7 +289,7 @@ public:
 	{
 		if( step < 0 || step > INT_MAX - 2 ) throw std::invalid_argument( "invalid step index" );
 		synchronize();
-		ctl_t ctl{ step, sum, c, std::int32_t( step % ( _p.delay + 2 ) ) };
+		ctl_t ctl{ step, sum, c, std::int32_t( step % _v.rsize ) };
 		SPICE_HIP( hipMemcpy( _ctl.data() + ( step & ( CLOCK_SLOTS - 1 ) ), &ctl, sizeof( ctl ), hipMemcpyHostToDevice ) );
 		SPICE_HIP( hipMemset( _counts.data(), 0, _counts.bytes() ) );
 		if constexpr( plastic )
@@ -440,7 +467,7 @@ public:
 		if( _slog_n == 0 ) return 0;
 		SPICE_HIP( hipMemcpy( off, _slog_off.data(), std::size_t( _slog_n ) * 8, hipMemcpyDeviceToHost ) );
 		std::uint32_t last = 0;
-		int const slot = int( ( _step - 1 ) % ( _p.delay + 2 ) );
+		int const slot = int( ( _step - 1 ) % _v.rsize );
 		SPICE_HIP( hipMemcpy( &last, _counts.data() + slot, 4, hipMemcpyDeviceToHost ) );
 		std::uint64_t const total = off[_slog_n - 1] + last;
 		off[_slog_n] = total;
@@ -562,7 +589,9 @@ private:
 	int _upd_block = SPICE_UPDATE_BLOCK;
 	int _grid_plast = 0; // plasticity workgroups of the delivery kernel
 	bool _overlap = false; // steps run as k_step_overlap kernels
-	bool _fused = false;   // steps run as k_step_fused kernels (decided by the launch shape)
+	int _window = 0;       // longest window of the window kernels that run the steps (0: none)
+	int _lanes_log2 = 4;   // window kernels: lanes that walk a row segment
+	launch_queue _queue;
 	launch_cfg _lc{};
 	dbuf<std::int32_t> _pivots;
 	dbuf<std::int32_t> _tile_ids;
@@ -614,8 +643,10 @@ private:
 			using A = typename S::template type<I>;
 			_sa[I].resize( std::max<std::int64_t>( _g.nnz, 1 ) * sizeof( A ) );
 		} );
-		_ring.resize( std::size_t( _p.delay + 2 ) * n );
-		_counts.resize( _p.delay + 2 );
+		_v.wcap = window_cap<Model>( _p.delay );
+		_v.rsize = ring_entries<Model>( _p.delay );
+		_ring.resize( std::size_t( _v.rsize ) * n );
+		_counts.resize( _v.rsize );
 		SPICE_HIP( hipMemsetAsync( _counts.data(), 0, _counts.bytes(), _s ) );
 		if constexpr( plastic )
 		{
@@ -830,19 +861,14 @@ private:
 		_grid_plast = plastic ? std::max( 1, _grid_flush * 256 / c.recv_block ) : 0; // the same waves as flush_grid
 		_lc = c;
 		v.upd_slot0 = upd_slot0();
-		// one kernel per step (k_step_fused): static models whose steps do not overlap, one
-		// delivery work item per tile, every tile a delivery tile, tiles of at most FUSE_CHUNKS
-		// workgroup widths
-		_fused = !plastic && !_overlap && c.recv_parts == 1 && v.nact == v.ntiles && c.tile_w <= TILE_MAX &&
-		         c.tile_w <= FUSE_CHUNKS * c.recv_block;
-		v.fused = _fused ? 1 : 0;
+		choose_window();
 		// statistics slots: one per workgroup of the widest step kernel (receive: per work item;
 		// eager plasticity: after those, one per plasticity workgroup or synchronization block;
-		// the overlapped step's update blocks, or the fused step's FUSE_CHUNKS per tile, after
-		// those), and enough for the update kernel's blocks
+		// the overlapped step's update blocks after those; windows: one per tile), and enough for
+		// the update kernel's blocks
 		std::size_t const slots =
 		    std::size_t( std::max( { _grid_update, _grid_upd, 2 * _grid_flush, 2 * _grid_tiles,
-		                             upd_slot0() + _grid_update, upd_slot0() + FUSE_CHUNKS * v.ntiles } ) ) *
+		                             upd_slot0() + _grid_update } ) ) *
 		    NSTAT; // (update blocks of >= 256 neurons)
 		if( slots > _bstats.size() )
 		{
@@ -887,10 +913,37 @@ private:
 		for( std::int32_t t = 0; t < v.ntiles; t++ )
 			if( f[std::size_t( t )] ) ids.push_back( t );
 		if( ids.empty() ) ids.push_back( 0 );
+		v.nact = std::int32_t( ids.size() );
+		for( std::int32_t t = 0; t < v.ntiles; t++ )
+			if( !f[std::size_t( t )] && ( t != ids[0] || v.nact > 1 ) ) ids.push_back( t );
 		_tile_ids.resize( ids.size() );
 		SPICE_HIP( hipMemcpy( _tile_ids.data(), ids.data(), ids.size() * 4, hipMemcpyHostToDevice ) );
 		v.tile_ids = _tile_ids.data();
-		v.nact = std::int32_t( ids.size() );
+	}
+
+	// Window kernels (_window: their longest window, 0: none) run the steps of static models: those
+	// whose delivery may run before its targets' update in windows of up to the delay, as long as
+	// the accumulators fit; the others step by step where one workgroup delivers a tile
+	// (recv_parts = 1) of at most 4 workgroup widths.
+	void choose_window()
+	{
+		_window = 0;
+		if constexpr( !plastic )
+		{
+			if( !_overlap && ( _lc.recv_parts != 1 || _lc.tile_w > 4 * _lc.recv_block ) ) return;
+			_window = 1;
+			with_window_kernel( [&]( auto kernel, auto bytes, int ) {
+				int w = _v.wcap;
+				while( w > 1 && bytes( w ) > WINDOW_LDS ) w = window_steps( w - 1 );
+				_window = w;
+				if( bytes( w ) > ( 64 << 10 ) )
+					SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( w ) ) ) );
+			} );
+			// lanes per segment: the power of two that holds the mean row segment of a tile
+			double const mean = _g.n > 0 ? double( _g.nnz ) / double( _g.n ) / _v.nact : 0.0;
+			_lanes_log2 = 2;
+			while( _lanes_log2 < 6 && double( 1 << _lanes_log2 ) < mean ) _lanes_log2++;
+		}
 	}
 
 	void initialize()
@@ -914,15 +967,9 @@ private:
 	// next delivery kernel (or a synchronization).
 	void launch_steps( std::int64_t t, std::int64_t len )
 	{
-		if( _fused )
+		if( _window )
 		{
-			for( std::int64_t k = 0; k < len; k++ )
-			{
-				if( fixed() )
-					launch_fused<true>( _vs[( t + k ) & ( CLOCK_SLOTS - 1 )], nullptr, nullptr );
-				else
-					launch_fused<false>( _vs[( t + k ) & ( CLOCK_SLOTS - 1 )], nullptr, nullptr );
-			}
+			for( std::int64_t k = 0; k < len; k++ ) launch_window( t + k, 1, nullptr, nullptr );
 			return;
 		}
 		if( !_overlap )
@@ -1051,29 +1098,48 @@ private:
 		}
 	}
 
-	// the fused step kernel (static models), with HIP events attached to its dispatch when
-	// start is not null
-	template <bool F>
-	void launch_fused( dview const & v, hipEvent_t start, hipEvent_t stop )
+	// The window of w steps from step t (static models), with HIP events attached to its dispatch
+	// when start is not null.
+	void launch_window( std::int64_t t, int w, hipEvent_t start, hipEvent_t stop )
 	{
 		if constexpr( !plastic )
 		{
-			std::int32_t const tiles = _grid_tiles, s0 = upd_slot0();
-			auto go = [&]( auto b ) {
-				constexpr int BS = decltype( b )::value;
+			if( _slog_ctl.size() ) throw std::logic_error( "nets with a spike log are stepped by a batch" );
+			dview v = _vs[t & ( CLOCK_SLOTS - 1 )];
+			v.ctl_next = _ctl.data() + ( ( t + w ) & ( CLOCK_SLOTS - 1 ) );
+			with_window_kernel( [&]( auto kernel, auto bytes, int bs ) {
+				// the ring entry of step t: the clock phase if the ring has CLOCK_SLOTS entries (a
+				// captured launch replays at any step of its phase), else known to eager launches only
+				std::int32_t const slot0 = _window > 1 || v.rsize == CLOCK_SLOTS ? std::int32_t( t % v.rsize ) : -1;
+				std::int32_t const W = w, lg = _lanes_log2;
+				void * args[] = { &v, const_cast<std::int32_t *>( &W ), const_cast<std::int32_t *>( &slot0 ), const_cast<std::int32_t *>( &lg ) };
+				void const * fn = reinterpret_cast<void const *>( kernel );
 				if( start )
-					launch_timed( reinterpret_cast<void const *>( &k_step_fused<Model, F, BS> ), unsigned( tiles ), BS, start, stop, v, tiles, s0 );
+					SPICE_HIP( hipExtLaunchKernel( fn, dim3( unsigned( v.ntiles ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s, start, stop, 0 ) );
 				else
-					SPICE_LAUNCH( ( k_step_fused<Model, F, BS><<<unsigned( tiles ), BS, 0, _s>>>( v, tiles, s0 ) ) );
-			};
-			int const bs = _lc.recv_block;
-			bs == 256 ? go( std::integral_constant<int, 256>{} ) : bs == 512 ? go( std::integral_constant<int, 512>{} ) : go( std::integral_constant<int, 1024>{} );
+					SPICE_HIP( hipLaunchKernel( fn, dim3( unsigned( v.ntiles ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s ) );
+			} );
 		}
 	}
 
-	// run_profiled for fused steps: every step's kernel -> kernel_ms[2]
-	template <bool F>
-	void run_profiled_fused( std::int64_t n, double * kernel_ms )
+	// f(window kernel, its LDS bytes for w steps, workgroup size) of the launch shape
+	template <typename F>
+	void with_window_kernel( F && f )
+	{
+		auto go = [&]( auto fx, auto b ) {
+			constexpr bool FX = decltype( fx )::value;
+			constexpr int BS = decltype( b )::value;
+			f( &k_window<Model, FX, BS>, [&]( int w ) { return window_lds<Model, FX>::bytes( BS, _lc.tile_w, w ); }, BS );
+		};
+		auto by_block = [&]( auto fx ) {
+			int const bs = _lc.recv_block;
+			bs == 256 ? go( fx, std::integral_constant<int, 256>{} ) : bs == 512 ? go( fx, std::integral_constant<int, 512>{} ) : go( fx, std::integral_constant<int, 1024>{} );
+		};
+		fixed() ? by_block( std::true_type{} ) : by_block( std::false_type{} );
+	}
+
+	// run_profiled for windows: every kernel -> kernel_ms[2]
+	void run_profiled_windows( std::int64_t n, double * kernel_ms )
 	{
 		constexpr int batch = 128;
 		synchronize(); // profiled steps run serially on the main stream
@@ -1081,13 +1147,15 @@ private:
 		try
 		{
 			for( auto & e : ev ) SPICE_HIP( hipEventCreate( &e ) );
-			for( std::int64_t done = 0; done < n; )
+			while( n > 0 )
 			{
-				int const k = int( std::min<std::int64_t>( batch, n - done ) );
-				for( int i = 0; i < k; i++ )
+				int k = 0;
+				for( ; k < batch && n > 0; k++ )
 				{
-					launch_fused<F>( _vs[_step & ( CLOCK_SLOTS - 1 )], ev[2 * i], ev[2 * i + 1] );
-					tick();
+					int const w = window_steps( std::min<std::int64_t>( n, _window ) );
+					launch_window( _step, w, ev[2 * k], ev[2 * k + 1] );
+					for( int i = 0; i < w; i++ ) tick();
+					n -= w;
 				}
 				SPICE_HIP( hipStreamSynchronize( _s ) );
 				for( int i = 0; i < k; i++ )
@@ -1096,7 +1164,6 @@ private:
 					SPICE_HIP( hipEventElapsedTime( &ms, ev[2 * i], ev[2 * i + 1] ) );
 					kernel_ms[2] += ms;
 				}
-				done += k;
 			}
 		}
 		catch( ... )

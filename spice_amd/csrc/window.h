@@ -1,0 +1,357 @@
+#pragma once
+// The window kernel: one launch simulates a window of W <= delay steps of a static network.
+//
+// A spike emitted at step T reaches its targets at T + D, so the arrivals of the steps
+// [T0, T0 + W), W <= D, are all known when the window starts, and a workgroup that owns a tile of
+// target neurons needs nothing from the others inside the window: it delivers the arrivals of all
+// W steps to its tile (LDS accumulators per step), then advances its neurons W steps with their
+// state in registers, then appends the tile's spikes of every step to the ring. One launch, one
+// chain of dependent loads (counts, ids, tile offsets, targets) and one read and write of the
+// neuron state per W steps instead of per step, and W times the loads in flight per workgroup.
+// With W = 1 (delay 1, or a receive() that reads its target) the workgroup delivers and then
+// updates one step.
+//
+// What bounds it: the dependent loads of a delivery (with W = 1), the rate of scattered row
+// segments (larger windows). A row's segment inside a tile is walked by a group of 2^lg lanes
+// (lg from the mean segment length), four segments per group in flight: no per-event search, and
+// an entry costs one load and one LDS atomic.
+#include "kernels.h"
+
+#include <algorithm>
+
+namespace spice::hipx
+{
+constexpr int WINDOW_MAX = 15;              // longest window (steps)
+constexpr std::size_t WINDOW_LDS = 64 << 10; // LDS of a window of more than one step: two workgroups per CU
+
+// The longest window of at most n steps: never a multiple of CLOCK_SLOTS, so that the clock a
+// window writes is not the slot its workgroups read.
+inline int window_steps( std::int64_t n )
+{
+	int const w = int( std::min<std::int64_t>( n, WINDOW_MAX ) );
+	return w % CLOCK_SLOTS == 0 ? w - 1 : w;
+}
+
+// One staged row segment of a chunk of spikes.
+struct alignas( 16 ) win_seg
+{
+	std::int64_t off;  // first target id in the row store (0 for an empty segment)
+	std::int32_t src;
+	std::int32_t meta; // length | step of the window << 16
+};
+
+template <typename Model, bool FIXED>
+struct window_lds
+{
+	using N = typename Model::neuron;
+	using word = acc_word<N, FIXED>;
+	static constexpr int nacc = __builtin_popcount( receive_mask_v<N> ) > 0 ? __builtin_popcount( receive_mask_v<N> ) : 1;
+	// byte offsets of the dynamic LDS: staged segments, accumulators [W][nacc][tile_w], spike
+	// masks [W][tile_w / 64], and the masks' exclusive prefix counts
+	HYBRID static std::size_t acc_at( int bs ) { return sizeof( win_seg ) * std::size_t( bs ); }
+	HYBRID static std::size_t mask_at( int bs, int tw, int w ) { return acc_at( bs ) + sizeof( word ) * std::size_t( nacc ) * std::size_t( tw ) * std::size_t( w ); }
+	HYBRID static std::size_t pre_at( int bs, int tw, int w ) { return mask_at( bs, tw, w ) + 8 * std::size_t( tw / 64 ) * std::size_t( w ); }
+	HYBRID static std::size_t bytes( int bs, int tw, int w ) { return pre_at( bs, tw, w ) + 4 * std::size_t( tw / 64 ) * std::size_t( w ); }
+};
+
+// Receive target inside a window: backend.atomic_add goes to the LDS accumulators of the
+// event's step, reads of the target (W = 1 only) to its state.
+template <typename Neuron, bool FIXED>
+struct win_iter
+{
+	dview const * v;
+	std::int32_t j, t0, stride;
+	acc_word<Neuron, FIXED> * acc; // [nacc][stride] of the event's step
+	template <int I>
+	__device__ auto get() const
+	{
+		using T = typename Neuron::template type<I>;
+		constexpr std::uint32_t mask = receive_mask_v<Neuron>;
+		constexpr int a = __builtin_popcount( mask & ( ( 1u << I ) - 1u ) );
+		using A = acc_type<T, FIXED>;
+		return tile_proxy<T, I, A, ( ( mask >> I ) & 1u ) != 0>{ v, j, reinterpret_cast<A *>( acc + a * stride ), t0, 0u };
+	}
+	__device__ uint_ id() const { return uint_( j ); }
+};
+
+__device__ inline std::uint32_t wave_inclusive_scan32( std::uint32_t x )
+{
+	int const l = lane_id();
+#pragma unroll
+	for( int d = 1; d < 64; d <<= 1 )
+	{
+		std::uint32_t const y = shfl_u32( x, l - d );
+		if( l >= d ) x += y;
+	}
+	return x;
+}
+
+// The window [T0, T0 + W) of the tile at place `pos` of v.tile_ids. slot0: the ring entry of T0
+// (-1: from the clock). lg: log2 of the lanes that walk a segment.
+template <typename Model, bool FIXED, int BS>
+__device__ inline void window_tile( dview const & v, std::int32_t pos, int W, std::int32_t slot0, int lg )
+{
+	using N = typename Model::neuron;
+	using L = window_lds<Model, FIXED>;
+	using word = typename L::word;
+	constexpr int nacc = L::nacc;
+	constexpr std::uint32_t rmask = receive_mask_v<N>;
+
+	extern __shared__ __align__( 16 ) unsigned char dyn[];
+	__shared__ std::uint32_t base[WINDOW_MAX + 1];
+	__shared__ std::uint32_t ev_total, spk_total;
+
+	int const tid = threadIdx.x, lane = lane_id();
+	std::int32_t const tws = v.tile_w; // stride of the LDS arrays
+	win_seg * const seg = reinterpret_cast<win_seg *>( dyn );
+	word * const acc = reinterpret_cast<word *>( dyn + L::acc_at( BS ) );
+	std::uint64_t * const masks = reinterpret_cast<std::uint64_t *>( dyn + L::mask_at( BS, tws, W ) );
+	std::uint32_t * const wpre = reinterpret_cast<std::uint32_t *>( dyn + L::pre_at( BS, tws, W ) );
+
+	std::int32_t const R = v.rsize;
+	ctl_t const clk = *v.ctl;
+	std::int64_t const T0 = clk.step;
+	if( slot0 < 0 ) slot0 = clk.rslot;
+	auto entry = [&]( std::int32_t k ) { // ring entry of T0 + k, -D <= k < 2 * WINDOW_MAX
+		std::int32_t const r = slot0 + k;
+		return r < 0 ? r + R : r >= R ? r - R : r;
+	};
+	std::int32_t const tile = v.tile_ids[pos];
+	bool const active = pos < v.nact; // some row has a target in the tile
+	std::int32_t const t0 = tile * tws;
+	std::int32_t const tw = ( v.N - t0 ) < tws ? ( v.N - t0 ) : tws;
+	snn_info const info = info_of( v );
+
+	// arrivals of the window's steps: lane q holds the count of step q, then the inclusive prefix.
+	// Entries of steps before 0 are empty (counts start at zero).
+	std::uint32_t incl = 0;
+	std::int32_t spec = 0; // W = 1: this thread's id, read beside the count it is checked against
+	if( active )
+	{
+		if( W == 1 ) spec = v.ring[std::int64_t( entry( -v.D ) ) * v.N + ( tid < v.N ? tid : 0 )];
+		if( lane < W ) incl = v.counts[entry( lane - v.D )];
+	}
+	for( int x = tid; x < int( sizeof( word ) * nacc * std::size_t( tws ) * std::size_t( W ) / 16 ); x += BS )
+		reinterpret_cast<uint4 *>( acc )[x] = uint4{ 0, 0, 0, 0 };
+	if( tid == 0 ) ev_total = spk_total = 0;
+	if( W > 1 )
+	{
+#pragma unroll
+		for( int d = 1; d < 16; d <<= 1 )
+		{
+			std::uint32_t const y = shfl_u32( incl, lane - d );
+			if( lane >= d ) incl += y;
+		}
+	}
+	std::int32_t const total = __builtin_amdgcn_readlane( std::int32_t( incl ), W - 1 );
+
+	// arrival k of the window: its source and step
+	auto fetch_id = [&]( std::int32_t k, std::int32_t & q ) {
+		std::int32_t const kk = k < total ? k : total - 1;
+		q = 0;
+		for( int m = 0; m < W - 1; m++ ) q += kk >= __builtin_amdgcn_readlane( std::int32_t( incl ), m ) ? 1 : 0;
+		std::int32_t const below = std::int32_t( shfl_u32( incl, q - 1 ) ); // (every lane takes part)
+		return v.ring[std::int64_t( entry( q - v.D ) ) * v.N + ( kk - ( q > 0 ? below : 0 ) )];
+	};
+
+	std::uint32_t ev = 0;
+	if( total > 0 )
+	{
+		std::int32_t src, q, a, b, src_n = 0, q_n = 0;
+		std::int64_t rp;
+		auto fetch_seg = [&]() {
+			std::int32_t const * pv = v.pivots + std::int64_t( src ) * ( v.ntiles + 1 ) + tile;
+			a = pv[0];
+			b = pv[1];
+			rp = v.row_ptr[src];
+		};
+		if( W == 1 )
+		{
+			src = tid < total ? spec : 0;
+			q = 0;
+		}
+		else
+			src = fetch_id( tid, q );
+		fetch_seg();
+		if( total > BS ) src_n = fetch_id( BS + tid, q_n );
+
+		int const G = 1 << lg, g = tid >> lg, l = tid & ( G - 1 ), ng = BS >> lg;
+		for( std::int32_t k0 = 0; k0 < total; k0 += BS )
+		{
+			std::int32_t const cnt = ( total - k0 ) < BS ? ( total - k0 ) : BS;
+			if( tid < cnt )
+			{
+				std::int32_t const len = b - a;
+				seg[tid] = win_seg{ len > 0 ? rp + a : 0, src, len | ( q << 16 ) };
+				ev += std::uint32_t( len );
+			}
+			__syncthreads(); // (and the accumulators are clear)
+			if( k0 + BS < total )
+			{
+				// the next chunk's tile offsets, and the ids of the one after it, beside the walk
+				src = src_n;
+				q = q_n;
+				fetch_seg();
+				if( k0 + 2 * BS < total ) src_n = fetch_id( k0 + 2 * BS + tid, q_n );
+			}
+			constexpr int U = 4; // segments per group in flight
+			for( std::int32_t c = 0; c < cnt; c += U * ng )
+			{
+				win_seg r[U];
+				std::int32_t len[U], most = 0;
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					std::int32_t const k = c + u * ng + g;
+					r[u] = seg[k < cnt ? k : 0];
+					len[u] = k < cnt ? ( r[u].meta & 0xffff ) : 0;
+					most = len[u] > most ? len[u] : most;
+				}
+				for( std::int32_t e = l;; e += G )
+				{
+					// (past a segment's end its first entry is read, a valid address, and ignored)
+					std::int32_t j[U];
+#pragma unroll
+					for( int u = 0; u < U; u++ ) j[u] = v.col[r[u].off + ( e < len[u] ? e : 0 )];
+#pragma unroll
+					for( int u = 0; u < U; u++ )
+					{
+						if( e >= len[u] ) continue;
+						int const s = r[u].meta >> 16;
+						tile_backend<FIXED> bak{ make_backend<FIXED>( v, std::uint32_t( r[u].src ), std::uint32_t( j[u] ), std::uint32_t( T0 + s ), util::TAG_RECEIVE ) };
+						deliver_event<N>( r[u].src, win_iter<N, FIXED>{ &v, j[u], t0, tws, acc + s * ( nacc * tws ) }, no_syn_iter{}, info, bak );
+					}
+					if( e - l + G >= most ) break;
+				}
+			}
+			__syncthreads(); // the next chunk overwrites the segments; the update reads the sums
+		}
+	}
+	else
+		__syncthreads(); // the accumulators are clear
+
+	// the tile's neurons, W steps each
+	int const nw = tws >> 6;
+	for( int x = tid; x < tws; x += BS )
+	{
+		std::uint32_t spikes = 0; // bit q: spiked at T0 + q
+		if( x < tw )
+		{
+			std::int64_t const i = t0 + x;
+			typename N::tuple_t s;
+			load_tuple<N>( s, v.na, i );
+			float sum = clk.sum, c = clk.c;
+			for( int q = 0; q < W; q++ )
+			{
+				// the step's compensated dt, then the next step's clock: exactly kahan_sum::add
+				float const dt = v.DT - c;
+				float const t = sum + dt;
+				c = ( t - sum ) - dt;
+				sum = t;
+				std::int64_t const T = T0 + q;
+				// the step's inputs; a split receive()'s gate is tested on the state that the
+				// delivery's receive() would have read
+				bool open = true;
+				if constexpr( gated_receive_v<N> ) open = N::accepts( reg_iter<typename N::tuple_t>{ s, std::uint32_t( i ) } );
+				util::for_n<N::size>( [&]( auto I ) {
+					if constexpr( ( ( rmask >> I ) & 1u ) != 0 )
+					{
+						using A = typename N::template type<I>;
+						using AC = acc_type<A, FIXED>;
+						constexpr int a = __builtin_popcount( rmask & ( ( 1u << I ) - 1u ) );
+						AC const in = reinterpret_cast<AC const *>( acc + ( q * nacc + a ) * tws )[x];
+						if constexpr( std::is_floating_point_v<A> && FIXED )
+						{
+							if( open ) std::get<I>( s ) = std::get<I>( s ) + float( in ) * __builtin_ldexpf( 1.0f, -v.shift );
+						}
+						else
+						{
+							if( open ) std::get<I>( s ) = A( std::get<I>( s ) + in );
+						}
+					}
+				} );
+				auto bak = make_backend<FIXED>(
+				    v, std::uint32_t( i ), std::uint32_t( T ), std::uint32_t( std::uint64_t( T ) >> 32 ), util::TAG_NEURON_UPDATE );
+				if( N::update( reg_iter<typename N::tuple_t>{ s, std::uint32_t( i ) }, dt, info, bak ) ) spikes |= 1u << q;
+			}
+			store_tuple<N>( s, v.na, i );
+		}
+		for( int q = 0; q < W; q++ )
+		{
+			std::uint64_t const m = ballot( ( spikes >> q ) & 1u );
+			if( lane == 0 ) masks[q * nw + ( x >> 6 )] = m;
+		}
+	}
+	{
+		std::uint32_t const t = wave_inclusive_scan32( ev );
+		if( lane == 63 && t ) atomicAdd( &ev_total, t );
+	}
+	__syncthreads();
+
+	// a wave per step: the masks' prefix counts, and one atomic reserves the tile's ring places
+	for( int q = tid >> 6; q < W; q += BS / 64 )
+	{
+		std::uint32_t const n = lane < nw ? std::uint32_t( __popcll( masks[q * nw + lane] ) ) : 0u;
+		std::uint32_t const in = wave_inclusive_scan32( n );
+		if( lane < nw ) wpre[q * nw + lane] = in - n;
+		if( lane == 63 && in )
+		{
+			base[q] = atomicAdd( &v.counts[entry( q )], in );
+			atomicAdd( &spk_total, in );
+		}
+	}
+	if( tile == 0 )
+	{
+		// the counters of the steps after the window (no window before them reads those entries),
+		// and the clock of the step after it
+		if( tid < v.wcap ) v.counts[entry( W + tid )] = 0;
+		if( tid == 0 )
+		{
+			float sum = clk.sum, c = clk.c;
+			for( int q = 0; q < W; q++ )
+			{
+				float const y = v.DT - c;
+				float const t = sum + y;
+				c = ( t - sum ) - y;
+				sum = t;
+			}
+			v.ctl_next->c = c;
+			v.ctl_next->sum = sum;
+			v.ctl_next->step = T0 + W;
+			v.ctl_next->rslot = entry( W );
+		}
+	}
+	__syncthreads();
+	for( int x = tid; x < tws; x += BS )
+		for( int q = 0; q < W; q++ )
+		{
+			std::uint64_t const m = masks[q * nw + ( x >> 6 )];
+			if( ( m >> lane ) & 1ull )
+				v.ring[std::int64_t( entry( q ) ) * v.N + base[q] + wpre[q * nw + ( x >> 6 )] + std::uint32_t( lanes_below( m ) )] = t0 + x;
+		}
+	if( tid == 0 )
+	{
+		// this tile's statistics slot, no result awaited
+		if( ev_total ) atomicAdd( &v.bstats[std::int64_t( pos ) * NSTAT + ST_EVENTS], static_cast<unsigned long long>( ev_total ) );
+		if( spk_total ) atomicAdd( &v.bstats[std::int64_t( pos ) * NSTAT + ST_SPIKES], static_cast<unsigned long long>( spk_total ) );
+	}
+}
+
+// Workgroups go to the XCDs round robin, each with an L2 of its own: workgroup b of n takes the
+// place that gives each XCD one contiguous range of tiles, so a spike's tile offsets and the
+// memory lines shared by neighbouring segments of its row are fetched into one L2.
+constexpr int XCDS = 8;
+__device__ inline std::int32_t xcd_place( std::int32_t b, std::int32_t n )
+{
+	std::int32_t const x = b % XCDS, per = n / XCDS, more = n % XCDS;
+	return x * per + ( x < more ? x : more ) + b / XCDS;
+}
+
+// One workgroup per tile: those with incoming synapses first.
+template <typename Model, bool FIXED, int BS>
+__global__ __launch_bounds__( BS ) void k_window( dview v, std::int32_t W, std::int32_t slot0, std::int32_t lg )
+{
+	std::int32_t const b = blockIdx.x;
+	window_tile<Model, FIXED, BS>( v, b < v.nact ? xcd_place( b, v.nact ) : b, W, slot0, lg );
+}
+} // namespace spice::hipx
