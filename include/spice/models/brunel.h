@@ -66,13 +66,26 @@ struct brunel : model
 			return util::get<Twait>( n ) <= 0;
 		}
 
+		// excitatory and inhibitory sources: two fixed weights
+		static constexpr int input_classes = 2;
+		static constexpr int input_attr[input_classes] = { V, V };
+
+		HYBRID static int_ input_class( int_ src, snn_info info )
+		{
+			int_ const nexc = static_cast<int_>( 0.9f * info.num_neurons );
+			return src < nexc ? 0 : 1;
+		}
+		HYBRID static float input_value( int c, snn_info info )
+		{
+			float const Wex = 0.0001f * 20'000 / info.num_neurons;  // V
+			float const Win = -0.0005f * 20'000 / info.num_neurons; // V
+			return c == 0 ? Wex : Win;
+		}
+
 		template <typename Iter, typename SynIter, typename Backend>
 		HYBRID static void deliver( int_ src, Iter dst, SynIter &&, snn_info info, Backend & bak )
 		{
-			int_ const nexc = static_cast<int_>( 0.9f * info.num_neurons );
-			float const Wex = 0.0001f * 20'000 / info.num_neurons;  // V
-			float const Win = -0.0005f * 20'000 / info.num_neurons; // V
-			bak.atomic_add( util::get<V>( dst ), src < nexc ? Wex : Win );
+			bak.atomic_add( util::get<V>( dst ), input_value( input_class( src, info ), info ) );
 		}
 
 		template <typename Iter, typename SynIter, typename Backend>

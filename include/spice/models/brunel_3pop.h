@@ -80,12 +80,25 @@ struct brunel_3pop : model
 			return util::get<Twait>( n ) <= 0;
 		}
 
-		template <typename Iter, typename SynIter, typename Backend>
-		HYBRID static void deliver( int_ src, Iter dst, SynIter &&, snn_info info, Backend & bak )
+		// excitatory and inhibitory sources: two fixed weights
+		static constexpr int input_classes = 2;
+		static constexpr int input_attr[input_classes] = { V, V };
+
+		HYBRID static int_ input_class( int_ src, snn_info info )
+		{
+			return src < num_exc_end( info ) ? 0 : 1;
+		}
+		HYBRID static float input_value( int c, snn_info info )
 		{
 			float const Wex = 0.0001f * 50'000 / info.num_neurons;  // V
 			float const Win = -0.0005f * 50'000 / info.num_neurons; // V
-			bak.atomic_add( util::get<V>( dst ), src < num_exc_end( info ) ? Wex : Win );
+			return c == 0 ? Wex : Win;
+		}
+
+		template <typename Iter, typename SynIter, typename Backend>
+		HYBRID static void deliver( int_ src, Iter dst, SynIter &&, snn_info info, Backend & bak )
+		{
+			bak.atomic_add( util::get<V>( dst ), input_value( input_class( src, info ), info ) );
 		}
 
 		template <typename Iter, typename SynIter, typename Backend>

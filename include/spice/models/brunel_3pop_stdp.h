@@ -21,7 +21,10 @@ struct brunel_3pop_stdp : model
 
 	struct neuron : brunel_3pop::neuron
 	{
-		// both halves of the split receive() are redefined (the base's deliver() has fixed weights)
+		// both halves of the split receive() are redefined (the base's deliver() has fixed weights,
+		// and thus input classes)
+		static constexpr int input_classes = 0;
+
 		template <typename Iter, typename SynIter, typename Backend>
 		HYBRID static void deliver( int_, Iter dst, SynIter && syn, snn_info info, Backend & bak )
 		{

@@ -44,6 +44,17 @@
 //     static constexpr std::uint32_t receive_reads = 0;
 // (receive() reads nothing of its target) allows the same without a gate.
 //
+// Optional input classes, for models without per-synapse state: a neuron type whose inputs take
+// one of a few values, chosen by the source, may declare
+//     static constexpr int input_classes = K;
+//     static constexpr int input_attr[K] = { ... };      the attribute class c's inputs add to
+//     static int_ input_class( int_ src, snn_info );     the class of a source's inputs, 0 .. K - 1
+//     static T input_value( int c, snn_info );           what each input of class c adds
+// with receive() (or deliver()) == atomic_add( get<input_attr[c]>( dst ), input_value( c ) ) for
+// c = input_class( src ), and a T that is the attribute's type. The GPU may then count a step's
+// inputs of each class and form their sum from the counts (in fp32: the same additions, class by
+// class).
+//
 // Optional trait of a neuron-trace synapse (trace_synapse below):
 //     static constexpr int refractory_steps = R;
 // promises that a neuron that is an endpoint of a plastic synapse and spikes at step t neither
@@ -203,6 +214,16 @@ template <typename N>
 struct gated_receive_of<N, std::void_t<decltype( N::gated_receive )>> : std::bool_constant<N::gated_receive>
 {
 };
+template <typename N, typename = void>
+struct input_classes_of
+{
+	static constexpr int value = 0;
+};
+template <typename N>
+struct input_classes_of<N, std::void_t<decltype( N::input_classes )>>
+{
+	static constexpr int value = N::input_classes;
+};
 template <typename S, typename = void>
 struct refractory_steps_of
 {
@@ -231,4 +252,8 @@ inline constexpr int refractory_steps_v = detail::refractory_steps_of<Synapse>::
 
 template <typename Model>
 inline constexpr bool is_plastic_v = Model::synapse::size > 0;
+
+// Input classes of a model without per-synapse state (0: none declared).
+template <typename Model>
+inline constexpr int input_classes_v = is_plastic_v<Model> ? 0 : detail::input_classes_of<typename Model::neuron>::value;
 } // namespace spice

@@ -16,6 +16,11 @@ struct synth : model
 		};
 
 		static constexpr std::uint32_t receive_reads = 0; // receive() reads nothing of its target
+		static constexpr int input_classes = 1;
+		static constexpr int input_attr[input_classes] = { N };
+
+		HYBRID static int_ input_class( int_, snn_info ) { return 0; }
+		HYBRID static int input_value( int, snn_info ) { return 1; }
 
 		template <typename Iter, typename Backend>
 		HYBRID static void init( Iter n, snn_info, Backend & )
@@ -30,9 +35,9 @@ struct synth : model
 		}
 
 		template <typename Iter, typename SynIter, typename Backend>
-		HYBRID static void receive( int_, Iter dst, SynIter &&, snn_info, Backend & bak )
+		HYBRID static void receive( int_, Iter dst, SynIter &&, snn_info info, Backend & bak )
 		{
-			bak.atomic_add( util::get<N>( dst ), 1 );
+			bak.atomic_add( util::get<N>( dst ), input_value( 0, info ) );
 		}
 	};
 };

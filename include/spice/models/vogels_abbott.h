@@ -70,17 +70,31 @@ struct vogels_abbott : model
 			return spiked;
 		}
 
+		// excitatory and inhibitory sources: a fixed weight each, to a conductance each
+		static constexpr int input_classes = 2;
+		static constexpr int input_attr[input_classes] = { Gex, Gin };
+
+		HYBRID static int_ input_class( int_ src, snn_info info )
+		{
+			int_ const nexc = static_cast<int_>( 0.8f * info.num_neurons );
+			return src < nexc ? 0 : 1;
+		}
+		HYBRID static float input_value( int c, snn_info info )
+		{
+			float const Wex = 0.4f * 16'000'000 / ( (long_)info.num_neurons * info.num_neurons ); // S
+			float const Win = 5.1f * 16'000'000 / ( (long_)info.num_neurons * info.num_neurons ); // S
+			return c == 0 ? Wex : Win;
+		}
+
 		template <typename Iter, typename SynIter, typename Backend>
 		HYBRID static void receive( int_ src, Iter dst, SynIter &&, snn_info info, Backend & bak )
 		{
 			using util::get;
-			float const Wex = 0.4f * 16'000'000 / ( (long_)info.num_neurons * info.num_neurons ); // S
-			float const Win = 5.1f * 16'000'000 / ( (long_)info.num_neurons * info.num_neurons ); // S
-			int_ const nexc = static_cast<int_>( 0.8f * info.num_neurons );
-			if( src < nexc )
-				bak.atomic_add( get<Gex>( dst ), Wex );
+			int_ const c = input_class( src, info );
+			if( c == 0 )
+				bak.atomic_add( get<Gex>( dst ), input_value( c, info ) );
 			else
-				bak.atomic_add( get<Gin>( dst ), Win );
+				bak.atomic_add( get<Gin>( dst ), input_value( c, info ) );
 		}
 	};
 };

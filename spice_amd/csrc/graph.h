@@ -9,10 +9,11 @@
 
 namespace spice::hipx
 {
+constexpr std::int64_t COL_PAD = 4;
 struct csr_dev
 {
 	dbuf<std::int64_t> row_ptr; // N + 1
-	dbuf<std::int32_t> col;     // E
+	dbuf<std::int32_t> col;     // E (+ COL_PAD, so that a 16-byte read of the last entries stays inside)
 	std::int64_t n = 0, nnz = 0, width = 0;
 };
 

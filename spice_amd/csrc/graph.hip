@@ -197,7 +197,7 @@ csr_dev generate_csr( std::vector<conn> const & conns, std::int64_t n, std::int6
 		    dconns.data(), int( conns.size() ), n, width, seed, deg.data() ) );
 	exclusive_scan_i32_to_i64( deg.data(), g.row_ptr.data(), n, s );
 	SPICE_HIP( hipMemcpy( &g.nnz, g.row_ptr.data() + n, sizeof( std::int64_t ), hipMemcpyDeviceToHost ) );
-	g.col.resize( g.nnz > 0 ? g.nnz : 1 );
+	g.col.resize( g.nnz + COL_PAD );
 	if( n > 0 && g.nnz > 0 )
 	{
 		std::int64_t const blocks = ( n + 3 ) / 4; // 4 waves (rows) per block
@@ -258,7 +258,7 @@ csr_dev upload_csr( std::int64_t const * row_ptr, std::int32_t const * col, std:
 	g.width = width;
 	g.nnz = row_ptr[n];
 	g.row_ptr.resize( n + 1 );
-	g.col.resize( g.nnz > 0 ? g.nnz : 1 );
+	g.col.resize( g.nnz + COL_PAD );
 	SPICE_HIP( hipMemcpyAsync( g.row_ptr.data(), row_ptr, ( n + 1 ) * sizeof( std::int64_t ), hipMemcpyHostToDevice, s ) );
 	if( g.nnz > 0 )
 		SPICE_HIP( hipMemcpyAsync( g.col.data(), col, g.nnz * sizeof( std::int32_t ), hipMemcpyHostToDevice, s ) );

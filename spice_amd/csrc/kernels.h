@@ -477,8 +477,10 @@ constexpr int TILE_WIDE = 8192;
 // Delivery workgroups have 256 or 1024 threads (a launch shape): they stage that many spikes
 // per pass in LDS.
 
-// Per row r and tile t: offset (within the row) of the first target >= t * tile_w, for
-// t = 0 .. ntiles (the last entry is the row length). One wave per row, binary searches.
+// Per row r and tile t: place in col of the first target >= t * tile_w, for t = 0 .. ntiles (the
+// last entry is the row's end). One wave per row, binary searches. (Places, not offsets in the
+// row: a staged segment then costs one memory request, two neighbouring entries, and none for
+// where its row starts.)
 static inline __global__ __launch_bounds__( 256 ) void k_pivots( dview v )
 {
 	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
@@ -498,7 +500,7 @@ static inline __global__ __launch_bounds__( 256 ) void k_pivots( dview v )
 			else
 				b = m;
 		}
-		v.pivots[r * ( v.ntiles + 1 ) + t] = a;
+		v.pivots[r * ( v.ntiles + 1 ) + t] = lo + a;
 	}
 }
 
@@ -507,7 +509,7 @@ static inline __global__ __launch_bounds__( 256 ) void k_tile_active( dview v, s
 {
 	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
 	if( r >= v.N ) return;
-	std::int32_t const * pv = v.pivots + r * ( v.ntiles + 1 );
+	std::int64_t const * pv = v.pivots + r * ( v.ntiles + 1 );
 	for( int t = lane_id(); t < v.ntiles; t += 64 )
 		if( pv[t + 1] > pv[t] ) flag[t] = 1;
 }
@@ -797,10 +799,9 @@ __device__ inline void receive_tile( dview const & v, std::int32_t work )
 			if( tid < cnt )
 			{
 				src = spk[c0 + tid];
-				std::int32_t const * pv = v.pivots + std::int64_t( src ) * ( v.ntiles + 1 ) + tile;
-				std::int32_t const a = pv[0], b = pv[1];
-				beg = v.row_ptr[src] + a;
-				len = b - a;
+				std::int64_t const * pv = v.pivots + std::int64_t( src ) * ( v.ntiles + 1 ) + tile;
+				beg = pv[0];
+				len = std::int32_t( pv[1] - beg );
 				if constexpr( deferred )
 				{
 					pend = catch_up && ( v.fl8[prev + src] & F8_ARRIVED );

@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <memory>
@@ -115,6 +116,21 @@ template <typename Model>
 int ring_entries( int delay )
 {
 	return std::max( 4, delay + 2 * window_cap<Model>( delay ) );
+}
+
+// Targets per delivery tile of a new network. Static models (window kernels): one tile per CU, as
+// every tile stages all of the window's arrivals and a wider one does it less often (synth 1e9:
+// 29 us per step with 251 tiles of 3,200, 50 with 391 of 2,048), but none wider than its kernel
+// takes; windows of several steps, whose accumulators take LDS per step, two per CU beyond that.
+// Plastic models: about two tiles per CU, of 256 at least.
+template <typename Model>
+int default_tile_w( std::int64_t n, int delay, int cus )
+{
+	auto const per = [&]( std::int64_t tiles ) { return ( ( n + tiles - 1 ) / tiles + 63 ) / 64 * 64; };
+	if( is_plastic_v<Model> ) return int( std::clamp<std::int64_t>( per( 2 * cus ), 256, TILE_MAX ) );
+	bool const ahead = overlap_capable_v<Model> && delay >= 2;
+	std::int64_t const most = ahead ? TILE_MAX : 4 * 1024;
+	return int( std::clamp<std::int64_t>( per( ahead && per( cus ) > most ? 2 * cus : cus ), 64, most ) );
 }
 
 template <typename Model>
@@ -593,7 +609,7 @@ private:
 	int _lanes_log2 = 4;   // window kernels: lanes that walk a row segment
 	launch_queue _queue;
 	launch_cfg _lc{};
-	dbuf<std::int32_t> _pivots;
+	dbuf<std::int64_t> _pivots;
 	dbuf<std::int32_t> _tile_ids;
 	std::int64_t _step = 0;
 	util::kahan_sum<float> _clock;
@@ -801,7 +817,7 @@ private:
 	}
 
 	// Launch shapes (zero fields: the defaults). tile_w: targets per delivery tile (the
-	// receive workgroup's LDS accumulators; ~2 tiles per CU by default); flush_slots: target
+	// receive workgroup's LDS accumulators; see default_tile_w); flush_slots: target
 	// slots per flush work item (one wave), so a flushed row of length L is split into about
 	// L / flush_slots items; flush_grid: persistent flush workgroups (8 per CU by default).
 	launch_cfg default_launch() const
@@ -809,14 +825,20 @@ private:
 		int const cus = device_cu_count();
 		std::int64_t const n = _g.n;
 		launch_cfg c;
-		c.tile_w = int( std::min<std::int64_t>( TILE_MAX, std::max<std::int64_t>( 256, ( ( n + 2 * cus - 1 ) / ( 2 * cus ) + 63 ) / 64 * 64 ) ) );
+		c.tile_w = default_tile_w<Model>( n, _p.delay, cus );
 		c.flush_slots = 256;
 		double const mean_row = n > 0 ? double( _g.nnz ) / double( n ) : 0.0;
 		std::int64_t const fparts = std::max( 1, int( mean_row / c.flush_slots + 0.5 ) );
 		c.flush_grid = int( std::min<std::int64_t>( 8 * cus, std::max<std::int64_t>( 1, ( n * fparts + 3 ) / 4 ) ) );
-		// small nets: few events per tile, so more and smaller delivery workgroups
-		c.recv_block = n <= 65536 ? 256 : 1024;
 		c.recv_parts = 1;
+		if( !plastic )
+			// window kernels: 16 waves where a tile has a CU to itself, 8 where several share one or
+			// the tile is small (Vogels 1e9, delay 8: 7.6 us per step with 250 tiles of 896 and 16
+			// waves, 8.9 with 8; Brunel 1e10, 495 tiles of 640: 19.4 with 16, 17.3 with 8)
+			c.recv_block = c.tile_w > 2048 || ( c.tile_w >= 512 && ( n + c.tile_w - 1 ) / c.tile_w <= cus ) ? 1024 : 512;
+		else
+			// small nets: few events per tile, so more and smaller delivery workgroups
+			c.recv_block = n <= 65536 ? 256 : 1024;
 		return c;
 	}
 
@@ -933,16 +955,21 @@ private:
 			if( !_overlap && ( _lc.recv_parts != 1 || _lc.tile_w > 4 * _lc.recv_block ) ) return;
 			_window = 1;
 			with_window_kernel( [&]( auto kernel, auto bytes, int ) {
+				// the LDS of a CU, shared by the workgroups that a CU gets
+				std::size_t const per_cu = std::size_t( std::clamp( ( _v.ntiles + device_cu_count() - 1 ) / device_cu_count(), 1, 3 ) );
+				std::size_t const room = ( LDS_PER_CU - 4096 ) / per_cu;
 				int w = _v.wcap;
-				while( w > 1 && bytes( w ) > WINDOW_LDS ) w = window_steps( w - 1 );
+				while( w > 1 && bytes( w ) > room ) w = window_steps( w - 1 );
 				_window = w;
 				if( bytes( w ) > ( 64 << 10 ) )
 					SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( w ) ) ) );
 			} );
-			// lanes per segment: the power of two that holds the mean row segment of a tile
+			// lanes per segment: the power of two whose reads hold a segment two standard deviations
+			// longer than the mean, so that few take a second round (Vogels 1e9, delay 8, 17.9
+			// targets per segment: 8.9 us per step with 4 lanes, 7.5 with 8, 8.3 with 16)
 			double const mean = _g.n > 0 ? double( _g.nnz ) / double( _g.n ) / _v.nact : 0.0;
-			_lanes_log2 = 2;
-			while( _lanes_log2 < 6 && double( 1 << _lanes_log2 ) < mean ) _lanes_log2++;
+			_lanes_log2 = 0;
+			while( _lanes_log2 < 5 && double( WIN_VEC << _lanes_log2 ) < mean + 2.0 * std::sqrt( mean ) ) _lanes_log2++;
 		}
 	}
 

@@ -54,14 +54,14 @@ inline std::uint64_t estimate_job_bytes( int model, std::int64_t n, std::int64_t
 		using M = decltype( m );
 		using Nn = typename M::neuron;
 		using Ss = typename M::synapse;
-		std::uint64_t const N = std::uint64_t( n ), E = N * std::uint64_t( width );
+		std::uint64_t const N = std::uint64_t( n ), E = N * std::uint64_t( width ) + COL_PAD;
 		std::uint64_t const cus = 256;
-		std::uint64_t const tile_w = std::min<std::uint64_t>( TILE_MAX, std::max<std::uint64_t>( 256, ( ( N + 2 * cus - 1 ) / ( 2 * cus ) + 63 ) / 64 * 64 ) );
+		std::uint64_t const tile_w = std::uint64_t( default_tile_w<M>( n, delay, int( cus ) ) );
 		std::uint64_t const ntiles = ( N + tile_w - 1 ) / tile_w;
 		std::uint64_t b = 8 * ( N + 1 ) + 4 * E + 4 * N;                 // CSR (+ generator degrees)
 		b += N * Nn::size_in_bytes + N * Nn::size * ( fixed ? 8 : 4 );    // neurons + accumulators
 		b += E * Ss::size_in_bytes;                                        // synapses
-		b += 4 * N * std::uint64_t( ring_entries<M>( delay ) ) + 4 * N * ( ntiles + 1 ); // ring, pivots
+		b += 4 * N * std::uint64_t( ring_entries<M>( delay ) ) + 8 * N * ( ntiles + 1 ); // ring, pivots
 		if constexpr( is_plastic_v<M> )
 		{
 			b += 8 * HWORDS * N + 36 * N;

@@ -12,9 +12,14 @@
 // updates one step.
 //
 // What bounds it: the dependent loads of a delivery (with W = 1), the rate of scattered row
-// segments (larger windows). A row's segment inside a tile is walked by a group of 2^lg lanes
-// (lg from the mean segment length), four segments per group in flight: no per-event search, and
-// an entry costs one load and one LDS atomic.
+// segments (larger windows). A row's segment inside a tile is walked by a group of 2^lg lanes of
+// WIN_VEC entries each (lg from the mean segment length), several segments per group in flight: no
+// per-event search, and an entry costs a quarter of a load and one LDS atomic.
+//
+// Accumulators: models with input classes (model.h) count the inputs of each class, others add
+// the inputs up, in 64 bits (doubles, or fixed point). No 32-bit float atomics: ds_add_f32 takes
+// 193 cycles per wave instruction on gfx950 (three per lane, whatever the addresses), ds_add_f64
+// 21 and ds_add_u32 7 at random addresses, and was what a Vogels-Abbott delivery waited for.
 #include "kernels.h"
 
 #include <algorithm>
@@ -22,7 +27,7 @@
 namespace spice::hipx
 {
 constexpr int WINDOW_MAX = 15;              // longest window (steps)
-constexpr std::size_t WINDOW_LDS = 64 << 10; // LDS of a window of more than one step: two workgroups per CU
+constexpr std::size_t LDS_PER_CU = 160 << 10;
 
 // The longest window of at most n steps: never a multiple of CLOCK_SLOTS, so that the clock a
 // window writes is not the slot its workgroups read.
@@ -40,12 +45,21 @@ struct alignas( 16 ) win_seg
 	std::int32_t meta; // length | step of the window << 16
 };
 
+constexpr int WIN_VEC = 4;   // consecutive targets a lane reads at once (the row store is padded by as many)
+constexpr int WIN_TABLE = 64; // partial sums kept per input class
+
+// What an input of attribute type T is accumulated in.
+template <typename T, bool FIXED>
+using win_acc = std::conditional_t<std::is_floating_point_v<T>, std::conditional_t<FIXED, long long, double>, T>;
+
 template <typename Model, bool FIXED>
 struct window_lds
 {
 	using N = typename Model::neuron;
-	using word = acc_word<N, FIXED>;
-	static constexpr int nacc = __builtin_popcount( receive_mask_v<N> ) > 0 ? __builtin_popcount( receive_mask_v<N> ) : 1;
+	static constexpr int classes = input_classes_v<Model>;
+	// accumulators per neuron and step: a count per class, or a sum per received attribute
+	static constexpr int nacc = classes > 0 ? classes : ( __builtin_popcount( receive_mask_v<N> ) > 0 ? __builtin_popcount( receive_mask_v<N> ) : 1 );
+	using word = std::conditional_t<( classes > 0 ), std::uint32_t, unsigned long long>;
 	// byte offsets of the dynamic LDS: staged segments, accumulators [W][nacc][tile_w], spike
 	// masks [W][tile_w / 64], and the masks' exclusive prefix counts
 	HYBRID static std::size_t acc_at( int bs ) { return sizeof( win_seg ) * std::size_t( bs ); }
@@ -54,25 +68,62 @@ struct window_lds
 	HYBRID static std::size_t bytes( int bs, int tw, int w ) { return pre_at( bs, tw, w ) + 4 * std::size_t( tw / 64 ) * std::size_t( w ); }
 };
 
-// Receive target inside a window: backend.atomic_add goes to the LDS accumulators of the
-// event's step, reads of the target (W = 1 only) to its state.
+// Receive target inside a window (models without input classes): backend.atomic_add goes to the
+// LDS accumulators of the event's step, reads of the target (W = 1 only) to its state.
 template <typename Neuron, bool FIXED>
 struct win_iter
 {
 	dview const * v;
 	std::int32_t j, t0, stride;
-	acc_word<Neuron, FIXED> * acc; // [nacc][stride] of the event's step
+	unsigned long long * acc; // [nacc][stride] of the event's step
 	template <int I>
 	__device__ auto get() const
 	{
 		using T = typename Neuron::template type<I>;
 		constexpr std::uint32_t mask = receive_mask_v<Neuron>;
 		constexpr int a = __builtin_popcount( mask & ( ( 1u << I ) - 1u ) );
-		using A = acc_type<T, FIXED>;
+		using A = win_acc<T, FIXED>;
 		return tile_proxy<T, I, A, ( ( mask >> I ) & 1u ) != 0>{ v, j, reinterpret_cast<A *>( acc + a * stride ), t0, 0u };
 	}
 	__device__ uint_ id() const { return uint_( j ); }
 };
+
+// The sum of n inputs of class c, as adding them one after the other to zero gives it: for fp32
+// from a table of the first sums.
+template <typename Model, bool FIXED, typename T>
+__device__ inline auto class_sum( std::uint32_t n, T value, float const * table, int shift )
+{
+	if constexpr( !std::is_floating_point_v<T> )
+		return T( T( n ) * value );
+	else if constexpr( FIXED )
+		return (long long)( (unsigned long long)( n ) * (unsigned long long)( (long long)__builtin_rint( double( value ) * double( 1ull << shift ) ) ) );
+	else
+	{
+		T x = table[n < WIN_TABLE ? n : WIN_TABLE - 1];
+		for( std::uint32_t k = WIN_TABLE - 1; k < n; k++ ) x += value;
+		return x;
+	}
+}
+
+// WIN_VEC consecutive target ids, from any entry of the row store.
+struct targets
+{
+	std::int32_t id[WIN_VEC];
+};
+__device__ inline targets load_targets( std::int32_t const * p )
+{
+	targets t;
+	__builtin_memcpy( &t, p, sizeof( t ) ); // one 16-byte load (4-byte alignment suffices)
+	return t;
+}
+
+// Orders a wave's LDS writes before its own later LDS reads (and reads before writes): the LDS
+// serves a wave's instructions in order, so only the compiler has to keep them.
+__device__ inline void wave_lds_fence()
+{
+	__builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
+	__builtin_amdgcn_wave_barrier();
+}
 
 __device__ inline std::uint32_t wave_inclusive_scan32( std::uint32_t x )
 {
@@ -100,6 +151,9 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W, st
 	extern __shared__ __align__( 16 ) unsigned char dyn[];
 	__shared__ std::uint32_t base[WINDOW_MAX + 1];
 	__shared__ std::uint32_t ev_total, spk_total;
+	// fp32 input classes: the sum of the first k inputs of class c
+	constexpr bool tables = L::classes > 0 && !FIXED;
+	__shared__ float table[tables ? L::classes * WIN_TABLE : 1];
 
 	int const tid = threadIdx.x, lane = lane_id();
 	std::int32_t const tws = v.tile_w; // stride of the LDS arrays
@@ -125,15 +179,23 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W, st
 	// arrivals of the window's steps: lane q holds the count of step q, then the inclusive prefix.
 	// Entries of steps before 0 are empty (counts start at zero).
 	std::uint32_t incl = 0;
-	std::int32_t spec = 0; // W = 1: this thread's id, read beside the count it is checked against
-	if( active )
-	{
-		if( W == 1 ) spec = v.ring[std::int64_t( entry( -v.D ) ) * v.N + ( tid < v.N ? tid : 0 )];
-		if( lane < W ) incl = v.counts[entry( lane - v.D )];
-	}
+	if( active && lane < W ) incl = v.counts[entry( lane - v.D )];
 	for( int x = tid; x < int( sizeof( word ) * nacc * std::size_t( tws ) * std::size_t( W ) / 16 ); x += BS )
 		reinterpret_cast<uint4 *>( acc )[x] = uint4{ 0, 0, 0, 0 };
 	if( tid == 0 ) ev_total = spk_total = 0;
+	if constexpr( tables )
+	{
+		if( tid < L::classes )
+		{
+			float const x = float( N::input_value( tid, info ) );
+			float t = 0.0f;
+			for( int k = 0; k < WIN_TABLE; k++ )
+			{
+				table[tid * WIN_TABLE + k] = t;
+				t += x;
+			}
+		}
+	}
 	if( W > 1 )
 	{
 #pragma unroll
@@ -154,45 +216,49 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W, st
 		return v.ring[std::int64_t( entry( q - v.D ) ) * v.N + ( kk - ( q > 0 ? below : 0 ) )];
 	};
 
+	// Delivery, wave by wave: a wave stages up to 64 of the window's arrivals at a time (one segment
+	// each) in its own part of the LDS and walks them; the next ones' ids and segment bounds are
+	// read beside the walk. No wave waits for another before the update.
 	std::uint32_t ev = 0;
-	if( total > 0 )
+	__syncthreads(); // the accumulators are clear
+	constexpr int NW = BS / 64;
+	int const wave = tid >> 6;
+	// arrivals per wave and round: few ones are spread over all waves
+	std::int32_t const per = total >= 64 * NW ? 64 : ( total + NW - 1 ) / NW;
+	std::int32_t k0 = wave * per;
+	std::int32_t const mylane = lane < per ? lane : per - 1; // (the lanes past a round's arrivals repeat its last)
+	if( k0 < total )
 	{
-		std::int32_t src, q, a, b, src_n = 0, q_n = 0;
-		std::int64_t rp;
+		win_seg * const mine = seg + wave * 64;
+		std::int32_t src, q = 0, src_n = 0, q_n = 0;
+		std::int64_t a, b;
 		auto fetch_seg = [&]() {
-			std::int32_t const * pv = v.pivots + std::int64_t( src ) * ( v.ntiles + 1 ) + tile;
+			std::int64_t const * pv = v.pivots + std::int64_t( src ) * ( v.ntiles + 1 ) + tile;
 			a = pv[0];
 			b = pv[1];
-			rp = v.row_ptr[src];
 		};
-		if( W == 1 )
-		{
-			src = tid < total ? spec : 0;
-			q = 0;
-		}
-		else
-			src = fetch_id( tid, q );
+		src = fetch_id( k0 + mylane, q );
 		fetch_seg();
-		if( total > BS ) src_n = fetch_id( BS + tid, q_n );
+		if( k0 + NW * per < total ) src_n = fetch_id( k0 + NW * per + mylane, q_n );
 
-		int const G = 1 << lg, g = tid >> lg, l = tid & ( G - 1 ), ng = BS >> lg;
-		for( std::int32_t k0 = 0; k0 < total; k0 += BS )
+		int const G = 1 << lg, g = lane >> lg, l = lane & ( G - 1 ), ng = 64 >> lg;
+		for( ; k0 < total; k0 += NW * per )
 		{
-			std::int32_t const cnt = ( total - k0 ) < BS ? ( total - k0 ) : BS;
-			if( tid < cnt )
+			std::int32_t const cnt = ( total - k0 ) < per ? ( total - k0 ) : per;
+			std::int32_t const len = lane < cnt ? std::int32_t( b - a ) : 0;
+			if constexpr( L::classes > 0 )
+				// in the place of the source: where the class's counters of the step start (for target 0)
+				mine[lane] = win_seg{ len > 0 ? a : 0, ( q * nacc + N::input_class( src, info ) ) * tws - t0, len };
+			else
+				mine[lane] = win_seg{ len > 0 ? a : 0, src, len | ( q << 16 ) };
+			ev += std::uint32_t( len );
+			wave_lds_fence();
+			if( k0 + NW * per < total )
 			{
-				std::int32_t const len = b - a;
-				seg[tid] = win_seg{ len > 0 ? rp + a : 0, src, len | ( q << 16 ) };
-				ev += std::uint32_t( len );
-			}
-			__syncthreads(); // (and the accumulators are clear)
-			if( k0 + BS < total )
-			{
-				// the next chunk's tile offsets, and the ids of the one after it, beside the walk
 				src = src_n;
 				q = q_n;
 				fetch_seg();
-				if( k0 + 2 * BS < total ) src_n = fetch_id( k0 + 2 * BS + tid, q_n );
+				if( k0 + 2 * NW * per < total ) src_n = fetch_id( k0 + 2 * NW * per + mylane, q_n );
 			}
 			constexpr int U = 4; // segments per group in flight
 			for( std::int32_t c = 0; c < cnt; c += U * ng )
@@ -203,32 +269,38 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W, st
 				for( int u = 0; u < U; u++ )
 				{
 					std::int32_t const k = c + u * ng + g;
-					r[u] = seg[k < cnt ? k : 0];
-					len[u] = k < cnt ? ( r[u].meta & 0xffff ) : 0;
+					r[u] = mine[k & 63]; // (records from cnt on are empty)
+					len[u] = k < 64 ? ( r[u].meta & 0xffff ) : 0;
 					most = len[u] > most ? len[u] : most;
 				}
-				for( std::int32_t e = l;; e += G )
+				for( std::int32_t e = l * WIN_VEC;; e += G * WIN_VEC )
 				{
-					// (past a segment's end its first entry is read, a valid address, and ignored)
-					std::int32_t j[U];
+					// (past a segment's end its first entries are read, at valid addresses, and ignored)
+					targets j[U];
 #pragma unroll
-					for( int u = 0; u < U; u++ ) j[u] = v.col[r[u].off + ( e < len[u] ? e : 0 )];
+					for( int u = 0; u < U; u++ ) j[u] = load_targets( v.col + r[u].off + ( e < len[u] ? e : 0 ) );
 #pragma unroll
 					for( int u = 0; u < U; u++ )
-					{
-						if( e >= len[u] ) continue;
-						int const s = r[u].meta >> 16;
-						tile_backend<FIXED> bak{ make_backend<FIXED>( v, std::uint32_t( r[u].src ), std::uint32_t( j[u] ), std::uint32_t( T0 + s ), util::TAG_RECEIVE ) };
-						deliver_event<N>( r[u].src, win_iter<N, FIXED>{ &v, j[u], t0, tws, acc + s * ( nacc * tws ) }, no_syn_iter{}, info, bak );
-					}
-					if( e - l + G >= most ) break;
+#pragma unroll
+						for( int x = 0; x < WIN_VEC; x++ )
+						{
+							if( e + x >= len[u] ) continue;
+							if constexpr( L::classes > 0 )
+								atomicAdd( acc + ( r[u].src + j[u].id[x] ), 1u );
+							else
+							{
+								int const s = r[u].meta >> 16;
+								tile_backend<FIXED> bak{ make_backend<FIXED>( v, std::uint32_t( r[u].src ), std::uint32_t( j[u].id[x] ), std::uint32_t( T0 + s ), util::TAG_RECEIVE ) };
+								deliver_event<N>( r[u].src, win_iter<N, FIXED>{ &v, j[u].id[x], t0, tws, acc + s * ( nacc * tws ) }, no_syn_iter{}, info, bak );
+							}
+						}
+					if( e - l * WIN_VEC + G * WIN_VEC >= most ) break;
 				}
 			}
-			__syncthreads(); // the next chunk overwrites the segments; the update reads the sums
+			wave_lds_fence(); // the next round overwrites the records
 		}
 	}
-	else
-		__syncthreads(); // the accumulators are clear
+	__syncthreads(); // the sums are complete
 
 	// the tile's neurons, W steps each
 	int const nw = tws >> 6;
@@ -257,9 +329,19 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W, st
 					if constexpr( ( ( rmask >> I ) & 1u ) != 0 )
 					{
 						using A = typename N::template type<I>;
-						using AC = acc_type<A, FIXED>;
-						constexpr int a = __builtin_popcount( rmask & ( ( 1u << I ) - 1u ) );
-						AC const in = reinterpret_cast<AC const *>( acc + ( q * nacc + a ) * tws )[x];
+						using AC = std::conditional_t<std::is_floating_point_v<A>, std::conditional_t<FIXED, long long, A>, A>;
+						AC in = AC( 0 );
+						if constexpr( L::classes > 0 )
+							util::for_n<L::classes>( [&]( auto C ) {
+								if constexpr( N::input_attr[C] == int( I ) )
+									in = AC( in + class_sum<Model, FIXED>( acc[( q * nacc + C ) * tws + x], A( N::input_value( C, info ) ),
+									                                       table + ( tables ? C * WIN_TABLE : 0 ), v.shift ) );
+							} );
+						else
+						{
+							constexpr int a = __builtin_popcount( rmask & ( ( 1u << I ) - 1u ) );
+							in = AC( reinterpret_cast<win_acc<A, FIXED> const *>( acc + ( q * nacc + a ) * tws )[x] );
+						}
 						if constexpr( std::is_floating_point_v<A> && FIXED )
 						{
 							if( open ) std::get<I>( s ) = std::get<I>( s ) + float( in ) * __builtin_ldexpf( 1.0f, -v.shift );

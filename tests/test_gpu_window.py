@@ -1,0 +1,68 @@
+"""Window kernels (static networks: up to `delay` steps per launch, each tile delivered and
+updated by one workgroup) against the CPU checker, fixed point and so bit for bit: delays below,
+at and above the longest window and at multiples of the clock's slots, tiles of one wave, ragged
+last tiles, tiles without inputs, wide tiles, rows with many and with no targets in a tile; runs
+that end inside a window; and fp32 inputs past the tabulated sums."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from spice_amd import Layout, Snn
+from tests.helpers import assert_state_equal, brunel_ref_layout, three_pop_layout
+
+pytestmark = pytest.mark.gpu
+
+DT = 1e-4
+RUNS = (1, 2, 3, 4, 5, 7, 8, 15, 16, 29, 30, 31, 60, 1, 89)  # 301 steps
+
+
+@pytest.mark.parametrize("model,layout,delay,launch", [
+    ("brunel_3pop", three_pop_layout(1500), 2, (0, 0)),
+    ("brunel_3pop", three_pop_layout(1500), 3, (64, 256)),
+    ("brunel_3pop", three_pop_layout(1111), 4, (128, 1024)),
+    ("brunel_3pop", three_pop_layout(2000), 15, (1024, 256)),
+    ("brunel_3pop", three_pop_layout(1500), 16, (192, 512)),
+    ("brunel_3pop", three_pop_layout(777), 40, (0, 0)),
+    ("brunel", brunel_ref_layout(1500), 15, (64, 512)),  # half of the tiles receive nothing
+    ("vogels_abbott", ([1300], [(0, 0, 0.3)]), 8, (256, 512)),
+    ("vogels_abbott", ([2500], [(0, 0, 0.02)]), 5, (64, 256)),
+    ("vogels_abbott", ([4200], [(0, 0, 0.02)]), 1, (4096, 1024)),
+    ("synth", ([3000], [(0, 0, 0.001)]), 7, (64, 1024)),  # most segments empty
+    ("synth", ([500], [(0, 0, 1.0)]), 12, (512, 256)),  # every row in full
+    ("synth", ([65], [(0, 0, 0.5)]), 1, (0, 0)),
+    ("synth", ([40], [(0, 0, 0.0)]), 3, (0, 0)),  # no synapse at all
+])
+def test_windows_bit_exact(gpu, model, layout, delay, launch):
+    h = O.CpuSnn(model, layout, DT, delay, seed=81, fixed_point=True)
+    d = Snn(model, Layout(*layout), DT, delay, seed=81, fixed_point=True)
+    d.set_launch(tile_w=launch[0], recv_block=launch[1])
+    done = 0
+    for n in RUNS:
+        d.run(n)
+        h.run(n)
+        done += n
+        assert d.clock() == h.clock()
+        assert_state_equal(d.neurons(), h.neurons(), f"{model} after {done} steps")
+    for i in range(3):
+        np.testing.assert_array_equal(np.sort(d.step(True)), np.sort(h.step(True)), err_msg=f"step {done + i}")
+    ms = d.run_profiled(20)
+    h.run(20)
+    assert ms["receive"] == 0 and ms["update"] == 0 and ms["step"] > 0
+    assert_state_equal(d.neurons(), h.neurons(), "after profiled steps")
+    d.close(), h.close()
+
+
+@pytest.mark.parametrize("delay", [1, 6])
+def test_fp32_inputs_past_the_tabulated_sums(gpu, delay):
+    """Vogels-Abbott in fp32: the whole population's first spike gives every neuron hundreds of
+    inputs of one value in one step, whose fp32 sum is the same in any order of adding them."""
+    lay = ([900], [(0, 0, 0.4)])
+    h = O.CpuSnn("vogels_abbott", lay, DT, delay, seed=5)
+    d = Snn("vogels_abbott", Layout(*lay), DT, delay, seed=5)
+    for n in (130, 5, 5, 5, 40):
+        d.run(n)
+        h.run(n)
+        assert_state_equal(d.neurons(), h.neurons(), f"after {d.clock()[0]} steps")
+    st = d.stats()
+    assert st["spikes"] >= 900 and st["events"] > 64 * 900
+    d.close(), h.close()
