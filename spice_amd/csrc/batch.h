@@ -46,20 +46,13 @@ public:
 		_fixed = _nets[0]->fixed();
 		for( auto * n : _nets )
 			if( n->fixed() != _fixed ) throw std::invalid_argument( "all nets of a batch use the same accumulation mode" );
-		// Many nets already fill the GPU, so then a batched net does not need many small
-		// delivery tiles: each net gets about max(64, 64 x CUs / nets) tiles (fewer workgroups,
-		// each with a fixed staging cost). On a sweep of two 256-net batches 64 tiles per net
-		// beat 16, 32, 128 and 256; a batch of a few nets keeps its nets' own tiles. Fixed-point
-		// results do not depend on the tile width (fp32 sums are reordered, as by any launch
-		// shape); a net keeps wider tiles it already has, and keeps the new width afterwards.
-		std::int64_t const tiles_per_net = std::max<std::int64_t>( 64, std::int64_t( SPICE_BATCH_ITEMS_PER_CU ) * device_cu_count() / std::int64_t( _nets.size() ) );
 		for( auto * n : _nets )
 		{
 			launch_cfg c = n->get_launch();
-			int const tw = int( std::clamp<std::int64_t>( ( n->num_neurons() / tiles_per_net + 63 ) / 64 * 64, 64, TILE_MAX ) );
-			if( tw > c.tile_w || c.tile_w > TILE_MAX ) // (the batched kernels hold tiles of up to TILE_MAX)
+			int const tw = batch_tile_w( n->num_neurons(), c.tile_w, std::int64_t( _nets.size() ) );
+			if( tw != c.tile_w )
 			{
-				c.tile_w = c.tile_w > TILE_MAX ? TILE_MAX : tw;
+				c.tile_w = tw;
 				n->set_launch( c );
 			}
 		}
@@ -68,18 +61,20 @@ public:
 		for( std::size_t k = 0; k < _nets.size(); k++ )
 		{
 			hip_net<Model> & n = *_nets[k];
-			for( int t = 0; t < n.num_tiles() * n.num_receive_parts(); t++ ) // (tile, part) work items
+			// static models: windows, one workgroup per tile; plastic ones: (tile, part) work items of
+			// the tiles with incoming synapses
+			for( int t = 0; t < ( plastic ? n.num_tiles() * n.num_receive_parts() : n.num_all_tiles() ); t++ )
 			{
 				tn.push_back( std::int32_t( k ) );
 				tl.push_back( t );
 			}
-			for( int b = 0; b < n.num_update_blocks(); b++ )
-			{
-				bn.push_back( std::int32_t( k ) );
-				bl.push_back( b );
-			}
 			if constexpr( plastic )
 			{
+				for( int b = 0; b < n.num_update_blocks(); b++ )
+				{
+					bn.push_back( std::int32_t( k ) );
+					bl.push_back( b );
+				}
 				int const nf = n.num_batch_flush_blocks();
 				for( int b = 0; b < nf; b++ )
 				{
@@ -98,6 +93,26 @@ public:
 		// batched update blocks' size)
 		_overlap = recv_block == 256;
 		for( auto * n : _nets ) _overlap = _overlap && n->overlapped();
+		if constexpr( !plastic )
+		{
+			// the longest window that suits every net and whose LDS leaves room for four workgroups
+			// on a CU
+			_window = WINDOW_MAX;
+			int widest = 64;
+			for( auto * n : _nets )
+			{
+				_window = std::min( _window, n->longest_window() );
+				widest = std::max( widest, int( n->get_launch().tile_w ) );
+				_logged = _logged || n->logged();
+			}
+			auto bytes = [&]( int w ) { return _fixed ? window_lds<Model, true>::bytes( window_block, widest, w ) : window_lds<Model, false>::bytes( window_block, widest, w ); };
+			while( _window > 1 && bytes( _window ) > LDS_PER_CU / 4 ) _window = window_steps( _window - 1 );
+			_lds = bytes( _window );
+			if( _lds > ( 64 << 10 ) )
+				SPICE_HIP( hipFuncSetAttribute( _fixed ? reinterpret_cast<void const *>( &k_batch_window<Model, true, window_block> )
+				                                       : reinterpret_cast<void const *>( &k_batch_window<Model, false, window_block> ),
+				                                hipFuncAttributeMaxDynamicSharedMemorySize, int( _lds ) ) );
+		}
 		upload( _tile_net, tn );
 		upload( _tile_local, tl );
 		upload( _block_net, bn );
@@ -111,10 +126,27 @@ public:
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 	}
 
+	// Delivery tile width of a net of n neurons (at `tile_w` now) in a batch of nnets. Many nets
+	// already fill the GPU, so then a batched net does not need many small delivery tiles: fewer
+	// workgroups, each with a fixed staging cost (every tile stages all of a window's arrivals). A
+	// batch of a few nets keeps its nets' own tiles. Fixed-point results do not depend on the tile
+	// width (fp32 sums are reordered, as by any launch shape); a net keeps wider tiles it already
+	// has (of up to TILE_MAX, what the batched kernels hold), and keeps the new width afterwards.
+	// Plastic models: about max(64, 64 x CUs / nets) tiles per net (on a sweep of two 256-net
+	// batches 64 tiles per net beat 16, 32, 128 and 256).
+	static int batch_tile_w( std::int64_t n, int tile_w, std::int64_t nnets )
+	{
+		std::int64_t const tiles = plastic ? std::max<std::int64_t>( 64, std::int64_t( SPICE_BATCH_ITEMS_PER_CU ) * device_cu_count() / nnets )
+		                                   : std::max<std::int64_t>( 1, window_tiles_per_cu * device_cu_count() / nnets );
+		int const tw = int( std::clamp<std::int64_t>( ( n / tiles + 63 ) / 64 * 64, 64, TILE_MAX ) );
+		return std::min( std::max( tw, tile_w ), TILE_MAX );
+	}
+
 	~hip_batch() override
 	{
 		if( _s ) (void)hipStreamSynchronize( _s );
 		_graphs.clear();
+		_queue.clear();
 		if( _s && _own_stream ) (void)hipStreamDestroy( _s );
 	}
 
@@ -122,6 +154,13 @@ public:
 	{
 		if( n < 0 ) throw std::invalid_argument( "negative step count" );
 		if( n == 0 ) return;
+		if( _window > 1 )
+		{
+			launch_windows( _step, n );
+			_step += n;
+			for( auto * net : _nets ) net->advance_host( n );
+			return;
+		}
 		if( _graphs.empty() ) _graphs.capture( _s, [&]( int t, int len ) { launch_steps( t, len ); } );
 		_graphs.run( _s, _step, n, [&] { _step++; } );
 		for( auto * net : _nets ) net->advance_host( n );
@@ -153,6 +192,16 @@ private:
 	step_graphs _graphs;
 	bool _fixed = false;
 	bool _overlap = false; // every net runs overlapped steps: so does the batch
+	// static models: windows of up to _window steps
+	static constexpr int window_block = 256;
+	// tiles of all nets, per CU: 48 nets of 1e4 to 1e7 synapses take, at 4 / 8 / 16 / 64, 2.6 / 1.8 /
+	// 1.8 / 1.9 us per step in windows of 15 steps and 11.0 / 10.6 / 14.5 / 18.3 step by step (10.3
+	// and 14.7 with a delivery and an update kernel, or an overlapped one, per step)
+	static constexpr std::int64_t window_tiles_per_cu = 8;
+	int _window = 0;
+	bool _logged = false; // some net has a spike log
+	std::size_t _lds = 0;
+	launch_queue _queue;
 	std::int64_t _step = 0;
 	std::int32_t _ntiles = 0, _nblocks = 0, _nflush = 0;
 	int _grid_tiles = 0;
@@ -167,10 +216,47 @@ private:
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 	}
 
-	// Same schedules as hip_net::launch_steps: two kernels per step (delivery with step t - 1's
-	// plasticity, update), or the overlapped sequence (delivery of step t, one overlapped
-	// kernel per step boundary, the last update).
+	// n steps from batch step t in windows; each appends its predecessor's spikes to the nets'
+	// logs, and a last kernel the last one's.
+	void launch_windows( std::int64_t t, std::int64_t n )
+	{
+		int before = 0;
+		while( n > 0 )
+		{
+			int const w = window_steps( std::min<std::int64_t>( n, _window ) );
+			if( _fixed )
+				launch_window_t<true>( t, w, before );
+			else
+				launch_window_t<false>( t, w, before );
+			if( _window > 1 ) _queue.launched( _s );
+			before = w;
+			t += w;
+			n -= w;
+		}
+		if( _logged ) SPICE_LAUNCH( k_batch_log<<<unsigned( _nets.size() ), 256, 0, _s>>>( _views[t & ( CLOCK_SLOTS - 1 )].data(), before ) );
+	}
+
+	template <bool F>
+	void launch_window_t( std::int64_t t, int w, int before )
+	{
+		unsigned const grid = unsigned( _ntiles ) + ( _logged && before ? unsigned( _nets.size() ) : 0u );
+		if constexpr( !plastic )
+			SPICE_LAUNCH( ( k_batch_window<Model, F, window_block><<<grid, window_block, _lds, _s>>>( _views[t & ( CLOCK_SLOTS - 1 )].data(), _tile_net.data(),
+			                                                                                      _tile_local.data(), _ntiles, w, before ) ) );
+	}
+
+	// Same schedules as hip_net::launch_steps: windows of one step, two kernels per step (delivery
+	// with step t - 1's plasticity, update), or the overlapped sequence (delivery of step t, one
+	// overlapped kernel per step boundary, the last update).
 	void launch_steps( std::int64_t t, std::int64_t len )
+	{
+		if constexpr( !plastic )
+			launch_windows( t, len );
+		else
+			launch_plastic_steps( t, len );
+	}
+
+	void launch_plastic_steps( std::int64_t t, std::int64_t len )
 	{
 		for( std::int64_t k = 0; k < len; k++ )
 		{
@@ -234,7 +320,9 @@ batch_iface * make_batch( std::vector<net_params> const & ps, std::vector<csr_de
 		SPICE_HIP( hipStreamCreateWithFlags( &ns, hipStreamNonBlocking ) );
 		try
 		{
-			nets.emplace_back( new hip_net<Model>( ps[k], std::move( gs[k] ), ns ) );
+			launch_cfg first; // at the width that the batch will want
+			first.tile_w = hip_batch<Model>::batch_tile_w( gs[k].n, default_tile_w<Model>( gs[k].n, ps[k].delay, device_cu_count() ), std::int64_t( ps.size() ) );
+			nets.emplace_back( new hip_net<Model>( ps[k], std::move( gs[k] ), ns, first ) );
 		}
 		catch( ... )
 		{

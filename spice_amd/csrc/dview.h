@@ -107,6 +107,7 @@ struct dview
 	std::int32_t upd_slot0; // first statistics slot of the update blocks of an overlapped kernel
 	std::int32_t rsize;     // entries of the spike ring
 	std::int32_t wcap;      // longest window of steps run by one kernel
+	std::int32_t wlanes;    // windows: log2 of the lanes that walk a row segment
 	std::uint32_t flags;
 	std::uint64_t seed;
 	float param[4]; // per-net model parameters (snn_info::param)
@@ -141,6 +142,7 @@ struct dview
 	tp_entry const * tp_ent;
 	std::int64_t * caught;
 
+	ctl_t * ctl0;     // the clock slots
 	ctl_t * ctl;      // this step's clock
 	ctl_t * ctl_next; // the next step's clock (written by k_update)
 	ctl_t * ctl_prev; // the previous step's clock (its dt for the lazy flush of that step)

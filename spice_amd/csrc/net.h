@@ -143,7 +143,8 @@ class hip_net final : public net_iface
 	static constexpr bool nodefer = eager_nodefer_v<Model>; // every eager event applied by the passes
 
 public:
-	hip_net( net_params const & p, csr_dev && g, hipStream_t stream )
+	// first: launch shapes to start with (zero fields: the defaults)
+	hip_net( net_params const & p, csr_dev && g, hipStream_t stream, launch_cfg first = {} )
 	    : _p( p )
 	    , _g( std::move( g ) )
 	    , _s( stream )
@@ -157,7 +158,7 @@ public:
 		static_assert( N::size <= MAXA && S::size <= MAXA, "at most 16 neuron/synapse attributes" );
 		// the update of step T runs beside the delivery of step T + 1 (see k_step_overlap)
 		_overlap = overlap_capable_v<Model> && p.delay >= 2;
-		allocate();
+		allocate( first );
 		initialize();
 	}
 
@@ -553,6 +554,9 @@ public:
 	// ---- used by hip_batch (batched stepping of many nets) ----
 	dview const & view( int slot ) const { return _vs[slot & ( CLOCK_SLOTS - 1 )]; }
 	int num_tiles() const { return _v.nact; } // the delivery's tiles (those with incoming synapses)
+	int num_all_tiles() const { return _v.ntiles; }
+	int longest_window() const { return _v.wcap; }
+	bool logged() const { return _slog_ctl.size() > 0; }
 	int num_receive_parts() const { return _v.rparts; }
 	int num_update_blocks() const { return _grid_update; }
 	// flush workgroups of this net inside a batch: about two per expected work item wave
@@ -606,7 +610,6 @@ private:
 	int _grid_plast = 0; // plasticity workgroups of the delivery kernel
 	bool _overlap = false; // steps run as k_step_overlap kernels
 	int _window = 0;       // longest window of the window kernels that run the steps (0: none)
-	int _lanes_log2 = 4;   // window kernels: lanes that walk a row segment
 	launch_queue _queue;
 	launch_cfg _lc{};
 	dbuf<std::int64_t> _pivots;
@@ -642,7 +645,7 @@ private:
 		if( a < 0 || a >= n ) throw std::invalid_argument( "attribute index out of range" );
 	}
 
-	void allocate()
+	void allocate( launch_cfg const & first )
 	{
 		std::int64_t const n = _g.n;
 		util::for_n<N::size>( [&]( auto I ) {
@@ -741,6 +744,7 @@ private:
 		v.po_count = _po_count.data();
 		v.tp_ptr = _tp_ptr.data();
 		v.caught = _caught.data();
+		v.ctl0 = _ctl.data();
 		v.ctl = _ctl.data();
 		v.ctl_next = _ctl.data() + 1;
 
@@ -748,7 +752,7 @@ private:
 		_grid_update = int( ( n + 255 ) / 256 );
 		_upd_block = n >= UPDATE_LARGE_N ? UPDATE_BLOCK_LARGE : SPICE_UPDATE_BLOCK;
 		_grid_upd = int( ( n + _upd_block - 1 ) / _upd_block );
-		apply_launch( launch_cfg{} );
+		apply_launch( first );
 	}
 
 	// Eager plasticity state at a clock (re)start: zero traces and flags, no pending lists.
@@ -952,6 +956,12 @@ private:
 		_window = 0;
 		if constexpr( !plastic )
 		{
+			// lanes per segment: the power of two whose reads hold a segment two standard deviations
+			// longer than the mean, so that few take a second round (Vogels 1e9, delay 8, 17.9
+			// targets per segment: 8.9 us per step with 4 lanes, 7.5 with 8, 8.3 with 16)
+			double const mean = _g.n > 0 ? double( _g.nnz ) / double( _g.n ) / _v.nact : 0.0;
+			_v.wlanes = 0;
+			while( _v.wlanes < 5 && double( WIN_VEC << _v.wlanes ) < mean + 2.0 * std::sqrt( mean ) ) _v.wlanes++;
 			if( !_overlap && ( _lc.recv_parts != 1 || _lc.tile_w > 4 * _lc.recv_block ) ) return;
 			_window = 1;
 			with_window_kernel( [&]( auto kernel, auto bytes, int ) {
@@ -964,12 +974,6 @@ private:
 				if( bytes( w ) > ( 64 << 10 ) )
 					SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( w ) ) ) );
 			} );
-			// lanes per segment: the power of two whose reads hold a segment two standard deviations
-			// longer than the mean, so that few take a second round (Vogels 1e9, delay 8, 17.9
-			// targets per segment: 8.9 us per step with 4 lanes, 7.5 with 8, 8.3 with 16)
-			double const mean = _g.n > 0 ? double( _g.nnz ) / double( _g.n ) / _v.nact : 0.0;
-			_lanes_log2 = 0;
-			while( _lanes_log2 < 5 && double( WIN_VEC << _lanes_log2 ) < mean + 2.0 * std::sqrt( mean ) ) _lanes_log2++;
 		}
 	}
 
@@ -1133,13 +1137,9 @@ private:
 		{
 			if( _slog_ctl.size() ) throw std::logic_error( "nets with a spike log are stepped by a batch" );
 			dview v = _vs[t & ( CLOCK_SLOTS - 1 )];
-			v.ctl_next = _ctl.data() + ( ( t + w ) & ( CLOCK_SLOTS - 1 ) );
 			with_window_kernel( [&]( auto kernel, auto bytes, int bs ) {
-				// the ring entry of step t: the clock phase if the ring has CLOCK_SLOTS entries (a
-				// captured launch replays at any step of its phase), else known to eager launches only
-				std::int32_t const slot0 = _window > 1 || v.rsize == CLOCK_SLOTS ? std::int32_t( t % v.rsize ) : -1;
-				std::int32_t const W = w, lg = _lanes_log2;
-				void * args[] = { &v, const_cast<std::int32_t *>( &W ), const_cast<std::int32_t *>( &slot0 ), const_cast<std::int32_t *>( &lg ) };
+				std::int32_t W = w;
+				void * args[] = { &v, &W };
 				void const * fn = reinterpret_cast<void const *>( kernel );
 				if( start )
 					SPICE_HIP( hipExtLaunchKernel( fn, dim3( unsigned( v.ntiles ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s, start, stop, 0 ) );

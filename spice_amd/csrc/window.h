@@ -137,10 +137,13 @@ __device__ inline std::uint32_t wave_inclusive_scan32( std::uint32_t x )
 	return x;
 }
 
-// The window [T0, T0 + W) of the tile at place `pos` of v.tile_ids. slot0: the ring entry of T0
-// (-1: from the clock). lg: log2 of the lanes that walk a segment.
+// Ring entry of the view's step. A ring of CLOCK_SLOTS entries (delay 1) has it at the clock's
+// place, known before the clock is read.
+__device__ inline std::int32_t window_entry( dview const & v ) { return v.rsize == CLOCK_SLOTS ? std::int32_t( v.ctl - v.ctl0 ) : v.ctl->rslot; }
+
+// The window [T0, T0 + W) of the tile at place `pos` of v.tile_ids.
 template <typename Model, bool FIXED, int BS>
-__device__ inline void window_tile( dview const & v, std::int32_t pos, int W, std::int32_t slot0, int lg )
+__device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 {
 	using N = typename Model::neuron;
 	using L = window_lds<Model, FIXED>;
@@ -165,7 +168,8 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W, st
 	std::int32_t const R = v.rsize;
 	ctl_t const clk = *v.ctl;
 	std::int64_t const T0 = clk.step;
-	if( slot0 < 0 ) slot0 = clk.rslot;
+	std::int32_t const slot0 = window_entry( v );
+	int const lg = v.wlanes;
 	auto entry = [&]( std::int32_t k ) { // ring entry of T0 + k, -D <= k < 2 * WINDOW_MAX
 		std::int32_t const r = slot0 + k;
 		return r < 0 ? r + R : r >= R ? r - R : r;
@@ -397,10 +401,11 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W, st
 				c = ( t - sum ) - y;
 				sum = t;
 			}
-			v.ctl_next->c = c;
-			v.ctl_next->sum = sum;
-			v.ctl_next->step = T0 + W;
-			v.ctl_next->rslot = entry( W );
+			ctl_t * const next = v.ctl0 + ( ( v.ctl - v.ctl0 + W ) & ( CLOCK_SLOTS - 1 ) );
+			next->c = c;
+			next->sum = sum;
+			next->step = T0 + W;
+			next->rslot = entry( W );
 		}
 	}
 	__syncthreads();
@@ -431,9 +436,47 @@ __device__ inline std::int32_t xcd_place( std::int32_t b, std::int32_t n )
 
 // One workgroup per tile: those with incoming synapses first.
 template <typename Model, bool FIXED, int BS>
-__global__ __launch_bounds__( BS ) void k_window( dview v, std::int32_t W, std::int32_t slot0, std::int32_t lg )
+__global__ __launch_bounds__( BS ) void k_window( dview v, std::int32_t W )
 {
 	std::int32_t const b = blockIdx.x;
-	window_tile<Model, FIXED, BS>( v, b < v.nact ? xcd_place( b, v.nact ) : b, W, slot0, lg );
+	window_tile<Model, FIXED, BS>( v, b < v.nact ? xcd_place( b, v.nact ) : b, W );
 }
+
+// Appends the spikes of the n steps before the view's step to the net's spike log (one workgroup;
+// the counts of a window's steps are final only when its kernel has ended, so the log is written
+// by the next one, or by a kernel of its own after the last).
+__device__ inline void log_steps( dview const & v, int n )
+{
+	if( !v.slog ) return;
+	std::int64_t const k0 = v.ctl->step - n - v.slog->t0; // first of the steps' places in the log's window
+	if( k0 < 0 || k0 + n > v.slog->nsteps ) return;
+	std::int32_t const slot0 = window_entry( v );
+	auto entry = [&]( std::int32_t k ) { return slot0 + k < 0 ? slot0 + k + v.rsize : slot0 + k; };
+	std::uint64_t base = k0 == 0 ? 0ull : v.slog_off[k0 - 1] + v.counts[entry( -n - 1 )];
+	std::uint64_t const cap = v.slog->cap;
+	for( int q = 0; q < n; q++ )
+	{
+		std::uint32_t const cnt = v.counts[entry( q - n )];
+		std::int32_t const * ids = v.ring + std::int64_t( entry( q - n ) ) * v.N;
+		if( threadIdx.x == 0 ) v.slog_off[k0 + q] = base;
+		for( std::uint32_t i = threadIdx.x; i < cnt; i += blockDim.x )
+			if( base + i < cap ) v.slog_ids[base + i] = ids[i];
+		base += cnt;
+	}
+}
+
+// Batched windows: workgroup b < ntiles runs the tile at place tile_pos[b] of net tile_net[b], the
+// rest append net b - ntiles's spikes of the nlog steps before the window to its log.
+template <typename Model, bool FIXED, int BS>
+__global__ __launch_bounds__( BS ) void k_batch_window( dview const * views, std::int32_t const * tile_net, std::int32_t const * tile_pos,
+                                                        std::int32_t ntiles, std::int32_t W, std::int32_t nlog )
+{
+	std::int32_t const b = blockIdx.x;
+	if( b < ntiles )
+		window_tile<Model, FIXED, BS>( views[tile_net[b]], tile_pos[b], W );
+	else
+		log_steps( views[b - ntiles], nlog );
+}
+
+static __global__ __launch_bounds__( 256 ) void k_batch_log( dview const * views, std::int32_t nlog ) { log_steps( views[blockIdx.x], nlog ); }
 } // namespace spice::hipx
