@@ -29,6 +29,7 @@ template <typename Model>
 class hip_batch final : public batch_iface
 {
 	static constexpr bool plastic = is_plastic_v<Model>;
+	static constexpr bool windowed = windowed_v<Model>; // steps run as windows
 	// delivery workgroup size: most tiles of a sweep belong to small nets and carry few events,
 	// so more, smaller workgroups shorten the launch's critical path
 	static constexpr int recv_block = SPICE_BATCH_RECV_BLOCK;
@@ -61,20 +62,21 @@ public:
 		for( std::size_t k = 0; k < _nets.size(); k++ )
 		{
 			hip_net<Model> & n = *_nets[k];
-			// static models: windows, one workgroup per tile; plastic ones: (tile, part) work items of
-			// the tiles with incoming synapses
-			for( int t = 0; t < ( plastic ? n.num_tiles() * n.num_receive_parts() : n.num_all_tiles() ); t++ )
+			// windows: one workgroup per tile; two-kernel steps: (tile, part) work items of the tiles
+			// with incoming synapses
+			for( int t = 0; t < ( windowed ? n.num_all_tiles() : n.num_tiles() * n.num_receive_parts() ); t++ )
 			{
 				tn.push_back( std::int32_t( k ) );
 				tl.push_back( t );
 			}
-			if constexpr( plastic )
-			{
+			if constexpr( !windowed )
 				for( int b = 0; b < n.num_update_blocks(); b++ )
 				{
 					bn.push_back( std::int32_t( k ) );
 					bl.push_back( b );
 				}
+			if constexpr( plastic )
+			{
 				int const nf = n.num_batch_flush_blocks();
 				for( int b = 0; b < nf; b++ )
 				{
@@ -89,19 +91,15 @@ public:
 		_ntiles = std::int32_t( tn.size() );
 		_nblocks = std::int32_t( bn.size() );
 		_nflush = std::int32_t( fn.size() );
-		// (the overlapped kernel's update workgroups have the delivery's size: 256 threads, the
-		// batched update blocks' size)
-		_overlap = recv_block == 256;
-		for( auto * n : _nets ) _overlap = _overlap && n->overlapped();
-		if constexpr( !plastic )
+		if constexpr( windowed )
 		{
 			// the longest window that suits every net and whose LDS leaves room for four workgroups
 			// on a CU
-			_window = WINDOW_MAX;
 			int widest = 64;
+			_window = WINDOW_MAX;
 			for( auto * n : _nets )
 			{
-				_window = std::min( _window, n->longest_window() );
+				_window = std::min( _window, window_cap<Model>( n->params().delay ) );
 				widest = std::max( widest, int( n->get_launch().tile_w ) );
 				_logged = _logged || n->logged();
 			}
@@ -156,7 +154,11 @@ public:
 		if( n == 0 ) return;
 		if( _window > 1 )
 		{
-			launch_windows( _step, n );
+			std::int64_t single = 0; // (state imported into a net may ask for a few steps one by one)
+			for( auto * net : _nets ) single = std::max( single, net->single_steps_left() );
+			single = std::min( single, n );
+			launch_windows( _step, single, 1 );
+			launch_windows( _step + single, n - single, _window );
 			_step += n;
 			for( auto * net : _nets ) net->advance_host( n );
 			return;
@@ -191,8 +193,7 @@ private:
 	bool _own_stream = false;
 	step_graphs _graphs;
 	bool _fixed = false;
-	bool _overlap = false; // every net runs overlapped steps: so does the batch
-	// static models: windows of up to _window steps
+	// windows of up to _window steps (0: two-kernel steps)
 	static constexpr int window_block = 256;
 	// tiles of all nets, per CU: 48 nets of 1e4 to 1e7 synapses take, at 4 / 8 / 16 / 64, 2.6 / 1.8 /
 	// 1.8 / 1.9 us per step in windows of 15 steps and 11.0 / 10.6 / 14.5 / 18.3 step by step (10.3
@@ -216,14 +217,15 @@ private:
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 	}
 
-	// n steps from batch step t in windows; each appends its predecessor's spikes to the nets'
-	// logs, and a last kernel the last one's.
-	void launch_windows( std::int64_t t, std::int64_t n )
+	// n steps from batch step t in windows of up to `most`; each appends its predecessor's spikes
+	// to the nets' logs, and a last kernel the last one's.
+	void launch_windows( std::int64_t t, std::int64_t n, int most )
 	{
+		if( n == 0 ) return;
 		int before = 0;
 		while( n > 0 )
 		{
-			int const w = window_steps( std::min<std::int64_t>( n, _window ) );
+			int const w = window_steps( std::min<std::int64_t>( n, most ) );
 			if( _fixed )
 				launch_window_t<true>( t, w, before );
 			else
@@ -239,60 +241,25 @@ private:
 	template <bool F>
 	void launch_window_t( std::int64_t t, int w, int before )
 	{
-		unsigned const grid = unsigned( _ntiles ) + ( _logged && before ? unsigned( _nets.size() ) : 0u );
-		if constexpr( !plastic )
-			SPICE_LAUNCH( ( k_batch_window<Model, F, window_block><<<grid, window_block, _lds, _s>>>( _views[t & ( CLOCK_SLOTS - 1 )].data(), _tile_net.data(),
-			                                                                                      _tile_local.data(), _ntiles, w, before ) ) );
+		unsigned const grid = unsigned( _ntiles + _nflush ) + ( _logged && before ? unsigned( _nets.size() ) : 0u );
+		if constexpr( windowed )
+			SPICE_LAUNCH( ( k_batch_window<Model, F, window_block><<<grid, window_block, _lds, _s>>>(
+			    _views[t & ( CLOCK_SLOTS - 1 )].data(), _tile_net.data(), _tile_local.data(), _ntiles, w, before, _flush_net.data(),
+			    _flush_local.data(), _flush_count.data(), _nflush ) ) );
 	}
 
-	// Same schedules as hip_net::launch_steps: windows of one step, two kernels per step (delivery
-	// with step t - 1's plasticity, update), or the overlapped sequence (delivery of step t, one
-	// overlapped kernel per step boundary, the last update).
+	// Same schedules as hip_net::launch_steps: windows of one step, or two kernels per step
+	// (delivery with step t - 1's plasticity, update).
 	void launch_steps( std::int64_t t, std::int64_t len )
 	{
-		if constexpr( !plastic )
-			launch_windows( t, len );
+		if constexpr( windowed )
+			launch_windows( t, len, 1 );
 		else
-			launch_plastic_steps( t, len );
-	}
-
-	void launch_plastic_steps( std::int64_t t, std::int64_t len )
-	{
-		for( std::int64_t k = 0; k < len; k++ )
-		{
-			if( _overlap ) break;
-			if( _fixed )
-				launch_step_t<true>( t + k );
-			else
-				launch_step_t<false>( t + k );
-		}
-		if( !_overlap ) return;
-		for( std::int64_t k = 0; k <= len; k++ )
-		{
-			if( _fixed )
-				launch_overlap_t<true>( t, len, k );
-			else
-				launch_overlap_t<false>( t, len, k );
-		}
-	}
-
-	template <bool F>
-	void launch_overlap_t( std::int64_t t, std::int64_t len, std::int64_t k )
-	{
-		if( k == 0 )
-		{
-			// delivery of step t only: step t - 1's plasticity runs beside the first update
-			dview const * v = _views[t & ( CLOCK_SLOTS - 1 )].data();
-			SPICE_LAUNCH( k_batch_receive<Model, F, recv_block><<<unsigned( _grid_tiles ), recv_block, 0, _s>>>(
-			    v, _tile_net.data(), _tile_local.data(), _ntiles, _grid_tiles, _flush_net.data(), _flush_local.data(), _flush_count.data() ) );
-			return;
-		}
-		dview const * v = _views[( t + k - 1 ) & ( CLOCK_SLOTS - 1 )].data(); // updates step t + k - 1
-		std::int32_t const grecv = k < len ? _grid_tiles : 0, nplast = plastic ? _nflush : 0;
-		unsigned const grid = unsigned( grecv + nplast + _nblocks );
-		SPICE_LAUNCH( k_batch_step_overlap<Model, F, recv_block><<<grid, recv_block, 0, _s>>>(
-		    v, _tile_net.data(), _tile_local.data(), _ntiles, grecv, _flush_net.data(), _flush_local.data(), _flush_count.data(), nplast,
-		    _block_net.data(), _block_local.data() ) );
+			for( std::int64_t k = 0; k < len; k++ )
+				if( _fixed )
+					launch_step_t<true>( t + k );
+				else
+					launch_step_t<false>( t + k );
 	}
 
 	template <bool F>

@@ -28,13 +28,20 @@
 //   fl_*     int32[2][N] rows queued at this step (spike arrived, or history window full),
 //                        with their (synced, pend) at that time; lists by step parity,
 //                        counters [4] by step mod 4
-// eager plasticity (neuron-trace synapses), all [2][N] arrays by step parity:
+// eager plasticity (neuron-trace synapses) with deferred events, all [2][N] by step parity:
 //   xtr/ytr  f32[2][N]   neuron-local pre/post traces after step T
 //   fl8      u8[2][N]    bit 0: spiked at T, bit 1: its spike arrives at T, bit 2: at T + 1
-//                        (bit 2 only for models whose deliveries apply deferred events)
-//   fl_id    int32[2][N] rows whose spike arrived at T (and, with deferred events, does not
-//                        arrive at T + 1)
+//   fl_id    int32[2][N] rows whose spike arrived at T and does not arrive at T + 1
 //   po_id    int32[2][N] neurons that spiked at T and have incoming plastic synapses
+// eager plasticity in windows (refractory endpoints), k = the window's number:
+//   xtr/ytr  f32[4][N]   traces before the window's first step, by k mod 4
+//   fl8      u8[2][N]    by k mod 2: 1 + the step of the window at which the neuron's spike
+//                        arrived (0: none)
+//   sp8      u8[2][N]    by k mod 2: 1 + the step of the window at which the neuron spiked
+//   fl_id    int32[2][N] rows whose spike arrived in the window
+//   po_id    int32[2][N] neurons that spiked in the window and have incoming plastic synapses
+//                        (their counters by k mod 4)
+// both:
 //   tp_ptr   int64[N+1], tp_ent {src, offset in src's row}[P]: the P plastic synapses by target
 // both:
 //   caught   int64       step whose plasticity work (and, eager, deferred events of the rows
@@ -59,6 +66,10 @@ struct ctl_t
 	float sum;         // Kahan sum of dt over completed steps
 	float c;           // Kahan compensation
 	std::int32_t rslot; // spike ring entry of this step: step mod rsize
+	// windows of plastic models: this window's number, and of the window before it (the one whose
+	// plasticity passes are due) the steps (0: none) and the clock at its start
+	std::int32_t wseq, wprev;
+	float psum, pc;
 };
 
 // Device counters live in per-block slots: block b of any step kernel adds its block-reduced
@@ -102,9 +113,6 @@ struct dview
 	std::int32_t fparts; // work items per flushed row
 	std::int32_t pparts; // work items per spiking target (eager plasticity)
 	std::int32_t rparts; // delivery workgroups per tile (the step's spike list split between them)
-	std::int32_t overlap; // 1: the update of step T runs beside the delivery of T + 1 (it writes
-	                      // the spike log's step offsets then; otherwise the delivery does)
-	std::int32_t upd_slot0; // first statistics slot of the update blocks of an overlapped kernel
 	std::int32_t rsize;     // entries of the spike ring
 	std::int32_t wcap;      // longest window of steps run by one kernel
 	std::int32_t wlanes;    // windows: log2 of the lanes that walk a row segment
@@ -136,6 +144,7 @@ struct dview
 	float * xtr;
 	float * ytr;
 	std::uint8_t * fl8;
+	std::uint8_t * sp8;
 	std::int32_t * po_id;
 	std::uint32_t * po_count; // [4]
 	std::int64_t const * tp_ptr;

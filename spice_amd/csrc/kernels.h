@@ -1,8 +1,9 @@
 #pragma once
 // Model-templated step kernels for gfx950 (subsystems b, c, d).
 //
-// Per step T (step index read from device memory, see dview.h), two kernels on one stream, or
-// (overlapped steps) one kernel per step boundary that holds the work of both:
+// Static models, and plastic ones with refractory endpoints, run the window kernels of window.h.
+// The others (and launch shapes that split a tile's spikes between workgroups), per step T (step
+// index read from device memory, see dview.h), two kernels on one stream:
 //   k_receive_tiled<M> : delivers the spikes emitted at T - D. One workgroup per (target tile,
 //                  part of the step's spike list): the spikes' row segments inside the tile
 //                  are walked as one flat index space and M::neuron::receive accumulates
@@ -19,11 +20,6 @@
 //                  plasticity work. Block 0 writes step T + 1's clock and empties its counters,
 //                  so the same launches are valid at every step and are captured once into a
 //                  HIP graph.
-//   k_step_overlap<M>: for models whose delivery may run before its targets' update (receive()
-//                  split into a gate the update tests, or reading nothing of the target; for
-//                  plastic models, eager with refractory endpoints) and a delay of at least 2:
-//                  the update of step T, the delivery of step T + 1 and the plasticity passes
-//                  of step T - 1 in one kernel, one kernel per step boundary.
 //
 // Reference counterparts: _process_neurons (spice/cuda/algorithm.cu:181-230),
 // _process_spikes HNDL_SPKS / UPDT_SYNS (algorithm.cu:238-313), _gather (algorithm.cu:340-384),
@@ -278,6 +274,19 @@ __device__ inline bool store_changed( typename Decl::tuple_t const & before, typ
 	return any;
 }
 
+// Whether two synapse states are the same, bit for bit.
+template <typename Decl>
+__device__ inline bool same_bits( typename Decl::tuple_t const & a, typename Decl::tuple_t const & b )
+{
+	bool same = true;
+	util::for_n<Decl::size>( [&]( auto I ) {
+		using T = typename Decl::template type<I>;
+		using B = std::conditional_t<sizeof( T ) == 8, std::uint64_t, std::uint32_t>;
+		same = same && __builtin_bit_cast( B, std::get<I>( a ) ) == __builtin_bit_cast( B, std::get<I>( b ) );
+	} );
+	return same;
+}
+
 // ---- spike history and lazy plasticity --------------------------------------------------
 // Spike history (plastic models): bit (t mod HISTORY) of ring word ((t mod HISTORY) / 64) of
 // neuron j is set iff j spiked at step t, valid for the last HISTORY steps. Lazy plasticity
@@ -375,12 +384,8 @@ __device__ inline void replay(
 // they touch no row that delivery reads, and they read only step T's traces and flags (arrays
 // by step parity), which the update of step T + 1 writes only after that kernel.
 
-//
 // A synapse type promising refractory endpoints (refractory_steps >= 2, see model.h) needs no
-// deferred events: the pre pass of step T takes every row whose spike arrives at T, the post
-// pass every other source, and the delivery only reads weights. A weight it reads may still
-// get an event of step T - 1 or T applied beside it, but only one whose target does not take
-// this delivery's input.
+// deferred events: the passes apply every event, and the delivery only reads weights (window.h).
 
 // flag bits of fl8
 constexpr std::uint8_t F8_SPIKED = 1, F8_ARRIVED = 2, F8_ARRIVES_NEXT = 4;
@@ -390,8 +395,8 @@ template <typename Model>
 inline constexpr bool eager_nodefer_v =
     is_plastic_v<Model> && has_neuron_traces_v<typename Model::synapse> && refractory_steps_v<typename Model::synapse> >= 2;
 
-// The update of step T may run beside the delivery of step T + 1 (given a delay of at least 2
-// steps): delivery reads nothing that the update writes -- no target state (receive() split
+// The delivery of a step may run before the update of the steps before it (given a delay of at
+// least 2 steps): it reads nothing that those updates write -- no target state (receive() split
 // into a gate the update tests, or declared to read nothing) and, for plastic models, no weight
 // whose pending events matter.
 template <typename Model>
@@ -694,9 +699,8 @@ __device__ inline void deliver_event( A &&... a )
 // entry's segment found from a bitmap of segment starts, or for very large chunks by binary
 // search). receive() accumulates into
 // LDS with LDS atomics; at the end the tile's sums go to the global accumulators with plain
-// stores: one workgroup owns each tile, so no global atomics are needed. AHEAD: the kernel's
-// clock is step T - 1's (the overlapped step kernel delivers the next step beside the update).
-template <typename Model, bool FIXED, int BS, bool AHEAD = false, int TM = TILE_MAX>
+// stores: one workgroup owns each tile, so no global atomics are needed.
+template <typename Model, bool FIXED, int BS, int TM = TILE_MAX>
 __device__ inline void receive_tile( dview const & v, std::int32_t work )
 {
 	// work item = (active tile, part): the tile's spike list is split into v.rparts parts,
@@ -734,10 +738,11 @@ __device__ inline void receive_tile( dview const & v, std::int32_t work )
 	__shared__ std::uint64_t seg_total;
 	constexpr bool eager = plastic && has_neuron_traces_v<S>;
 	constexpr bool lazy = plastic && !eager;
-	constexpr bool deferred = eager && !eager_nodefer_v<Model>; // delivery applies step T - 1's events
+	constexpr bool deferred = eager; // delivery applies step T - 1's events
 	// record and target id of each entry loaded without branches (entries past the chunk's end
 	// read its last entry and are ignored)
-	constexpr bool flat = !plastic || ( eager && !deferred );
+	constexpr bool flat = !plastic;
+	static_assert( !eager_nodefer_v<Model>, "models whose passes apply every event run windows" );
 	__shared__ std::int32_t seg_synced[lazy ? BS : 1];
 	__shared__ std::int32_t seg_pend[lazy || deferred ? BS : 1]; // deferred: the row's spike also arrived at T - 1
 	__shared__ float seg_xf[deferred ? BS : 1];                  // deferred: the row's pre trace after T - 1
@@ -745,17 +750,17 @@ __device__ inline void receive_tile( dview const & v, std::int32_t work )
 	__shared__ float tile_y[deferred ? TM : 1];            // deferred: the tile's post traces after T - 1
 	__shared__ std::uint64_t wsum[BS / 64];
 
-	std::int64_t const T = v.ctl->step + ( AHEAD ? 1 : 0 );
-	int const slot = ring_at( v, ( AHEAD ? 1 : 0 ) - v.D ); // ring entry of step T - D
+	std::int64_t const T = v.ctl->step;
+	int const slot = ring_at( v, -v.D ); // ring entry of step T - D
 	std::int32_t const nall = T < v.D ? 0 : std::int32_t( v.counts[slot] );
 	std::int32_t const s_beg = std::int32_t( std::int64_t( nall ) * part / v.rparts );
 	std::int32_t const nspk = std::int32_t( std::int64_t( nall ) * ( part + 1 ) / v.rparts ) - s_beg;
-	if( !v.overlap && v.slog && work == 0 && threadIdx.x == 0 )
+	if( v.slog && work == 0 && threadIdx.x == 0 )
 	{
 		// spike log: step T's ids start where step T-1's (final by now) end
 		std::int64_t const k = T - v.slog->t0;
 		if( k >= 0 && k < v.slog->nsteps )
-			v.slog_off[k] = k == 0 ? 0ull : v.slog_off[k - 1] + v.counts[ring_at( v, ( AHEAD ? 1 : 0 ) - 1 )];
+			v.slog_off[k] = k == 0 ? 0ull : v.slog_off[k - 1] + v.counts[ring_at( v, -1 )];
 	}
 	std::int32_t const * spk = v.ring + std::int64_t( slot ) * v.N + s_beg;
 	float const dt = step_dt( v );
@@ -946,24 +951,6 @@ __device__ inline void receive_tile( dview const & v, std::int32_t work )
 						deliver_event<N>( s, dst, itr, info, bak );
 					}
 				}
-				else if constexpr( eager )
-				{
-					// neuron-trace synapses without deferred events: the synapse state of all U
-					// entries (valid addresses, see above), then delivery
-					typename S::tuple_t sy[U];
-#pragma unroll
-					for( int u = 0; u < U; u++ ) load_tuple<S, ( SPICE_NT & 4 ) != 0>( sy[u], v.sa, e[u] );
-#pragma unroll
-					for( int u = 0; u < U; u++ )
-					{
-						if( !ok[u] ) continue;
-						std::int32_t const s = sv[u];
-						tile_backend<FIXED> bak{ make_backend<FIXED>( v, std::uint32_t( s ), std::uint32_t( j[u] ), std::uint32_t( T ), util::TAG_RECEIVE ) };
-						tile_iter<N, FIXED, TM> dst{ &v, j[u], t0, acc, stage };
-						reg_iter<typename S::tuple_t> itr{ sy[u], std::uint32_t( e[u] ) };
-						deliver_event<N>( s, dst, itr, info, bak );
-					}
-				}
 				else if constexpr( !plastic )
 				{
 					// the staged attribute values of all U targets first (one LDS round), then
@@ -1082,38 +1069,10 @@ __global__ __launch_bounds__( BS ) void k_receive_tiled( dview v, std::int32_t g
 	if( std::int32_t( blockIdx.x ) < grecv )
 	{
 		std::int32_t const nwork = v.nact * v.rparts;
-		for( std::int32_t w = blockIdx.x; w < nwork; w += grecv ) receive_tile<Model, FIXED, BS, false, TM>( v, w );
+		for( std::int32_t w = blockIdx.x; w < nwork; w += grecv ) receive_tile<Model, FIXED, BS, TM>( v, w );
 	}
 	else if constexpr( is_plastic_v<Model> )
 		plasticity_prev_block<Model, FIXED>( v, blockIdx.x - grecv, gridDim.x - grecv );
-}
-
-template <typename Model, bool FIXED>
-__device__ inline void update_block( dview const & v, std::int64_t blk, std::int64_t slot );
-
-// The overlapped step (overlap_capable_v models, delay >= 2), clock of step T: workgroups
-// [0, nrecv) deliver step T + 1, [nrecv, nrecv + nplast) run step T - 1's plasticity passes,
-// the rest update the neurons of step T (blockDim.x neurons each; statistics slots from
-// upd_slot0). None reads what another writes: the accumulators, plasticity lists, traces and
-// flags are kept by step parity, the delivery reads ring entries of earlier steps and no target
-// state (the update tests receive()'s gate), and the passes touch only weights whose targets
-// do not take that delivery's input. With nrecv = 0 the kernel ends a run of overlapped steps
-// (the last update, beside the passes of the step before it).
-template <typename Model, bool FIXED, int BS>
-__global__ __launch_bounds__( BS ) void k_step_overlap( dview v, std::int32_t nrecv, std::int32_t nplast, std::int32_t upd_slot0 )
-{
-	std::int32_t const b = blockIdx.x;
-	if( b < nrecv )
-	{
-		std::int32_t const nwork = v.nact * v.rparts;
-		for( std::int32_t w = b; w < nwork; w += nrecv ) receive_tile<Model, FIXED, BS, true>( v, w );
-	}
-	else if( b < nrecv + nplast )
-	{
-		if constexpr( is_plastic_v<Model> ) plasticity_prev_block<Model, FIXED>( v, b - nrecv, nplast );
-	}
-	else
-		update_block<Model, FIXED>( v, b - nrecv - nplast, upd_slot0 + ( b - nrecv - nplast ) );
 }
 
 // Batched delivery: global work item gt belongs to net tile_net[gt] (local work item
@@ -1136,37 +1095,6 @@ __global__ __launch_bounds__( BS ) void k_batch_receive( dview const * views, st
 		plasticity_prev_block<Model, FIXED>( views[block_net[b]], block_local[b], block_count[b] );
 	}
 }
-
-// Batched overlapped step (every net of the batch overlapped): k_step_overlap over the nets'
-// tables -- workgroups [0, grecv) deliver each net's next step (work items round robin),
-// [grecv, grecv + nplast) run plasticity block flush_local[b] of the flush_count[b] blocks of
-// net flush_net[b], the rest update neuron block upd_local[u] of net upd_net[u] (256 neurons).
-// grecv = 0: the last update of a run, beside the passes of the step before it.
-template <typename Model, bool FIXED, int BS>
-__global__ __launch_bounds__( BS ) void k_batch_step_overlap( dview const * views, std::int32_t const * tile_net, std::int32_t const * tile_local,
-                                                              std::int32_t ntiles, std::int32_t grecv, std::int32_t const * flush_net,
-                                                              std::int32_t const * flush_local, std::int32_t const * flush_count, std::int32_t nplast,
-                                                              std::int32_t const * upd_net, std::int32_t const * upd_local )
-{
-	std::int32_t const b = blockIdx.x;
-	if( b < grecv )
-	{
-		for( std::int32_t gt = b; gt < ntiles; gt += grecv ) receive_tile<Model, FIXED, BS, true>( views[tile_net[gt]], tile_local[gt] );
-	}
-	else if( b < grecv + nplast )
-	{
-		if constexpr( is_plastic_v<Model> )
-			plasticity_prev_block<Model, FIXED>( views[flush_net[b - grecv]], flush_local[b - grecv], flush_count[b - grecv] );
-	}
-	else
-	{
-		std::int32_t const u = b - grecv - nplast;
-		dview const & v = views[upd_net[u]];
-		update_block<Model, FIXED>( v, upd_local[u], v.upd_slot0 + upd_local[u] );
-	}
-}
-
-
 
 // Neuron update of neurons [first, first + min(count, blockDim.x)) (blockDim.x <= 1024) at step
 // T; statistics go to slot `slot`. The range that starts at neuron 0 also clears the next
@@ -1219,7 +1147,7 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 		if constexpr( plastic )
 		{
 			if( T >= v.D ) h_arr = v.hring[( ( ( T - v.D ) & ( HISTORY - 1 ) ) >> 6 ) * N64 + i];
-			if( !eager_nodefer_v<Model> && T + 1 >= v.D && v.D != 1 ) h_next = v.hring[( ( ( T + 1 - v.D ) & ( HISTORY - 1 ) ) >> 6 ) * N64 + i];
+			if( T + 1 >= v.D && v.D != 1 ) h_next = v.hring[( ( ( T + 1 - v.D ) & ( HISTORY - 1 ) ) >> 6 ) * N64 + i];
 			h_now = v.hring[hcur];
 			has_plastic = v.hasp[i];
 			if constexpr( eager )
@@ -1269,9 +1197,9 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 		{
 			// this neuron's spike of step T - D reaches its synapses now
 			bool const arrived = T >= v.D && ( ( h_arr >> ( ( T - v.D ) & 63 ) ) & 1ull );
-			// and its spike of step T + 1 - D at the next step (recorded already unless D = 1); only
-			// models with deferred events (or lazy plasticity) leave such rows to that delivery
-			bool const arrives_next = !eager_nodefer_v<Model> && T + 1 >= v.D &&
+			// and its spike of step T + 1 - D at the next step (recorded already unless D = 1): such
+			// rows are left to that delivery
+			bool const arrives_next = T + 1 >= v.D &&
 			                          ( v.D == 1 ? spiked : ( ( h_next >> ( ( T + 1 - v.D ) & 63 ) ) & 1ull ) != 0 );
 			{ // record this step in the history ring (overwriting step T - HISTORY)
 				unsigned long long const bit = 1ull << ( T & 63 );
@@ -1287,9 +1215,9 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 				v.xtr[cur + i] = fmaf( x_prev, d, arrived ? 1.0f : 0.0f );
 				v.ytr[cur + i] = fmaf( y_prev, d, spiked ? 1.0f : 0.0f );
 				v.fl8[cur + i] = std::uint8_t( ( spiked ? F8_SPIKED : 0 ) | ( arrived ? F8_ARRIVED : 0 ) | ( arrives_next ? F8_ARRIVES_NEXT : 0 ) );
-				// pre pass: a row whose spike arrives now, unless (deferred events) it arrives again
-				// at T + 1 and that delivery applies this step's events of the row; post pass: a
-				// spiking neuron with incoming plastic synapses
+				// pre pass: a row whose spike arrives now, unless it arrives again at T + 1 and that
+				// delivery applies this step's events of the row; post pass: a spiking neuron with
+				// incoming plastic synapses
 				flush = arrived && !arrives_next && has_plastic;
 				post = spiked && in_hi > in_lo;
 			}
@@ -1335,7 +1263,7 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 	// atomic per block on the step's counter, mbcnt gives each spiking lane its slot.
 	__shared__ unsigned wcount[16][3]; // at most 1024 threads
 	__shared__ unsigned bbase[3];
-	__shared__ std::uint64_t lbase; // overlapped step: where step T's ids start in the spike log
+	__shared__ std::uint64_t lbase; // where step T's ids start in the spike log
 	int const w = threadIdx.x >> 6;
 	std::uint64_t const m = ballot( spiked );
 	std::uint64_t const fm = plastic ? ballot( flush ) : 0ull;
@@ -1352,22 +1280,9 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 		// (the spike log's loads go out before the counter atomics: they do not depend on them)
 		if( v.slog )
 		{
-			// where step T's ids start in the log: written by this step's delivery kernel, or
-			// (the overlapped step, whose delivery of step T ran beside step T - 1's update) here,
-			// from step T - 1's offset and count, both final (written by an earlier kernel; this
-			// update clears the counts of steps after T, not of T - 1)
+			// where step T's ids start in the log: written by this step's delivery kernel
 			std::int64_t const k = T - v.slog->t0;
-			std::uint64_t base = 0;
-			if( k >= 0 && k < v.slog->nsteps )
-			{
-				if( !v.overlap )
-					base = v.slog_off[k];
-				else
-				{
-					base = k == 0 ? 0ull : v.slog_off[k - 1] + v.counts[ring_at( v, -1 )];
-					if( first == 0 ) v.slog_off[k] = base;
-				}
-			}
+			std::uint64_t const base = k >= 0 && k < v.slog->nsteps ? v.slog_off[k] : 0ull;
 			lbase = base;
 		}
 		unsigned t0 = 0, t1 = 0, t2 = 0;

@@ -103,12 +103,11 @@ inline int device_cu_count()
 	return cus;
 }
 
-// Longest window of steps one kernel may run (k_window): static models whose delivery may run
-// before its targets' update, up to the delay.
+// Longest window of steps one kernel may run (k_window).
 template <typename Model>
 int window_cap( int delay )
 {
-	return !is_plastic_v<Model> && overlap_capable_v<Model> && delay >= 2 ? window_steps( delay ) : 1;
+	return windowed_v<Model> && delay >= 2 ? std::max( 1, window_steps( std::min( delay, longest_window_v<Model> ) ) ) : 1;
 }
 // Entries of the spike ring: the delay and two windows; four at least, so that with a delay of
 // one step the entry of a step is its clock slot, known without reading the clock.
@@ -118,18 +117,18 @@ int ring_entries( int delay )
 	return std::max( 4, delay + 2 * window_cap<Model>( delay ) );
 }
 
-// Targets per delivery tile of a new network. Static models (window kernels): one tile per CU, as
+// Targets per delivery tile of a new network. Window kernels: one tile per CU, as
 // every tile stages all of the window's arrivals and a wider one does it less often (synth 1e9:
 // 29 us per step with 251 tiles of 3,200, 50 with 391 of 2,048), but none wider than its kernel
 // takes; windows of several steps, whose accumulators take LDS per step, two per CU beyond that.
-// Plastic models: about two tiles per CU, of 256 at least.
+// Two-kernel plastic steps: about two tiles per CU, of 256 at least.
 template <typename Model>
 int default_tile_w( std::int64_t n, int delay, int cus )
 {
 	auto const per = [&]( std::int64_t tiles ) { return ( ( n + tiles - 1 ) / tiles + 63 ) / 64 * 64; };
-	if( is_plastic_v<Model> ) return int( std::clamp<std::int64_t>( per( 2 * cus ), 256, TILE_MAX ) );
+	if( !windowed_v<Model> ) return int( std::clamp<std::int64_t>( per( 2 * cus ), 256, TILE_MAX ) );
 	bool const ahead = overlap_capable_v<Model> && delay >= 2;
-	std::int64_t const most = ahead ? TILE_MAX : 4 * 1024;
+	std::int64_t const most = ahead || is_plastic_v<Model> ? TILE_MAX : 4 * 1024;
 	return int( std::clamp<std::int64_t>( per( ahead && per( cus ) > most ? 2 * cus : cus ), 64, most ) );
 }
 
@@ -140,7 +139,7 @@ class hip_net final : public net_iface
 	using S = typename Model::synapse;
 	static constexpr bool plastic = is_plastic_v<Model>;
 	static constexpr bool traced = plastic && has_neuron_traces_v<S>;
-	static constexpr bool nodefer = eager_nodefer_v<Model>; // every eager event applied by the passes
+	static constexpr bool windowed = windowed_v<Model>; // steps run as windows (static models: at most launch shapes)
 
 public:
 	// first: launch shapes to start with (zero fields: the defaults)
@@ -156,8 +155,7 @@ public:
 			throw std::invalid_argument( "plastic models support delays of at most 255 steps" );
 		if( _g.n < 1 || _g.n > INT_MAX - 1024 ) throw std::invalid_argument( "invalid neuron count" );
 		static_assert( N::size <= MAXA && S::size <= MAXA, "at most 16 neuron/synapse attributes" );
-		// the update of step T runs beside the delivery of step T + 1 (see k_step_overlap)
-		_overlap = overlap_capable_v<Model> && p.delay >= 2;
+		_ahead = overlap_capable_v<Model> && p.delay >= 2;
 		allocate( first );
 		initialize();
 	}
@@ -191,7 +189,7 @@ public:
 			// windows are long enough to be launched one by one (a launch costs the host a few us)
 			while( n > 0 )
 			{
-				int const w = window_steps( std::min<std::int64_t>( n, _window ) );
+				int const w = window_steps( std::min<std::int64_t>( n, window_now() ) );
 				launch_window( _step, w, nullptr, nullptr );
 				_queue.launched( _s );
 				for( int i = 0; i < w; i++ ) tick();
@@ -205,64 +203,16 @@ public:
 
 	// Runs n steps eagerly, each kernel with HIP events attached to its dispatch on the net's
 	// stream, and adds the summed kernel durations (ms) to kernel_ms[0..2]: receive (delivery,
-	// with the previous step's plasticity), update, and 0; overlapped steps: the first delivery,
-	// the last update (with the passes of the step before it), and the n - 1 overlapped step
-	// kernels; windows: 0, 0 and the window kernels.
+	// with the previous step's plasticity), update, and 0. Windows of static models: 0, 0 and the
+	// window kernels; of plastic ones: the first window, the last one, and those between (a run
+	// of fewer than three windows: all in [2]).
 	void run_profiled( std::int64_t n, double * kernel_ms ) override
 	{
 		if( n < 0 ) throw std::invalid_argument( "negative step count" );
 		if( _window )
-		{
 			run_profiled_windows( n, kernel_ms );
-			return;
-		}
-		if( _overlap )
-		{
-			if( fixed() )
-				run_profiled_overlap<true>( n, kernel_ms );
-			else
-				run_profiled_overlap<false>( n, kernel_ms );
-			return;
-		}
-		constexpr int batch = 128, ev_per_step = 4;
-		synchronize(); // profiled steps run serially on the main stream
-		std::vector<hipEvent_t> ev( batch * ev_per_step, nullptr );
-		try
-		{
-			for( auto & e : ev ) SPICE_HIP( hipEventCreate( &e ) );
-			for( std::int64_t done = 0; done < n; )
-			{
-				int const k = int( std::min<std::int64_t>( batch, n - done ) );
-				for( int i = 0; i < k; i++ )
-				{
-					hipEvent_t * e = &ev[i * ev_per_step];
-					if( fixed() )
-						launch_step_events<true>( e, _vs[_step & ( CLOCK_SLOTS - 1 )] );
-					else
-						launch_step_events<false>( e, _vs[_step & ( CLOCK_SLOTS - 1 )] );
-					tick();
-				}
-				SPICE_HIP( hipStreamSynchronize( _s ) );
-				for( int i = 0; i < k; i++ )
-				{
-					hipEvent_t * e = &ev[i * ev_per_step];
-					for( int q = 0; q < 2; q++ ) // kernel_ms[2] stays 0: plasticity runs inside the delivery kernel
-					{
-						float ms = 0;
-						SPICE_HIP( hipEventElapsedTime( &ms, e[2 * q], e[2 * q + 1] ) );
-						kernel_ms[q] += ms;
-					}
-				}
-				done += k;
-			}
-		}
-		catch( ... )
-		{
-			for( auto & e : ev )
-				if( e ) (void)hipEventDestroy( e );
-			throw;
-		}
-		for( auto & e : ev ) (void)hipEventDestroy( e );
+		else
+			run_profiled_steps( n, kernel_ms );
 	}
 
 	void copy_spikes( std::int32_t * out, std::uint64_t cap, std::uint64_t * count ) override
@@ -306,7 +256,7 @@ public:
 	{
 		if( step < 0 || step > INT_MAX - 2 ) throw std::invalid_argument( "invalid step index" );
 		synchronize();
-		ctl_t ctl{ step, sum, c, std::int32_t( step % _v.rsize ) };
+		ctl_t ctl{ step, sum, c, std::int32_t( step % _v.rsize ), 0, 0, 0.0f, 0.0f };
 		SPICE_HIP( hipMemcpy( _ctl.data() + ( step & ( CLOCK_SLOTS - 1 ) ), &ctl, sizeof( ctl ), hipMemcpyHostToDevice ) );
 		SPICE_HIP( hipMemset( _counts.data(), 0, _counts.bytes() ) );
 		if constexpr( plastic )
@@ -331,7 +281,11 @@ public:
 
 	void get_stats( spice_stats * out ) override
 	{
-		synchronize();
+		// (windows of different lengths leave different amounts of plasticity due: count all of it)
+		if( windowed )
+			sync_synapses();
+		else
+			synchronize();
 		std::vector<unsigned long long> b( _bstats.size() );
 		SPICE_HIP( hipMemcpyAsync( b.data(), _bstats.data(), _bstats.bytes(), hipMemcpyDeviceToHost, _s ) );
 		SPICE_HIP( hipStreamSynchronize( _s ) );
@@ -392,6 +346,15 @@ public:
 		check_attr( a, int( N::size ) );
 		if( bytes != std::uint64_t( _g.n ) * attr_bytes<N>( a ) ) throw std::invalid_argument( "buffer size mismatch" );
 		synchronize();
+		if constexpr( plastic && windowed )
+			if( _step > 0 )
+			{
+				// The imported state need not keep the refractory promise towards spikes before it, so
+				// no event may still be due, and until those spikes have arrived windows are of one
+				// step (which relies on the promise for two steps only).
+				sync_synapses();
+				_single_until = _step + _p.delay + _v.wcap;
+			}
 		SPICE_HIP( hipMemcpy( _na[a].data(), in, bytes, hipMemcpyHostToDevice ) );
 	}
 
@@ -499,7 +462,7 @@ public:
 		for( int a = 0; a < MAXA; a++ ) b += _na[a].bytes() + _acc[a].bytes() + _sa[a].bytes();
 		b += _ring.bytes() + _counts.bytes() + _hring.bytes() + _last_spk.bytes() + _synced.bytes() + _pend.bytes() +
 		     _fl_id.bytes() + _fl_synced.bytes() + _fl_pend.bytes() + _hasp.bytes() + _pl_lo.bytes() + _pl_hi.bytes() +
-		     _fl_count.bytes() + _xtr.bytes() + _ytr.bytes() + _fl8.bytes() + _po_id.bytes() + _po_count.bytes() +
+		     _fl_count.bytes() + _xtr.bytes() + _ytr.bytes() + _fl8.bytes() + _sp8.bytes() + _po_id.bytes() + _po_count.bytes() +
 		     _tp_ptr.bytes() + _caught.bytes() + _tp_ent.bytes() + _ctl.bytes() + _bstats.bytes() +
 		     _pivots.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
 		return b;
@@ -513,9 +476,8 @@ public:
 		apply_launch( c );
 	}
 	bool is_plastic() const override { return plastic; }
-	bool overlapped() const { return _overlap; }
-	// widest delivery tile: wide tiles for the two-kernel step of static models
-	int max_tile_w() const override { return !plastic && !_overlap ? TILE_WIDE : TILE_MAX; }
+	// widest delivery tile: wide tiles for static models that run step by step
+	int max_tile_w() const override { return !plastic && !_ahead ? TILE_WIDE : TILE_MAX; }
 
 	net_iface * clone() const override
 	{
@@ -555,7 +517,7 @@ public:
 	dview const & view( int slot ) const { return _vs[slot & ( CLOCK_SLOTS - 1 )]; }
 	int num_tiles() const { return _v.nact; } // the delivery's tiles (those with incoming synapses)
 	int num_all_tiles() const { return _v.ntiles; }
-	int longest_window() const { return _v.wcap; }
+	std::int64_t single_steps_left() const { return std::max<std::int64_t>( 0, _single_until - _step ); }
 	bool logged() const { return _slog_ctl.size() > 0; }
 	int num_receive_parts() const { return _v.rparts; }
 	int num_update_blocks() const { return _grid_update; }
@@ -564,7 +526,7 @@ public:
 	// of their spike; eager: arriving rows and spiking targets), at most the net's own grid
 	int num_batch_flush_blocks() const
 	{
-		std::int64_t const items = traced ? ( _g.n / 256 + 1 ) * ( _v.fparts + _v.pparts ) : ( _g.n / FLUSH_AGE + _g.n / 256 + 1 ) * _v.fparts;
+		std::int64_t const items = traced ? ( _g.n / 256 + 1 ) * _v.wcap * ( _v.fparts + _v.pparts ) : ( _g.n / FLUSH_AGE + _g.n / 256 + 1 ) * _v.fparts;
 		return int( std::clamp<std::int64_t>( ( items + 1 ) / 2, 1, _grid_flush ) );
 	}
 	bool fixed() const { return ( _p.flags & SPICE_FLAG_FIXED_POINT ) != 0; }
@@ -589,8 +551,8 @@ private:
 	dbuf<std::uint8_t> _hasp;
 	dbuf<std::int32_t> _pl_lo, _pl_hi;
 	dbuf<std::uint32_t> _fl_count;
-	dbuf<float> _xtr, _ytr;                    // eager: [2][N] traces by step parity
-	dbuf<std::uint8_t> _fl8;                   // eager: [2][N] step flags
+	dbuf<float> _xtr, _ytr;                    // eager: traces, [2][N] by step parity or [4][N] by window
+	dbuf<std::uint8_t> _fl8, _sp8;             // eager: [2][N] step flags, or the windows' arrivals and spikes
 	dbuf<std::int32_t> _po_id;                 // eager: [2][N] spiking targets
 	dbuf<std::uint32_t> _po_count;             // eager: [4]
 	dbuf<std::int64_t> _tp_ptr;                // eager: by-target index offsets
@@ -608,7 +570,8 @@ private:
 	int _grid_upd = 0; // workgroups of this net's own update kernel (_upd_block threads)
 	int _upd_block = SPICE_UPDATE_BLOCK;
 	int _grid_plast = 0; // plasticity workgroups of the delivery kernel
-	bool _overlap = false; // steps run as k_step_overlap kernels
+	bool _ahead = false; // the delivery of a step may run before the updates of earlier steps
+	std::int64_t _single_until = 0; // windows of one step before this step (see import_neuron_attr)
 	int _window = 0;       // longest window of the window kernels that run the steps (0: none)
 	launch_queue _queue;
 	launch_cfg _lc{};
@@ -660,7 +623,7 @@ private:
 		} );
 		util::for_n<S::size>( [&]( auto I ) {
 			using A = typename S::template type<I>;
-			_sa[I].resize( std::max<std::int64_t>( _g.nnz, 1 ) * sizeof( A ) );
+			_sa[I].resize( ( _g.nnz + COL_PAD ) * sizeof( A ) ); // (read in pieces like the row store)
 		} );
 		_v.wcap = window_cap<Model>( _p.delay );
 		_v.rsize = ring_entries<Model>( _p.delay );
@@ -681,9 +644,10 @@ private:
 			reset_caught();
 			if constexpr( traced )
 			{
-				_xtr.resize( 2 * n );
-				_ytr.resize( 2 * n );
+				_xtr.resize( ( windowed ? 4 : 2 ) * n );
+				_ytr.resize( ( windowed ? 4 : 2 ) * n );
 				_fl8.resize( 2 * n );
+				if( windowed ) _sp8.resize( 2 * n );
 				_po_id.resize( 2 * n );
 				_po_count.resize( CLOCK_SLOTS );
 				_tp_ptr.resize( n + 1 );
@@ -711,7 +675,6 @@ private:
 		v.D = _p.delay;
 		v.width = std::int32_t( std::min<std::int64_t>( _g.width, INT_MAX ) );
 		v.shift = 40;
-		v.overlap = _overlap ? 1 : 0;
 		v.DT = _p.dt;
 		v.flags = _p.flags;
 		v.seed = _p.seed;
@@ -740,6 +703,7 @@ private:
 		v.xtr = _xtr.data();
 		v.ytr = _ytr.data();
 		v.fl8 = _fl8.data();
+		v.sp8 = _sp8.data();
 		v.po_id = _po_id.data();
 		v.po_count = _po_count.data();
 		v.tp_ptr = _tp_ptr.data();
@@ -760,6 +724,7 @@ private:
 	{
 		for( auto * b : { &_xtr, &_ytr } ) SPICE_HIP( hipMemsetAsync( b->data(), 0, b->bytes(), _s ) );
 		SPICE_HIP( hipMemsetAsync( _fl8.data(), 0, _fl8.bytes(), _s ) );
+		if( windowed ) SPICE_HIP( hipMemsetAsync( _sp8.data(), 0, _sp8.bytes(), _s ) );
 		SPICE_HIP( hipMemsetAsync( _po_count.data(), 0, _po_count.bytes(), _s ) );
 	}
 
@@ -830,16 +795,22 @@ private:
 		std::int64_t const n = _g.n;
 		launch_cfg c;
 		c.tile_w = default_tile_w<Model>( n, _p.delay, cus );
-		c.flush_slots = 256;
+		// plasticity beside a window's tiles: four workgroups of 256 threads per CU; work items of 128
+		// slots or entries, which one round of a wave's loads holds twice over (STDP 1e8, delay 1:
+		// 13.0 us per step, 16.2 with 256, 23.6 with 512), or of 512 where a window has items enough
+		// for every wave anyway (1e9, delay 15, steps 2,000-12,000: 24.9, 25.3 with 256, 26.5 with 128)
 		double const mean_row = n > 0 ? double( _g.nnz ) / double( n ) : 0.0;
+		c.flush_slots = !windowed ? 256 : _v.wcap > 1 && mean_row >= 8192.0 ? 512 : 128;
 		std::int64_t const fparts = std::max( 1, int( mean_row / c.flush_slots + 0.5 ) );
-		c.flush_grid = int( std::min<std::int64_t>( 8 * cus, std::max<std::int64_t>( 1, ( n * fparts + 3 ) / 4 ) ) );
+		c.flush_grid = int( std::min<std::int64_t>( ( windowed ? 4 : 8 ) * cus, std::max<std::int64_t>( 1, ( n * fparts + 3 ) / 4 ) ) );
 		c.recv_parts = 1;
 		if( !plastic )
 			// window kernels: 16 waves where a tile has a CU to itself, 8 where several share one or
 			// the tile is small (Vogels 1e9, delay 8: 7.6 us per step with 250 tiles of 896 and 16
 			// waves, 8.9 with 8; Brunel 1e10, 495 tiles of 640: 19.4 with 16, 17.3 with 8)
 			c.recv_block = c.tile_w > 2048 || ( c.tile_w >= 512 && ( n + c.tile_w - 1 ) / c.tile_w <= cus ) ? 1024 : 512;
+		else if( windowed )
+			c.recv_block = 512; // (STDP 1e9: 24.3 us per step, 27.4 with 1,024 threads)
 		else
 			// small nets: few events per tile, so more and smaller delivery workgroups
 			c.recv_block = n <= 65536 ? 256 : 1024;
@@ -886,16 +857,14 @@ private:
 		_grid_tiles = std::max( 1, std::min( v.nact * v.rparts, ( 16 * 1024 / c.recv_block ) * cus ) );
 		_grid_plast = plastic ? std::max( 1, _grid_flush * 256 / c.recv_block ) : 0; // the same waves as flush_grid
 		_lc = c;
-		v.upd_slot0 = upd_slot0();
 		choose_window();
 		// statistics slots: one per workgroup of the widest step kernel (receive: per work item;
-		// eager plasticity: after those, one per plasticity workgroup or synchronization block;
-		// the overlapped step's update blocks after those; windows: one per tile), and enough for
-		// the update kernel's blocks
+		// plasticity: after those, one per plasticity workgroup or synchronization block; windows:
+		// one per tile, then the passes' workgroups; update: per block)
 		std::size_t const slots =
 		    std::size_t( std::max( { _grid_update, _grid_upd, 2 * _grid_flush, 2 * _grid_tiles,
-		                             upd_slot0() + _grid_update } ) ) *
-		    NSTAT; // (update blocks of >= 256 neurons)
+		                             v.ntiles * v.rparts + std::max( _grid_plast, _grid_flush ) } ) ) *
+		    NSTAT;
 		if( slots > _bstats.size() )
 		{
 			std::vector<unsigned long long> keep( NSTAT, 0ull );
@@ -947,14 +916,14 @@ private:
 		v.tile_ids = _tile_ids.data();
 	}
 
-	// Window kernels (_window: their longest window, 0: none) run the steps of static models: those
-	// whose delivery may run before its targets' update in windows of up to the delay, as long as
-	// the accumulators fit; the others step by step where one workgroup delivers a tile
+	// Window kernels (_window: their longest window, 0: none) run the steps of models whose
+	// delivery may run before its targets' update in windows of up to the delay, as long as the
+	// accumulators fit; other static models' step by step where one workgroup delivers a tile
 	// (recv_parts = 1) of at most 4 workgroup widths.
 	void choose_window()
 	{
 		_window = 0;
-		if constexpr( !plastic )
+		if constexpr( windowed )
 		{
 			// lanes per segment: the power of two whose reads hold a segment two standard deviations
 			// longer than the mean, so that few take a second round (Vogels 1e9, delay 8, 17.9
@@ -962,7 +931,7 @@ private:
 			double const mean = _g.n > 0 ? double( _g.nnz ) / double( _g.n ) / _v.nact : 0.0;
 			_v.wlanes = 0;
 			while( _v.wlanes < 5 && double( WIN_VEC << _v.wlanes ) < mean + 2.0 * std::sqrt( mean ) ) _v.wlanes++;
-			if( !_overlap && ( _lc.recv_parts != 1 || _lc.tile_w > 4 * _lc.recv_block ) ) return;
+			if( !plastic && !_ahead && ( _lc.recv_parts != 1 || _lc.tile_w > 4 * _lc.recv_block ) ) return;
 			_window = 1;
 			with_window_kernel( [&]( auto kernel, auto bytes, int ) {
 				// the LDS of a CU, shared by the workgroups that a CU gets
@@ -987,96 +956,75 @@ private:
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 	}
 
-	// First statistics slot of the overlapped step's update blocks (after the delivery work
-	// items and the plasticity workgroups).
-	int upd_slot0() const { return _v.ntiles * _v.rparts + std::max( _grid_plast, _grid_flush ); }
+	// Windows at this step: of one step while imported neuron state may break the promise that
+	// longer ones rely on.
+	int window_now() const { return _step < _single_until ? 1 : _window; }
 
-	// Enqueues steps t .. t + len - 1. Two kernels per step, or (overlapped steps) the delivery
-	// of step t, then one k_step_overlap per step boundary (update of T, delivery of T + 1,
-	// passes of T - 1), then the last update with the passes of the step before it: len + 1
-	// kernels, and as with the two-kernel step the passes of the last step are left to the
-	// next delivery kernel (or a synchronization).
+	// Enqueues steps t .. t + len - 1: windows of one step, or two kernels per step. The passes of
+	// the last step of a plastic model are left to the next kernel (or a synchronization).
 	void launch_steps( std::int64_t t, std::int64_t len )
 	{
-		if( _window )
-		{
-			for( std::int64_t k = 0; k < len; k++ ) launch_window( t + k, 1, nullptr, nullptr );
-			return;
-		}
-		if( !_overlap )
-		{
-			for( std::int64_t k = 0; k < len; k++ ) launch_step( t + k );
-			return;
-		}
-		for( std::int64_t k = 0; k <= len; k++ )
+		for( std::int64_t k = 0; k < len; k++ )
+			if( _window )
+				launch_window( t + k, 1, nullptr, nullptr );
+			else
+				launch_step( t + k );
+	}
+
+	// Enqueues the kernels of step `t` (t mod 4 selects the clock slot): delivery (plastic
+	// models: with step t - 1's plasticity work in the same kernel), then the neuron update.
+	void launch_step( std::int64_t t )
+	{
+		[[maybe_unused]] dview const & v = _vs[t & ( CLOCK_SLOTS - 1 )];
+		if constexpr( !plastic || !windowed )
 		{
 			if( fixed() )
-				launch_overlap_kernel<true>( t, len, k, nullptr, nullptr );
+			{
+				launch_receive<true>( v );
+				launch_update<true>( v, nullptr, nullptr );
+			}
 			else
-				launch_overlap_kernel<false>( t, len, k, nullptr, nullptr );
+			{
+				launch_receive<false>( v );
+				launch_update<false>( v, nullptr, nullptr );
+			}
 		}
 	}
 
-	// Kernel k (0 .. len) of the overlapped sequence of steps t .. t + len - 1 (see
-	// launch_steps), with HIP events attached to its dispatch when start is not null.
-	template <bool F>
-	void launch_overlap_kernel( std::int64_t t, std::int64_t len, std::int64_t k, hipEvent_t start, hipEvent_t stop )
+	// run_profiled for two-kernel steps
+	void run_profiled_steps( std::int64_t n, double * kernel_ms )
 	{
-		int const bs = _lc.recv_block;
-		if( k == 0 )
-		{
-			// delivery of step t only: step t - 1's passes run beside the first update
-			dview const & v = _vs[t & ( CLOCK_SLOTS - 1 )];
-			std::int32_t const tiles = _grid_tiles;
-			auto go = [&]( auto b ) {
-				constexpr int BS = decltype( b )::value;
-				if( start )
-					launch_timed( reinterpret_cast<void const *>( &k_receive_tiled<Model, F, BS> ), unsigned( tiles ), BS, start, stop, v, tiles );
-				else
-					SPICE_LAUNCH( ( k_receive_tiled<Model, F, BS><<<unsigned( tiles ), BS, 0, _s>>>( v, tiles ) ) );
-			};
-			bs == 256 ? go( std::integral_constant<int, 256>{} ) : bs == 512 ? go( std::integral_constant<int, 512>{} ) : go( std::integral_constant<int, 1024>{} );
-			return;
-		}
-		std::int64_t const T = t + k - 1; // this kernel updates step T
-		dview const & v = _vs[T & ( CLOCK_SLOTS - 1 )];
-		std::int32_t const nrecv = k < len ? _grid_tiles : 0; // the last kernel delivers nothing
-		std::int32_t const nplast = _grid_plast, s0 = upd_slot0();
-		unsigned const grid = unsigned( nrecv + nplast + int( ( _g.n + bs - 1 ) / bs ) );
-		auto go = [&]( auto b ) {
-			constexpr int BS = decltype( b )::value;
-			if( start )
-				launch_timed( reinterpret_cast<void const *>( &k_step_overlap<Model, F, BS> ), grid, BS, start, stop, v, nrecv, nplast, s0 );
-			else
-				SPICE_LAUNCH( ( k_step_overlap<Model, F, BS><<<grid, BS, 0, _s>>>( v, nrecv, nplast, s0 ) ) );
-		};
-		bs == 256 ? go( std::integral_constant<int, 256>{} ) : bs == 512 ? go( std::integral_constant<int, 512>{} ) : go( std::integral_constant<int, 1024>{} );
-	}
-
-	// run_profiled for overlapped steps: kernel 0 -> kernel_ms[0], kernels 1 .. n - 1 ->
-	// kernel_ms[2], kernel n -> kernel_ms[1].
-	template <bool F>
-	void run_profiled_overlap( std::int64_t n, double * kernel_ms )
-	{
-		if( n == 0 ) return;
-		constexpr int batch = 128;
-		synchronize();
-		std::int64_t const t0 = _step;
-		std::vector<hipEvent_t> ev( 2 * batch, nullptr );
+		constexpr int batch = 128, ev_per_step = 4;
+		synchronize(); // profiled steps run serially on the main stream
+		std::vector<hipEvent_t> ev( batch * ev_per_step, nullptr );
 		try
 		{
 			for( auto & e : ev ) SPICE_HIP( hipEventCreate( &e ) );
-			for( std::int64_t done = 0; done <= n; )
+			for( std::int64_t done = 0; done < n; )
 			{
-				int const k = int( std::min<std::int64_t>( batch, n + 1 - done ) );
-				for( int i = 0; i < k; i++ ) launch_overlap_kernel<F>( t0, n, done + i, ev[2 * i], ev[2 * i + 1] );
+				int const k = int( std::min<std::int64_t>( batch, n - done ) );
+				for( int i = 0; i < k; i++ )
+				{
+					hipEvent_t * e = &ev[i * ev_per_step];
+					if constexpr( !plastic || !windowed )
+					{
+						if( fixed() )
+							launch_step_events<true>( e, _vs[_step & ( CLOCK_SLOTS - 1 )] );
+						else
+							launch_step_events<false>( e, _vs[_step & ( CLOCK_SLOTS - 1 )] );
+					}
+					tick();
+				}
 				SPICE_HIP( hipStreamSynchronize( _s ) );
 				for( int i = 0; i < k; i++ )
 				{
-					float ms = 0;
-					SPICE_HIP( hipEventElapsedTime( &ms, ev[2 * i], ev[2 * i + 1] ) );
-					std::int64_t const idx = done + i;
-					kernel_ms[idx == 0 ? 0 : idx == n ? 1 : 2] += ms;
+					hipEvent_t * e = &ev[i * ev_per_step];
+					for( int q = 0; q < 2; q++ ) // kernel_ms[2] stays 0: plasticity runs inside the delivery kernel
+					{
+						float ms = 0;
+						SPICE_HIP( hipEventElapsedTime( &ms, e[2 * q], e[2 * q + 1] ) );
+						kernel_ms[q] += ms;
+					}
 				}
 				done += k;
 			}
@@ -1088,24 +1036,6 @@ private:
 			throw;
 		}
 		for( auto & e : ev ) (void)hipEventDestroy( e );
-		for( std::int64_t i = 0; i < n; i++ ) tick();
-	}
-
-	// Enqueues the kernels of step `t` (t mod 4 selects the clock slot): delivery (plastic
-	// models: with step t - 1's plasticity work in the same kernel), then the neuron update.
-	void launch_step( std::int64_t t )
-	{
-		dview const & v = _vs[t & ( CLOCK_SLOTS - 1 )];
-		if( fixed() )
-		{
-			launch_receive<true>( v );
-			launch_update<true>( v, nullptr, nullptr );
-		}
-		else
-		{
-			launch_receive<false>( v );
-			launch_update<false>( v, nullptr, nullptr );
-		}
 	}
 
 	// the neuron update kernel of the two-kernel step (workgroups of _upd_block threads), with
@@ -1129,11 +1059,11 @@ private:
 		}
 	}
 
-	// The window of w steps from step t (static models), with HIP events attached to its dispatch
-	// when start is not null.
+	// The window of w steps from step t, with HIP events attached to its dispatch when start is not
+	// null.
 	void launch_window( std::int64_t t, int w, hipEvent_t start, hipEvent_t stop )
 	{
-		if constexpr( !plastic )
+		if constexpr( windowed )
 		{
 			if( _slog_ctl.size() ) throw std::logic_error( "nets with a spike log are stepped by a batch" );
 			dview v = _vs[t & ( CLOCK_SLOTS - 1 )];
@@ -1142,9 +1072,9 @@ private:
 				void * args[] = { &v, &W };
 				void const * fn = reinterpret_cast<void const *>( kernel );
 				if( start )
-					SPICE_HIP( hipExtLaunchKernel( fn, dim3( unsigned( v.ntiles ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s, start, stop, 0 ) );
+					SPICE_HIP( hipExtLaunchKernel( fn, dim3( unsigned( v.ntiles + _grid_plast ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s, start, stop, 0 ) );
 				else
-					SPICE_HIP( hipLaunchKernel( fn, dim3( unsigned( v.ntiles ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s ) );
+					SPICE_HIP( hipLaunchKernel( fn, dim3( unsigned( v.ntiles + _grid_plast ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s ) );
 			} );
 		}
 	}
@@ -1165,7 +1095,7 @@ private:
 		fixed() ? by_block( std::true_type{} ) : by_block( std::false_type{} );
 	}
 
-	// run_profiled for windows: every kernel -> kernel_ms[2]
+	// run_profiled for windows
 	void run_profiled_windows( std::int64_t n, double * kernel_ms )
 	{
 		constexpr int batch = 128;
@@ -1174,12 +1104,14 @@ private:
 		try
 		{
 			for( auto & e : ev ) SPICE_HIP( hipEventCreate( &e ) );
+			double first = 0.0, last = 0.0, sum = 0.0;
+			std::int64_t windows = 0;
 			while( n > 0 )
 			{
 				int k = 0;
 				for( ; k < batch && n > 0; k++ )
 				{
-					int const w = window_steps( std::min<std::int64_t>( n, _window ) );
+					int const w = window_steps( std::min<std::int64_t>( n, window_now() ) );
 					launch_window( _step, w, ev[2 * k], ev[2 * k + 1] );
 					for( int i = 0; i < w; i++ ) tick();
 					n -= w;
@@ -1189,9 +1121,15 @@ private:
 				{
 					float ms = 0;
 					SPICE_HIP( hipEventElapsedTime( &ms, ev[2 * i], ev[2 * i + 1] ) );
-					kernel_ms[2] += ms;
+					if( windows++ == 0 ) first = ms;
+					last = ms;
+					sum += ms;
 				}
 			}
+			bool const ends = plastic && windows >= 3;
+			kernel_ms[0] += ends ? first : 0.0;
+			kernel_ms[1] += ends ? last : 0.0;
+			kernel_ms[2] += ends ? sum - first - last : sum;
 		}
 		catch( ... )
 		{
@@ -1271,15 +1209,22 @@ private:
 				// recorded in `caught` so the next delivery kernel skips the former
 				std::int64_t const now = _step - 1;
 				dview const & v = _vs[_step & ( CLOCK_SLOTS - 1 )]; // a view of step now + 1
-				std::int64_t const slot0 = std::int64_t( v.ntiles ) * v.rparts;
-				if constexpr( traced )
+				[[maybe_unused]] std::int64_t const slot0 = std::int64_t( v.ntiles ) * v.rparts;
+				if constexpr( windowed )
+				{
+					if( fixed() )
+						SPICE_LAUNCH( ( k_window_passes<Model, true><<<_grid_flush, 256, 0, _s>>>( v ) ) );
+					else
+						SPICE_LAUNCH( ( k_window_passes<Model, false><<<_grid_flush, 256, 0, _s>>>( v ) ) );
+				}
+				else if constexpr( traced )
 				{
 					if( fixed() )
 						SPICE_LAUNCH( k_stdp<Model, true><<<_grid_flush, 256, 0, _s>>>( v, now, slot0 ) );
 					else
 						SPICE_LAUNCH( k_stdp<Model, false><<<_grid_flush, 256, 0, _s>>>( v, now, slot0 ) );
-					// deferred events of the rows arriving next (none when the passes apply all)
-					if constexpr( !nodefer ) SPICE_LAUNCH( k_sync_eager<Model><<<unsigned( ( _g.n + 3 ) / 4 ), 256, 0, _s>>>( _v, now ) );
+					// deferred events of the rows arriving next
+					SPICE_LAUNCH( k_sync_eager<Model><<<unsigned( ( _g.n + 3 ) / 4 ), 256, 0, _s>>>( _v, now ) );
 				}
 				else
 				{

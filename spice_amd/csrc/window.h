@@ -52,6 +52,20 @@ constexpr int WIN_TABLE = 64; // partial sums kept per input class
 template <typename T, bool FIXED>
 using win_acc = std::conditional_t<std::is_floating_point_v<T>, std::conditional_t<FIXED, long long, double>, T>;
 
+// Models whose steps run as windows: static ones, and plastic ones whose passes apply every event.
+template <typename Model>
+inline constexpr bool windowed_v = !is_plastic_v<Model> || eager_nodefer_v<Model>;
+
+// Longest window (steps, before the clock's restriction): 1 unless the delivery may run before its
+// targets' update. Plastic models: an input is read beside the passes of the window before, and
+// before this window's, so no event of its synapse may fall into the 2 W - 1 steps before it
+// unless the input is dropped: a post event's target is refractory for R steps, and a pre event's
+// source does not spike twice within R.
+template <typename Model>
+constexpr int longest_window_v = !overlap_capable_v<Model> ? 1
+                                 : is_plastic_v<Model>     ? ( refractory_steps_v<typename Model::synapse> + 1 ) / 2
+                                                           : WINDOW_MAX;
+
 template <typename Model, bool FIXED>
 struct window_lds
 {
@@ -64,8 +78,10 @@ struct window_lds
 	// masks [W][tile_w / 64], and the masks' exclusive prefix counts
 	HYBRID static std::size_t acc_at( int bs ) { return sizeof( win_seg ) * std::size_t( bs ); }
 	HYBRID static std::size_t mask_at( int bs, int tw, int w ) { return acc_at( bs ) + sizeof( word ) * std::size_t( nacc ) * std::size_t( tw ) * std::size_t( w ); }
-	HYBRID static std::size_t pre_at( int bs, int tw, int w ) { return mask_at( bs, tw, w ) + 8 * std::size_t( tw / 64 ) * std::size_t( w ); }
-	HYBRID static std::size_t bytes( int bs, int tw, int w ) { return pre_at( bs, tw, w ) + 4 * std::size_t( tw / 64 ) * std::size_t( w ); }
+	// rows of masks: the window's steps, then (plastic models) the arriving rows and the spiking targets
+	HYBRID static int rows( int w ) { return w + ( is_plastic_v<Model> ? 2 : 0 ); }
+	HYBRID static std::size_t pre_at( int bs, int tw, int w ) { return mask_at( bs, tw, w ) + 8 * std::size_t( tw / 64 ) * std::size_t( rows( w ) ); }
+	HYBRID static std::size_t bytes( int bs, int tw, int w ) { return pre_at( bs, tw, w ) + 4 * std::size_t( tw / 64 ) * std::size_t( rows( w ) ); }
 };
 
 // Receive target inside a window (models without input classes): backend.atomic_add goes to the
@@ -117,6 +133,23 @@ __device__ inline targets load_targets( std::int32_t const * p )
 	return t;
 }
 
+// The state of WIN_VEC consecutive synapses.
+template <typename S>
+struct synapses
+{
+	typename S::tuple_t s[WIN_VEC];
+	__device__ void load( void * const * arr, std::int64_t i )
+	{
+		util::for_n<S::size>( [&]( auto I ) {
+			using T = typename S::template type<I>;
+			T t[WIN_VEC];
+			__builtin_memcpy( t, static_cast<T const *>( arr[I] ) + i, sizeof( t ) );
+#pragma unroll
+			for( int x = 0; x < WIN_VEC; x++ ) std::get<I>( s[x] ) = t[x];
+		} );
+	}
+};
+
 // Orders a wave's LDS writes before its own later LDS reads (and reads before writes): the LDS
 // serves a wave's instructions in order, so only the compiler has to keep them.
 __device__ inline void wave_lds_fence()
@@ -146,13 +179,15 @@ template <typename Model, bool FIXED, int BS>
 __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 {
 	using N = typename Model::neuron;
+	using S = typename Model::synapse;
 	using L = window_lds<Model, FIXED>;
 	using word = typename L::word;
+	constexpr bool plastic = is_plastic_v<Model>;
 	constexpr int nacc = L::nacc;
 	constexpr std::uint32_t rmask = receive_mask_v<N>;
 
 	extern __shared__ __align__( 16 ) unsigned char dyn[];
-	__shared__ std::uint32_t base[WINDOW_MAX + 1];
+	__shared__ std::uint32_t base[WINDOW_MAX + 2];
 	__shared__ std::uint32_t ev_total, spk_total;
 	// fp32 input classes: the sum of the first k inputs of class c
 	constexpr bool tables = L::classes > 0 && !FIXED;
@@ -264,7 +299,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 				fetch_seg();
 				if( k0 + 2 * NW * per < total ) src_n = fetch_id( k0 + 2 * NW * per + mylane, q_n );
 			}
-			constexpr int U = 4; // segments per group in flight
+			constexpr int U = plastic ? 2 : 4; // segments per group in flight (with weights, 4 measured 3 % slower)
 			for( std::int32_t c = 0; c < cnt; c += U * ng )
 			{
 				win_seg r[U];
@@ -283,6 +318,12 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 					targets j[U];
 #pragma unroll
 					for( int u = 0; u < U; u++ ) j[u] = load_targets( v.col + r[u].off + ( e < len[u] ? e : 0 ) );
+					synapses<S> sy[U];
+					if constexpr( plastic )
+					{
+#pragma unroll
+						for( int u = 0; u < U; u++ ) sy[u].load( v.sa, r[u].off + ( e < len[u] ? e : 0 ) );
+					}
 #pragma unroll
 					for( int u = 0; u < U; u++ )
 #pragma unroll
@@ -295,7 +336,11 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 							{
 								int const s = r[u].meta >> 16;
 								tile_backend<FIXED> bak{ make_backend<FIXED>( v, std::uint32_t( r[u].src ), std::uint32_t( j[u].id[x] ), std::uint32_t( T0 + s ), util::TAG_RECEIVE ) };
-								deliver_event<N>( r[u].src, win_iter<N, FIXED>{ &v, j[u].id[x], t0, tws, acc + s * ( nacc * tws ) }, no_syn_iter{}, info, bak );
+								win_iter<N, FIXED> dst{ &v, j[u].id[x], t0, tws, acc + s * ( nacc * tws ) };
+								if constexpr( plastic )
+									deliver_event<N>( r[u].src, dst, reg_iter<typename S::tuple_t>{ sy[u].s[x], std::uint32_t( r[u].off + e + x ) }, info, bak );
+								else
+									deliver_event<N>( r[u].src, dst, no_syn_iter{}, info, bak );
 							}
 						}
 					if( e - l * WIN_VEC + G * WIN_VEC >= most ) break;
@@ -316,6 +361,26 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 			std::int64_t const i = t0 + x;
 			typename N::tuple_t s;
 			load_tuple<N>( s, v.na, i );
+			// plastic models: the arrivals of this neuron's own spikes (of the steps from T0 - D), its
+			// traces, and the history words that the window's steps go to
+			std::uint32_t arrivals = 0;
+			float xt = 0.0f, yt = 0.0f;
+			unsigned long long h0 = 0, h1 = 0;
+			std::int64_t const hw0 = ( T0 & ( HISTORY - 1 ) ) >> 6, hw1 = ( ( T0 + W - 1 ) & ( HISTORY - 1 ) ) >> 6;
+			bool has_out = false, has_in = false;
+			if constexpr( plastic )
+			{
+				int const b = int( ( T0 - v.D ) & ( HISTORY - 1 ) ), sh = b & 63;
+				unsigned long long a = v.hring[std::int64_t( b >> 6 ) * v.N + i] >> sh;
+				if( sh + W > 64 ) a |= v.hring[std::int64_t( ( ( b >> 6 ) + 1 ) & ( HWORDS - 1 ) ) * v.N + i] << ( 64 - sh );
+				arrivals = std::uint32_t( a ) & ( ( 1u << W ) - 1u );
+				h0 = v.hring[hw0 * v.N + i];
+				if( hw1 != hw0 ) h1 = v.hring[hw1 * v.N + i];
+				xt = v.xtr[( clk.wseq & 3 ) * std::int64_t( v.N ) + i];
+				yt = v.ytr[( clk.wseq & 3 ) * std::int64_t( v.N ) + i];
+				has_out = v.hasp[i];
+				has_in = v.tp_ptr[i + 1] > v.tp_ptr[i];
+			}
 			float sum = clk.sum, c = clk.c;
 			for( int q = 0; q < W; q++ )
 			{
@@ -358,11 +423,38 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 				} );
 				auto bak = make_backend<FIXED>(
 				    v, std::uint32_t( i ), std::uint32_t( T ), std::uint32_t( std::uint64_t( T ) >> 32 ), util::TAG_NEURON_UPDATE );
-				if( N::update( reg_iter<typename N::tuple_t>{ s, std::uint32_t( i ) }, dt, info, bak ) ) spikes |= 1u << q;
+				bool const spiked = N::update( reg_iter<typename N::tuple_t>{ s, std::uint32_t( i ) }, dt, info, bak );
+				if( spiked ) spikes |= 1u << q;
+				if constexpr( plastic )
+				{
+					float const d = S::trace_decay( dt );
+					xt = fmaf( xt, d, ( arrivals >> q ) & 1u ? 1.0f : 0.0f );
+					yt = fmaf( yt, d, spiked ? 1.0f : 0.0f );
+				}
 			}
 			store_tuple<N>( s, v.na, i );
+			if constexpr( plastic )
+			{
+				// the steps' history bits (over those of the steps HISTORY before)
+				unsigned long long const all = ( 1ull << W ) - 1ull;
+				int const sh = int( T0 & 63 );
+				unsigned long long const n0 = ( h0 & ~( all << sh ) ) | ( (unsigned long long)( spikes ) << sh );
+				if( n0 != h0 ) v.hring[hw0 * v.N + i] = n0;
+				if( hw1 != hw0 )
+				{
+					unsigned long long const n1 = ( h1 & ~( all >> ( 64 - sh ) ) ) | ( (unsigned long long)( spikes ) >> ( 64 - sh ) );
+					if( n1 != h1 ) v.hring[hw1 * v.N + i] = n1;
+				}
+				std::int64_t const nx = ( ( clk.wseq + 1 ) & 3 ) * std::int64_t( v.N ) + i, par = ( clk.wseq & 1 ) * std::int64_t( v.N ) + i;
+				v.xtr[nx] = xt;
+				v.ytr[nx] = yt;
+				v.fl8[par] = std::uint8_t( arrivals ? __builtin_ctz( arrivals ) + 1 : 0 );
+				v.sp8[par] = std::uint8_t( spikes ? __builtin_ctz( spikes ) + 1 : 0 );
+				if( has_out && arrivals ) spikes |= 1u << W;
+				if( has_in && ( spikes & std::uint32_t( all ) ) ) spikes |= 2u << W;
+			}
 		}
-		for( int q = 0; q < W; q++ )
+		for( int q = 0; q < L::rows( W ); q++ )
 		{
 			std::uint64_t const m = ballot( ( spikes >> q ) & 1u );
 			if( lane == 0 ) masks[q * nw + ( x >> 6 )] = m;
@@ -375,15 +467,18 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	__syncthreads();
 
 	// a wave per step: the masks' prefix counts, and one atomic reserves the tile's ring places
-	for( int q = tid >> 6; q < W; q += BS / 64 )
+	for( int q = tid >> 6; q < L::rows( W ); q += BS / 64 )
 	{
 		std::uint32_t const n = lane < nw ? std::uint32_t( __popcll( masks[q * nw + lane] ) ) : 0u;
 		std::uint32_t const in = wave_inclusive_scan32( n );
 		if( lane < nw ) wpre[q * nw + lane] = in - n;
 		if( lane == 63 && in )
 		{
-			base[q] = atomicAdd( &v.counts[entry( q )], in );
-			atomicAdd( &spk_total, in );
+			std::uint32_t * count = &v.counts[entry( q < W ? q : 0 )];
+			if constexpr( plastic )
+				if( q >= W ) count = ( q == W ? v.fl_count : v.po_count ) + ( clk.wseq & 3 );
+			base[q] = atomicAdd( count, in );
+			if( q < W ) atomicAdd( &spk_total, in );
 		}
 	}
 	if( tile == 0 )
@@ -406,15 +501,28 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 			next->sum = sum;
 			next->step = T0 + W;
 			next->rslot = entry( W );
+			if constexpr( plastic )
+			{
+				next->wseq = clk.wseq + 1;
+				next->wprev = W;
+				next->psum = clk.sum;
+				next->pc = clk.c;
+				// the next window's list counters (last read by the passes of window wseq - 3)
+				v.fl_count[( clk.wseq + 1 ) & 3] = 0;
+				v.po_count[( clk.wseq + 1 ) & 3] = 0;
+			}
 		}
 	}
 	__syncthreads();
 	for( int x = tid; x < tws; x += BS )
-		for( int q = 0; q < W; q++ )
+		for( int q = 0; q < L::rows( W ); q++ )
 		{
 			std::uint64_t const m = masks[q * nw + ( x >> 6 )];
-			if( ( m >> lane ) & 1ull )
-				v.ring[std::int64_t( entry( q ) ) * v.N + base[q] + wpre[q * nw + ( x >> 6 )] + std::uint32_t( lanes_below( m ) )] = t0 + x;
+			if( !( ( m >> lane ) & 1ull ) ) continue;
+			std::int32_t * list = v.ring + std::int64_t( entry( q < W ? q : 0 ) ) * v.N;
+			if constexpr( plastic )
+				if( q >= W ) list = ( q == W ? v.fl_id : v.po_id ) + ( clk.wseq & 1 ) * std::int64_t( v.N );
+			list[base[q] + wpre[q * nw + ( x >> 6 )] + std::uint32_t( lanes_below( m ) )] = t0 + x;
 		}
 	if( tid == 0 )
 	{
@@ -434,12 +542,216 @@ __device__ inline std::int32_t xcd_place( std::int32_t b, std::int32_t n )
 	return x * per + ( x < more ? x : more ) + b / XCDS;
 }
 
-// One workgroup per tile: those with incoming synapses first.
+// Plasticity of the window before the view's step: a pre pass over the plastic slots of the rows
+// whose spike arrived in it, and a post pass over the incoming plastic synapses (by-target index) of
+// the neurons that spiked in it, leaving out sources that arrived in it (the pre pass has those).
+// Refractory endpoints have at most one arrival and one spike each in a window, so a synapse has at
+// most a pre event (at step a) and a post event (at step b), applied in step order in one
+// read-modify-write; the traces at a and b are the per-step recurrence continued from the window's
+// start. One index space of work items, (row, part) then (target, part), taken round robin by the
+// waves of workgroups blk, blk + nblk, ...; statistics go to slots slot0 + blk. Bound by the rate
+// of random memory lines: the post pass's weights (profiles/random_line_probe.md).
+template <typename Model, bool FIXED>
+__device__ inline void window_passes( dview const & v, std::int64_t blk, std::int64_t nblk, std::int64_t slot0 )
+{
+	using S = typename Model::synapse;
+	constexpr int U = 4; // synapses per lane in flight
+	ctl_t const clk = *v.ctl;
+	int const W = clk.wprev;
+	std::int64_t const Tp = clk.step - W; // the window's first step
+	if( W == 0 || *v.caught == clk.step - 1 ) return;
+	std::int32_t const k = clk.wseq - 1; // its number
+	std::int64_t const par = ( k & 1 ) * std::int64_t( v.N ), tr = ( k & 3 ) * std::int64_t( v.N );
+	std::int64_t const npre = std::int64_t( v.fl_count[k & 3] ) * v.fparts;
+	std::int64_t const nitems = npre + std::int64_t( v.po_count[k & 3] ) * v.pparts;
+	snn_info const info = info_of( v );
+	int const lane = lane_id();
+	// lane q: the decay of the window's step q
+	float decay = 0.0f;
+	{
+		float sum = clk.psum, c = clk.pc;
+		for( int q = 0; q < W; q++ )
+		{
+			float const dt = v.DT - c;
+			float const t = sum + dt;
+			c = ( t - sum ) - dt;
+			sum = t;
+			if( lane == q ) decay = S::trace_decay( dt );
+		}
+	}
+	auto decay_of = [&]( int q ) { return __builtin_bit_cast( float, __builtin_amdgcn_readlane( __builtin_bit_cast( std::int32_t, decay ), q ) ); };
+	auto backend = [&]( std::int64_t e, int q ) {
+		return make_backend<FIXED>( v, std::uint32_t( e ), std::uint32_t( std::uint64_t( e ) >> 32 ), std::uint32_t( Tp + q ), util::TAG_SYNAPSE_UPDATE );
+	};
+	std::int64_t const wave0 = uniform64( ( blk * blockDim.x + threadIdx.x ) >> 6 );
+	std::int64_t const nwaves = nblk * ( blockDim.x >> 6 );
+	unsigned long long touched = 0, written = 0, words = 0, rows = 0;
+	// one event; counts it, and whether it changed the synapse
+	auto event = [&]( typename S::tuple_t & sy, std::int64_t e, int q, bool pre, bool post, float x, float y ) {
+		typename S::tuple_t const before = sy;
+		auto bak = backend( e, q );
+		S::on_event( reg_iter<typename S::tuple_t>{ sy, std::uint32_t( e ) }, pre, post, x, y, info, bak );
+		touched++;
+		written += same_bits<S>( before, sy ) ? 0 : 1;
+	};
+	for( std::int64_t it = wave0; it < nitems; it += nwaves )
+	{
+		if( it < npre )
+		{
+			std::int64_t const f = it / v.fparts;
+			std::int64_t const p = it - f * v.fparts;
+			std::int32_t const s = uniform( v.fl_id[par + f] );
+			int const a = uniform( v.fl8[par + s] ) - 1;
+			std::int64_t const r0 = v.row_ptr[s];
+			std::int64_t const lo = r0 + v.pl_lo[s], hi = r0 + v.pl_hi[s];
+			std::int64_t const chunk = ( ( hi - lo + v.fparts - 1 ) / v.fparts + 63 ) & ~std::int64_t( 63 );
+			std::int64_t const beg = lo + p * chunk;
+			std::int64_t const end = beg + chunk < hi ? beg + chunk : hi;
+			// lane q: the row's pre trace after step q
+			float xs = 0.0f;
+			{
+				float x = v.xtr[tr + s];
+				for( int q = 0; q < W; q++ )
+				{
+					x = fmaf( x, decay_of( q ), q == a ? 1.0f : 0.0f );
+					if( lane == q ) xs = x;
+				}
+			}
+			for( std::int64_t first = beg; first < end; first += 64 * U )
+			{
+				std::int32_t j[U];
+				bool ok[U];
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					std::int64_t const e = first + lane + 64 * u;
+					ok[u] = e < end;
+					j[u] = v.col[ok[u] ? e : beg];
+				}
+				typename S::tuple_t sy[U];
+				int b[U];
+				float y[U];
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					std::int64_t const e = first + lane + 64 * u;
+					ok[u] = ok[u] && S::plastic( s, j[u], info );
+					load_tuple<S>( sy[u], v.sa, ok[u] ? e : beg );
+					b[u] = int( v.sp8[par + j[u]] ) - 1;
+					y[u] = v.ytr[tr + j[u]];
+				}
+				// the targets' post traces after step a, the row's pre trace after their steps b
+				for( int q = 0; q <= a; q++ )
+				{
+					float const dq = decay_of( q );
+#pragma unroll
+					for( int u = 0; u < U; u++ ) y[u] = fmaf( y[u], dq, q == b[u] ? 1.0f : 0.0f );
+				}
+				float xb[U];
+#pragma unroll
+				for( int u = 0; u < U; u++ ) xb[u] = __builtin_bit_cast( float, shfl_u32( __builtin_bit_cast( std::uint32_t, xs ), b[u] < 0 ? 0 : b[u] ) );
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					if( !ok[u] ) continue;
+					std::int64_t const e = first + lane + 64 * u;
+					typename S::tuple_t const before = sy[u];
+					bool const post = b[u] >= 0;
+					if( post && b[u] < a ) event( sy[u], e, b[u], false, true, xb[u], 0.0f );
+					event( sy[u], e, a, true, b[u] == a, b[u] == a ? xb[u] : 0.0f, y[u] );
+					if( post && b[u] > a ) event( sy[u], e, b[u], false, true, xb[u], 0.0f );
+					store_changed<S>( before, sy[u], v.sa, e );
+				}
+			}
+			if( lane == 0 )
+			{
+				if( end > beg ) words += std::uint64_t( end - beg ); // target ids
+				if( p == 0 ) rows++;
+			}
+		}
+		else
+		{
+			std::int64_t const g = it - npre;
+			std::int64_t const f = g / v.pparts;
+			std::int64_t const p = g - f * v.pparts;
+			std::int32_t const d = uniform( v.po_id[par + f] );
+			int const b = uniform( v.sp8[par + d] ) - 1;
+			std::int64_t const lo = v.tp_ptr[d], hi = v.tp_ptr[d + 1];
+			std::int64_t const chunk = ( ( hi - lo + v.pparts - 1 ) / v.pparts + 63 ) & ~std::int64_t( 63 );
+			std::int64_t const beg = lo + p * chunk;
+			std::int64_t const end = beg + chunk < hi ? beg + chunk : hi;
+			for( std::int64_t first = beg; first < end; first += 64 * U )
+			{
+				tp_entry te[U];
+				bool ok[U];
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					std::int64_t const x = first + lane + 64 * u;
+					ok[u] = x < end;
+					te[u] = v.tp_ent[ok[u] ? x : beg];
+				}
+				// the source's arrival, row start and trace: independent loads, issued together
+				std::int64_t e[U];
+				float xv[U];
+				std::uint8_t a8[U];
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					a8[u] = v.fl8[par + te[u].src];
+					e[u] = v.row_ptr[te[u].src] + te[u].off;
+					xv[u] = v.xtr[tr + te[u].src];
+				}
+				typename S::tuple_t sy[U];
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					ok[u] = ok[u] && a8[u] == 0;
+					if( ok[u] ) load_tuple<S>( sy[u], v.sa, e[u] );
+				}
+				for( int q = 0; q <= b; q++ )
+				{
+					float const dq = decay_of( q );
+#pragma unroll
+					for( int u = 0; u < U; u++ ) xv[u] = fmaf( xv[u], dq, 0.0f ); // (no arrival in the window)
+				}
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					if( !ok[u] ) continue;
+					typename S::tuple_t const before = sy[u];
+					event( sy[u], e[u], b, false, true, xv[u], 0.0f );
+					store_changed<S>( before, sy[u], v.sa, e[u] );
+				}
+			}
+			if( lane == 0 )
+			{
+				if( end > beg ) words += 2 * std::uint64_t( end - beg ); // (source, offset) entries
+				if( p == 0 ) rows++;
+			}
+		}
+	}
+	block_add_stats<4>( v, slot0 + blk, { touched, written, words, rows }, { ST_FLUSH_SYN, ST_FLUSH_WRITTEN, ST_FLUSH_SLOTS, ST_FLUSH_ROWS } );
+}
+
+// The passes on their own (a synchronization before a state export applies those of the last
+// window, which the next window's kernel would otherwise run beside it).
+template <typename Model, bool FIXED>
+__global__ __launch_bounds__( 256 ) void k_window_passes( dview v )
+{
+	window_passes<Model, FIXED>( v, blockIdx.x, gridDim.x, v.ntiles );
+}
+
+// One workgroup per tile, those with incoming synapses first; then (plastic models) the
+// workgroups of the passes of the window before.
 template <typename Model, bool FIXED, int BS>
 __global__ __launch_bounds__( BS ) void k_window( dview v, std::int32_t W )
 {
 	std::int32_t const b = blockIdx.x;
-	window_tile<Model, FIXED, BS>( v, b < v.nact ? xcd_place( b, v.nact ) : b, W );
+	if( b < v.ntiles )
+		window_tile<Model, FIXED, BS>( v, b < v.nact ? xcd_place( b, v.nact ) : b, W );
+	else if constexpr( is_plastic_v<Model> )
+		window_passes<Model, FIXED>( v, b - v.ntiles, std::int32_t( gridDim.x ) - v.ntiles, v.ntiles );
 }
 
 // Appends the spikes of the n steps before the view's step to the net's spike log (one workgroup;
@@ -466,16 +778,28 @@ __device__ inline void log_steps( dview const & v, int n )
 }
 
 // Batched windows: workgroup b < ntiles runs the tile at place tile_pos[b] of net tile_net[b], the
-// rest append net b - ntiles's spikes of the nlog steps before the window to its log.
+// next nplast run passes block pass_local[.] of the pass_count[.] blocks of net pass_net[.], the
+// rest append net b - ntiles - nplast's spikes of the nlog steps before the window to its log.
 template <typename Model, bool FIXED, int BS>
 __global__ __launch_bounds__( BS ) void k_batch_window( dview const * views, std::int32_t const * tile_net, std::int32_t const * tile_pos,
-                                                        std::int32_t ntiles, std::int32_t W, std::int32_t nlog )
+                                                        std::int32_t ntiles, std::int32_t W, std::int32_t nlog, std::int32_t const * pass_net,
+                                                        std::int32_t const * pass_local, std::int32_t const * pass_count, std::int32_t nplast )
 {
 	std::int32_t const b = blockIdx.x;
 	if( b < ntiles )
+	{
 		window_tile<Model, FIXED, BS>( views[tile_net[b]], tile_pos[b], W );
-	else
-		log_steps( views[b - ntiles], nlog );
+		return;
+	}
+	std::int32_t const p = b - ntiles;
+	if constexpr( is_plastic_v<Model> )
+		if( p < nplast )
+		{
+			dview const & v = views[pass_net[p]];
+			window_passes<Model, FIXED>( v, pass_local[p], pass_count[p], v.ntiles );
+			return;
+		}
+	log_steps( views[p - nplast], nlog );
 }
 
 static __global__ __launch_bounds__( 256 ) void k_batch_log( dview const * views, std::int32_t nlog ) { log_steps( views[blockIdx.x], nlog ); }

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
-from spice_amd import Layout, Snn
+from spice_amd import Batch, Layout, Snn
 from tests.helpers import assert_state_equal, brunel_ref_layout, three_pop_layout
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +66,52 @@ def test_fp32_inputs_past_the_tabulated_sums(gpu, delay):
     st = d.stats()
     assert st["spikes"] >= 900 and st["events"] > 64 * 900
     d.close(), h.close()
+
+
+@pytest.mark.parametrize("delay,launch", [(1, (0, 0, 0, 0)), (2, (64, 256, 64, 1)), (3, (128, 512, 64, 7)), (9, (0, 0, 0, 0)), (10, (448, 1024, 1024, 300)),
+                                          (12, (64, 512, 128, 64)), (255, (0, 0, 0, 0))])
+def test_plastic_windows_bit_exact(gpu, delay, launch):
+    """Pair STDP in windows (of up to 10 steps: the refractory promise allows (19 + 1) / 2), the
+    passes of each beside the next: state and every weight against the checker's dense per-step
+    plasticity, at window lengths on both sides of the clock's slots, over history words' ends
+    and the ring of 256 steps, weights exported between windows."""
+    lay = three_pop_layout(900)
+    h = O.CpuSnn("brunel_3pop_stdp", lay, DT, delay, seed=33, fixed_point=True)
+    d = Snn("brunel_3pop_stdp", Layout(*lay), DT, delay, seed=33, fixed_point=True)
+    d.set_launch(tile_w=launch[0], recv_block=launch[1], flush_slots=launch[2], flush_grid=launch[3])
+    for k, n in enumerate((60, 1, 2, 3, 4, 9, 10, 11, 21, 64, 130, 5, 200)):
+        d.run(n)
+        h.run(n)
+        assert_state_equal(d.neurons(), h.neurons(), f"after run {k}")
+        if k % 3 == 0:
+            assert_state_equal(d.synapses(ell=False), h.synapses(ell=False), f"weights after run {k}")
+    assert_state_equal(d.synapses(ell=False), h.synapses(ell=False), "weights")
+    d.close(), h.close()
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_imported_state_that_breaks_the_refractory_promise(gpu, batched):
+    """Neuron state imported in mid-run lets neurons spike and accept input a few steps after a
+    spike; windows rely on 19 refractory steps, so the steps until those spikes have arrived run
+    one by one. Against the checker, weights included."""
+    lay = three_pop_layout(700)
+    h = O.CpuSnn("brunel_3pop_stdp", lay, DT, 15, seed=3, fixed_point=True)
+    if batched:
+        b = Batch("brunel_3pop_stdp", [(Layout(*lay), 15, 3), (Layout(*lay), 15, 4)], DT, fixed_point=True)
+        run, net = b.run, b.net(0)
+    else:
+        net = Snn("brunel_3pop_stdp", Layout(*lay), DT, 15, seed=3, fixed_point=True)
+        run = net.run
+    run(157)
+    h.run(157)
+    for n in (40, 23, 60):
+        s = h.neurons()
+        s["V"] = np.full_like(s["V"], 0.021)
+        s["Twait"] = np.full_like(s["Twait"], 4)
+        net.set_neurons(s)
+        h.set_neurons(s)
+        run(n)
+        h.run(n)
+        assert_state_equal(net.neurons(), h.neurons(), "neurons")
+    assert_state_equal(net.synapses(ell=False), h.synapses(ell=False), "weights")
+    h.close()
