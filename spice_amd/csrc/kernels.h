@@ -1666,22 +1666,7 @@ __global__ __launch_bounds__( 256 ) void k_sync_eager( dview v, std::int64_t now
 	}
 }
 
-// ---- by-target index of the plastic synapses (eager plasticity) ----------------------------
-// Counts every target's incoming plastic synapses; one wave per source row.
-template <typename Model>
-__global__ __launch_bounds__( 256 ) void k_tp_count( dview v, std::uint32_t * cnt )
-{
-	using S = typename Model::synapse;
-	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
-	if( r >= v.N ) return;
-	snn_info const info = info_of( v );
-	for( std::int64_t e = v.row_ptr[r] + lane_id(); e < v.row_ptr[r + 1]; e += 64 )
-	{
-		std::int32_t const j = v.col[e];
-		if( S::plastic( std::int32_t( r ), j, info ) ) atomicAdd( &cnt[j], 1u );
-	}
-}
-
+// ---- by-target index of the plastic synapses (built by the tile kernels of window.h) ----------
 // ptr[0..n] = exclusive prefix sums of cnt[0..n-1]; one workgroup of 1024 threads, each
 // summing a contiguous slice (n is a neuron count: this runs once per network).
 static inline __global__ __launch_bounds__( 1024 ) void k_tp_scan( std::uint32_t const * cnt, std::int64_t * ptr, std::int64_t n )
@@ -1711,28 +1696,6 @@ static inline __global__ __launch_bounds__( 1024 ) void k_tp_scan( std::uint32_t
 	{
 		ptr[i] = run;
 		run += cnt[i];
-	}
-}
-
-// Fills the index: every plastic synapse appends (source, offset in the source's row) to its
-// target's list (cursor: a copy of ptr), in arbitrary order; the host then sorts each list by
-// source.
-template <typename Model>
-__global__ __launch_bounds__( 256 ) void k_tp_fill( dview v, unsigned long long * cursor, tp_entry * ent )
-{
-	using S = typename Model::synapse;
-	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
-	if( r >= v.N ) return;
-	snn_info const info = info_of( v );
-	std::int64_t const r0 = v.row_ptr[r];
-	for( std::int64_t e = r0 + lane_id(); e < v.row_ptr[r + 1]; e += 64 )
-	{
-		std::int32_t const j = v.col[e];
-		if( S::plastic( std::int32_t( r ), j, info ) )
-		{
-			unsigned long long const k = atomicAdd( &cursor[j], 1ull );
-			ent[k] = tp_entry{ std::int32_t( e - r0 ), std::int32_t( r ) };
-		}
 	}
 }
 } // namespace spice::hipx

@@ -15,8 +15,6 @@
 #include <spice/util/numeric.h>
 #include <spice_hip.h>
 
-#include <hipcub/hipcub.hpp>
-
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -712,7 +710,6 @@ private:
 		v.ctl = _ctl.data();
 		v.ctl_next = _ctl.data() + 1;
 
-		if constexpr( traced ) build_by_target();
 		_grid_update = int( ( n + 255 ) / 256 );
 		_upd_block = n >= UPDATE_LARGE_N ? UPDATE_BLOCK_LARGE : SPICE_UPDATE_BLOCK;
 		_grid_upd = int( ( n + _upd_block - 1 ) / _upd_block );
@@ -737,52 +734,27 @@ private:
 		_caught_host = -1;
 	}
 
-	// By-target index of the plastic synapses: count per target, prefix sums, fill.
+	// By-target index of the plastic synapses: count per target, prefix sums, fill (after the
+	// tiles and the rows' plastic flags are known).
 	void build_by_target()
 	{
 		std::int64_t const n = _g.n;
-		unsigned const rows_grid = unsigned( ( n + 3 ) / 4 ); // one wave per row
 		dbuf<std::uint32_t> cnt( n );
-		SPICE_HIP( hipMemsetAsync( cnt.data(), 0, cnt.bytes(), _s ) );
-		SPICE_LAUNCH( k_tp_count<Model><<<rows_grid, 256, 0, _s>>>( _v, cnt.data() ) );
+		SPICE_HIP( hipMemsetAsync( cnt.data(), 0, cnt.bytes(), _s ) ); // (tiles without inputs are not walked)
+		SPICE_LAUNCH( ( k_tp_tile<Model, true><<<unsigned( _v.nact ), TP_BLOCK, 0, _s>>>( _v, cnt.data(), nullptr ) ) );
 		SPICE_LAUNCH( k_tp_scan<<<1, 1024, 0, _s>>>( cnt.data(), _tp_ptr.data(), n ) );
-		std::int64_t total = 0;
-		SPICE_HIP( hipMemcpyAsync( &total, _tp_ptr.data() + n, 8, hipMemcpyDeviceToHost, _s ) );
-		SPICE_HIP( hipStreamSynchronize( _s ) );
-		_tp_total = total;
-		_tp_ent.resize( std::size_t( std::max<std::int64_t>( total, 1 ) ) );
-		_v.tp_ent = _tp_ent.data();
-		if( total > 0 )
-		{
-			dbuf<unsigned long long> cursor( n );
-			SPICE_HIP( hipMemcpyAsync( cursor.data(), _tp_ptr.data(), 8 * n, hipMemcpyDeviceToDevice, _s ) );
-			SPICE_LAUNCH( k_tp_fill<Model><<<rows_grid, 256, 0, _s>>>( _v, cursor.data(), _tp_ent.data() ) );
-			SPICE_HIP( hipStreamSynchronize( _s ) ); // before the temporaries are freed
-		}
-		if( total > 1 && total <= INT_MAX )
-		{
-			// each target's list sorted by source: neighbouring entries of a post-pass wave then
-			// gather neighbouring traces, flags and row starts (fewer cache lines), and the index
-			// does not depend on the order of the fill's atomics. Radix sort on the source bits
-			// of the entries read as 64-bit words (the sort counts items in int: an index of more
-			// than 2^31 entries keeps the fill's order, which is equally correct).
-			int const bits = 64 - __builtin_clzll( static_cast<unsigned long long>( std::max<std::int64_t>( n - 1, 1 ) ) );
-			auto const * keys = reinterpret_cast<unsigned long long const *>( _tp_ent.data() );
-			dbuf<unsigned long long> sorted{ std::size_t( total ) };
-			std::size_t tb = 0;
-			SPICE_HIP( hipcub::DeviceSegmentedRadixSort::SortKeys( nullptr, tb, keys, sorted.data(), int( total ), int( n ), _tp_ptr.data(),
-			                                                       _tp_ptr.data() + 1, 32, 32 + bits, _s ) );
-			dbuf<char> temp( std::max<std::size_t>( tb, 1 ) );
-			SPICE_HIP( hipcub::DeviceSegmentedRadixSort::SortKeys( temp.data(), tb, keys, sorted.data(), int( total ), int( n ), _tp_ptr.data(),
-			                                                       _tp_ptr.data() + 1, 32, 32 + bits, _s ) );
-			SPICE_HIP( hipMemcpyAsync( _tp_ent.data(), sorted.data(), std::size_t( total ) * 8, hipMemcpyDeviceToDevice, _s ) );
-			SPICE_HIP( hipStreamSynchronize( _s ) ); // before the temporaries are freed
-		}
-		// targets with incoming plastic synapses (the mean in-degree sets the post-pass split)
 		std::vector<std::int64_t> ptr( n + 1 );
-		SPICE_HIP( hipMemcpy( ptr.data(), _tp_ptr.data(), ptr.size() * 8, hipMemcpyDeviceToHost ) );
+		SPICE_HIP( hipMemcpyAsync( ptr.data(), _tp_ptr.data(), ptr.size() * 8, hipMemcpyDeviceToHost, _s ) );
+		SPICE_HIP( hipStreamSynchronize( _s ) );
+		_tp_total = ptr[n];
+		_tp_ent.resize( std::size_t( std::max<std::int64_t>( _tp_total, 1 ) ) );
+		_v.tp_ent = _tp_ent.data();
+		if( _tp_total > 0 ) SPICE_LAUNCH( ( k_tp_tile<Model, false><<<unsigned( _v.nact ), TP_BLOCK, 0, _s>>>( _v, nullptr, _tp_ent.data() ) ) );
+		// targets with incoming plastic synapses (the mean in-degree sets the post-pass split)
 		_tp_targets = 0;
 		for( std::int64_t i = 0; i < n; i++ ) _tp_targets += ptr[i + 1] > ptr[i];
+		SPICE_HIP( hipStreamSynchronize( _s ) );
+		apply_launch( _lc ); // the views, and the post pass's split
 	}
 
 	// Launch shapes (zero fields: the defaults). tile_w: targets per delivery tile (the
@@ -923,7 +895,6 @@ private:
 	void choose_window()
 	{
 		_window = 0;
-		if constexpr( windowed )
 		{
 			// lanes per segment: the power of two whose reads hold a segment two standard deviations
 			// longer than the mean, so that few take a second round (Vogels 1e9, delay 8, 17.9
@@ -931,6 +902,9 @@ private:
 			double const mean = _g.n > 0 ? double( _g.nnz ) / double( _g.n ) / _v.nact : 0.0;
 			_v.wlanes = 0;
 			while( _v.wlanes < 5 && double( WIN_VEC << _v.wlanes ) < mean + 2.0 * std::sqrt( mean ) ) _v.wlanes++;
+		}
+		if constexpr( windowed )
+		{
 			if( !plastic && !_ahead && ( _lc.recv_parts != 1 || _lc.tile_w > 4 * _lc.recv_block ) ) return;
 			_window = 1;
 			with_window_kernel( [&]( auto kernel, auto bytes, int ) {
@@ -952,6 +926,7 @@ private:
 		if constexpr( plastic )
 		{
 			SPICE_LAUNCH( k_init_synapses<Model><<<unsigned( ( _g.n + 3 ) / 4 ), 256, 0, _s>>>( _v ) );
+			if constexpr( traced ) build_by_target();
 		}
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 	}
