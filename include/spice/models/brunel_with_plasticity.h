@@ -65,11 +65,27 @@ struct brunel_with_plasticity : model
 			return false;
 		}
 
+		// receive() = accepts() ? deliver() : nothing (split so that the GPU may test the gate
+		// in the neuron update)
+		static constexpr bool gated_receive = true;
+
+		template <typename Iter>
+		HYBRID static bool accepts( Iter n )
+		{
+			return util::get<Twait>( n ) <= 0;
+		}
+
 		template <typename Iter, typename SynIter, typename Backend>
-		HYBRID static void receive( int_, Iter dst, SynIter && syn, snn_info info, Backend & bak )
+		HYBRID static void deliver( int_, Iter dst, SynIter && syn, snn_info info, Backend & bak )
 		{
 			using util::get;
-			if( get<Twait>( dst ) <= 0 ) bak.atomic_add( get<V>( dst ), get<W>( syn ) * 20'000 / info.num_neurons );
+			bak.atomic_add( get<V>( dst ), get<W>( syn ) * 20'000 / info.num_neurons );
+		}
+
+		template <typename Iter, typename SynIter, typename Backend>
+		HYBRID static void receive( int_ src, Iter dst, SynIter && syn, snn_info info, Backend & bak )
+		{
+			if( accepts( dst ) ) deliver( src, dst, syn, info, bak );
 		}
 	};
 
@@ -85,24 +101,51 @@ struct brunel_with_plasticity : model
 			get<Zpost>( syn ) = 1.0f;
 		}
 
+		// update(): the traces first, then the weight
+		static constexpr int pre_trace = Zpre, post_trace = Zpost;
+		static constexpr float trace_init = 1.0f;
+		// after a spike at t, Twait = 20 closes a LIF neuron's gate for the inputs of t + 1 .. t + 20
+		// and its next spike comes at t + 20 at the earliest
+		static constexpr int refractory_steps = 19;
+
+		HYBRID static bool refractory( int_ neuron, snn_info info ) { return neuron >= info.num_neurons / 2; }
+
+		HYBRID static float trace_decay( float dt )
+		{
+			float const TstdpInv = 1.0f / 0.02f;
+			return 1 - dt * TstdpInv;
+		}
+
+		// exp(-z) is 0 in single precision for every z > 104
+		HYBRID static bool inert( bool const pre, bool const post, float const a, float const b, float const dt )
+		{
+			float const dtInv = 1.0f / dt;
+			return ( !post || a * dtInv > 110.0f ) && ( !pre || b * dtInv > 110.0f );
+		}
+
 		template <typename Iter, typename Backend>
-		HYBRID static void update(
-		    Iter && syn, int_ const nsteps, bool const pre, bool const post, float const dt, snn_info, Backend & bak )
+		HYBRID static void on_event( Iter && syn, bool const pre, bool const post, float const dt, snn_info, Backend & bak )
 		{
 			using util::get;
-			float const TstdpInv = 1.0f / 0.02f;
 			float const dtInv = 1.0f / dt;
-			float const decay = bak.pow( 1 - dt * TstdpInv, nsteps );
-
-			get<Zpre>( syn ) = bak.fma( get<Zpre>( syn ), decay, pre );
-			get<Zpost>( syn ) = bak.fma( get<Zpost>( syn ), decay, post );
-
 			float const w = get<W>( syn );
 			get<W>( syn ) = bak.clamp(
 			    w - pre * 0.0202f * w * bak.exp( -get<Zpost>( syn ) * dtInv ) +
 			        post * 0.01f * ( 1.0f - w ) * bak.exp( -get<Zpre>( syn ) * dtInv ),
 			    0.0f,
 			    0.0003f );
+		}
+
+		template <typename Iter, typename Backend>
+		HYBRID static void update(
+		    Iter && syn, int_ const nsteps, bool const pre, bool const post, float const dt, snn_info info, Backend & bak )
+		{
+			using util::get;
+			float const decay = bak.pow( trace_decay( dt ), nsteps );
+
+			get<Zpre>( syn ) = bak.fma( get<Zpre>( syn ), decay, pre );
+			get<Zpost>( syn ) = bak.fma( get<Zpost>( syn ), decay, post );
+			on_event( syn, pre, post, dt, info, bak );
 		}
 
 		HYBRID static bool plastic( int_ const src, int_ const dst, snn_info const info )

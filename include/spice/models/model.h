@@ -44,6 +44,26 @@
 //     static constexpr std::uint32_t receive_reads = 0;
 // (receive() reads nothing of its target) allows the same without a gate.
 //
+// Optional factored traces of a per-synapse type (synapse<...>): where update() advances two trace
+// attributes by the flags alone and changes the others at events only, the traces of all plastic
+// synapses of a source (and of a target) are the same, and a synapse type may declare
+//     static constexpr int pre_trace = A, post_trace = B;   the trace attributes
+//     static constexpr float trace_init = z;                what init() gives them, everywhere
+//     static constexpr int refractory_steps = R;            the promise below, for the neurons with
+//     static bool refractory( int_ neuron, snn_info );      this set
+//     static float trace_decay( dt );
+//     static void on_event( syn, pre, post, dt, info, backend );
+// with update( n, pre, post ) == { A <- fma( A, trace_decay( dt )^n, pre ); B <- fma( B, ..., post );
+// on_event( pre, post ) }, where on_event reads A only if post is set and B only if pre is set, changes
+// neither, and changes nothing when neither is set. The GPU then keeps the traces per neuron and
+// applies on_event at events, if every plastic synapse joins neurons with refractory() set (imported
+// synapse state that is not of this form goes back to the per-synapse contract).
+//
+// Such a type may also declare
+//     static bool inert( bool pre, bool post, float a, float b, float dt );
+// set if on_event surely leaves every synapse as it is whose state an event-free step does (a, b: its
+// traces; a is given where post is set, b where pre is): the GPU then does not read the synapse.
+//
 // Optional input classes, for models without per-synapse state: a neuron type whose inputs take
 // one of a few values, chosen by the source, may declare
 //     static constexpr int input_classes = K;
@@ -55,7 +75,7 @@
 // inputs of each class and form their sum from the counts (in fp32: the same additions, class by
 // class).
 //
-// Optional trait of a neuron-trace synapse (trace_synapse below):
+// Optional trait of a neuron-trace synapse (trace_synapse below), or of factored traces:
 //     static constexpr int refractory_steps = R;
 // promises that a neuron that is an endpoint of a plastic synapse and spikes at step t neither
 // spikes nor accepts input at steps t + 1 .. t + R. With R >= 2 a plastic synapse's events of
@@ -145,6 +165,37 @@ struct has_neuron_traces<S, std::void_t<decltype( S::neuron_traces )>> : std::bo
 {
 };
 } // namespace detail
+
+namespace detail
+{
+template <typename S, typename = void>
+struct has_factored_traces : std::false_type
+{
+};
+template <typename S>
+struct has_factored_traces<S, std::void_t<decltype( S::pre_trace )>> : std::true_type
+{
+};
+} // namespace detail
+
+namespace detail
+{
+template <typename S, typename = void>
+struct has_inert : std::false_type
+{
+};
+template <typename S>
+struct has_inert<S, std::void_t<decltype( S::inert( false, false, 0.0f, 0.0f, 0.0f ) )>> : std::true_type
+{
+};
+} // namespace detail
+
+template <typename Synapse>
+inline constexpr bool has_inert_v = detail::has_inert<Synapse>::value;
+
+// True for per-synapse types that declare factored traces.
+template <typename Synapse>
+inline constexpr bool has_factored_traces_v = detail::has_factored_traces<Synapse>::value;
 
 // True for synapse types derived from trace_synapse<...>.
 template <typename Synapse>

@@ -57,6 +57,21 @@ public:
 				n->set_launch( c );
 			}
 		}
+		build();
+	}
+
+	// Device tables of the nets' workgroups and views. Windows, unless a net's plasticity went back
+	// to the per-synapse contract (hip_net::make_lazy): then every net's does, and steps are two
+	// kernels.
+	void build()
+	{
+		_windows = windowed;
+		if constexpr( factored_v<Model> )
+		{
+			for( auto * n : _nets ) _windows = _windows && !n->lazy();
+			if( !_windows )
+				for( auto * n : _nets ) n->make_lazy();
+		}
 		std::vector<std::int32_t> tn, tl, bn, bl, fn, fl, fc;
 		std::vector<dview> vs[CLOCK_SLOTS];
 		for( std::size_t k = 0; k < _nets.size(); k++ )
@@ -64,12 +79,12 @@ public:
 			hip_net<Model> & n = *_nets[k];
 			// windows: one workgroup per tile; two-kernel steps: (tile, part) work items of the tiles
 			// with incoming synapses
-			for( int t = 0; t < ( windowed ? n.num_all_tiles() : n.num_tiles() * n.num_receive_parts() ); t++ )
+			for( int t = 0; t < ( _windows ? n.num_all_tiles() : n.num_tiles() * n.num_receive_parts() ); t++ )
 			{
 				tn.push_back( std::int32_t( k ) );
 				tl.push_back( t );
 			}
-			if constexpr( !windowed )
+			if( !_windows )
 				for( int b = 0; b < n.num_update_blocks(); b++ )
 				{
 					bn.push_back( std::int32_t( k ) );
@@ -85,12 +100,14 @@ public:
 					fc.push_back( nf );
 				}
 			}
-			// batch step t runs net step host_step + t: clock slot (host_step + t) mod 4
-			for( int p = 0; p < CLOCK_SLOTS; p++ ) vs[p].push_back( n.view( int( ( n.host_step() + p ) & ( CLOCK_SLOTS - 1 ) ) ) );
+			// batch step t runs net step host_step + (t - _step): the clock slot of that
+			for( int p = 0; p < CLOCK_SLOTS; p++ ) vs[( _step + p ) & ( CLOCK_SLOTS - 1 )].push_back( n.view( int( ( n.host_step() + p ) & ( CLOCK_SLOTS - 1 ) ) ) );
 		}
 		_ntiles = std::int32_t( tn.size() );
 		_nblocks = std::int32_t( bn.size() );
 		_nflush = std::int32_t( fn.size() );
+		_window = 0;
+		_graphs.clear();
 		if constexpr( windowed )
 		{
 			// the longest window that suits every net and whose LDS leaves room for four workgroups
@@ -106,6 +123,7 @@ public:
 			auto bytes = [&]( int w ) { return _fixed ? window_lds<Model, true>::bytes( window_block, widest, w ) : window_lds<Model, false>::bytes( window_block, widest, w ); };
 			while( _window > 1 && bytes( _window ) > LDS_PER_CU / 4 ) _window = window_steps( _window - 1 );
 			_lds = bytes( _window );
+			if( !_windows ) _window = 0;
 			if( _lds > ( 64 << 10 ) )
 				SPICE_HIP( hipFuncSetAttribute( _fixed ? reinterpret_cast<void const *>( &k_batch_window<Model, true, window_block> )
 				                                       : reinterpret_cast<void const *>( &k_batch_window<Model, false, window_block> ),
@@ -130,12 +148,12 @@ public:
 	// batch of a few nets keeps its nets' own tiles. Fixed-point results do not depend on the tile
 	// width (fp32 sums are reordered, as by any launch shape); a net keeps wider tiles it already
 	// has (of up to TILE_MAX, what the batched kernels hold), and keeps the new width afterwards.
-	// Plastic models: about max(64, 64 x CUs / nets) tiles per net (on a sweep of two 256-net
+	// Two-kernel steps: about max(64, 64 x CUs / nets) tiles per net (on a sweep of two 256-net
 	// batches 64 tiles per net beat 16, 32, 128 and 256).
 	static int batch_tile_w( std::int64_t n, int tile_w, std::int64_t nnets )
 	{
-		std::int64_t const tiles = plastic ? std::max<std::int64_t>( 64, std::int64_t( SPICE_BATCH_ITEMS_PER_CU ) * device_cu_count() / nnets )
-		                                   : std::max<std::int64_t>( 1, window_tiles_per_cu * device_cu_count() / nnets );
+		std::int64_t const tiles = windowed ? std::max<std::int64_t>( 1, window_tiles_per_cu * device_cu_count() / nnets )
+		                                    : std::max<std::int64_t>( 64, std::int64_t( SPICE_BATCH_ITEMS_PER_CU ) * device_cu_count() / nnets );
 		int const tw = int( std::clamp<std::int64_t>( ( n / tiles + 63 ) / 64 * 64, 64, TILE_MAX ) );
 		return std::min( std::max( tw, tile_w ), TILE_MAX );
 	}
@@ -152,13 +170,28 @@ public:
 	{
 		if( n < 0 ) throw std::invalid_argument( "negative step count" );
 		if( n == 0 ) return;
+		if constexpr( factored_v<Model> )
+		{
+			bool lazy = false;
+			for( auto * net : _nets ) lazy = lazy || net->lazy();
+			if( lazy && _windows )
+			{
+				synchronize();
+				build();
+			}
+		}
+		// (state imported into a net may ask for a few steps one by one)
+		std::int64_t single = 0;
+		for( auto * net : _nets ) single = std::max( single, net->single_steps_left() );
+		single = std::min( single, n );
+		if( single ) launch_windows( _step, single, 1, true );
+		_step += single;
+		for( auto * net : _nets ) net->advance_host( single );
+		n -= single;
+		if( n == 0 ) return;
 		if( _window > 1 )
 		{
-			std::int64_t single = 0; // (state imported into a net may ask for a few steps one by one)
-			for( auto * net : _nets ) single = std::max( single, net->single_steps_left() );
-			single = std::min( single, n );
-			launch_windows( _step, single, 1 );
-			launch_windows( _step + single, n - single, _window );
+			launch_windows( _step, n, _window );
 			_step += n;
 			for( auto * net : _nets ) net->advance_host( n );
 			return;
@@ -193,6 +226,7 @@ private:
 	bool _own_stream = false;
 	step_graphs _graphs;
 	bool _fixed = false;
+	bool _windows = false; // steps run as windows
 	// windows of up to _window steps (0: two-kernel steps)
 	static constexpr int window_block = 256;
 	// tiles of all nets, per CU: 48 nets of 1e4 to 1e7 synapses take, at 4 / 8 / 16 / 64, 2.6 / 1.8 /
@@ -218,18 +252,20 @@ private:
 	}
 
 	// n steps from batch step t in windows of up to `most`; each appends its predecessor's spikes
-	// to the nets' logs, and a last kernel the last one's.
-	void launch_windows( std::int64_t t, std::int64_t n, int most )
+	// to the nets' logs, and a last kernel the last one's. alone: the passes before each in kernels
+	// of their own.
+	void launch_windows( std::int64_t t, std::int64_t n, int most, bool alone = false )
 	{
-		if( n == 0 ) return;
 		int before = 0;
 		while( n > 0 )
 		{
 			int const w = window_steps( std::min<std::int64_t>( n, most ) );
+			if( alone )
+				for( auto * net : _nets ) net->launch_passes( net->host_step() + ( t - _step ), _s );
 			if( _fixed )
-				launch_window_t<true>( t, w, before );
+				launch_window_t<true>( t, w, before, alone );
 			else
-				launch_window_t<false>( t, w, before );
+				launch_window_t<false>( t, w, before, alone );
 			if( _window > 1 ) _queue.launched( _s );
 			before = w;
 			t += w;
@@ -239,39 +275,44 @@ private:
 	}
 
 	template <bool F>
-	void launch_window_t( std::int64_t t, int w, int before )
+	void launch_window_t( std::int64_t t, int w, int before, bool alone )
 	{
-		unsigned const grid = unsigned( _ntiles + _nflush ) + ( _logged && before ? unsigned( _nets.size() ) : 0u );
+		std::int32_t const nplast = alone ? 0 : _nflush;
+		unsigned const grid = unsigned( _ntiles + nplast ) + ( _logged && before ? unsigned( _nets.size() ) : 0u );
 		if constexpr( windowed )
 			SPICE_LAUNCH( ( k_batch_window<Model, F, window_block><<<grid, window_block, _lds, _s>>>(
 			    _views[t & ( CLOCK_SLOTS - 1 )].data(), _tile_net.data(), _tile_local.data(), _ntiles, w, before, _flush_net.data(),
-			    _flush_local.data(), _flush_count.data(), _nflush ) ) );
+			    _flush_local.data(), _flush_count.data(), nplast ) ) );
 	}
 
 	// Same schedules as hip_net::launch_steps: windows of one step, or two kernels per step
 	// (delivery with step t - 1's plasticity, update).
 	void launch_steps( std::int64_t t, std::int64_t len )
 	{
-		if constexpr( windowed )
+		if( _windows )
+		{
 			launch_windows( t, len, 1 );
-		else
-			for( std::int64_t k = 0; k < len; k++ )
-				if( _fixed )
-					launch_step_t<true>( t + k );
-				else
-					launch_step_t<false>( t + k );
+			return;
+		}
+		for( std::int64_t k = 0; k < len; k++ )
+			if( _fixed )
+				launch_step_t<true>( t + k );
+			else
+				launch_step_t<false>( t + k );
 	}
 
 	template <bool F>
 	void launch_step_t( std::int64_t t )
 	{
-		dview const * v = _views[t & ( CLOCK_SLOTS - 1 )].data();
-		unsigned const grid = unsigned( _grid_tiles + ( plastic ? _nflush : 0 ) );
-		SPICE_LAUNCH( k_batch_receive<Model, F, recv_block><<<grid, recv_block, 0, _s>>>( v, _tile_net.data(), _tile_local.data(), _ntiles, _grid_tiles,
-		                                                                                    _flush_net.data(), _flush_local.data(), _flush_count.data() ) );
-		SPICE_LAUNCH( k_batch_update<Model, F><<<_nblocks, 256, 0, _s>>>( v, _block_net.data(), _block_local.data() ) );
+		if constexpr( !windowed || factored_v<Model> )
+		{
+			dview const * v = _views[t & ( CLOCK_SLOTS - 1 )].data();
+			unsigned const grid = unsigned( _grid_tiles + ( plastic ? _nflush : 0 ) );
+			SPICE_LAUNCH( k_batch_receive<Model, F, recv_block><<<grid, recv_block, 0, _s>>>( v, _tile_net.data(), _tile_local.data(), _ntiles, _grid_tiles,
+			                                                                                    _flush_net.data(), _flush_local.data(), _flush_count.data() ) );
+			SPICE_LAUNCH( k_batch_update<Model, F><<<_nblocks, 256, 0, _s>>>( v, _block_net.data(), _block_local.data() ) );
+		}
 	}
-
 };
 
 // Builds the nets of a batch (each gets its own stream for setup) and the batch, which owns
@@ -288,7 +329,7 @@ batch_iface * make_batch( std::vector<net_params> const & ps, std::vector<csr_de
 		try
 		{
 			launch_cfg first; // at the width that the batch will want
-			first.tile_w = hip_batch<Model>::batch_tile_w( gs[k].n, default_tile_w<Model>( gs[k].n, ps[k].delay, device_cu_count() ), std::int64_t( ps.size() ) );
+			first.tile_w = hip_batch<Model>::batch_tile_w( gs[k].n, default_tile_w<Model>( gs[k].n, gs[k].targets, ps[k].delay, device_cu_count() ), std::int64_t( ps.size() ) );
 			nets.emplace_back( new hip_net<Model>( ps[k], std::move( gs[k] ), ns, first ) );
 		}
 		catch( ... )

@@ -645,7 +645,7 @@ static job_spec job_spec_of( spice_job_desc const & j )
 
 static std::uint64_t job_estimate( job_spec const & s, std::int64_t chunk )
 {
-	return estimate_job_bytes( s.p.model, s.n, s.width, s.p.delay, ( s.p.flags & SPICE_FLAG_FIXED_POINT ) != 0, chunk, s.p.dt );
+	return estimate_job_bytes( s.p.model, s.n, s.width, target_range( s.conns ), s.p.delay, ( s.p.flags & SPICE_FLAG_FIXED_POINT ) != 0, chunk, s.p.dt );
 }
 
 static serve::scheduler<hip_exec> & sched_of( spice_server * sv )

@@ -15,7 +15,21 @@ struct csr_dev
 	dbuf<std::int64_t> row_ptr; // N + 1
 	dbuf<std::int32_t> col;     // E (+ COL_PAD, so that a 16-byte read of the last entries stays inside)
 	std::int64_t n = 0, nnz = 0, width = 0;
+	std::int64_t targets = 0; // neurons between the first and the last one that a row may target
 };
+
+// csr_dev::targets of a generated graph.
+inline std::int64_t target_range( std::vector<util::gen::conn> const & conns )
+{
+	std::int64_t first = INT64_MAX, last = 0;
+	for( auto const & c : conns )
+		if( c.mean > 0.0 && c.src_last > c.src_first && c.dst_last > c.dst_first )
+		{
+			first = c.dst_first < first ? c.dst_first : first;
+			last = c.dst_last > last ? c.dst_last : last;
+		}
+	return last > first ? last - first : 0;
+}
 
 // Builds the CSR adjacency for the flattened connections on the device:
 // degrees (one thread per row) -> exclusive scan -> targets (one wave per row).

@@ -187,6 +187,7 @@ csr_dev generate_csr( std::vector<conn> const & conns, std::int64_t n, std::int6
 	csr_dev g;
 	g.n = n;
 	g.width = width;
+	g.targets = target_range( conns );
 	g.row_ptr.resize( n + 1 );
 	dbuf<conn> dconns( conns.size() > 0 ? conns.size() : 1 );
 	if( !conns.empty() )
@@ -257,6 +258,14 @@ csr_dev upload_csr( std::int64_t const * row_ptr, std::int32_t const * col, std:
 	g.n = n;
 	g.width = width;
 	g.nnz = row_ptr[n];
+	std::int64_t first = n, last = -1; // (rows are sorted by target)
+	for( std::int64_t r = 0; r < n; r++ )
+		if( row_ptr[r + 1] > row_ptr[r] )
+		{
+			first = col[row_ptr[r]] < first ? col[row_ptr[r]] : first;
+			last = col[row_ptr[r + 1] - 1] > last ? col[row_ptr[r + 1] - 1] : last;
+		}
+	g.targets = last >= first ? last - first + 1 : 0;
 	g.row_ptr.resize( n + 1 );
 	g.col.resize( g.nnz + COL_PAD );
 	SPICE_HIP( hipMemcpyAsync( g.row_ptr.data(), row_ptr, ( n + 1 ) * sizeof( std::int64_t ), hipMemcpyHostToDevice, s ) );

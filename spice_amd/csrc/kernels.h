@@ -274,7 +274,37 @@ __device__ inline bool store_changed( typename Decl::tuple_t const & before, typ
 	return any;
 }
 
-// Whether two synapse states are the same, bit for bit.
+// Attribute I of a synapse type is a factored trace (kept per neuron, not per synapse).
+template <typename S>
+constexpr bool is_factored_attr( int I )
+{
+	if constexpr( has_factored_traces_v<S> )
+		return I == S::pre_trace || I == S::post_trace;
+	else
+		return false;
+}
+
+// load_tuple / store_changed of the attributes kept per synapse.
+template <typename S>
+__device__ inline void load_synapse( typename S::tuple_t & s, void * const * arr, std::int64_t i )
+{
+	util::for_n<S::size>( [&]( auto I ) {
+		using T = typename S::template type<I>;
+		if constexpr( !is_factored_attr<S>( int( I ) ) ) std::get<I>( s ) = ld<T>( arr[I], i );
+	} );
+}
+template <typename S>
+__device__ inline void store_synapse( typename S::tuple_t const & before, typename S::tuple_t const & after, void * const * arr, std::int64_t i )
+{
+	util::for_n<S::size>( [&]( auto I ) {
+		using T = typename S::template type<I>;
+		using B = std::conditional_t<sizeof( T ) == 8, std::uint64_t, std::uint32_t>;
+		if constexpr( !is_factored_attr<S>( int( I ) ) )
+			if( __builtin_bit_cast( B, std::get<I>( after ) ) != __builtin_bit_cast( B, std::get<I>( before ) ) ) st<T>( arr[I], i, std::get<I>( after ) );
+	} );
+}
+
+// Whether two synapse states are the same, bit for bit (attributes kept per synapse).
 template <typename Decl>
 __device__ inline bool same_bits( typename Decl::tuple_t const & a, typename Decl::tuple_t const & b )
 {
@@ -282,7 +312,7 @@ __device__ inline bool same_bits( typename Decl::tuple_t const & a, typename Dec
 	util::for_n<Decl::size>( [&]( auto I ) {
 		using T = typename Decl::template type<I>;
 		using B = std::conditional_t<sizeof( T ) == 8, std::uint64_t, std::uint32_t>;
-		same = same && __builtin_bit_cast( B, std::get<I>( a ) ) == __builtin_bit_cast( B, std::get<I>( b ) );
+		if constexpr( !is_factored_attr<Decl>( int( I ) ) ) same = same && __builtin_bit_cast( B, std::get<I>( a ) ) == __builtin_bit_cast( B, std::get<I>( b ) );
 	} );
 	return same;
 }
@@ -395,13 +425,22 @@ template <typename Model>
 inline constexpr bool eager_nodefer_v =
     is_plastic_v<Model> && has_neuron_traces_v<typename Model::synapse> && refractory_steps_v<typename Model::synapse> >= 2;
 
+// Per-synapse types with factored traces (model.h): run as neuron-trace synapses, in windows,
+// unless a net's layout or imported state is not of that form (hip_net::make_lazy).
+template <typename Model>
+inline constexpr bool factored_v = is_plastic_v<Model> && has_factored_traces_v<typename Model::synapse> && refractory_steps_v<typename Model::synapse> >= 2;
+
+// Plastic models whose steps run as windows.
+template <typename Model>
+inline constexpr bool windowed_plastic_v = eager_nodefer_v<Model> || factored_v<Model>;
+
 // The delivery of a step may run before the update of the steps before it (given a delay of at
 // least 2 steps): it reads nothing that those updates write -- no target state (receive() split
 // into a gate the update tests, or declared to read nothing) and, for plastic models, no weight
 // whose pending events matter.
 template <typename Model>
 inline constexpr bool overlap_capable_v =
-    input_ahead_of_update_v<typename Model::neuron> && ( !is_plastic_v<Model> || eager_nodefer_v<Model> );
+    input_ahead_of_update_v<typename Model::neuron> && ( !is_plastic_v<Model> || windowed_plastic_v<Model> );
 
 // ---- kernels -------------------------------------------------------------------------------
 
@@ -417,9 +456,11 @@ __global__ __launch_bounds__( 256 ) void k_init_neurons( dview v )
 	store_tuple<N>( s, v.na, i );
 }
 
-// One wave per source row: synapse init + "row has a plastic synapse" flag.
+// One wave per source row: synapse init (of the attributes that are kept per synapse: sa[I] is not
+// null) + "row has a plastic synapse" flag. *broken (factored traces) is set if a plastic synapse
+// joins a neuron that does not keep the refractory promise.
 template <typename Model>
-__global__ __launch_bounds__( 256 ) void k_init_synapses( dview v )
+__global__ __launch_bounds__( 256 ) void k_init_synapses( dview v, std::int32_t * broken )
 {
 	using S = typename Model::synapse;
 	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
@@ -434,9 +475,14 @@ __global__ __launch_bounds__( 256 ) void k_init_synapses( dview v )
 		auto bak = make_backend<false>(
 		    v, std::uint32_t( e ), std::uint32_t( std::uint64_t( e ) >> 32 ), 0u, util::TAG_SYNAPSE_INIT );
 		S::init( reg_iter<typename S::tuple_t>{ s, std::uint32_t( e ) }, int_( r ), j, info, bak );
-		store_tuple<S>( s, v.sa, e );
+		util::for_n<S::size>( [&]( auto I ) {
+			using T = typename S::template type<I>;
+			if( v.sa[I] ) st<T>( v.sa[I], e, std::get<I>( s ) );
+		} );
 		if( S::plastic( int_( r ), j, info ) )
 		{
+			if constexpr( factored_v<Model> )
+				if( !S::refractory( int_( r ), info ) || !S::refractory( j, info ) ) *broken = 1;
 			first = e < first ? e : first;
 			last = e;
 		}

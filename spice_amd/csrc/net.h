@@ -119,12 +119,14 @@ int ring_entries( int delay )
 // every tile stages all of the window's arrivals and a wider one does it less often (synth 1e9:
 // 29 us per step with 251 tiles of 3,200, 50 with 391 of 2,048), but none wider than its kernel
 // takes; windows of several steps, whose accumulators take LDS per step, two per CU beyond that.
-// Two-kernel plastic steps: about two tiles per CU, of 256 at least.
+// targets: the neurons that have inputs (csr_dev::targets; the other tiles cost little). Two-kernel
+// plastic steps: about two tiles per CU, of 256 at least.
+inline int lazy_tile_w( std::int64_t n, int cus ) { return int( std::clamp<std::int64_t>( ( ( n + 2 * cus - 1 ) / ( 2 * cus ) + 63 ) / 64 * 64, 256, TILE_MAX ) ); }
 template <typename Model>
-int default_tile_w( std::int64_t n, int delay, int cus )
+int default_tile_w( std::int64_t n, std::int64_t targets, int delay, int cus )
 {
-	auto const per = [&]( std::int64_t tiles ) { return ( ( n + tiles - 1 ) / tiles + 63 ) / 64 * 64; };
-	if( !windowed_v<Model> ) return int( std::clamp<std::int64_t>( per( 2 * cus ), 256, TILE_MAX ) );
+	auto const per = [&]( std::int64_t tiles ) { return ( ( targets + tiles - 1 ) / tiles + 63 ) / 64 * 64; };
+	if( !windowed_v<Model> ) return lazy_tile_w( n, cus );
 	bool const ahead = overlap_capable_v<Model> && delay >= 2;
 	std::int64_t const most = ahead || is_plastic_v<Model> ? TILE_MAX : 4 * 1024;
 	return int( std::clamp<std::int64_t>( per( ahead && per( cus ) > most ? 2 * cus : cus ), 64, most ) );
@@ -138,6 +140,8 @@ class hip_net final : public net_iface
 	static constexpr bool plastic = is_plastic_v<Model>;
 	static constexpr bool traced = plastic && has_neuron_traces_v<S>;
 	static constexpr bool windowed = windowed_v<Model>; // steps run as windows (static models: at most launch shapes)
+	static constexpr bool factored = factored_v<Model>; // factored traces (a net may go back to the per-synapse contract)
+	static constexpr bool eager = traced || factored;   // traces kept per neuron
 
 public:
 	// first: launch shapes to start with (zero fields: the defaults)
@@ -145,6 +149,7 @@ public:
 	    : _p( p )
 	    , _g( std::move( g ) )
 	    , _s( stream )
+	    , _lazy( plastic && !eager )
 	{
 		if( !( p.dt > 0.0f ) ) throw std::invalid_argument( "dt must be positive" );
 		if( p.flags & ~std::uint32_t( SPICE_FLAG_FIXED_POINT ) ) throw std::invalid_argument( "unknown flags" );
@@ -170,7 +175,10 @@ public:
 	void step( std::int32_t ** dspk, std::uint32_t ** dcnt ) override
 	{
 		std::int64_t const t = _step;
-		launch_steps( t, 1 );
+		if( t < _single_until )
+			launch_window( t, 1, nullptr, nullptr, true );
+		else
+			launch_steps( t, 1 );
 		tick();
 		int const slot = int( t % _v.rsize );
 		if( dspk ) *dspk = _ring.data() + std::int64_t( slot ) * _g.n;
@@ -181,13 +189,20 @@ public:
 	void run( std::int64_t n ) override
 	{
 		if( n < 0 ) throw std::invalid_argument( "negative step count" );
+		while( n > 0 && _step < _single_until )
+		{
+			launch_window( _step, 1, nullptr, nullptr, true );
+			_queue.launched( _s );
+			tick();
+			n--;
+		}
 		if( n == 0 ) return;
 		if( _window > 1 )
 		{
 			// windows are long enough to be launched one by one (a launch costs the host a few us)
 			while( n > 0 )
 			{
-				int const w = window_steps( std::min<std::int64_t>( n, window_now() ) );
+				int const w = window_steps( std::min<std::int64_t>( n, _window ) );
 				launch_window( _step, w, nullptr, nullptr );
 				_queue.launched( _s );
 				for( int i = 0; i < w; i++ ) tick();
@@ -253,6 +268,14 @@ public:
 	void set_clock( std::int64_t step, float sum, float c ) override
 	{
 		if( step < 0 || step > INT_MAX - 2 ) throw std::invalid_argument( "invalid step index" );
+		if( factored && !_lazy )
+		{
+			// (the traces are synapse state: kept, as windows number them from 0 again)
+			sync_synapses();
+			std::int64_t const from = trace_slot() * _g.n;
+			if( from )
+				for( auto * b : { &_xtr, &_ytr } ) SPICE_HIP( hipMemcpy( b->data(), b->data() + from, std::size_t( _g.n ) * 4, hipMemcpyDeviceToDevice ) );
+		}
 		synchronize();
 		ctl_t ctl{ step, sum, c, std::int32_t( step % _v.rsize ), 0, 0, 0.0f, 0.0f };
 		SPICE_HIP( hipMemcpy( _ctl.data() + ( step & ( CLOCK_SLOTS - 1 ) ), &ctl, sizeof( ctl ), hipMemcpyHostToDevice ) );
@@ -262,16 +285,10 @@ public:
 			SPICE_HIP( hipMemset( _hring.data(), 0, _hring.bytes() ) );
 			SPICE_HIP( hipMemset( _fl_count.data(), 0, _fl_count.bytes() ) );
 			reset_caught();
-			if constexpr( traced )
-				reset_eager();
-			else
-			{
-				SPICE_HIP( hipMemset( _last_spk.data(), 0xff, _last_spk.bytes() ) );
-				std::vector<std::int32_t> synced( _g.n, std::int32_t( step - 1 ) );
-				SPICE_HIP( hipMemcpy( _synced.data(), synced.data(), _synced.bytes(), hipMemcpyHostToDevice ) );
-				SPICE_HIP( hipMemset( _pend.data(), 0, _pend.bytes() ) );
-			}
+			if constexpr( eager ) reset_eager( traced );
+			if( _lazy ) reset_lazy( std::int32_t( step - 1 ) );
 		}
+		_single_until = 0;
 		_step = step;
 		_clock.set( sum, c );
 		_dt_last = 0.0f;
@@ -280,7 +297,7 @@ public:
 	void get_stats( spice_stats * out ) override
 	{
 		// (windows of different lengths leave different amounts of plasticity due: count all of it)
-		if( windowed )
+		if( windowed && !_lazy )
 			sync_synapses();
 		else
 			synchronize();
@@ -345,11 +362,10 @@ public:
 		if( bytes != std::uint64_t( _g.n ) * attr_bytes<N>( a ) ) throw std::invalid_argument( "buffer size mismatch" );
 		synchronize();
 		if constexpr( plastic && windowed )
-			if( _step > 0 )
+			if( _step > 0 && !_lazy )
 			{
-				// The imported state need not keep the refractory promise towards spikes before it, so
-				// no event may still be due, and until those spikes have arrived windows are of one
-				// step (which relies on the promise for two steps only).
+				// The imported state need not keep the refractory promise towards spikes before it:
+				// until those have arrived, steps run one by one, the passes of each before the next.
 				sync_synapses();
 				_single_until = _step + _p.delay + _v.wcap;
 			}
@@ -363,13 +379,22 @@ public:
 		if( bytes != ( ell ? std::uint64_t( _g.n * _g.width ) : std::uint64_t( _g.nnz ) ) * sz )
 			throw std::invalid_argument( "buffer size mismatch" );
 		sync_synapses();
+		dbuf<float> expanded; // a factored trace as synapse attribute
+		char const * src = _sa[a].data();
+		if constexpr( factored )
+			if( !_lazy && is_factored_attr<S>( a ) )
+			{
+				expanded.resize( std::size_t( _g.nnz ) + 1 );
+				expand_trace( a, expanded.data() );
+				src = reinterpret_cast<char const *>( expanded.data() );
+			}
 		if( !ell )
 		{
-			if( _g.nnz ) SPICE_HIP( hipMemcpy( out, _sa[a].data(), bytes, hipMemcpyDeviceToHost ) );
+			if( _g.nnz ) SPICE_HIP( hipMemcpy( out, src, bytes, hipMemcpyDeviceToHost ) );
 			return;
 		}
 		std::vector<char> csr( _g.nnz * sz );
-		if( _g.nnz ) SPICE_HIP( hipMemcpy( csr.data(), _sa[a].data(), csr.size(), hipMemcpyDeviceToHost ) );
+		if( _g.nnz ) SPICE_HIP( hipMemcpy( csr.data(), src, csr.size(), hipMemcpyDeviceToHost ) );
 		std::vector<std::int64_t> rp( _g.n + 1 );
 		SPICE_HIP( hipMemcpy( rp.data(), _g.row_ptr.data(), rp.size() * 8, hipMemcpyDeviceToHost ) );
 		char * o = static_cast<char *>( out );
@@ -387,7 +412,7 @@ public:
 		sync_synapses();
 		if( !ell )
 		{
-			if( _g.nnz ) SPICE_HIP( hipMemcpy( _sa[a].data(), in, bytes, hipMemcpyHostToDevice ) );
+			store_synapse_attr( a, in );
 			return;
 		}
 		std::vector<std::int64_t> rp( _g.n + 1 );
@@ -396,7 +421,7 @@ public:
 		char const * src = static_cast<char const *>( in );
 		for( std::int64_t r = 0; r < _g.n; r++ )
 			std::memcpy( csr.data() + rp[r] * sz, src + r * _g.width * sz, ( rp[r + 1] - rp[r] ) * sz );
-		if( _g.nnz ) SPICE_HIP( hipMemcpy( _sa[a].data(), csr.data(), csr.size(), hipMemcpyHostToDevice ) );
+		store_synapse_attr( a, csr.data() );
 	}
 
 	// ---- spike log ----
@@ -489,6 +514,7 @@ public:
 			g.n = _g.n;
 			g.nnz = _g.nnz;
 			g.width = _g.width;
+			g.targets = _g.targets;
 			g.row_ptr.resize( _g.row_ptr.size() );
 			g.col.resize( _g.col.size() );
 			SPICE_HIP( hipMemcpyAsync( g.row_ptr.data(), _g.row_ptr.data(), _g.row_ptr.bytes(), hipMemcpyDeviceToDevice, s ) );
@@ -496,6 +522,17 @@ public:
 			SPICE_HIP( hipStreamSynchronize( s ) );
 			auto * c = new hip_net( _p, std::move( g ), s );
 			s = nullptr; // owned by c
+			if constexpr( factored )
+			{
+				if( _lazy )
+					c->make_lazy();
+				else
+				{
+					std::int64_t const from = trace_slot() * _g.n;
+					SPICE_HIP( hipMemcpy( c->_xtr.data(), _xtr.data() + from, std::size_t( _g.n ) * 4, hipMemcpyDeviceToDevice ) );
+					SPICE_HIP( hipMemcpy( c->_ytr.data(), _ytr.data() + from, std::size_t( _g.n ) * 4, hipMemcpyDeviceToDevice ) );
+				}
+			}
 			for( int a = 0; a < MAXA; a++ )
 			{
 				if( _na[a].bytes() ) SPICE_HIP( hipMemcpy( c->_na[a].data(), _na[a].data(), _na[a].bytes(), hipMemcpyDeviceToDevice ) );
@@ -516,6 +553,48 @@ public:
 	int num_tiles() const { return _v.nact; } // the delivery's tiles (those with incoming synapses)
 	int num_all_tiles() const { return _v.ntiles; }
 	std::int64_t single_steps_left() const { return std::max<std::int64_t>( 0, _single_until - _step ); }
+	bool lazy() const { return _lazy; }
+
+	// The passes due before step t in a kernel of their own.
+	void launch_passes( std::int64_t t, hipStream_t s )
+	{
+		if constexpr( plastic && windowed )
+		{
+			dview const & v = _vs[t & ( CLOCK_SLOTS - 1 )];
+			if( fixed() )
+				SPICE_LAUNCH( ( k_window_passes<Model, true><<<_grid_flush, 256, 0, s>>>( v ) ) );
+			else
+				SPICE_LAUNCH( ( k_window_passes<Model, false><<<_grid_flush, 256, 0, s>>>( v ) ) );
+		}
+	}
+
+	// Factored traces back to the per-synapse contract: the traces become synapse attributes, and
+	// steps run as two kernels with lazy plasticity. For a layout whose plastic synapses join
+	// neurons that do not keep the refractory promise, and for imported synapse state that is not of
+	// the factored form.
+	void make_lazy()
+	{
+		if constexpr( factored )
+		{
+			if( _lazy ) return;
+			bool const fresh = _step == 0;
+			sync_synapses();
+			_tp_ent.release();
+			_tp_total = _tp_targets = 0;
+			for( int a : { int( S::pre_trace ), int( S::post_trace ) } )
+			{
+				_sa[a].resize( std::size_t( _g.nnz + COL_PAD ) * sizeof( float ) );
+				_v.sa[a] = _sa[a].data();
+				expand_trace( a, reinterpret_cast<float *>( _sa[a].data() ) );
+			}
+			_lazy = true;
+			_single_until = 0;
+			alloc_lazy();
+			reset_lazy( std::int32_t( _step - 1 ) );
+			SPICE_HIP( hipMemset( _fl_count.data(), 0, _fl_count.bytes() ) );
+			apply_launch( fresh ? launch_cfg{} : _lc );
+		}
+	}
 	bool logged() const { return _slog_ctl.size() > 0; }
 	int num_receive_parts() const { return _v.rparts; }
 	int num_update_blocks() const { return _grid_update; }
@@ -524,7 +603,7 @@ public:
 	// of their spike; eager: arriving rows and spiking targets), at most the net's own grid
 	int num_batch_flush_blocks() const
 	{
-		std::int64_t const items = traced ? ( _g.n / 256 + 1 ) * _v.wcap * ( _v.fparts + _v.pparts ) : ( _g.n / FLUSH_AGE + _g.n / 256 + 1 ) * _v.fparts;
+		std::int64_t const items = !_lazy ? ( _g.n / 256 + 1 ) * _v.wcap * ( _v.fparts + _v.pparts ) : ( _g.n / FLUSH_AGE + _g.n / 256 + 1 ) * _v.fparts;
 		return int( std::clamp<std::int64_t>( ( items + 1 ) / 2, 1, _grid_flush ) );
 	}
 	bool fixed() const { return ( _p.flags & SPICE_FLAG_FIXED_POINT ) != 0; }
@@ -569,7 +648,8 @@ private:
 	int _upd_block = SPICE_UPDATE_BLOCK;
 	int _grid_plast = 0; // plasticity workgroups of the delivery kernel
 	bool _ahead = false; // the delivery of a step may run before the updates of earlier steps
-	std::int64_t _single_until = 0; // windows of one step before this step (see import_neuron_attr)
+	std::int64_t _single_until = 0; // steps run one by one before this step (see import_neuron_attr)
+	bool _lazy = false; // plasticity by the per-synapse contract
 	int _window = 0;       // longest window of the window kernels that run the steps (0: none)
 	launch_queue _queue;
 	launch_cfg _lc{};
@@ -621,7 +701,7 @@ private:
 		} );
 		util::for_n<S::size>( [&]( auto I ) {
 			using A = typename S::template type<I>;
-			_sa[I].resize( ( _g.nnz + COL_PAD ) * sizeof( A ) ); // (read in pieces like the row store)
+			if constexpr( !factored || !is_factored_attr<S>( int( I ) ) ) _sa[I].resize( ( _g.nnz + COL_PAD ) * sizeof( A ) ); // (read in pieces like the row store)
 		} );
 		_v.wcap = window_cap<Model>( _p.delay );
 		_v.rsize = ring_entries<Model>( _p.delay );
@@ -640,7 +720,7 @@ private:
 			SPICE_HIP( hipMemsetAsync( _hring.data(), 0, _hring.bytes(), _s ) );
 			SPICE_HIP( hipMemsetAsync( _fl_count.data(), 0, _fl_count.bytes(), _s ) );
 			reset_caught();
-			if constexpr( traced )
+			if constexpr( eager )
 			{
 				_xtr.resize( ( windowed ? 4 : 2 ) * n );
 				_ytr.resize( ( windowed ? 4 : 2 ) * n );
@@ -649,20 +729,12 @@ private:
 				_po_id.resize( 2 * n );
 				_po_count.resize( CLOCK_SLOTS );
 				_tp_ptr.resize( n + 1 );
-				reset_eager();
+				reset_eager( true );
 			}
-			else
+			if( _lazy )
 			{
-				_last_spk.resize( n );
-				_synced.resize( n );
-				_pend.resize( n );
-				_fl_synced.resize( 2 * n );
-				_fl_pend.resize( 2 * n );
-				SPICE_HIP( hipMemsetAsync( _last_spk.data(), 0xff, _last_spk.bytes(), _s ) ); // -1
-				SPICE_HIP( hipMemsetAsync( _pend.data(), 0, _pend.bytes(), _s ) );
-				std::vector<std::int32_t> synced( n, -1 );
-				SPICE_HIP( hipMemcpyAsync( _synced.data(), synced.data(), _synced.bytes(), hipMemcpyHostToDevice, _s ) );
-				SPICE_HIP( hipStreamSynchronize( _s ) ); // `synced` is a host temporary
+				alloc_lazy();
+				reset_lazy( -1 );
 			}
 		}
 		_ctl.resize( CLOCK_SLOTS );
@@ -716,13 +788,98 @@ private:
 		apply_launch( first );
 	}
 
-	// Eager plasticity state at a clock (re)start: zero traces and flags, no pending lists.
-	void reset_eager()
+	// Eager plasticity state at a clock (re)start: initial traces (if asked), no flags or lists.
+	void reset_eager( bool traces )
 	{
-		for( auto * b : { &_xtr, &_ytr } ) SPICE_HIP( hipMemsetAsync( b->data(), 0, b->bytes(), _s ) );
+		if( traces )
+			for( auto * b : { &_xtr, &_ytr } )
+			{
+				if constexpr( factored )
+					SPICE_LAUNCH( k_fill<<<unsigned( ( b->size() + 255 ) / 256 ), 256, 0, _s>>>( b->data(), std::int64_t( b->size() ), S::trace_init ) );
+				else
+					SPICE_HIP( hipMemsetAsync( b->data(), 0, b->bytes(), _s ) );
+			}
 		SPICE_HIP( hipMemsetAsync( _fl8.data(), 0, _fl8.bytes(), _s ) );
 		if( windowed ) SPICE_HIP( hipMemsetAsync( _sp8.data(), 0, _sp8.bytes(), _s ) );
 		SPICE_HIP( hipMemsetAsync( _po_count.data(), 0, _po_count.bytes(), _s ) );
+	}
+
+	// Lazy plasticity's bookkeeping, every row current through step `synced`.
+	void alloc_lazy()
+	{
+		std::int64_t const n = _g.n;
+		_last_spk.resize( n );
+		_synced.resize( n );
+		_pend.resize( n );
+		_fl_synced.resize( 2 * n );
+		_fl_pend.resize( 2 * n );
+		_v.last_spk = _last_spk.data();
+		_v.synced = _synced.data();
+		_v.pend = _pend.data();
+		_v.fl_synced = _fl_synced.data();
+		_v.fl_pend = _fl_pend.data();
+	}
+	void reset_lazy( std::int32_t synced )
+	{
+		SPICE_HIP( hipMemsetAsync( _last_spk.data(), 0xff, _last_spk.bytes(), _s ) ); // -1
+		SPICE_HIP( hipMemsetAsync( _pend.data(), 0, _pend.bytes(), _s ) );
+		std::vector<std::int32_t> rows( _g.n, synced );
+		SPICE_HIP( hipMemcpyAsync( _synced.data(), rows.data(), _synced.bytes(), hipMemcpyHostToDevice, _s ) );
+		SPICE_HIP( hipStreamSynchronize( _s ) ); // `rows` is a host temporary
+	}
+
+	// The place (0 .. 3) of the current traces: that of the next window's number.
+	std::int64_t trace_slot() const
+	{
+		ctl_t c{};
+		SPICE_HIP( hipMemcpy( &c, _ctl.data() + ( _step & ( CLOCK_SLOTS - 1 ) ), sizeof( c ), hipMemcpyDeviceToHost ) );
+		return c.wseq & 3;
+	}
+
+	// Factored trace attribute a of every synapse (synapses synchronized).
+	void expand_trace( int a, float * out )
+	{
+		if constexpr( factored )
+		{
+			std::int64_t const at = trace_slot() * _g.n;
+			SPICE_LAUNCH( k_expand_trace<Model><<<unsigned( ( _g.n + 3 ) / 4 ), 256, 0, _s>>>( _v, _xtr.data() + at, _ytr.data() + at, a, out ) );
+			SPICE_HIP( hipStreamSynchronize( _s ) );
+		}
+	}
+
+	// Imported attribute a of every synapse, in CSR order (synapses synchronized).
+	void store_synapse_attr( int a, void const * in )
+	{
+		std::size_t const bytes = std::size_t( _g.nnz ) * attr_bytes<S>( a );
+		if constexpr( factored )
+			if( !_lazy && _g.nnz )
+			{
+				dbuf<char> tmp( bytes );
+				SPICE_HIP( hipMemcpy( tmp.data(), in, bytes, hipMemcpyHostToDevice ) );
+				unsigned const rows = unsigned( ( _g.n + 3 ) / 4 );
+				dbuf<std::int32_t> bad( 1 );
+				SPICE_HIP( hipMemsetAsync( bad.data(), 0, 4, _s ) );
+				dbuf<float> t( std::size_t( _g.n ) );
+				dbuf<float> & kept = a == S::pre_trace ? _xtr : _ytr;
+				std::int64_t const at = trace_slot() * _g.n;
+				if( is_factored_attr<S>( a ) )
+				{
+					SPICE_HIP( hipMemcpyAsync( t.data(), kept.data() + at, t.bytes(), hipMemcpyDeviceToDevice, _s ) );
+					SPICE_LAUNCH( k_gather_trace<Model><<<rows, 256, 0, _s>>>( _v, a, reinterpret_cast<float const *>( tmp.data() ), t.data() ) );
+				}
+				SPICE_LAUNCH( k_check_factored<Model><<<rows, 256, 0, _s>>>( _v, a, tmp.data(), t.data(), bad.data() ) );
+				std::int32_t b = 0;
+				SPICE_HIP( hipMemcpyAsync( &b, bad.data(), 4, hipMemcpyDeviceToHost, _s ) );
+				SPICE_HIP( hipStreamSynchronize( _s ) );
+				if( b )
+					make_lazy();
+				else if( is_factored_attr<S>( a ) )
+				{
+					SPICE_HIP( hipMemcpy( kept.data() + at, t.data(), t.bytes(), hipMemcpyDeviceToDevice ) );
+					return;
+				}
+			}
+		if( bytes ) SPICE_HIP( hipMemcpy( _sa[a].data(), in, bytes, hipMemcpyHostToDevice ) );
 	}
 
 	// Nothing synchronized yet (plastic models).
@@ -766,22 +923,24 @@ private:
 		int const cus = device_cu_count();
 		std::int64_t const n = _g.n;
 		launch_cfg c;
-		c.tile_w = default_tile_w<Model>( n, _p.delay, cus );
+		c.tile_w = _lazy ? lazy_tile_w( n, cus ) : default_tile_w<Model>( n, _g.targets, _p.delay, cus );
 		// plasticity beside a window's tiles: four workgroups of 256 threads per CU; work items of 128
 		// slots or entries, which one round of a wave's loads holds twice over (STDP 1e8, delay 1:
 		// 13.0 us per step, 16.2 with 256, 23.6 with 512), or of 512 where a window has items enough
-		// for every wave anyway (1e9, delay 15, steps 2,000-12,000: 24.9, 25.3 with 256, 26.5 with 128)
+		// for every wave anyway (1e9, delay 15, steps 2,000-12,000: 24.9, 25.3 with 256, 26.5 with 128;
+		// brunel_with_plasticity 6e8: 13.1, 13.9 and 15.9)
 		double const mean_row = n > 0 ? double( _g.nnz ) / double( n ) : 0.0;
-		c.flush_slots = !windowed ? 256 : _v.wcap > 1 && mean_row >= 8192.0 ? 512 : 128;
+		bool const win = windowed && !_lazy;
+		c.flush_slots = !win ? 256 : _v.wcap > 1 && mean_row >= 5000.0 ? 512 : 128;
 		std::int64_t const fparts = std::max( 1, int( mean_row / c.flush_slots + 0.5 ) );
-		c.flush_grid = int( std::min<std::int64_t>( ( windowed ? 4 : 8 ) * cus, std::max<std::int64_t>( 1, ( n * fparts + 3 ) / 4 ) ) );
+		c.flush_grid = int( std::min<std::int64_t>( ( win ? 4 : 8 ) * cus, std::max<std::int64_t>( 1, ( n * fparts + 3 ) / 4 ) ) );
 		c.recv_parts = 1;
 		if( !plastic )
 			// window kernels: 16 waves where a tile has a CU to itself, 8 where several share one or
 			// the tile is small (Vogels 1e9, delay 8: 7.6 us per step with 250 tiles of 896 and 16
 			// waves, 8.9 with 8; Brunel 1e10, 495 tiles of 640: 19.4 with 16, 17.3 with 8)
-			c.recv_block = c.tile_w > 2048 || ( c.tile_w >= 512 && ( n + c.tile_w - 1 ) / c.tile_w <= cus ) ? 1024 : 512;
-		else if( windowed )
+			c.recv_block = c.tile_w > 2048 || ( c.tile_w >= 512 && ( _g.targets + c.tile_w - 1 ) / c.tile_w <= cus ) ? 1024 : 512;
+		else if( win )
 			c.recv_block = 512; // (STDP 1e9: 24.3 us per step, 27.4 with 1,024 threads)
 		else
 			// small nets: few events per tile, so more and smaller delivery workgroups
@@ -905,6 +1064,7 @@ private:
 		}
 		if constexpr( windowed )
 		{
+			if( plastic && _lazy ) return;
 			if( !plastic && !_ahead && ( _lc.recv_parts != 1 || _lc.tile_w > 4 * _lc.recv_block ) ) return;
 			_window = 1;
 			with_window_kernel( [&]( auto kernel, auto bytes, int ) {
@@ -925,15 +1085,19 @@ private:
 		SPICE_LAUNCH( k_init_neurons<Model><<<_grid_update, 256, 0, _s>>>( _v ) );
 		if constexpr( plastic )
 		{
-			SPICE_LAUNCH( k_init_synapses<Model><<<unsigned( ( _g.n + 3 ) / 4 ), 256, 0, _s>>>( _v ) );
-			if constexpr( traced ) build_by_target();
+			dbuf<std::int32_t> broken( 1 );
+			SPICE_HIP( hipMemsetAsync( broken.data(), 0, 4, _s ) );
+			SPICE_LAUNCH( k_init_synapses<Model><<<unsigned( ( _g.n + 3 ) / 4 ), 256, 0, _s>>>( _v, broken.data() ) );
+			std::int32_t b = 0;
+			SPICE_HIP( hipMemcpyAsync( &b, broken.data(), 4, hipMemcpyDeviceToHost, _s ) );
+			SPICE_HIP( hipStreamSynchronize( _s ) );
+			if( b )
+				make_lazy();
+			else if constexpr( eager )
+				build_by_target();
 		}
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 	}
-
-	// Windows at this step: of one step while imported neuron state may break the promise that
-	// longer ones rely on.
-	int window_now() const { return _step < _single_until ? 1 : _window; }
 
 	// Enqueues steps t .. t + len - 1: windows of one step, or two kernels per step. The passes of
 	// the last step of a plastic model are left to the next kernel (or a synchronization).
@@ -951,7 +1115,7 @@ private:
 	void launch_step( std::int64_t t )
 	{
 		[[maybe_unused]] dview const & v = _vs[t & ( CLOCK_SLOTS - 1 )];
-		if constexpr( !plastic || !windowed )
+		if constexpr( !plastic || !windowed || factored )
 		{
 			if( fixed() )
 			{
@@ -981,7 +1145,7 @@ private:
 				for( int i = 0; i < k; i++ )
 				{
 					hipEvent_t * e = &ev[i * ev_per_step];
-					if constexpr( !plastic || !windowed )
+					if constexpr( !plastic || !windowed || factored )
 					{
 						if( fixed() )
 							launch_step_events<true>( e, _vs[_step & ( CLOCK_SLOTS - 1 )] );
@@ -1035,11 +1199,12 @@ private:
 	}
 
 	// The window of w steps from step t, with HIP events attached to its dispatch when start is not
-	// null.
-	void launch_window( std::int64_t t, int w, hipEvent_t start, hipEvent_t stop )
+	// null. alone: the passes before it in a kernel of their own first.
+	void launch_window( std::int64_t t, int w, hipEvent_t start, hipEvent_t stop, bool alone = false )
 	{
 		if constexpr( windowed )
 		{
+			if( alone ) launch_passes( t, _s );
 			if( _slog_ctl.size() ) throw std::logic_error( "nets with a spike log are stepped by a batch" );
 			dview v = _vs[t & ( CLOCK_SLOTS - 1 )];
 			with_window_kernel( [&]( auto kernel, auto bytes, int bs ) {
@@ -1047,9 +1212,9 @@ private:
 				void * args[] = { &v, &W };
 				void const * fn = reinterpret_cast<void const *>( kernel );
 				if( start )
-					SPICE_HIP( hipExtLaunchKernel( fn, dim3( unsigned( v.ntiles + _grid_plast ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s, start, stop, 0 ) );
+					SPICE_HIP( hipExtLaunchKernel( fn, dim3( unsigned( v.ntiles + ( alone ? 0 : _grid_plast ) ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s, start, stop, 0 ) );
 				else
-					SPICE_HIP( hipLaunchKernel( fn, dim3( unsigned( v.ntiles + _grid_plast ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s ) );
+					SPICE_HIP( hipLaunchKernel( fn, dim3( unsigned( v.ntiles + ( alone ? 0 : _grid_plast ) ) ), dim3( unsigned( bs ) ), args, bytes( w ), _s ) );
 			} );
 		}
 	}
@@ -1086,8 +1251,9 @@ private:
 				int k = 0;
 				for( ; k < batch && n > 0; k++ )
 				{
-					int const w = window_steps( std::min<std::int64_t>( n, window_now() ) );
-					launch_window( _step, w, ev[2 * k], ev[2 * k + 1] );
+					bool const single = _step < _single_until;
+					int const w = single ? 1 : window_steps( std::min<std::int64_t>( n, _window ) );
+					launch_window( _step, w, ev[2 * k], ev[2 * k + 1], single );
 					for( int i = 0; i < w; i++ ) tick();
 					n -= w;
 				}
@@ -1185,14 +1351,9 @@ private:
 				std::int64_t const now = _step - 1;
 				dview const & v = _vs[_step & ( CLOCK_SLOTS - 1 )]; // a view of step now + 1
 				[[maybe_unused]] std::int64_t const slot0 = std::int64_t( v.ntiles ) * v.rparts;
-				if constexpr( windowed )
-				{
-					if( fixed() )
-						SPICE_LAUNCH( ( k_window_passes<Model, true><<<_grid_flush, 256, 0, _s>>>( v ) ) );
-					else
-						SPICE_LAUNCH( ( k_window_passes<Model, false><<<_grid_flush, 256, 0, _s>>>( v ) ) );
-				}
-				else if constexpr( traced )
+				if( windowed && !_lazy )
+					launch_passes( _step, _s );
+				else if constexpr( traced && !windowed )
 				{
 					if( fixed() )
 						SPICE_LAUNCH( k_stdp<Model, true><<<_grid_flush, 256, 0, _s>>>( v, now, slot0 ) );
@@ -1201,7 +1362,7 @@ private:
 					// deferred events of the rows arriving next
 					SPICE_LAUNCH( k_sync_eager<Model><<<unsigned( ( _g.n + 3 ) / 4 ), 256, 0, _s>>>( _v, now ) );
 				}
-				else
+				else if constexpr( !traced )
 				{
 					if( fixed() )
 						SPICE_LAUNCH( k_flush<Model, true><<<_grid_flush, 256, 0, _s>>>( v, now, slot0 ) );

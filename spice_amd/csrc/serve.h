@@ -48,7 +48,8 @@ inline std::uint64_t spike_log_capacity( std::int64_t n, std::int64_t chunk, flo
 
 // Upper bound of a job's device memory (admission reservation): every buffer of a hip_net
 // with E <= N * width edges, plus the spike log and per-allocation slack.
-inline std::uint64_t estimate_job_bytes( int model, std::int64_t n, std::int64_t width, int delay, bool fixed, std::int64_t chunk, float dt )
+// (targets: csr_dev::targets.)
+inline std::uint64_t estimate_job_bytes( int model, std::int64_t n, std::int64_t width, std::int64_t targets, int delay, bool fixed, std::int64_t chunk, float dt )
 {
 	return dispatch_model( model, [&]( auto m ) -> std::uint64_t {
 		using M = decltype( m );
@@ -56,7 +57,8 @@ inline std::uint64_t estimate_job_bytes( int model, std::int64_t n, std::int64_t
 		using Ss = typename M::synapse;
 		std::uint64_t const N = std::uint64_t( n ), E = N * std::uint64_t( width ) + COL_PAD;
 		std::uint64_t const cus = 256;
-		std::uint64_t const tile_w = std::uint64_t( default_tile_w<M>( n, delay, int( cus ) ) );
+		std::uint64_t tile_w = std::uint64_t( default_tile_w<M>( n, targets, delay, int( cus ) ) );
+		if( factored_v<M> ) tile_w = std::min<std::uint64_t>( tile_w, std::uint64_t( lazy_tile_w( n, int( cus ) ) ) ); // (per-synapse contract)
 		std::uint64_t const ntiles = ( N + tile_w - 1 ) / tile_w;
 		std::uint64_t b = 8 * ( N + 1 ) + 4 * E + 4 * N;                 // CSR (+ generator degrees)
 		b += N * Nn::size_in_bytes + N * Nn::size * ( fixed ? 8 : 4 );    // neurons + accumulators
@@ -65,9 +67,10 @@ inline std::uint64_t estimate_job_bytes( int model, std::int64_t n, std::int64_t
 		if constexpr( is_plastic_v<M> )
 		{
 			b += 8 * HWORDS * N + 36 * N;
-			// eager: traces, flags and target lists by parity, by-target index (at most every
-			// edge) with its offsets and build temporaries (the sort's second buffer and work space)
-			if constexpr( has_neuron_traces_v<Ss> ) b += 17 * E + 48 * N + ( 64 << 20 );
+			// eager: traces, flags and target lists, by-target index (at most every edge) with its
+			// offsets and counters; factored traces: the index takes the place of the traces, which
+			// the per-synapse contract (without an index) keeps per synapse
+			if constexpr( has_neuron_traces_v<Ss> || factored_v<M> ) b += ( has_neuron_traces_v<Ss> ? 8 * E : 0 ) + 64 * N;
 		}
 		b += 8 * NSTAT * ( N / 256 + 8 * cus + ntiles + 1 );             // statistics slots
 		b += 4 * spike_log_capacity( n, chunk, dt ) + 8 * std::uint64_t( chunk ) + 64;

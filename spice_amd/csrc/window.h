@@ -54,7 +54,7 @@ using win_acc = std::conditional_t<std::is_floating_point_v<T>, std::conditional
 
 // Models whose steps run as windows: static ones, and plastic ones whose passes apply every event.
 template <typename Model>
-inline constexpr bool windowed_v = !is_plastic_v<Model> || eager_nodefer_v<Model>;
+inline constexpr bool windowed_v = !is_plastic_v<Model> || windowed_plastic_v<Model>;
 
 // Longest window (steps, before the clock's restriction): 1 unless the delivery may run before its
 // targets' update. Plastic models: an input is read beside the passes of the window before, and
@@ -142,8 +142,8 @@ struct synapses
 	{
 		util::for_n<S::size>( [&]( auto I ) {
 			using T = typename S::template type<I>;
-			T t[WIN_VEC];
-			__builtin_memcpy( t, static_cast<T const *>( arr[I] ) + i, sizeof( t ) );
+			T t[WIN_VEC] = {};
+			if constexpr( !is_factored_attr<S>( int( I ) ) ) __builtin_memcpy( t, static_cast<T const *>( arr[I] ) + i, sizeof( t ) );
 #pragma unroll
 			for( int x = 0; x < WIN_VEC; x++ ) std::get<I>( s[x] ) = t[x];
 		} );
@@ -566,8 +566,8 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 	std::int64_t const nitems = npre + std::int64_t( v.po_count[k & 3] ) * v.pparts;
 	snn_info const info = info_of( v );
 	int const lane = lane_id();
-	// lane q: the decay of the window's step q
-	float decay = 0.0f;
+	// lane q: the dt of the window's step q and the traces' decay in it
+	float decay = 0.0f, dts = 0.0f;
 	{
 		float sum = clk.psum, c = clk.pc;
 		for( int q = 0; q < W; q++ )
@@ -576,7 +576,11 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 			float const t = sum + dt;
 			c = ( t - sum ) - dt;
 			sum = t;
-			if( lane == q ) decay = S::trace_decay( dt );
+			if( lane == q )
+			{
+				dts = dt;
+				decay = S::trace_decay( dt );
+			}
 		}
 	}
 	auto decay_of = [&]( int q ) { return __builtin_bit_cast( float, __builtin_amdgcn_readlane( __builtin_bit_cast( std::int32_t, decay ), q ) ); };
@@ -586,11 +590,20 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 	std::int64_t const wave0 = uniform64( ( blk * blockDim.x + threadIdx.x ) >> 6 );
 	std::int64_t const nwaves = nblk * ( blockDim.x >> 6 );
 	unsigned long long touched = 0, written = 0, words = 0, rows = 0;
-	// one event; counts it, and whether it changed the synapse
-	auto event = [&]( typename S::tuple_t & sy, std::int64_t e, int q, bool pre, bool post, float x, float y ) {
+	auto dt_of = [&]( int q ) { return __builtin_bit_cast( float, shfl_u32( __builtin_bit_cast( std::uint32_t, dts ), q < 0 ? 0 : q ) ); };
+	// one event (of step q, whose dt is given where the rule takes it); counts it, and whether it
+	// changed the synapse
+	auto event = [&]( typename S::tuple_t & sy, std::int64_t e, int q, float dt, bool pre, bool post, float x, float y ) {
 		typename S::tuple_t const before = sy;
 		auto bak = backend( e, q );
-		S::on_event( reg_iter<typename S::tuple_t>{ sy, std::uint32_t( e ) }, pre, post, x, y, info, bak );
+		if constexpr( factored_v<Model> )
+		{
+			std::get<S::pre_trace>( sy ) = x;
+			std::get<S::post_trace>( sy ) = y;
+			S::on_event( reg_iter<typename S::tuple_t>{ sy, std::uint32_t( e ) }, pre, post, dt, info, bak );
+		}
+		else
+			S::on_event( reg_iter<typename S::tuple_t>{ sy, std::uint32_t( e ) }, pre, post, x, y, info, bak );
 		touched++;
 		written += same_bits<S>( before, sy ) ? 0 : 1;
 	};
@@ -636,7 +649,7 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 				{
 					std::int64_t const e = first + lane + 64 * u;
 					ok[u] = ok[u] && S::plastic( s, j[u], info );
-					load_tuple<S>( sy[u], v.sa, ok[u] ? e : beg );
+					if constexpr( !has_inert_v<S> ) load_synapse<S>( sy[u], v.sa, ok[u] ? e : beg );
 					b[u] = int( v.sp8[par + j[u]] ) - 1;
 					y[u] = v.ytr[tr + j[u]];
 				}
@@ -647,9 +660,30 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 #pragma unroll
 					for( int u = 0; u < U; u++ ) y[u] = fmaf( y[u], dq, q == b[u] ? 1.0f : 0.0f );
 				}
-				float xb[U];
+				float xb[U], db[U];
+				float const da = dt_of( a );
+#pragma unroll
+				for( int u = 0; u < U; u++ ) db[u] = factored_v<Model> ? dt_of( b[u] ) : 0.0f;
 #pragma unroll
 				for( int u = 0; u < U; u++ ) xb[u] = __builtin_bit_cast( float, shfl_u32( __builtin_bit_cast( std::uint32_t, xs ), b[u] < 0 ? 0 : b[u] ) );
+				if constexpr( has_inert_v<S> )
+				{
+					// events that cannot change the synapse do not read it
+#pragma unroll
+					for( int u = 0; u < U; u++ )
+					{
+						if( !ok[u] ) continue;
+						bool const post = b[u] >= 0;
+						if( b[u] == a ? S::inert( true, true, xb[u], y[u], da ) : S::inert( true, false, 0.0f, y[u], da ) && ( !post || S::inert( false, true, xb[u], 0.0f, db[u] ) ) )
+						{
+							ok[u] = false;
+							touched += post && b[u] != a ? 2 : 1;
+						}
+					}
+#pragma unroll
+					for( int u = 0; u < U; u++ )
+						if( ok[u] ) load_synapse<S>( sy[u], v.sa, first + lane + 64 * u );
+				}
 #pragma unroll
 				for( int u = 0; u < U; u++ )
 				{
@@ -657,10 +691,10 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 					std::int64_t const e = first + lane + 64 * u;
 					typename S::tuple_t const before = sy[u];
 					bool const post = b[u] >= 0;
-					if( post && b[u] < a ) event( sy[u], e, b[u], false, true, xb[u], 0.0f );
-					event( sy[u], e, a, true, b[u] == a, b[u] == a ? xb[u] : 0.0f, y[u] );
-					if( post && b[u] > a ) event( sy[u], e, b[u], false, true, xb[u], 0.0f );
-					store_changed<S>( before, sy[u], v.sa, e );
+					if( post && b[u] < a ) event( sy[u], e, b[u], db[u], false, true, xb[u], 0.0f );
+					event( sy[u], e, a, da, true, b[u] == a, b[u] == a ? xb[u] : 0.0f, y[u] );
+					if( post && b[u] > a ) event( sy[u], e, b[u], db[u], false, true, xb[u], 0.0f );
+					store_synapse<S>( before, sy[u], v.sa, e );
 				}
 			}
 			if( lane == 0 )
@@ -676,6 +710,7 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 			std::int64_t const p = g - f * v.pparts;
 			std::int32_t const d = uniform( v.po_id[par + f] );
 			int const b = uniform( v.sp8[par + d] ) - 1;
+			float const dt_b = dt_of( b );
 			std::int64_t const lo = v.tp_ptr[d], hi = v.tp_ptr[d + 1];
 			std::int64_t const chunk = ( ( hi - lo + v.pparts - 1 ) / v.pparts + 63 ) & ~std::int64_t( 63 );
 			std::int64_t const beg = lo + p * chunk;
@@ -702,26 +737,32 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 					e[u] = v.row_ptr[te[u].src] + te[u].off;
 					xv[u] = v.xtr[tr + te[u].src];
 				}
-				typename S::tuple_t sy[U];
-#pragma unroll
-				for( int u = 0; u < U; u++ )
-				{
-					ok[u] = ok[u] && a8[u] == 0;
-					if( ok[u] ) load_tuple<S>( sy[u], v.sa, e[u] );
-				}
 				for( int q = 0; q <= b; q++ )
 				{
 					float const dq = decay_of( q );
 #pragma unroll
 					for( int u = 0; u < U; u++ ) xv[u] = fmaf( xv[u], dq, 0.0f ); // (no arrival in the window)
 				}
+				typename S::tuple_t sy[U];
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					ok[u] = ok[u] && a8[u] == 0;
+					if constexpr( has_inert_v<S> )
+						if( ok[u] && S::inert( false, true, xv[u], 0.0f, dt_b ) ) // the event cannot change the synapse
+						{
+							ok[u] = false;
+							touched++;
+						}
+					if( ok[u] ) load_synapse<S>( sy[u], v.sa, e[u] );
+				}
 #pragma unroll
 				for( int u = 0; u < U; u++ )
 				{
 					if( !ok[u] ) continue;
 					typename S::tuple_t const before = sy[u];
-					event( sy[u], e[u], b, false, true, xv[u], 0.0f );
-					store_changed<S>( before, sy[u], v.sa, e[u] );
+					event( sy[u], e[u], b, dt_b, false, true, xv[u], 0.0f );
+					store_synapse<S>( before, sy[u], v.sa, e[u] );
 				}
 			}
 			if( lane == 0 )
@@ -752,6 +793,79 @@ __global__ __launch_bounds__( BS ) void k_window( dview v, std::int32_t W )
 		window_tile<Model, FIXED, BS>( v, b < v.nact ? xcd_place( b, v.nact ) : b, W );
 	else if constexpr( is_plastic_v<Model> )
 		window_passes<Model, FIXED>( v, b - v.ntiles, std::int32_t( gridDim.x ) - v.ntiles, v.ntiles );
+}
+
+// ---- factored traces as synapse attributes (exports, imports, the per-synapse contract) -----
+// out[e] = factored trace attribute `attr` of synapse e: the trace of its source or target where the
+// synapse is plastic, init()'s value elsewhere. x, y: the traces now. One wave per row.
+template <typename Model>
+__global__ __launch_bounds__( 256 ) void k_expand_trace( dview v, float const * x, float const * y, int attr, float * out )
+{
+	using S = typename Model::synapse;
+	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
+	if( r >= v.N ) return;
+	snn_info const info = info_of( v );
+	for( std::int64_t e = v.row_ptr[r] + lane_id(); e < v.row_ptr[r + 1]; e += 64 )
+	{
+		std::int32_t const j = v.col[e];
+		out[e] = !S::plastic( std::int32_t( r ), j, info ) ? S::trace_init : attr == S::pre_trace ? x[r] : y[j];
+	}
+}
+
+// Gathers a factored trace from an imported attribute, in[e]: t[source or target] = the value of some
+// plastic synapse of it.
+template <typename Model>
+__global__ __launch_bounds__( 256 ) void k_gather_trace( dview v, int attr, float const * in, float * t )
+{
+	using S = typename Model::synapse;
+	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
+	if( r >= v.N || !v.hasp[r] ) return;
+	snn_info const info = info_of( v );
+	for( std::int64_t e = v.row_ptr[r] + lane_id(); e < v.row_ptr[r + 1]; e += 64 )
+	{
+		std::int32_t const j = v.col[e];
+		if( S::plastic( std::int32_t( r ), j, info ) ) t[attr == S::pre_trace ? r : j] = in[e];
+	}
+}
+
+// *bad = 1 unless imported attribute `attr` keeps the factored form: a trace the same for all
+// plastic synapses of a neuron (t, from k_gather_trace) and init()'s value elsewhere; any other
+// attribute unchanged by an event-free step.
+template <typename Model>
+__global__ __launch_bounds__( 256 ) void k_check_factored( dview v, int attr, void const * in, float const * t, std::int32_t * bad )
+{
+	using S = typename Model::synapse;
+	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
+	if( r >= v.N ) return;
+	snn_info const info = info_of( v );
+	for( std::int64_t e = v.row_ptr[r] + lane_id(); e < v.row_ptr[r + 1]; e += 64 )
+	{
+		std::int32_t const j = v.col[e];
+		bool const plastic = S::plastic( std::int32_t( r ), j, info );
+		if( is_factored_attr<S>( attr ) )
+		{
+			float const want = !plastic ? S::trace_init : t[attr == S::pre_trace ? r : std::int64_t( j )];
+			if( __builtin_bit_cast( std::uint32_t, want ) != static_cast<std::uint32_t const *>( in )[e] ) *bad = 1;
+		}
+		else if( plastic )
+		{
+			typename S::tuple_t sy{};
+			util::for_n<S::size>( [&]( auto I ) {
+				using T = typename S::template type<I>;
+				if constexpr( !is_factored_attr<S>( int( I ) ) ) std::get<I>( sy ) = ld<T>( int( I ) == attr ? in : v.sa[I], e );
+			} );
+			typename S::tuple_t const before = sy;
+			auto bak = make_backend<false>( v, std::uint32_t( e ), std::uint32_t( std::uint64_t( e ) >> 32 ), 0u, util::TAG_SYNAPSE_UPDATE );
+			S::on_event( reg_iter<typename S::tuple_t>{ sy, std::uint32_t( e ) }, false, false, v.DT, info, bak );
+			if( !same_bits<S>( before, sy ) ) *bad = 1;
+		}
+	}
+}
+
+static inline __global__ __launch_bounds__( 256 ) void k_fill( float * p, std::int64_t n, float x )
+{
+	std::int64_t const i = std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x;
+	if( i < n ) p[i] = x;
 }
 
 // ---- by-target index of the plastic synapses (eager plasticity) ----------------------------
