@@ -330,7 +330,9 @@ batch_iface * make_batch( std::vector<net_params> const & ps, std::vector<csr_de
 		{
 			launch_cfg first; // at the width that the batch will want
 			first.tile_w = hip_batch<Model>::batch_tile_w( gs[k].n, default_tile_w<Model>( gs[k].n, gs[k].targets, ps[k].delay, device_cu_count() ), std::int64_t( ps.size() ) );
-			nets.emplace_back( new hip_net<Model>( ps[k], std::move( gs[k] ), ns, first ) );
+			net_params p = ps[k];
+			p.records = false; // (memory for every net)
+			nets.emplace_back( new hip_net<Model>( p, std::move( gs[k] ), ns, first ) );
 		}
 		catch( ... )
 		{

@@ -162,6 +162,11 @@ struct dview
 	std::int32_t * tile_ids; // [ntiles]: the tiles with incoming synapses (the delivery's), then the others
 	std::int32_t nact;
 
+	// segment records (window.h): per row and tile 2^rec_lg bytes, the
+	// segment's length and targets in 16 bits (0: none built, the segments are read from col)
+	unsigned char const * recs;
+	std::int32_t rec_lg;
+
 	slog_t * slog; // nullptr: no spike log
 	std::int32_t * slog_ids;
 	std::uint64_t * slog_off;

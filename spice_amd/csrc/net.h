@@ -35,6 +35,7 @@ struct net_params
 	std::uint64_t seed;
 	std::uint32_t flags;
 	float param[4];
+	bool records = true; // segment records (window.h) where they pay: memory for speed
 };
 
 struct launch_cfg
@@ -114,6 +115,8 @@ int ring_entries( int delay )
 {
 	return std::max( 4, delay + 2 * window_cap<Model>( delay ) );
 }
+
+constexpr int REC_TILE = 768; // widest tile that segment records alone are a reason for (default_launch)
 
 // Targets per delivery tile of a new network. Window kernels: one tile per CU, as
 // every tile stages all of the window's arrivals and a wider one does it less often (synth 1e9:
@@ -487,7 +490,7 @@ public:
 		     _fl_id.bytes() + _fl_synced.bytes() + _fl_pend.bytes() + _hasp.bytes() + _pl_lo.bytes() + _pl_hi.bytes() +
 		     _fl_count.bytes() + _xtr.bytes() + _ytr.bytes() + _fl8.bytes() + _sp8.bytes() + _po_id.bytes() + _po_count.bytes() +
 		     _tp_ptr.bytes() + _caught.bytes() + _tp_ent.bytes() + _ctl.bytes() + _bstats.bytes() +
-		     _pivots.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
+		     _pivots.bytes() + _recs.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
 		return b;
 	}
 
@@ -654,6 +657,7 @@ private:
 	launch_queue _queue;
 	launch_cfg _lc{};
 	dbuf<std::int64_t> _pivots;
+	dbuf<unsigned char> _recs; // segment records
 	dbuf<std::int32_t> _tile_ids;
 	std::int64_t _step = 0;
 	util::kahan_sum<float> _clock;
@@ -924,6 +928,14 @@ private:
 		std::int64_t const n = _g.n;
 		launch_cfg c;
 		c.tile_w = _lazy ? lazy_tile_w( n, cus ) : default_tile_w<Model>( n, _g.targets, _p.delay, cus );
+		if constexpr( input_classes_v<Model> > 0 )
+			if( _v.wcap == 1 && _p.records && _g.targets > 0 && double( _g.nnz ) / double( n ) * REC_TILE / double( _g.targets ) <= 40.0 )
+				// Step by step, with segment records that fit: rather fewer and wider tiles, as all of
+				// them reserve their spikes' places on one address, 9 ns apart (us per step of Vogels
+				// nets of 22,361, 70,711 and 100,000 neurons: 6.6, 7.0 and 7.9 with a tile per CU, 5.8,
+				// 6.6 and 7.4 with 768 targets; 4,000: 5.5 with 64, 5.75 with 768. Brunel, 100,000, whose
+				// segments of 77 targets in such a tile have no records: 11.1 with 256, 11.4 with 768)
+				c.tile_w = int( std::clamp<std::int64_t>( ( ( _g.targets + 95 ) / 96 + 63 ) / 64 * 64, c.tile_w, std::max( c.tile_w, REC_TILE ) ) );
 		// plasticity beside a window's tiles: four workgroups of 256 threads per CU; work items of 128
 		// slots or entries, which one round of a wave's loads holds twice over (STDP 1e8, delay 1:
 		// 13.0 us per step, 16.2 with 256, 23.6 with 512), or of 512 where a window has items enough
@@ -969,6 +981,7 @@ private:
 		std::int64_t const n = _g.n;
 		dview & v = _v;
 		bool const retile = c.tile_w != v.tile_w;
+		int const had_window = _window;
 		if( retile )
 		{
 			std::int32_t const ntiles = std::int32_t( ( n + c.tile_w - 1 ) / c.tile_w );
@@ -989,6 +1002,7 @@ private:
 		_grid_plast = plastic ? std::max( 1, _grid_flush * 256 / c.recv_block ) : 0; // the same waves as flush_grid
 		_lc = c;
 		choose_window();
+		if( retile || ( _window > 0 ) != ( had_window > 0 ) ) build_records();
 		// statistics slots: one per workgroup of the widest step kernel (receive: per work item;
 		// plasticity: after those, one per plasticity workgroup or synchronization block; windows:
 		// one per tile, then the passes' workgroups; update: per block)
@@ -1077,6 +1091,53 @@ private:
 				if( bytes( w ) > ( 64 << 10 ) )
 					SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( w ) ) ) );
 			} );
+		}
+	}
+
+	// Segment records (window.h) of networks that run step by step, where segments are short: the
+	// smallest record that holds one 2.9 standard deviations longer than the mean. Not if the records took over twice
+	// the row store's memory, or more than half of the device's free memory, or if over 1 % of the
+	// segments did not fit (rows of very different lengths); not for served jobs, which are
+	// admitted by their memory.
+	void build_records()
+	{
+		_recs.release();
+		_v.recs = nullptr;
+		_v.rec_lg = 0;
+		if constexpr( input_classes_v<Model> > 0 )
+		{
+			double const mean = double( _g.nnz ) / double( _g.n ) / _v.nact, need = mean + 2.9 * std::sqrt( mean );
+			int lg = 4;
+			while( lg < 8 && rec_capacity( lg ) < need ) lg++;
+			std::uint64_t const segs = std::uint64_t( _g.n ) * std::uint64_t( _v.ntiles ), bytes = segs << lg;
+			if( _v.wcap > 1 || _window == 0 || !_p.records || lg > 7 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
+			if( bytes > ( std::uint64_t( 1 ) << 30 ) )
+			{
+				std::size_t room = 0, all = 0;
+				SPICE_HIP( hipMemGetInfo( &room, &all ) );
+				if( bytes > room / 2 ) return;
+			}
+			try
+			{
+				_recs.resize( bytes );
+			}
+			catch( std::bad_alloc const & )
+			{
+				return;
+			}
+			dbuf<unsigned long long> longs( 1 );
+			SPICE_HIP( hipMemsetAsync( longs.data(), 0, 8, _s ) );
+			SPICE_LAUNCH( k_records<<<unsigned( ( _g.n + 3 ) / 4 ), 256, 0, _s>>>( _v, _recs.data(), lg, longs.data() ) );
+			unsigned long long n = 0;
+			SPICE_HIP( hipMemcpyAsync( &n, longs.data(), 8, hipMemcpyDeviceToHost, _s ) );
+			SPICE_HIP( hipStreamSynchronize( _s ) );
+			if( n > segs / 100 )
+			{
+				_recs.release();
+				return;
+			}
+			_v.recs = _recs.data();
+			_v.rec_lg = lg;
 		}
 	}
 

@@ -121,7 +121,9 @@ public:
 			throw;
 		}
 		auto h = std::make_unique<handle>();
-		h->net.reset( make_net( s.p, std::move( g ), st ) );
+		net_params p = s.p;
+		p.records = false;
+		h->net.reset( make_net( p, std::move( g ), st ) );
 		h->model = s.p.model;
 		h->fixed = ( s.p.flags & SPICE_FLAG_FIXED_POINT ) != 0;
 		h->net->enable_spike_log( spike_log_capacity( s.n, _chunk_max, s.p.dt ), _chunk_max );

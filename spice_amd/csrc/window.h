@@ -66,6 +66,65 @@ constexpr int longest_window_v = !overlap_capable_v<Model> ? 1
                                  : is_plastic_v<Model>     ? ( refractory_steps_v<typename Model::synapse> + 1 ) / 2
                                                            : WINDOW_MAX;
 
+// ---- segment records -------------------------------------------------------------------------
+// For models with input classes a delivery needs of a row's segment in a tile only the targets, and
+// those fit 16 bits inside a tile. Where segments are short and the network runs step by step, each
+// (row, tile) gets a record of 2^lg bytes, 16 to 128: the segment's length, then its targets less
+// the tile's start. A segment then costs one aligned read instead of its bounds and, after them, an
+// unaligned piece of the row store; the chain of dependent accesses that bounds such a step loses
+// two links, as the arrivals' ids are read beside their count. A segment that does not fit has
+// REC_LONG for its length, then (at bytes 4 and 8) its true length and its place in col.
+// us per step, without and with: synth 1e9 (5 targets per segment) 30.1, 25.7; Vogels 1e8 7.8, 6.6.
+// Windows of several steps gain less (Vogels 1e9, delay 8: 7.55, 7.0) than the records cost where
+// a network is built (5 ms), so they have none. Spike lists per tile instead of one per step, which
+// need no atomic, were slower to read (8.5 and 28.3).
+constexpr std::uint16_t REC_LONG = 0xffff;
+HYBRID constexpr int rec_capacity( int lg ) { return ( 1 << lg ) / 2 - 1; }
+struct alignas( 16 ) rec_part // 16 bytes of a record
+{
+	std::uint16_t t[8];
+};
+
+// Builds the records, one wave per row, a lane per tile; *longs counts the segments that do not fit.
+static inline __global__ __launch_bounds__( 256 ) void k_records( dview v, unsigned char * recs, int lg, unsigned long long * longs )
+{
+	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
+	if( r >= v.N ) return;
+	std::int64_t const * pv = v.pivots + r * ( v.ntiles + 1 );
+	int const cap = rec_capacity( lg );
+	for( int t = lane_id(); t < v.ntiles; t += 64 )
+	{
+		std::int64_t const a = pv[t];
+		std::int32_t const len = std::int32_t( pv[t + 1] - a ), t0 = t * v.tile_w;
+		rec_part * const out = reinterpret_cast<rec_part *>( recs + ( ( r * v.ntiles + t ) << lg ) );
+		if( len > cap )
+		{
+			rec_part p{};
+			p.t[0] = REC_LONG;
+			__builtin_memcpy( &p.t[2], &len, 4 );
+			__builtin_memcpy( &p.t[4], &a, 8 );
+			out[0] = p;
+			atomicAdd( longs, 1ull );
+			continue;
+		}
+		std::int32_t const * c = v.col + a;
+		rec_part p{};
+		p.t[0] = std::uint16_t( len );
+		for( int i = 0; i < 1 << ( lg - 4 ); i++ )
+		{
+			// entries 8 i - 1 .. 8 i + 6 of the segment (the row store is padded past its end)
+#pragma unroll
+			for( int x = 0; x < 8; x++ )
+			{
+				int const e = 8 * i + x - 1;
+				if( e >= 0 && e < len ) p.t[x] = std::uint16_t( c[e] - t0 );
+			}
+			out[i] = p;
+			if( 8 * i + 7 >= len ) break; // (what follows is never read as a target)
+		}
+	}
+}
+
 template <typename Model, bool FIXED>
 struct window_lds
 {
@@ -218,7 +277,25 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	// arrivals of the window's steps: lane q holds the count of step q, then the inclusive prefix.
 	// Entries of steps before 0 are empty (counts start at zero).
 	std::uint32_t incl = 0;
+	// records: the first ids beside the count that tells which of them are this step's
+	constexpr int REC_U = 4; // arrivals per group of lanes in flight
+	std::int32_t early_id[REC_U] = {};
 	if( active && lane < W ) incl = v.counts[entry( lane - v.D )];
+	if constexpr( L::classes > 0 )
+		if( active && v.rec_lg )
+		{
+			int const gl = v.rec_lg - 4;
+#pragma unroll
+			for( int u = 0; u < REC_U; u++ )
+			{
+				std::int32_t const k = u * ( BS >> gl ) + ( tid >> gl );
+				early_id[u] = v.ring[std::int64_t( entry( -v.D ) ) * v.N + ( k < v.N ? k : 0 )];
+			}
+		}
+	// and the state of this thread's first neuron, used after the delivery
+	typename N::tuple_t early{};
+	bool const has_early = L::classes > 0 && v.rec_lg && tid < tw;
+	if( has_early ) load_tuple<N>( early, v.na, t0 + tid );
 	for( int x = tid; x < int( sizeof( word ) * nacc * std::size_t( tws ) * std::size_t( W ) / 16 ); x += BS )
 		reinterpret_cast<uint4 *>( acc )[x] = uint4{ 0, 0, 0, 0 };
 	if( tid == 0 ) ev_total = spk_total = 0;
@@ -244,7 +321,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 			if( lane >= d ) incl += y;
 		}
 	}
-	std::int32_t const total = __builtin_amdgcn_readlane( std::int32_t( incl ), W - 1 );
+	std::int32_t total = __builtin_amdgcn_readlane( std::int32_t( incl ), W - 1 );
 
 	// arrival k of the window: its source and step
 	auto fetch_id = [&]( std::int32_t k, std::int32_t & q ) {
@@ -255,11 +332,69 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 		return v.ring[std::int64_t( entry( q - v.D ) ) * v.N + ( kk - ( q > 0 ? below : 0 ) )];
 	};
 
+	std::uint32_t ev = 0;
+	if constexpr( L::classes > 0 )
+		if( v.rec_lg )
+		{
+			// Delivery from records: a group of 2^(rec_lg - 4) lanes per arrival, 16 bytes each, U
+			// arrivals per group in flight; nothing is staged.
+			constexpr int U = REC_U;
+			int const gl = v.rec_lg - 4, ng = BS >> gl, g = tid >> gl, l = tid & ( ( 1 << gl ) - 1 );
+			auto const * recs = reinterpret_cast<rec_part const *>( v.recs );
+			for( std::int32_t c = 0; c < total; c += U * ng )
+			{
+				rec_part r[U];
+				std::int32_t at[U]; // where the counters of the arrival's class and step start
+				bool ok[U];
+				std::int32_t src[U];
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					std::int32_t const k = c + u * ng + g;
+					ok[u] = k < total;
+					std::int32_t const id = c == 0 ? early_id[u] : v.ring[std::int64_t( entry( -v.D ) ) * v.N + ( ok[u] ? k : 0 )];
+					src[u] = ok[u] ? id : 0;
+				}
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					r[u] = rec_part{};
+					if( c + u * ng < total ) r[u] = recs[( ( std::int64_t( src[u] ) * v.ntiles + tile ) << gl ) + l];
+					at[u] = N::input_class( src[u], info ) * tws;
+				}
+				if( c == 0 ) __syncthreads(); // the accumulators are clear
+#pragma unroll
+				for( int u = 0; u < U; u++ )
+				{
+					if( c + u * ng >= total ) continue;
+					std::uint32_t head = r[u].t[0];
+					if( gl ) head = shfl_u32( head, lane & ~( ( 1 << gl ) - 1 ) );
+					int const len = ok[u] && head != REC_LONG ? int( head ) : 0;
+					if( l == 0 ) ev += std::uint32_t( len );
+					int const e0 = 8 * l - 1;
+#pragma unroll
+					for( int x = 0; x < 8; x++ )
+						if( ( x > 0 || l > 0 ) && e0 + x < len ) atomicAdd( acc + ( at[u] + r[u].t[x] ), 1u );
+					if( ok[u] && head == REC_LONG )
+					{
+						rec_part const whole = recs[( std::int64_t( src[u] ) * v.ntiles + tile ) << gl];
+						std::int32_t n;
+						std::int64_t off;
+						__builtin_memcpy( &n, &whole.t[2], 4 );
+						__builtin_memcpy( &off, &whole.t[4], 8 );
+						if( l == 0 ) ev += std::uint32_t( n );
+						for( std::int32_t e = l; e < n; e += 1 << gl ) atomicAdd( acc + ( at[u] + v.col[off + e] - t0 ), 1u );
+					}
+				}
+			}
+			if( total == 0 ) __syncthreads(); // the accumulators are clear
+			total = 0;                        // nothing is left for the walk below
+		}
+
 	// Delivery, wave by wave: a wave stages up to 64 of the window's arrivals at a time (one segment
 	// each) in its own part of the LDS and walks them; the next ones' ids and segment bounds are
 	// read beside the walk. No wave waits for another before the update.
-	std::uint32_t ev = 0;
-	__syncthreads(); // the accumulators are clear
+	if( L::classes == 0 || !v.rec_lg ) __syncthreads(); // the accumulators are clear
 	constexpr int NW = BS / 64;
 	int const wave = tid >> 6;
 	// arrivals per wave and round: few ones are spread over all waves
@@ -359,8 +494,8 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 		if( x < tw )
 		{
 			std::int64_t const i = t0 + x;
-			typename N::tuple_t s;
-			load_tuple<N>( s, v.na, i );
+			typename N::tuple_t s = early;
+			if( !has_early || x != tid ) load_tuple<N>( s, v.na, i );
 			// plastic models: the arrivals of this neuron's own spikes (of the steps from T0 - D), its
 			// traces, and the history words that the window's steps go to
 			std::uint32_t arrivals = 0;

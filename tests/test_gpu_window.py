@@ -52,6 +52,26 @@ def test_windows_bit_exact(gpu, model, layout, delay, launch):
     d.close(), h.close()
 
 
+@pytest.mark.parametrize("model", ["vogels_abbott", "synth"])
+@pytest.mark.parametrize("p", [0.004, 0.02, 0.05, 0.1, 0.3])
+def test_segment_records_bit_exact(gpu, model, p):
+    """Delay 1: records of 16, 32, 64 and 128 bytes (segments of 1 to 26 targets, some longer than
+    their record) and segments too long for any; the tiles change on the way (Vogels: all neurons
+    fire at step 139)."""
+    lay = ([2500], [(0, 0, p)])
+    h = O.CpuSnn(model, lay, DT, 1, seed=23, fixed_point=True)
+    d = Snn(model, Layout(*lay), DT, 1, seed=23, fixed_point=True)
+    for w, block in ((256, 512), (320, 256), (64, 1024)):
+        d.set_launch(tile_w=w, recv_block=block)
+        d.run(149)
+        h.run(149)
+        assert_state_equal(d.neurons(), h.neurons(), f"tiles of {w}")
+        s = h.step(True)
+        np.testing.assert_array_equal(np.sort(d.step(True)), np.sort(s))
+    assert d.stats()["events"] > 0
+    d.close(), h.close()
+
+
 @pytest.mark.parametrize("delay", [1, 6])
 def test_fp32_inputs_past_the_tabulated_sums(gpu, delay):
     """Vogels-Abbott in fp32: the whole population's first spike gives every neuron hundreds of
