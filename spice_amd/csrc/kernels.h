@@ -1744,4 +1744,13 @@ static inline __global__ __launch_bounds__( 1024 ) void k_tp_scan( std::uint32_t
 		run += cnt[i];
 	}
 }
+
+// The first min(*count, most) words of src (most of them without a count) to host memory, after
+// their number.
+static inline __global__ __launch_bounds__( 1024 ) void k_stage( std::uint32_t const * src, std::uint32_t const * count, std::uint32_t most, std::uint32_t * host )
+{
+	std::uint32_t const c = count ? *count : most, n = c < most ? c : most, at = blockIdx.x * blockDim.x + threadIdx.x;
+	for( std::uint32_t k = at; k < n; k += gridDim.x * blockDim.x ) host[1 + k] = src[k];
+	if( at == 0 ) host[0] = c;
+}
 } // namespace spice::hipx

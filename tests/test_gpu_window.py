@@ -135,3 +135,22 @@ def test_imported_state_that_breaks_the_refractory_promise(gpu, batched):
         assert_state_equal(net.neurons(), h.neurons(), "neurons")
     assert_state_equal(net.synapses(ell=False), h.synapses(ell=False), "weights")
     h.close()
+
+
+@pytest.mark.parametrize("n", [16384, 16385, 20000])
+def test_spikes_and_state_read_back(gpu, n):
+    """Steps whose spikes (all neurons' at step 139) and networks whose state just fit, or do not
+    fit, the pinned buffer of 16,384 words that small answers come through."""
+    lay = ([n], [(0, 0, 0.0005)])
+    h = O.CpuSnn("vogels_abbott", lay, DT, 1, seed=3, fixed_point=True)
+    d = Snn("vogels_abbott", Layout(*lay), DT, 1, seed=3, fixed_point=True)
+    d.run(135), h.run(135)
+    sizes = []
+    for i in range(10):
+        want = np.sort(h.step(True))
+        np.testing.assert_array_equal(np.sort(d.step(True)), want, err_msg=f"step {135 + i}")
+        np.testing.assert_array_equal(np.sort(d.step_spikes_of_last()), want)
+        assert_state_equal(d.neurons(), h.neurons(), f"step {135 + i}")
+        sizes.append(len(want))
+    assert min(sizes) == 0 and max(sizes) == n
+    d.close(), h.close()
