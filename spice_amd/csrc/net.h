@@ -21,6 +21,7 @@
 #include <cstdint>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -36,6 +37,41 @@ struct net_params
 	std::uint32_t flags;
 	float param[4];
 	bool records = true; // segment records (window.h) where they pay: memory for speed
+};
+
+// Pinned memory through which the nets of this process read small answers back (their number and
+// `words` words): one buffer, held by the nets that use it.
+struct host_stage
+{
+	static constexpr std::uint32_t words = 16384;
+	std::uint32_t * host = nullptr;
+	std::mutex busy;
+
+	host_stage() = default;
+	host_stage( host_stage const & ) = delete;
+	~host_stage()
+	{
+		if( host ) (void)hipHostFree( host );
+	}
+
+	// nullptr: no memory
+	static std::shared_ptr<host_stage> get()
+	{
+		static std::mutex m;
+		static std::weak_ptr<host_stage> last;
+		std::lock_guard<std::mutex> g( m );
+		if( auto s = last.lock() ) return s;
+		auto s = std::make_shared<host_stage>();
+		void * p = nullptr;
+		if( hipHostMalloc( &p, ( words + 1 ) * 4, hipHostMallocPortable ) != hipSuccess )
+		{
+			(void)hipGetLastError();
+			return nullptr;
+		}
+		s->host = static_cast<std::uint32_t *>( p );
+		last = s;
+		return s;
+	}
 };
 
 struct launch_cfg
@@ -172,7 +208,6 @@ public:
 		_graphs.clear();
 		_queue.clear();
 		if( _s ) (void)hipStreamDestroy( _s );
-		if( _stage ) (void)hipHostFree( _stage );
 	}
 
 	// ---- simulation ----
@@ -243,10 +278,11 @@ public:
 		std::int32_t const * ids = _ring.data() + std::int64_t( slot ) * _g.n;
 		std::uint32_t const * cnt = _counts.data() + slot;
 		std::uint32_t c = 0;
-		bool const staged = stage_to_host( ids, cnt, STAGE_WORDS );
-		if( staged )
-			c = _stage[0];
-		else
+		bool const staged = stage_to_host( ids, cnt, host_stage::words, [&]( std::uint32_t const * words, std::uint32_t n ) {
+			c = n;
+			if( out && c <= cap && c <= host_stage::words ) std::memcpy( out, words, std::size_t( c ) * 4 );
+		} );
+		if( !staged )
 		{
 			SPICE_HIP( hipMemcpyAsync( &c, cnt, 4, hipMemcpyDeviceToHost, _s ) );
 			SPICE_HIP( hipStreamSynchronize( _s ) );
@@ -255,11 +291,7 @@ public:
 		if( out && c )
 		{
 			if( c > cap ) throw std::invalid_argument( "spike buffer too small" );
-			if( staged && c <= STAGE_WORDS )
-			{
-				std::memcpy( out, _stage + 1, std::size_t( c ) * 4 );
-				return;
-			}
+			if( staged && c <= host_stage::words ) return;
 			SPICE_HIP( hipMemcpyAsync( out, ids, std::size_t( c ) * 4, hipMemcpyDeviceToHost, _s ) );
 			SPICE_HIP( hipStreamSynchronize( _s ) );
 		}
@@ -370,11 +402,9 @@ public:
 	{
 		check_attr( a, int( N::size ) );
 		if( bytes != std::uint64_t( _g.n ) * attr_bytes<N>( a ) ) throw std::invalid_argument( "buffer size mismatch" );
-		if( _stage && bytes % 4 == 0 && bytes / 4 <= STAGE_WORDS && stage_to_host( _na[a].data(), nullptr, std::uint32_t( bytes / 4 ) ) )
-		{
-			std::memcpy( out, _stage + 1, bytes );
+		if( bytes % 4 == 0 && bytes / 4 <= host_stage::words &&
+		    stage_to_host( _na[a].data(), nullptr, std::uint32_t( bytes / 4 ), [&]( std::uint32_t const * words, std::uint32_t ) { std::memcpy( out, words, bytes ); } ) )
 			return;
-		}
 		synchronize();
 		SPICE_HIP( hipMemcpy( out, _na[a].data(), bytes, hipMemcpyDeviceToHost ) );
 	}
@@ -675,10 +705,8 @@ private:
 	int _window = 0;       // longest window of the window kernels that run the steps (0: none)
 	launch_queue _queue;
 	launch_cfg _lc{};
-	// a step's spikes, or a small net's neuron state, on their way to host memory (stage_to_host)
-	static constexpr std::uint32_t STAGE_WORDS = 16384;
-	std::uint32_t * _stage = nullptr; // pinned: their number and STAGE_WORDS words
-	int _staged = 0;                  // calls that asked for it
+	std::shared_ptr<host_stage> _stage; // see stage_to_host
+	int _staged = 0;                    // calls that asked for it
 	dbuf<std::int64_t> _pivots;
 	dbuf<unsigned char> _recs; // segment records
 	dbuf<std::int32_t> _tile_ids;
@@ -1104,7 +1132,7 @@ private:
 			if( plastic && _lazy ) return;
 			if( !plastic && !_ahead && ( _lc.recv_parts != 1 || _lc.tile_w > 4 * _lc.recv_block ) ) return;
 			_window = 1;
-			with_window_kernel( [&]( auto kernel, auto bytes, int ) {
+			with_window_kernel( false, [&]( auto kernel, auto bytes, int ) {
 				// the LDS of a CU, shared by the workgroups that a CU gets
 				std::size_t const per_cu = std::size_t( std::clamp( ( _v.ntiles + device_cu_count() - 1 ) / device_cu_count(), 1, 3 ) );
 				std::size_t const room = ( LDS_PER_CU - 4096 ) / per_cu;
@@ -1114,30 +1142,32 @@ private:
 				if( bytes( w ) > ( 64 << 10 ) )
 					SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( w ) ) ) );
 			} );
+			with_window_kernel( true, [&]( auto kernel, auto bytes, int ) { // (one step)
+				if( bytes( 1 ) > ( 64 << 10 ) )
+					SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( 1 ) ) ) );
+			} );
 		}
 	}
 
-	// Writes *count words of src (n of them without a count), at most n, and their number to the
-	// pinned buffer and waits: one small kernel in place of a copy of the count, a wait, a copy of
-	// the words and another wait (a step of 4,000 neurons and its spikes: 47.6 us with the copies).
-	// false: no buffer, nothing was done. It is allocated by the second call, as doing so takes
-	// longer than a few copies.
-	bool stage_to_host( void const * src, std::uint32_t const * count, std::uint32_t n )
+	// take(words, their number) of *count words of src (n of them without a count; n given at most),
+	// by way of the pinned buffer: one small kernel and one wait in place of a copy of the count, a
+	// wait, a copy of the words and another wait (a step of 4,000 neurons and its spikes: 47.6 us
+	// with the copies, 22 without). false: nothing was done, as another thread has the buffer, or
+	// there is none -- the second call gets it, as allocating it takes longer than a few copies.
+	template <typename F>
+	bool stage_to_host( void const * src, std::uint32_t const * count, std::uint32_t n, F && take )
 	{
 		if( !_stage )
 		{
 			if( ++_staged < 2 ) return false;
-			void * p = nullptr;
-			if( hipHostMalloc( &p, ( STAGE_WORDS + 1 ) * 4, hipHostMallocDefault ) != hipSuccess )
-			{
-				(void)hipGetLastError();
-				_staged = 0;
-				return false;
-			}
-			_stage = static_cast<std::uint32_t *>( p );
+			_stage = host_stage::get();
+			if( !_stage ) return false;
 		}
-		SPICE_LAUNCH( k_stage<<<4, 1024, 0, _s>>>( static_cast<std::uint32_t const *>( src ), count, n, _stage ) );
+		std::unique_lock<std::mutex> one( _stage->busy, std::try_to_lock );
+		if( !one ) return false;
+		SPICE_LAUNCH( k_stage<<<4, 1024, 0, _s>>>( static_cast<std::uint32_t const *>( src ), count, n, _stage->host ) );
 		SPICE_HIP( hipStreamSynchronize( _s ) );
+		take( _stage->host + 1, _stage->host[0] );
 		return true;
 	}
 
@@ -1315,7 +1345,7 @@ private:
 			if( alone ) launch_passes( t, _s );
 			if( _slog_ctl.size() ) throw std::logic_error( "nets with a spike log are stepped by a batch" );
 			dview v = _vs[t & ( CLOCK_SLOTS - 1 )];
-			with_window_kernel( [&]( auto kernel, auto bytes, int bs ) {
+			with_window_kernel( v.rec_lg != 0, [&]( auto kernel, auto bytes, int bs ) {
 				std::int32_t W = w;
 				void * args[] = { &v, &W };
 				void const * fn = reinterpret_cast<void const *>( kernel );
@@ -1329,12 +1359,13 @@ private:
 
 	// f(window kernel, its LDS bytes for w steps, workgroup size) of the launch shape
 	template <typename F>
-	void with_window_kernel( F && f )
+	void with_window_kernel( bool records, F && f )
 	{
 		auto go = [&]( auto fx, auto b ) {
 			constexpr bool FX = decltype( fx )::value;
 			constexpr int BS = decltype( b )::value;
-			f( &k_window<Model, FX, BS>, [&]( int w ) { return window_lds<Model, FX>::bytes( BS, _lc.tile_w, w ); }, BS );
+			f( records ? &k_window<Model, FX, BS, ( input_classes_v<Model> > 0 )> : &k_window<Model, FX, BS>,
+			   [&]( int w ) { return window_lds<Model, FX>::bytes( BS, _lc.tile_w, w ); }, BS );
 		};
 		auto by_block = [&]( auto fx ) {
 			int const bs = _lc.recv_block;

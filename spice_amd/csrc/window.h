@@ -234,7 +234,7 @@ __device__ inline std::uint32_t wave_inclusive_scan32( std::uint32_t x )
 __device__ inline std::int32_t window_entry( dview const & v ) { return v.rsize == CLOCK_SLOTS ? std::int32_t( v.ctl - v.ctl0 ) : v.ctl->rslot; }
 
 // The window [T0, T0 + W) of the tile at place `pos` of v.tile_ids.
-template <typename Model, bool FIXED, int BS>
+template <typename Model, bool FIXED, int BS, bool REC = false>
 __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 {
 	using N = typename Model::neuron;
@@ -281,8 +281,8 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	constexpr int REC_U = 4; // arrivals per group of lanes in flight
 	std::int32_t early_id[REC_U] = {};
 	if( active && lane < W ) incl = v.counts[entry( lane - v.D )];
-	if constexpr( L::classes > 0 )
-		if( active && v.rec_lg )
+	if constexpr( REC )
+		if( active )
 		{
 			int const gl = v.rec_lg - 4;
 #pragma unroll
@@ -294,7 +294,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 		}
 	// and the state of this thread's first neuron, used after the delivery
 	typename N::tuple_t early{};
-	bool const has_early = L::classes > 0 && v.rec_lg && tid < tw;
+	bool const has_early = REC && tid < tw;
 	if( has_early ) load_tuple<N>( early, v.na, t0 + tid );
 	for( int x = tid; x < int( sizeof( word ) * nacc * std::size_t( tws ) * std::size_t( W ) / 16 ); x += BS )
 		reinterpret_cast<uint4 *>( acc )[x] = uint4{ 0, 0, 0, 0 };
@@ -333,8 +333,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	};
 
 	std::uint32_t ev = 0;
-	if constexpr( L::classes > 0 )
-		if( v.rec_lg )
+	if constexpr( REC )
 		{
 			// Delivery from records: a group of 2^(rec_lg - 4) lanes per arrival, 16 bytes each, U
 			// arrivals per group in flight; nothing is staged.
@@ -394,7 +393,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	// Delivery, wave by wave: a wave stages up to 64 of the window's arrivals at a time (one segment
 	// each) in its own part of the LDS and walks them; the next ones' ids and segment bounds are
 	// read beside the walk. No wave waits for another before the update.
-	if( L::classes == 0 || !v.rec_lg ) __syncthreads(); // the accumulators are clear
+	if constexpr( !REC ) __syncthreads(); // the accumulators are clear
 	constexpr int NW = BS / 64;
 	int const wave = tid >> 6;
 	// arrivals per wave and round: few ones are spread over all waves
@@ -920,12 +919,14 @@ __global__ __launch_bounds__( 256 ) void k_window_passes( dview v )
 
 // One workgroup per tile, those with incoming synapses first; then (plastic models) the
 // workgroups of the passes of the window before.
-template <typename Model, bool FIXED, int BS>
+// REC: one step, from segment records (an instance of its own: in the others the registers of
+// its delivery cost 2 % -- Brunel 1e6 0.88 us per step, 0.90 with it inside).
+template <typename Model, bool FIXED, int BS, bool REC = false>
 __global__ __launch_bounds__( BS ) void k_window( dview v, std::int32_t W )
 {
 	std::int32_t const b = blockIdx.x;
 	if( b < v.ntiles )
-		window_tile<Model, FIXED, BS>( v, b < v.nact ? xcd_place( b, v.nact ) : b, W );
+		window_tile<Model, FIXED, BS, REC>( v, b < v.nact ? xcd_place( b, v.nact ) : b, REC ? 1 : W );
 	else if constexpr( is_plastic_v<Model> )
 		window_passes<Model, FIXED>( v, b - v.ntiles, std::int32_t( gridDim.x ) - v.ntiles, v.ntiles );
 }
