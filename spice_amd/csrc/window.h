@@ -66,6 +66,18 @@ constexpr int longest_window_v = !overlap_capable_v<Model> ? 1
                                  : is_plastic_v<Model>     ? ( refractory_steps_v<typename Model::synapse> + 1 ) / 2
                                                            : WINDOW_MAX;
 
+// WIN_VEC consecutive target ids, from any entry of the row store.
+struct targets
+{
+	std::int32_t id[WIN_VEC];
+};
+__device__ inline targets load_targets( std::int32_t const * p )
+{
+	targets t;
+	__builtin_memcpy( &t, p, sizeof( t ) ); // one 16-byte load (4-byte alignment suffices)
+	return t;
+}
+
 // ---- segment records -------------------------------------------------------------------------
 // For models with input classes a delivery needs of a row's segment in a tile only the targets, and
 // those fit 16 bits inside a tile. Where segments are short and the network runs step by step, each
@@ -91,6 +103,7 @@ static inline __global__ __launch_bounds__( 256 ) void k_records( dview v, unsig
 	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
 	if( r >= v.N ) return;
 	std::int64_t const * pv = v.pivots + r * ( v.ntiles + 1 );
+	std::int64_t const nnz = v.row_ptr[v.N];
 	int const cap = rec_capacity( lg );
 	for( int t = lane_id(); t < v.ntiles; t += 64 )
 	{
@@ -107,20 +120,19 @@ static inline __global__ __launch_bounds__( 256 ) void k_records( dview v, unsig
 			atomicAdd( longs, 1ull );
 			continue;
 		}
-		std::int32_t const * c = v.col + a;
-		rec_part p{};
-		p.t[0] = std::uint16_t( len );
+		std::int32_t before = len; // what the part's first 16 bits hold: the length, then the target before the part's
 		for( int i = 0; i < 1 << ( lg - 4 ); i++ )
 		{
-			// entries 8 i - 1 .. 8 i + 6 of the segment (the row store is padded past its end)
+			// entries 8 i - 1 .. 8 i + 6 of the segment; a piece that starts past the last edge holds
+			// none of them (the row store is padded by one piece)
+			targets const c[2] = { load_targets( v.col + std::min( a + 8 * i, nnz ) ), load_targets( v.col + std::min( a + 8 * i + 4, nnz ) ) };
+			rec_part p;
+			p.t[0] = std::uint16_t( before );
 #pragma unroll
-			for( int x = 0; x < 8; x++ )
-			{
-				int const e = 8 * i + x - 1;
-				if( e >= 0 && e < len ) p.t[x] = std::uint16_t( c[e] - t0 );
-			}
+			for( int x = 0; x < 7; x++ ) p.t[x + 1] = std::uint16_t( c[x / 4].id[x % 4] - t0 ); // (past the segment's end: never read as a target)
+			before = c[1].id[3] - t0;
 			out[i] = p;
-			if( 8 * i + 7 >= len ) break; // (what follows is never read as a target)
+			if( 8 * i + 7 >= len ) break;
 		}
 	}
 }
@@ -178,18 +190,6 @@ __device__ inline auto class_sum( std::uint32_t n, T value, float const * table,
 		for( std::uint32_t k = WIN_TABLE - 1; k < n; k++ ) x += value;
 		return x;
 	}
-}
-
-// WIN_VEC consecutive target ids, from any entry of the row store.
-struct targets
-{
-	std::int32_t id[WIN_VEC];
-};
-__device__ inline targets load_targets( std::int32_t const * p )
-{
-	targets t;
-	__builtin_memcpy( &t, p, sizeof( t ) ); // one 16-byte load (4-byte alignment suffices)
-	return t;
 }
 
 // The state of WIN_VEC consecutive synapses.
