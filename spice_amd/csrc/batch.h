@@ -129,14 +129,28 @@ public:
 				                                       : reinterpret_cast<void const *>( &k_batch_window<Model, false, window_block> ),
 				                                hipFuncAttributeMaxDynamicSharedMemorySize, int( _lds ) ) );
 		}
-		upload( _tile_net, tn );
-		upload( _tile_local, tl );
-		upload( _block_net, bn );
-		upload( _block_local, bl );
-		upload( _flush_net, fn );
-		upload( _flush_local, fl );
-		upload( _flush_count, fc );
-		for( int p = 0; p < CLOCK_SLOTS; p++ ) upload( _views[p], vs[p] );
+		// all tables in one buffer and one copy
+		std::vector<unsigned char> all;
+		auto put = [&]( auto const & h ) { // the place of h's copy
+			std::size_t const at = ( all.size() + 255 ) / 256 * 256;
+			all.resize( at + h.size() * sizeof( h[0] ) );
+			if( !h.empty() ) std::memcpy( all.data() + at, h.data(), h.size() * sizeof( h[0] ) );
+			return at;
+		};
+		std::size_t at[7], at_views[CLOCK_SLOTS];
+		{
+			int k = 0;
+			for( auto const * h : { &tn, &tl, &bn, &bl, &fn, &fl, &fc } ) at[k++] = put( *h );
+		}
+		for( int p = 0; p < CLOCK_SLOTS; p++ ) at_views[p] = put( vs[p] );
+		_tables.resize( all.size() );
+		SPICE_HIP( hipMemcpyAsync( _tables.data(), all.data(), all.size(), hipMemcpyHostToDevice, _s ) );
+		{
+			int k = 0;
+			for( auto * table : { &_tile_net, &_tile_local, &_block_net, &_block_local, &_flush_net, &_flush_local, &_flush_count } )
+				*table = reinterpret_cast<std::int32_t const *>( _tables.data() + at[k++] );
+		}
+		for( int p = 0; p < CLOCK_SLOTS; p++ ) _views[p] = reinterpret_cast<dview const *>( _tables.data() + at_views[p] );
 		_grid_tiles = std::min( _ntiles, ( recv_block == 256 ? SPICE_BATCH_GRID_PER_CU : SPICE_BATCH_GRID_PER_CU / 4 ) * device_cu_count() );
 		for( auto * n : _nets ) n->synchronize();
 		SPICE_HIP( hipStreamSynchronize( _s ) );
@@ -205,7 +219,7 @@ public:
 	{
 		for( auto * net : _nets ) net->note_spike_log( nsteps ); // validates nsteps first
 		std::int32_t const n = std::int32_t( _nets.size() );
-		SPICE_LAUNCH( k_batch_log_window<<<unsigned( ( n + 255 ) / 256 ), 256, 0, _s>>>( _views[_step & ( CLOCK_SLOTS - 1 )].data(), n, nsteps ) );
+		SPICE_LAUNCH( k_batch_log_window<<<unsigned( ( n + 255 ) / 256 ), 256, 0, _s>>>( _views[_step & ( CLOCK_SLOTS - 1 )], n, nsteps ) );
 	}
 
 	void synchronize() override
@@ -240,16 +254,10 @@ private:
 	std::int64_t _step = 0;
 	std::int32_t _ntiles = 0, _nblocks = 0, _nflush = 0;
 	int _grid_tiles = 0;
-	dbuf<std::int32_t> _tile_net, _tile_local, _block_net, _block_local, _flush_net, _flush_local, _flush_count;
-	dbuf<dview> _views[CLOCK_SLOTS];
-
-	template <typename T>
-	void upload( dbuf<T> & d, std::vector<T> const & h )
-	{
-		d.resize( std::max<std::size_t>( h.size(), 1 ) );
-		if( !h.empty() ) SPICE_HIP( hipMemcpyAsync( d.data(), h.data(), h.size() * sizeof( T ), hipMemcpyHostToDevice, _s ) );
-		SPICE_HIP( hipStreamSynchronize( _s ) );
-	}
+	dbuf<unsigned char> _tables; // all of these:
+	std::int32_t const *_tile_net = nullptr, *_tile_local = nullptr, *_block_net = nullptr, *_block_local = nullptr;
+	std::int32_t const *_flush_net = nullptr, *_flush_local = nullptr, *_flush_count = nullptr;
+	dview const * _views[CLOCK_SLOTS] = {};
 
 	// n steps from batch step t in windows of up to `most`; each appends its predecessor's spikes
 	// to the nets' logs, and a last kernel the last one's. alone: the passes before each in kernels
@@ -271,7 +279,7 @@ private:
 			t += w;
 			n -= w;
 		}
-		if( _logged ) SPICE_LAUNCH( k_batch_log<<<unsigned( _nets.size() ), 256, 0, _s>>>( _views[t & ( CLOCK_SLOTS - 1 )].data(), before ) );
+		if( _logged ) SPICE_LAUNCH( k_batch_log<<<unsigned( _nets.size() ), 256, 0, _s>>>( _views[t & ( CLOCK_SLOTS - 1 )], before ) );
 	}
 
 	template <bool F>
@@ -281,8 +289,8 @@ private:
 		unsigned const grid = unsigned( _ntiles + nplast ) + ( _logged && before ? unsigned( _nets.size() ) : 0u );
 		if constexpr( windowed )
 			SPICE_LAUNCH( ( k_batch_window<Model, F, window_block><<<grid, window_block, _lds, _s>>>(
-			    _views[t & ( CLOCK_SLOTS - 1 )].data(), _tile_net.data(), _tile_local.data(), _ntiles, w, before, _flush_net.data(),
-			    _flush_local.data(), _flush_count.data(), nplast ) ) );
+			    _views[t & ( CLOCK_SLOTS - 1 )], _tile_net, _tile_local, _ntiles, w, before, _flush_net,
+			    _flush_local, _flush_count, nplast ) ) );
 	}
 
 	// Same schedules as hip_net::launch_steps: windows of one step, or two kernels per step
@@ -306,11 +314,11 @@ private:
 	{
 		if constexpr( !windowed || factored_v<Model> )
 		{
-			dview const * v = _views[t & ( CLOCK_SLOTS - 1 )].data();
+			dview const * v = _views[t & ( CLOCK_SLOTS - 1 )];
 			unsigned const grid = unsigned( _grid_tiles + ( plastic ? _nflush : 0 ) );
-			SPICE_LAUNCH( k_batch_receive<Model, F, recv_block><<<grid, recv_block, 0, _s>>>( v, _tile_net.data(), _tile_local.data(), _ntiles, _grid_tiles,
-			                                                                                    _flush_net.data(), _flush_local.data(), _flush_count.data() ) );
-			SPICE_LAUNCH( k_batch_update<Model, F><<<_nblocks, 256, 0, _s>>>( v, _block_net.data(), _block_local.data() ) );
+			SPICE_LAUNCH( k_batch_receive<Model, F, recv_block><<<grid, recv_block, 0, _s>>>( v, _tile_net, _tile_local, _ntiles, _grid_tiles,
+			                                                                                    _flush_net, _flush_local, _flush_count ) );
+			SPICE_LAUNCH( k_batch_update<Model, F><<<_nblocks, 256, 0, _s>>>( v, _block_net, _block_local ) );
 		}
 	}
 };

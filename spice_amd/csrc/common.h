@@ -8,6 +8,7 @@
 #include <stdexcept>
 #include <string>
 #include <utility>
+#include <vector>
 
 namespace spice::hipx
 {
@@ -27,6 +28,71 @@ inline void check( hipError_t e, char const * what )
 		::spice::hipx::check( hipGetLastError(), "kernel launch" );   \
 	} while( 0 )
 
+// Small buffers that live and end together: blocks of device memory, freed by the destructor. A
+// buffer that a thread allocates inside an arena::scope comes from the scope's arena, if it is
+// small (an allocation and its end take 20 us; a net has about twenty small buffers).
+class arena
+{
+public:
+	static constexpr size_t LARGEST = size_t( 128 ) << 10, BLOCK = size_t( 512 ) << 10;
+
+	class scope
+	{
+	public:
+		explicit scope( arena & a )
+		    : _before( std::exchange( current(), &a ) )
+		{
+		}
+		~scope() { current() = _before; }
+		scope( scope const & ) = delete;
+
+	private:
+		arena * _before;
+	};
+
+	arena() = default;
+	arena( arena const & ) = delete;
+	arena & operator=( arena const & ) = delete;
+	~arena()
+	{
+		for( void * b : _blocks ) (void)hipFree( b );
+	}
+
+	static arena *& current()
+	{
+		static thread_local arena * a = nullptr;
+		return a;
+	}
+
+	// At most LARGEST bytes, aligned to 256.
+	void * take( size_t bytes )
+	{
+		bytes = ( bytes + 255 ) / 256 * 256;
+		if( bytes > _left )
+		{
+			_blocks.reserve( _blocks.size() + 1 );
+			void * b = nullptr;
+			if( hipMalloc( &b, BLOCK ) != hipSuccess )
+			{
+				(void)hipGetLastError();
+				throw std::bad_alloc();
+			}
+			_blocks.push_back( b );
+			_at = static_cast<char *>( b );
+			_left = BLOCK;
+		}
+		void * const p = _at;
+		_at += bytes;
+		_left -= bytes;
+		return p;
+	}
+
+private:
+	std::vector<void *> _blocks;
+	char * _at = nullptr;
+	size_t _left = 0;
+};
+
 // Owning device allocation (reference counterpart: dbuffer, spice/cuda/util/dbuffer.h:17-90).
 template <typename T>
 class dbuf
@@ -40,6 +106,7 @@ public:
 	dbuf( dbuf && o ) noexcept
 	    : _p( std::exchange( o._p, nullptr ) )
 	    , _n( std::exchange( o._n, 0 ) )
+	    , _own( o._own )
 	{
 	}
 	dbuf & operator=( dbuf && o ) noexcept
@@ -47,6 +114,7 @@ public:
 		release();
 		_p = std::exchange( o._p, nullptr );
 		_n = std::exchange( o._n, 0 );
+		_own = o._own;
 		return *this;
 	}
 
@@ -54,6 +122,14 @@ public:
 	{
 		release();
 		if( n == 0 ) return;
+		arena * const a = arena::current();
+		_own = !a || n > arena::LARGEST / sizeof( T );
+		if( !_own )
+		{
+			_p = static_cast<T *>( a->take( n * sizeof( T ) ) );
+			_n = n;
+			return;
+		}
 		void * p = nullptr;
 		hipError_t e = hipMalloc( &p, n * sizeof( T ) );
 		if( e != hipSuccess )
@@ -66,7 +142,7 @@ public:
 	}
 	void release()
 	{
-		if( _p ) (void)hipFree( _p );
+		if( _p && _own ) (void)hipFree( _p );
 		_p = nullptr;
 		_n = 0;
 	}
@@ -78,6 +154,7 @@ public:
 private:
 	T * _p = nullptr;
 	size_t _n = 0;
+	bool _own = true; // not an arena's
 };
 
 // ---- wave64 helpers ----------------------------------------------------------------------

@@ -71,7 +71,8 @@ inline hipStream_t new_stream()
 	return s;
 }
 
-// The net takes ownership of `s` once constructed; on failure `s` is destroyed here.
+// The net takes ownership of `s` once constructed; on failure `s` is destroyed here (unless the
+// stream is the caller's: net_params::own_stream).
 inline net_iface * make_net( net_params const & p, csr_dev && g, hipStream_t s )
 {
 	try
@@ -90,7 +91,7 @@ inline net_iface * make_net( net_params const & p, csr_dev && g, hipStream_t s )
 	}
 	catch( ... )
 	{
-		(void)hipStreamDestroy( s );
+		if( p.own_stream ) (void)hipStreamDestroy( s );
 		throw;
 	}
 }

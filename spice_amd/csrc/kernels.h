@@ -1753,4 +1753,14 @@ static inline __global__ __launch_bounds__( 1024 ) void k_stage( std::uint32_t c
 	for( std::uint32_t k = at; k < n; k += gridDim.x * blockDim.x ) host[1 + k] = src[k];
 	if( at == 0 ) host[0] = c;
 }
+
+// A spike log's n steps to host memory: where each step's ids start (`start`), the end (the last
+// step has *last of them), and the ids, at most cap.
+static inline __global__ __launch_bounds__( 1024 ) void k_log_out( std::uint64_t const * start, std::int64_t n, std::uint32_t const * last, std::int32_t const * ids,
+                                                                 std::uint64_t cap, std::uint64_t * host_start, std::int32_t * host_ids )
+{
+	std::uint64_t const total = start[n - 1] + *last, copied = total < cap ? total : cap, at = blockIdx.x * blockDim.x + threadIdx.x, all = gridDim.x * blockDim.x;
+	for( std::uint64_t k = at; k <= std::uint64_t( n ); k += all ) host_start[k] = k < std::uint64_t( n ) ? start[k] : total;
+	for( std::uint64_t k = at; k < copied; k += all ) host_ids[k] = ids[k];
+}
 } // namespace spice::hipx

@@ -36,7 +36,8 @@ struct net_params
 	std::uint64_t seed;
 	std::uint32_t flags;
 	float param[4];
-	bool records = true; // segment records (window.h) where they pay: memory for speed
+	bool records = true;    // segment records (window.h) where they pay: memory for speed
+	bool own_stream = true; // the net destroys its stream (on failure: make_net does)
 };
 
 // Pinned memory through which the nets of this process read small answers back (their number and
@@ -108,9 +109,9 @@ struct net_iface
 	// Spike log (served jobs). enable_spike_log allocates a log of `cap` ids for windows of at
 	// most `max_steps` steps (before the first run); begin_spike_log opens a window over the
 	// next `nsteps` steps; once the net has run exactly those steps, read_spike_log copies the
-	// window out: off[0..nsteps] (off[k] = first id of step t0+k, off[nsteps] = total) and the
-	// ids, and returns the total (> cap: the log overflowed, ids past cap were dropped). No step
-	// of the net may be in flight during begin/read.
+	// window out, to pinned memory: off[0..nsteps] (off[k] = first id of step t0+k, off[nsteps] =
+	// total) and the ids, and returns the total (> cap: the log overflowed, ids past cap were
+	// dropped). No step of the net may be in flight during begin/read.
 	virtual void enable_spike_log( std::uint64_t cap, std::int64_t max_steps ) = 0;
 	virtual void begin_spike_log( std::int64_t nsteps ) = 0;
 	virtual std::uint64_t read_spike_log( std::uint64_t * off, std::int32_t * ids, std::uint64_t cap ) = 0;
@@ -198,6 +199,7 @@ public:
 		if( _g.n < 1 || _g.n > INT_MAX - 1024 ) throw std::invalid_argument( "invalid neuron count" );
 		static_assert( N::size <= MAXA && S::size <= MAXA, "at most 16 neuron/synapse attributes" );
 		_ahead = overlap_capable_v<Model> && p.delay >= 2;
+		arena::scope const small( _arena );
 		allocate( first );
 		initialize();
 	}
@@ -207,7 +209,7 @@ public:
 		if( _s ) (void)hipStreamSynchronize( _s );
 		_graphs.clear();
 		_queue.clear();
-		if( _s ) (void)hipStreamDestroy( _s );
+		if( _s && _p.own_stream ) (void)hipStreamDestroy( _s );
 	}
 
 	// ---- simulation ----
@@ -481,6 +483,7 @@ public:
 	{
 		if( !_graphs.empty() || _slog_ctl.size() ) throw std::logic_error( "the spike log is enabled once, before the first run" );
 		if( max_steps < 1 ) throw std::invalid_argument( "spike log window must hold at least one step" );
+		arena::scope const small( _arena );
 		_slog_ctl.resize( 1 );
 		_slog_ids.resize( std::max<std::uint64_t>( cap, 1 ) );
 		_slog_off.resize( std::size_t( max_steps ) );
@@ -520,14 +523,10 @@ public:
 		if( _step != _slog_t0 + _slog_n ) throw std::logic_error( "spike log window not completed" );
 		off[0] = 0;
 		if( _slog_n == 0 ) return 0;
-		SPICE_HIP( hipMemcpy( off, _slog_off.data(), std::size_t( _slog_n ) * 8, hipMemcpyDeviceToHost ) );
-		std::uint32_t last = 0;
-		int const slot = int( ( _step - 1 ) % _v.rsize );
-		SPICE_HIP( hipMemcpy( &last, _counts.data() + slot, 4, hipMemcpyDeviceToHost ) );
-		std::uint64_t const total = off[_slog_n - 1] + last;
-		off[_slog_n] = total;
-		std::uint64_t const n = std::min( { total, _slog_cap, cap } );
-		if( n ) SPICE_HIP( hipMemcpy( ids, _slog_ids.data(), std::size_t( n ) * 4, hipMemcpyDeviceToHost ) );
+		SPICE_LAUNCH( k_log_out<<<16, 1024, 0, _s>>>( _slog_off.data(), _slog_n, _counts.data() + ( _step - 1 ) % _v.rsize, _slog_ids.data(),
+		                                              std::min( _slog_cap, cap ), off, ids ) );
+		SPICE_HIP( hipStreamSynchronize( _s ) );
+		std::uint64_t const total = off[_slog_n];
 		return total;
 	}
 
@@ -572,7 +571,9 @@ public:
 			SPICE_HIP( hipMemcpyAsync( g.row_ptr.data(), _g.row_ptr.data(), _g.row_ptr.bytes(), hipMemcpyDeviceToDevice, s ) );
 			SPICE_HIP( hipMemcpyAsync( g.col.data(), _g.col.data(), _g.col.bytes(), hipMemcpyDeviceToDevice, s ) );
 			SPICE_HIP( hipStreamSynchronize( s ) );
-			auto * c = new hip_net( _p, std::move( g ), s );
+			net_params p = _p;
+			p.own_stream = true;
+			auto * c = new hip_net( p, std::move( g ), s );
 			s = nullptr; // owned by c
 			if constexpr( factored )
 			{
@@ -667,6 +668,7 @@ public:
 
 private:
 	net_params _p;
+	arena _arena; // the small ones of the buffers below
 	csr_dev _g;
 	hipStream_t _s = nullptr;
 	step_graphs _graphs;

@@ -102,6 +102,7 @@ public:
 	{
 		_batches.clear();
 		for( auto & kv : _streams ) (void)hipStreamDestroy( kv.second );
+		if( _build ) (void)hipStreamDestroy( _build );
 		if( _off ) (void)hipHostFree( _off );
 		if( _ids ) (void)hipHostFree( _ids );
 	}
@@ -109,21 +110,14 @@ public:
 	std::unique_ptr<handle> create( spec const & s, serve::job_record & r )
 	{
 		SPICE_HIP( hipSetDevice( _dev ) );
-		hipStream_t st = new_stream();
-		csr_dev g;
-		try
-		{
-			g = generate_csr( s.conns, s.n, s.width, s.p.seed, st );
-		}
-		catch( ... )
-		{
-			(void)hipStreamDestroy( st );
-			throw;
-		}
+		// one stream for the construction and the queries of all jobs (this thread's work, and never
+		// steps): creating one per job took 0.3 ms each
+		if( !_build ) _build = new_stream();
 		auto h = std::make_unique<handle>();
 		net_params p = s.p;
 		p.records = false;
-		h->net.reset( make_net( p, std::move( g ), st ) );
+		p.own_stream = false;
+		h->net.reset( make_net( p, generate_csr( s.conns, s.n, s.width, s.p.seed, _build ), _build ) );
 		h->model = s.p.model;
 		h->fixed = ( s.p.flags & SPICE_FLAG_FIXED_POINT ) != 0;
 		h->net->enable_spike_log( spike_log_capacity( s.n, _chunk_max, s.p.dt ), _chunk_max );
@@ -192,6 +186,7 @@ private:
 	std::int64_t _chunk_max;
 	int _dev = 0;
 	std::map<std::pair<int, bool>, hipStream_t> _streams;
+	hipStream_t _build = nullptr; // the nets'
 	std::vector<std::unique_ptr<batch_iface>> _batches;
 	std::uint64_t * _off = nullptr;
 	std::int32_t * _ids = nullptr;
