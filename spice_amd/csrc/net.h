@@ -1188,7 +1188,7 @@ private:
 			double const mean = double( _g.nnz ) / double( _g.n ) / _v.nact, need = mean + 2.9 * std::sqrt( mean );
 			int lg = 4;
 			while( lg < 8 && rec_capacity( lg ) < need ) lg++;
-			std::uint64_t const segs = std::uint64_t( _g.n ) * std::uint64_t( _v.ntiles ), bytes = segs << lg;
+			std::uint64_t const segs = std::uint64_t( _g.n ) * std::uint64_t( ( ( _v.ntiles - 1 ) >> REC_TILES ) + 1 ) << REC_TILES, bytes = segs << lg;
 			if( _v.wcap > 1 || _window == 0 || !_p.records || lg > 7 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
 			if( bytes > ( std::uint64_t( 1 ) << 30 ) )
 			{

@@ -86,16 +86,35 @@ __device__ inline targets load_targets( std::int32_t const * p )
 // unaligned piece of the row store; the chain of dependent accesses that bounds such a step loses
 // two links, as the arrivals' ids are read beside their count. A segment that does not fit has
 // REC_LONG for its length, then (at bytes 4 and 8) its true length and its place in col.
-// us per step, without and with: synth 1e9 (5 targets per segment) 30.1, 25.7; Vogels 1e8 7.8, 6.6.
+// us per step, without and with: synth 1e9 (5 targets per segment) 30.1, 21.7; Vogels 1e8 7.8, 6.5.
 // Windows of several steps gain less (Vogels 1e9, delay 8: 7.55, 7.0) than the records cost where
 // a network is built (5 ms), so they have none. Spike lists per tile instead of one per step, which
 // need no atomic, were slower to read (8.5 and 28.3).
 constexpr std::uint16_t REC_LONG = 0xffff;
 HYBRID constexpr int rec_capacity( int lg ) { return ( 1 << lg ) / 2 - 1; }
+// The place of row r's record of tile t: the records of 2^REC_TILES tiles of a row lie side by side,
+// then those of the next row. A tile's deliveries thus stay within one part of the memory, whose
+// page translations a CU can hold, and a line of small records still serves several tiles (synth
+// 1e9, 3.3 GB of records: 21.7 us per step with 8 tiles, 21.9 with 4, 23.3 with 32, 24.0 row by row).
+constexpr int REC_TILES = 3;
+__device__ inline std::int64_t rec_at( dview const & v, std::int64_t r, std::int32_t t )
+{
+	return ( ( std::int64_t( t >> REC_TILES ) * v.N + r ) << REC_TILES ) + ( t & ( ( 1 << REC_TILES ) - 1 ) );
+}
 struct alignas( 16 ) rec_part // 16 bytes of a record
 {
 	std::uint16_t t[8];
 };
+
+// The number of the x-th of the BS >> gl groups of lanes that deliver records to a tile: the tiles
+// that share lines begin at different arrivals, so that not all of them wait for the same line's
+// first read (synth 1e9, 24.0 us per step, 25.0 without).
+template <int BS>
+__device__ inline int rec_group( int x, int gl, std::int32_t tile )
+{
+	int const ng = BS >> gl;
+	return ( x + ( ( tile & ( ( 1 << REC_TILES ) - 1 ) ) * ng >> REC_TILES ) ) & ( ng - 1 );
+}
 
 // Builds the records, one wave per row, a lane per tile; *longs counts the segments that do not fit.
 static inline __global__ __launch_bounds__( 256 ) void k_records( dview v, unsigned char * recs, int lg, unsigned long long * longs )
@@ -109,7 +128,7 @@ static inline __global__ __launch_bounds__( 256 ) void k_records( dview v, unsig
 	{
 		std::int64_t const a = pv[t];
 		std::int32_t const len = std::int32_t( pv[t + 1] - a ), t0 = t * v.tile_w;
-		rec_part * const out = reinterpret_cast<rec_part *>( recs + ( ( r * v.ntiles + t ) << lg ) );
+		rec_part * const out = reinterpret_cast<rec_part *>( recs + ( rec_at( v, r, t ) << lg ) );
 		if( len > cap )
 		{
 			rec_part p{};
@@ -288,7 +307,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 #pragma unroll
 			for( int u = 0; u < REC_U; u++ )
 			{
-				std::int32_t const k = u * ( BS >> gl ) + ( tid >> gl );
+				std::int32_t const k = u * ( BS >> gl ) + rec_group<BS>( tid >> gl, gl, tile );
 				early_id[u] = v.ring[std::int64_t( entry( -v.D ) ) * v.N + ( k < v.N ? k : 0 )];
 			}
 		}
@@ -338,7 +357,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 			// Delivery from records: a group of 2^(rec_lg - 4) lanes per arrival, 16 bytes each, U
 			// arrivals per group in flight; nothing is staged.
 			constexpr int U = REC_U;
-			int const gl = v.rec_lg - 4, ng = BS >> gl, g = tid >> gl, l = tid & ( ( 1 << gl ) - 1 );
+			int const gl = v.rec_lg - 4, ng = BS >> gl, g = rec_group<BS>( tid >> gl, gl, tile ), l = tid & ( ( 1 << gl ) - 1 );
 			auto const * recs = reinterpret_cast<rec_part const *>( v.recs );
 			for( std::int32_t c = 0; c < total; c += U * ng )
 			{
@@ -358,7 +377,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 				for( int u = 0; u < U; u++ )
 				{
 					r[u] = rec_part{};
-					if( c + u * ng < total ) r[u] = recs[( ( std::int64_t( src[u] ) * v.ntiles + tile ) << gl ) + l];
+					if( c + u * ng < total ) r[u] = recs[( rec_at( v, src[u], tile ) << gl ) + l];
 					at[u] = N::input_class( src[u], info ) * tws;
 				}
 				if( c == 0 ) __syncthreads(); // the accumulators are clear
@@ -376,7 +395,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 						if( ( x > 0 || l > 0 ) && e0 + x < len ) atomicAdd( acc + ( at[u] + r[u].t[x] ), 1u );
 					if( ok[u] && head == REC_LONG )
 					{
-						rec_part const whole = recs[( std::int64_t( src[u] ) * v.ntiles + tile ) << gl];
+						rec_part const whole = recs[rec_at( v, src[u], tile ) << gl];
 						std::int32_t n;
 						std::int64_t off;
 						__builtin_memcpy( &n, &whole.t[2], 4 );
