@@ -10,7 +10,7 @@
 //   acc[a]   receive accumulators of attribute a  [2][N] by step parity: fp32 / int64 (fixed
 //                        point) / int32
 //   sa[a]    attribute a of every synapse         CSR order (plastic models only)
-//   ring     int32[rsize * N], counts uint32[rsize] spike ids of the last steps (entry t mod
+//   ring     int32[rsize * N], counts uint32[rsize * COUNT_STRIDE] spike ids of the last steps (entry t mod
 //                        rsize; rsize >= D + 2 wcap: the last step of a window of W <= wcap steps
 //                        clears the entries of the wcap steps after it, while step T - D's may
 //                        still be read; never-written entries are empty)
@@ -105,6 +105,12 @@ struct alignas( 8 ) tp_entry
 	std::int32_t off;
 	std::int32_t src;
 };
+
+// The spike counters of successive steps lie this many words apart: all tiles reserve their places
+// of all of a window's steps at about the same time, and atomics on one line wait for each other, 9
+// ns each (us per step with the counters side by side and apart: Vogels 1e9, delay 8, 250 tiles: 7.5
+// and 5.8; Brunel 1e10, 495 tiles: 18.0 and 17.2; brunel_with_plasticity 6e8: 13.1 and 12.5).
+constexpr int COUNT_STRIDE = 64;
 
 struct dview
 {

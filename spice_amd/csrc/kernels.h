@@ -798,7 +798,7 @@ __device__ inline void receive_tile( dview const & v, std::int32_t work )
 
 	std::int64_t const T = v.ctl->step;
 	int const slot = ring_at( v, -v.D ); // ring entry of step T - D
-	std::int32_t const nall = T < v.D ? 0 : std::int32_t( v.counts[slot] );
+	std::int32_t const nall = T < v.D ? 0 : std::int32_t( v.counts[slot * COUNT_STRIDE] );
 	std::int32_t const s_beg = std::int32_t( std::int64_t( nall ) * part / v.rparts );
 	std::int32_t const nspk = std::int32_t( std::int64_t( nall ) * ( part + 1 ) / v.rparts ) - s_beg;
 	if( v.slog && work == 0 && threadIdx.x == 0 )
@@ -806,7 +806,7 @@ __device__ inline void receive_tile( dview const & v, std::int32_t work )
 		// spike log: step T's ids start where step T-1's (final by now) end
 		std::int64_t const k = T - v.slog->t0;
 		if( k >= 0 && k < v.slog->nsteps )
-			v.slog_off[k] = k == 0 ? 0ull : v.slog_off[k - 1] + v.counts[ring_at( v, -1 )];
+			v.slog_off[k] = k == 0 ? 0ull : v.slog_off[k - 1] + v.counts[ring_at( v, -1 ) * COUNT_STRIDE];
 	}
 	std::int32_t const * spk = v.ring + std::int64_t( slot ) * v.N + s_beg;
 	float const dt = step_dt( v );
@@ -1157,7 +1157,7 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 	std::int64_t const T = v.ctl->step;
 	int const wslot = ring_at( v, 0 );
 	// the next wcap steps' counters (the entries were last delivered before this step)
-	if( first == 0 && std::int32_t( threadIdx.x ) < v.wcap ) v.counts[ring_at( v, 1 + std::int32_t( threadIdx.x ) )] = 0;
+	if( first == 0 && std::int32_t( threadIdx.x ) < v.wcap ) v.counts[ring_at( v, 1 + std::int32_t( threadIdx.x ) ) * COUNT_STRIDE] = 0;
 	if( first == 0 && threadIdx.x == 0 )
 	{
 		if constexpr( plastic ) v.fl_count[( T + 1 ) & 3] = 0; // step T - 1's flush may still read slot (T - 1) & 3
@@ -1342,7 +1342,7 @@ __device__ inline void update_range( dview const & v, std::int64_t first, std::i
 			t1 += b;
 			t2 += c;
 		}
-		bbase[0] = t0 ? atomicAdd( &v.counts[wslot], t0 ) : 0u;
+		bbase[0] = t0 ? atomicAdd( &v.counts[wslot * COUNT_STRIDE], t0 ) : 0u;
 		if constexpr( plastic ) bbase[1] = t1 ? atomicAdd( &v.fl_count[T & 3], t1 ) : 0u;
 		if constexpr( eager ) bbase[2] = t2 ? atomicAdd( &v.po_count[T & 3], t2 ) : 0u;
 		if( t0 ) v.bstats[slot * NSTAT + ST_SPIKES] += t0;
@@ -1688,7 +1688,7 @@ __global__ __launch_bounds__( 256 ) void k_sync_eager( dview v, std::int64_t now
 	std::int64_t const T = now + 1; // the step whose delivery would apply them
 	if( T < v.D ) return;
 	int const slot = ring_slot( v, T - v.D ); // spikes of step T - D
-	if( x >= std::int64_t( v.counts[slot] ) ) return;
+	if( x >= std::int64_t( v.counts[slot * COUNT_STRIDE] ) ) return;
 	std::int32_t const r = v.ring[std::int64_t( slot ) * v.N + x];
 	if( !v.hasp[r] ) return;
 	snn_info const info = info_of( v );

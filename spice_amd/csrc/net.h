@@ -223,7 +223,7 @@ public:
 		tick();
 		int const slot = int( t % _v.rsize );
 		if( dspk ) *dspk = _ring.data() + std::int64_t( slot ) * _g.n;
-		if( dcnt ) *dcnt = _counts.data() + slot;
+		if( dcnt ) *dcnt = _counts.data() + slot * COUNT_STRIDE;
 	}
 
 	// Replays captured step graphs (all of them captured at the first run; see graphs.h).
@@ -278,7 +278,7 @@ public:
 		}
 		int const slot = int( ( _step - 1 ) % _v.rsize );
 		std::int32_t const * ids = _ring.data() + std::int64_t( slot ) * _g.n;
-		std::uint32_t const * cnt = _counts.data() + slot;
+		std::uint32_t const * cnt = _counts.data() + slot * COUNT_STRIDE;
 		std::uint32_t c = 0;
 		bool const staged = stage_to_host( ids, cnt, host_stage::words, [&]( std::uint32_t const * words, std::uint32_t n ) {
 			c = n;
@@ -523,7 +523,7 @@ public:
 		if( _step != _slog_t0 + _slog_n ) throw std::logic_error( "spike log window not completed" );
 		off[0] = 0;
 		if( _slog_n == 0 ) return 0;
-		SPICE_LAUNCH( k_log_out<<<16, 1024, 0, _s>>>( _slog_off.data(), _slog_n, _counts.data() + ( _step - 1 ) % _v.rsize, _slog_ids.data(),
+		SPICE_LAUNCH( k_log_out<<<16, 1024, 0, _s>>>( _slog_off.data(), _slog_n, _counts.data() + ( _step - 1 ) % _v.rsize * COUNT_STRIDE, _slog_ids.data(),
 		                                              std::min( _slog_cap, cap ), off, ids ) );
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 		std::uint64_t const total = off[_slog_n];
@@ -763,7 +763,7 @@ private:
 		_v.wcap = window_cap<Model>( _p.delay );
 		_v.rsize = ring_entries<Model>( _p.delay );
 		_ring.resize( std::size_t( _v.rsize ) * n );
-		_counts.resize( _v.rsize );
+		_counts.resize( std::size_t( _v.rsize ) * COUNT_STRIDE );
 		SPICE_HIP( hipMemsetAsync( _counts.data(), 0, _counts.bytes(), _s ) );
 		if constexpr( plastic )
 		{

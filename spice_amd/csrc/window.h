@@ -299,7 +299,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	// records: the first ids beside the count that tells which of them are this step's
 	constexpr int REC_U = 4; // arrivals per group of lanes in flight
 	std::int32_t early_id[REC_U] = {};
-	if( active && lane < W ) incl = v.counts[entry( lane - v.D )];
+	if( active && lane < W ) incl = v.counts[entry( lane - v.D ) * COUNT_STRIDE];
 	if constexpr( REC )
 		if( active )
 		{
@@ -627,7 +627,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 		if( lane < nw ) wpre[q * nw + lane] = in - n;
 		if( lane == 63 && in )
 		{
-			std::uint32_t * count = &v.counts[entry( q < W ? q : 0 )];
+			std::uint32_t * count = &v.counts[entry( q < W ? q : 0 ) * COUNT_STRIDE];
 			if constexpr( plastic )
 				if( q >= W ) count = ( q == W ? v.fl_count : v.po_count ) + ( clk.wseq & 3 );
 			base[q] = atomicAdd( count, in );
@@ -638,7 +638,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	{
 		// the counters of the steps after the window (no window before them reads those entries),
 		// and the clock of the step after it
-		if( tid < v.wcap ) v.counts[entry( W + tid )] = 0;
+		if( tid < v.wcap ) v.counts[entry( W + tid ) * COUNT_STRIDE] = 0;
 		if( tid == 0 )
 		{
 			float sum = clk.sum, c = clk.c;
@@ -1123,11 +1123,11 @@ __device__ inline void log_steps( dview const & v, int n )
 	if( k0 < 0 || k0 + n > v.slog->nsteps ) return;
 	std::int32_t const slot0 = window_entry( v );
 	auto entry = [&]( std::int32_t k ) { return slot0 + k < 0 ? slot0 + k + v.rsize : slot0 + k; };
-	std::uint64_t base = k0 == 0 ? 0ull : v.slog_off[k0 - 1] + v.counts[entry( -n - 1 )];
+	std::uint64_t base = k0 == 0 ? 0ull : v.slog_off[k0 - 1] + v.counts[entry( -n - 1 ) * COUNT_STRIDE];
 	std::uint64_t const cap = v.slog->cap;
 	for( int q = 0; q < n; q++ )
 	{
-		std::uint32_t const cnt = v.counts[entry( q - n )];
+		std::uint32_t const cnt = v.counts[entry( q - n ) * COUNT_STRIDE];
 		std::int32_t const * ids = v.ring + std::int64_t( entry( q - n ) ) * v.N;
 		if( threadIdx.x == 0 ) v.slog_off[k0 + q] = base;
 		for( std::uint32_t i = threadIdx.x; i < cnt; i += blockDim.x )
