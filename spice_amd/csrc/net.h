@@ -159,15 +159,19 @@ constexpr int REC_TILE = 768; // widest tile that segment records alone are a re
 // every tile stages all of the window's arrivals and a wider one does it less often (synth 1e9:
 // 29 us per step with 251 tiles of 3,200, 50 with 391 of 2,048), but none wider than its kernel
 // takes; windows of several steps, whose accumulators take LDS per step, two per CU beyond that.
-// targets: the neurons that have inputs (csr_dev::targets; the other tiles cost little). Two-kernel
-// plastic steps: about two tiles per CU, of 256 at least.
+// targets: the neurons that have inputs (csr_dev::targets). The other tiles cost little, except in
+// windows of static models, whose workgroups of 1,024 threads (default_launch) have a CU each
+// (Brunel, 100,000 and 40,000 neurons of which half have inputs, us per step: 3.4 and 1.9 with a
+// tile per CU of all, 4.7 and 2.2 with one per CU of those). Two-kernel plastic steps: about two
+// tiles per CU, of 256 at least.
 inline int lazy_tile_w( std::int64_t n, int cus ) { return int( std::clamp<std::int64_t>( ( ( n + 2 * cus - 1 ) / ( 2 * cus ) + 63 ) / 64 * 64, 256, TILE_MAX ) ); }
 template <typename Model>
 int default_tile_w( std::int64_t n, std::int64_t targets, int delay, int cus )
 {
-	auto const per = [&]( std::int64_t tiles ) { return ( ( targets + tiles - 1 ) / tiles + 63 ) / 64 * 64; };
 	if( !windowed_v<Model> ) return lazy_tile_w( n, cus );
 	bool const ahead = overlap_capable_v<Model> && delay >= 2;
+	std::int64_t const tiled = ahead && !is_plastic_v<Model> ? n : targets;
+	auto const per = [&]( std::int64_t tiles ) { return ( ( tiled + tiles - 1 ) / tiles + 63 ) / 64 * 64; };
 	std::int64_t const most = ahead || is_plastic_v<Model> ? TILE_MAX : 4 * 1024;
 	return int( std::clamp<std::int64_t>( per( ahead && per( cus ) > most ? 2 * cus : cus ), 64, most ) );
 }
@@ -1001,10 +1005,14 @@ private:
 		c.flush_grid = int( std::min<std::int64_t>( ( win ? 4 : 8 ) * cus, std::max<std::int64_t>( 1, ( n * fparts + 3 ) / 4 ) ) );
 		c.recv_parts = 1;
 		if( !plastic )
-			// window kernels: 16 waves where a tile has a CU to itself, 8 where several share one or
-			// the tile is small (Vogels 1e9, delay 8: 7.6 us per step with 250 tiles of 896 and 16
-			// waves, 8.9 with 8; Brunel 1e10, 495 tiles of 640: 19.4 with 16, 17.3 with 8)
-			c.recv_block = c.tile_w > 2048 || ( c.tile_w >= 512 && ( _g.targets + c.tile_w - 1 ) / c.tile_w <= cus ) ? 1024 : 512;
+		{
+			// window kernels: 16 waves where a workgroup has a CU to itself, 8 where several share one
+			// or, step by step, the tile is small. us per step with 16 and 8 waves, Vogels 1e9 (delay 8,
+			// 250 tiles of 896): 5.9, 9.0; brunel_3pop 1e9 (224 of 448): 2.8, 3.6, and 1e7 (248 of 128):
+			// 1.2, 1.4; Brunel 1e10 (495 of 640): 18.7, 18.0; brunel_3pop 4e7 (313 of 64): 1.7, 1.2.
+			bool const alone = ( _v.wcap > 1 ? n : _g.targets ) <= std::int64_t( cus ) * c.tile_w;
+			c.recv_block = c.tile_w > 2048 || ( alone && ( _v.wcap > 1 || c.tile_w >= 512 ) ) ? 1024 : 512;
+		}
 		else if( win )
 			c.recv_block = 512; // (STDP 1e9: 24.3 us per step, 27.4 with 1,024 threads)
 		else
