@@ -50,7 +50,7 @@ public:
 		for( auto * n : _nets )
 		{
 			launch_cfg c = n->get_launch();
-			int const tw = batch_tile_w( n->num_neurons(), c.tile_w, std::int64_t( _nets.size() ) );
+			int const tw = batch_tile_w( n->num_neurons(), c.tile_w, std::int64_t( _nets.size() ), n->params().delay );
 			if( tw != c.tile_w )
 			{
 				c.tile_w = tw;
@@ -162,13 +162,16 @@ public:
 	// batch of a few nets keeps its nets' own tiles. Fixed-point results do not depend on the tile
 	// width (fp32 sums are reordered, as by any launch shape); a net keeps wider tiles it already
 	// has (of up to TILE_MAX, what the batched kernels hold), and keeps the new width afterwards.
-	// Two-kernel steps: about max(64, 64 x CUs / nets) tiles per net (on a sweep of two 256-net
+	// Static nets step by step (delay 1) 192 at least, as fewer tiles reserve their spikes' places on a net's one
+	// counter (us per step with 64 and 192: 20 nets of up to 10,000 neurons, brunel_3pop 9.2, 8.7,
+	// synth 8.5, 8.1, Vogels 8.5, 8.1). Two-kernel steps: about max(64, 64 x CUs / nets) tiles per net (on a sweep of two 256-net
 	// batches 64 tiles per net beat 16, 32, 128 and 256).
-	static int batch_tile_w( std::int64_t n, int tile_w, std::int64_t nnets )
+	static int batch_tile_w( std::int64_t n, int tile_w, std::int64_t nnets, int delay )
 	{
 		std::int64_t const tiles = windowed ? std::max<std::int64_t>( 1, window_tiles_per_cu * device_cu_count() / nnets )
 		                                    : std::max<std::int64_t>( 64, std::int64_t( SPICE_BATCH_ITEMS_PER_CU ) * device_cu_count() / nnets );
-		int const tw = int( std::clamp<std::int64_t>( ( n / tiles + 63 ) / 64 * 64, 64, TILE_MAX ) );
+		int const least = windowed && !plastic && window_cap<Model>( delay ) == 1 ? BATCH_TILE : 64;
+		int const tw = int( std::clamp<std::int64_t>( ( n / tiles + 63 ) / 64 * 64, least, TILE_MAX ) );
 		return std::min( std::max( tw, tile_w ), TILE_MAX );
 	}
 
@@ -337,9 +340,9 @@ batch_iface * make_batch( std::vector<net_params> const & ps, std::vector<csr_de
 		try
 		{
 			launch_cfg first; // at the width that the batch will want
-			first.tile_w = hip_batch<Model>::batch_tile_w( gs[k].n, default_tile_w<Model>( gs[k].n, gs[k].targets, ps[k].delay, device_cu_count() ), std::int64_t( ps.size() ) );
+			first.tile_w = hip_batch<Model>::batch_tile_w( gs[k].n, default_tile_w<Model>( gs[k].n, gs[k].targets, ps[k].delay, device_cu_count() ), std::int64_t( ps.size() ), ps[k].delay );
 			net_params p = ps[k];
-			p.records = false; // (memory for every net)
+			p.batched = true;
 			nets.emplace_back( new hip_net<Model>( p, std::move( gs[k] ), ns, first ) );
 		}
 		catch( ... )

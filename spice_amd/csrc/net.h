@@ -36,7 +36,7 @@ struct net_params
 	std::uint64_t seed;
 	std::uint32_t flags;
 	float param[4];
-	bool records = true;    // segment records (window.h) where they pay: memory for speed
+	bool batched = false;   // made for a batch: no segment records (memory for speed), tiles that a batch keeps
 	bool own_stream = true; // the net destroys its stream (on failure: make_net does)
 };
 
@@ -154,6 +154,7 @@ int ring_entries( int delay )
 }
 
 constexpr int REC_TILE = 768; // widest tile that segment records alone are a reason for (default_launch)
+constexpr int BATCH_TILE = 192; // narrowest tile of a batch's nets that run step by step (hip_batch::batch_tile_w)
 
 // Targets per delivery tile of a new network. Window kernels: one tile per CU, as
 // every tile stages all of the window's arrivals and a wider one does it less often (synth 1e9:
@@ -985,8 +986,9 @@ private:
 		std::int64_t const n = _g.n;
 		launch_cfg c;
 		c.tile_w = _lazy ? lazy_tile_w( n, cus ) : default_tile_w<Model>( n, _g.targets, _p.delay, cus );
+		if( _p.batched && windowed && !plastic && _v.wcap == 1 ) c.tile_w = std::max( c.tile_w, BATCH_TILE );
 		if constexpr( input_classes_v<Model> > 0 )
-			if( _v.wcap == 1 && _p.records && _g.targets > 0 && double( _g.nnz ) / double( n ) * REC_TILE / double( _g.targets ) <= 40.0 )
+			if( _v.wcap == 1 && !_p.batched && _g.targets > 0 && double( _g.nnz ) / double( n ) * REC_TILE / double( _g.targets ) <= 40.0 )
 				// Step by step, with segment records that fit: rather fewer and wider tiles, as all of
 				// them reserve their spikes' places on one address, 9 ns apart (us per step of Vogels
 				// nets of 22,361, 70,711 and 100,000 neurons: 6.6, 7.0 and 7.9 with a tile per CU, 5.8,
@@ -1197,7 +1199,7 @@ private:
 			int lg = 4;
 			while( lg < 8 && rec_capacity( lg ) < need ) lg++;
 			std::uint64_t const segs = std::uint64_t( _g.n ) * std::uint64_t( ( ( _v.ntiles - 1 ) >> REC_TILES ) + 1 ) << REC_TILES, bytes = segs << lg;
-			if( _v.wcap > 1 || _window == 0 || !_p.records || lg > 7 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
+			if( _v.wcap > 1 || _window == 0 || _p.batched || lg > 7 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
 			if( bytes > ( std::uint64_t( 1 ) << 30 ) )
 			{
 				std::size_t room = 0, all = 0;

@@ -115,7 +115,7 @@ public:
 		if( !_build ) _build = new_stream();
 		auto h = std::make_unique<handle>();
 		net_params p = s.p;
-		p.records = false;
+		p.batched = true;
 		p.own_stream = false;
 		h->net.reset( make_net( p, generate_csr( s.conns, s.n, s.width, s.p.seed, _build ), _build ) );
 		h->model = s.p.model;
