@@ -173,6 +173,9 @@ struct dview
 	unsigned char const * recs;
 	std::int32_t rec_lg;
 
+	std::uint16_t const * col16; // the low halves of col (window.h); nullptr: none
+	std::int32_t vec16;          // of them per lane: 4 or 8
+
 	slog_t * slog; // nullptr: no spike log
 	std::int32_t * slog_ids;
 	std::uint64_t * slog_off;

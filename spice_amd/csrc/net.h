@@ -543,7 +543,7 @@ public:
 		     _fl_id.bytes() + _fl_synced.bytes() + _fl_pend.bytes() + _hasp.bytes() + _pl_lo.bytes() + _pl_hi.bytes() +
 		     _fl_count.bytes() + _xtr.bytes() + _ytr.bytes() + _fl8.bytes() + _sp8.bytes() + _po_id.bytes() + _po_count.bytes() +
 		     _tp_ptr.bytes() + _caught.bytes() + _tp_ent.bytes() + _ctl.bytes() + _bstats.bytes() +
-		     _pivots.bytes() + _recs.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
+		     _pivots.bytes() + _recs.bytes() + _col16.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
 		return b;
 	}
 
@@ -716,6 +716,7 @@ private:
 	int _staged = 0;                    // calls that asked for it
 	dbuf<std::int64_t> _pivots;
 	dbuf<unsigned char> _recs; // segment records
+	dbuf<std::uint16_t> _col16;       // low halves of the row store
 	dbuf<std::int32_t> _tile_ids;
 	std::int64_t _step = 0;
 	util::kahan_sum<float> _clock;
@@ -1012,7 +1013,10 @@ private:
 			// or, step by step, the tile is small. us per step with 16 and 8 waves, Vogels 1e9 (delay 8,
 			// 250 tiles of 896): 5.9, 9.0; brunel_3pop 1e9 (224 of 448): 2.8, 3.6, and 1e7 (248 of 128):
 			// 1.2, 1.4; Brunel 1e10 (495 of 640): 18.7, 18.0; brunel_3pop 4e7 (313 of 64): 1.7, 1.2.
-			bool const alone = ( _v.wcap > 1 ? n : _g.targets ) <= std::int64_t( cus ) * c.tile_w;
+			// (workgroups of tiles without inputs come after the others: where those have a CU each and
+			// are no small ones, 16 waves too -- Brunel, 400,000 neurons, 481 tiles of 832: 9.9, 14.5)
+			std::int64_t const room = std::int64_t( cus ) * c.tile_w;
+			bool const alone = c.tile_w >= 256 ? _g.targets <= room : n <= room;
 			c.recv_block = c.tile_w > 2048 || ( alone && ( _v.wcap > 1 || c.tile_w >= 512 ) ) ? 1024 : 512;
 		}
 		else if( win )
@@ -1066,6 +1070,7 @@ private:
 		_lc = c;
 		choose_window();
 		if( retile || ( _window > 0 ) != ( had_window > 0 ) ) build_records();
+		build_halves();
 		// statistics slots: one per workgroup of the widest step kernel (receive: per work item;
 		// plasticity: after those, one per plasticity workgroup or synchronization block; windows:
 		// one per tile, then the passes' workgroups; update: per block)
@@ -1144,20 +1149,19 @@ private:
 			if( plastic && _lazy ) return;
 			if( !plastic && !_ahead && ( _lc.recv_parts != 1 || _lc.tile_w > 4 * _lc.recv_block ) ) return;
 			_window = 1;
-			with_window_kernel( false, [&]( auto kernel, auto bytes, int ) {
+			with_window_kernel( IDS32, [&]( auto, auto bytes, int ) {
 				// the LDS of a CU, shared by the workgroups that a CU gets
 				std::size_t const per_cu = std::size_t( std::clamp( ( _v.ntiles + device_cu_count() - 1 ) / device_cu_count(), 1, 3 ) );
 				std::size_t const room = ( LDS_PER_CU - 4096 ) / per_cu;
 				int w = _v.wcap;
 				while( w > 1 && bytes( w ) > room ) w = window_steps( w - 1 );
 				_window = w;
-				if( bytes( w ) > ( 64 << 10 ) )
-					SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( w ) ) ) );
 			} );
-			with_window_kernel( true, [&]( auto kernel, auto bytes, int ) { // (one step)
-				if( bytes( 1 ) > ( 64 << 10 ) )
-					SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( 1 ) ) ) );
-			} );
+			for( int form : { IDS32, IDS16, IDS16X8, RECORDS } )
+				with_window_kernel( form, [&]( auto kernel, auto bytes, int ) {
+					if( bytes( _window ) > ( 64 << 10 ) )
+						SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( _window ) ) ) );
+				} );
 		}
 	}
 
@@ -1183,9 +1187,50 @@ private:
 		return true;
 	}
 
+	// The low halves of the row store (window.h), for windows without records. us per step without
+	// them, with 4 per lane and with 8, at this mean length of a segment: 2.6 (Vogels, 30,000
+	// neurons, delay 2) 3.9, 4.1, 4.3; 6 (brunel_3pop 1e6) 0.86, 0.85, 0.93; 18 (Vogels 1e9, delay
+	// 8) 5.8, 4.8, 5.3; 45 (brunel_3pop 1e9) 2.8, 2.5, 2.5; 50 (200,000 neurons) 3.4, 3.0, 3.2; 64
+	// (Brunel 1e10) 17.2, 14.9, 12.5. None if they took more than a fifth of the free memory; none for
+	// the nets of a batch, whose kernel reads the row store.
+	void build_halves()
+	{
+		_v.col16 = nullptr;
+		if constexpr( input_classes_v<Model> > 0 )
+		{
+			if( _window == 0 || _v.rec_lg || _p.batched || _g.nnz == 0 ) return;
+			// (lanes per segment: see choose_window)
+			double const mean = double( _g.nnz ) / double( _g.n ) / _v.nact;
+			if( mean < 4.0 ) return;
+			if( !_col16.size() )
+			{
+				std::size_t const n = std::size_t( _g.nnz ) + 8;
+				if( n > ( std::size_t( 1 ) << 29 ) )
+				{
+					std::size_t room = 0, all = 0;
+					SPICE_HIP( hipMemGetInfo( &room, &all ) );
+					if( 2 * n > room / 5 ) return;
+				}
+				try
+				{
+					_col16.resize( n );
+				}
+				catch( std::bad_alloc const & )
+				{
+					return;
+				}
+				SPICE_LAUNCH( k_halves<<<unsigned( std::min<std::size_t>( ( n / 8 + 255 ) / 256, 256 * 32 ) ), 256, 0, _s>>>( _g.col.data(), _g.nnz, _col16.data() ) );
+			}
+			_v.col16 = _col16.data();
+			_v.vec16 = mean >= 56.0 ? 8 : 4;
+			_v.wlanes = 0;
+			while( _v.wlanes < 5 && double( _v.vec16 << _v.wlanes ) < mean + ( mean < 20.0 ? 2.0 : 1.0 ) * std::sqrt( mean ) + ( _v.vec16 == 8 ? 4.0 : 0.0 ) ) _v.wlanes++;
+		}
+	}
+
 	// Segment records (window.h) of networks that run step by step, where segments are short: the
 	// smallest record that holds one 2.9 standard deviations longer than the mean. Not if the records took over twice
-	// the row store's memory, or more than half of the device's free memory, or if over 1 % of the
+	// the row store's memory, or more than a fifth of the free memory, or if over 1 % of the
 	// segments did not fit (rows of very different lengths); not for served jobs, which are
 	// admitted by their memory.
 	void build_records()
@@ -1204,7 +1249,7 @@ private:
 			{
 				std::size_t room = 0, all = 0;
 				SPICE_HIP( hipMemGetInfo( &room, &all ) );
-				if( bytes > room / 2 ) return;
+				if( bytes > room / 5 ) return;
 			}
 			try
 			{
@@ -1357,7 +1402,7 @@ private:
 			if( alone ) launch_passes( t, _s );
 			if( _slog_ctl.size() ) throw std::logic_error( "nets with a spike log are stepped by a batch" );
 			dview v = _vs[t & ( CLOCK_SLOTS - 1 )];
-			with_window_kernel( v.rec_lg != 0, [&]( auto kernel, auto bytes, int bs ) {
+			with_window_kernel( v.rec_lg ? RECORDS : !v.col16 ? IDS32 : v.vec16 == 8 ? IDS16X8 : IDS16, [&]( auto kernel, auto bytes, int bs ) {
 				std::int32_t W = w;
 				void * args[] = { &v, &W };
 				void const * fn = reinterpret_cast<void const *>( kernel );
@@ -1371,12 +1416,13 @@ private:
 
 	// f(window kernel, its LDS bytes for w steps, workgroup size) of the launch shape
 	template <typename F>
-	void with_window_kernel( bool records, F && f )
+	void with_window_kernel( int form, F && f )
 	{
 		auto go = [&]( auto fx, auto b ) {
 			constexpr bool FX = decltype( fx )::value;
 			constexpr int BS = decltype( b )::value;
-			f( records ? &k_window<Model, FX, BS, ( input_classes_v<Model> > 0 )> : &k_window<Model, FX, BS>,
+			constexpr bool cl = input_classes_v<Model> > 0;
+			f( form == RECORDS ? &k_window<Model, FX, BS, cl ? RECORDS : IDS32> : form == IDS16 ? &k_window<Model, FX, BS, cl ? IDS16 : IDS32> : form == IDS16X8 ? &k_window<Model, FX, BS, cl ? IDS16X8 : IDS32> : &k_window<Model, FX, BS>,
 			   [&]( int w ) { return window_lds<Model, FX>::bytes( BS, _lc.tile_w, w ); }, BS );
 		};
 		auto by_block = [&]( auto fx ) {

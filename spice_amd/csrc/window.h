@@ -78,6 +78,36 @@ __device__ inline targets load_targets( std::int32_t const * p )
 	return t;
 }
 
+// ---- what a delivery reads of a row's segment in a tile --------------------------------------
+enum { IDS32, IDS16, IDS16X8, RECORDS }; // the row store; its halves, 4 or 8 per lane (models with input classes); segment records
+
+// The low halves of the target ids, which tell a target within a tile (of at most 65,536); n of them
+// are read at once: 4 from any place, 8 from a multiple of 8 (the store is padded by 8).
+template <int n>
+struct halves
+{
+	std::uint16_t id[n];
+};
+template <int n>
+__device__ inline halves<n> load_halves( std::uint16_t const * p )
+{
+	halves<n> h;
+	__builtin_memcpy( &h, n == 8 ? __builtin_assume_aligned( p, 16 ) : p, sizeof( h ) );
+	return h;
+}
+static inline __global__ __launch_bounds__( 256 ) void k_halves( std::int32_t const * col, std::int64_t n, std::uint16_t * out )
+{
+	for( std::int64_t i = ( std::int64_t( blockIdx.x ) * 256 + threadIdx.x ) * 8; i < n; i += std::int64_t( gridDim.x ) * 256 * 8 )
+	{
+		// (the row store is padded by one piece of 4)
+		targets const c[2] = { load_targets( col + i ), load_targets( col + std::min( i + 4, n ) ) };
+		halves<8> h;
+#pragma unroll
+		for( int x = 0; x < 8; x++ ) h.id[x] = std::uint16_t( c[x / 4].id[x % 4] );
+		__builtin_memcpy( out + i, &h, sizeof( h ) );
+	}
+}
+
 // ---- segment records -------------------------------------------------------------------------
 // For models with input classes a delivery needs of a row's segment in a tile only the targets, and
 // those fit 16 bits inside a tile. Where segments are short and the network runs step by step, each
@@ -253,9 +283,10 @@ __device__ inline std::uint32_t wave_inclusive_scan32( std::uint32_t x )
 __device__ inline std::int32_t window_entry( dview const & v ) { return v.rsize == CLOCK_SLOTS ? std::int32_t( v.ctl - v.ctl0 ) : v.ctl->rslot; }
 
 // The window [T0, T0 + W) of the tile at place `pos` of v.tile_ids.
-template <typename Model, bool FIXED, int BS, bool REC = false>
+template <typename Model, bool FIXED, int BS, int FORM = IDS32>
 __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 {
+	constexpr bool REC = FORM == RECORDS;
 	using N = typename Model::neuron;
 	using S = typename Model::synapse;
 	using L = window_lds<Model, FIXED>;
@@ -440,7 +471,9 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 			std::int32_t const len = lane < cnt ? std::int32_t( b - a ) : 0;
 			if constexpr( L::classes > 0 )
 				// in the place of the source: where the class's counters of the step start (for target 0)
-				mine[lane] = win_seg{ len > 0 ? a : 0, ( q * nacc + N::input_class( src, info ) ) * tws - t0, len };
+				// (IDS16X8 also: the piece that the segment begins in, its end from there on, its place there)
+				mine[lane] = win_seg{ len > 0 ? a & ~std::int64_t( FORM == IDS16X8 ? 7 : 0 ) : 0, ( q * nacc + N::input_class( src, info ) ) * tws - ( FORM == IDS32 ? t0 : 0 ),
+				                      FORM == IDS16X8 && len > 0 ? ( len + ( int( a ) & 7 ) ) | ( int( a ) & 7 ) << 16 : len };
 			else
 				mine[lane] = win_seg{ len > 0 ? a : 0, src, len | ( q << 16 ) };
 			ev += std::uint32_t( len );
@@ -452,6 +485,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 				fetch_seg();
 				if( k0 + 2 * NW * per < total ) src_n = fetch_id( k0 + 2 * NW * per + mylane, q_n );
 			}
+			constexpr int V = FORM == IDS16X8 ? 8 : WIN_VEC; // entries per lane
 			constexpr int U = plastic ? 2 : 4; // segments per group in flight (with weights, 4 measured 3 % slower)
 			for( std::int32_t c = 0; c < cnt; c += U * ng )
 			{
@@ -465,9 +499,22 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 					len[u] = k < 64 ? ( r[u].meta & 0xffff ) : 0;
 					most = len[u] > most ? len[u] : most;
 				}
-				for( std::int32_t e = l * WIN_VEC;; e += G * WIN_VEC )
+				for( std::int32_t e = l * V;; e += G * V )
 				{
 					// (past a segment's end its first entries are read, at valid addresses, and ignored)
+					if constexpr( FORM == IDS16 || FORM == IDS16X8 )
+					{
+						halves<V> j[U];
+#pragma unroll
+						for( int u = 0; u < U; u++ ) j[u] = load_halves<V>( v.col16 + r[u].off + ( e < len[u] ? e : 0 ) );
+#pragma unroll
+						for( int u = 0; u < U; u++ )
+#pragma unroll
+							for( int x = 0; x < V; x++ )
+								if( e + x < len[u] && ( V == WIN_VEC || e + x >= r[u].meta >> 16 ) ) atomicAdd( acc + ( r[u].src + ( ( j[u].id[x] - t0 ) & 0xffff ) ), 1u );
+						if( e - l * V + G * V >= most ) break;
+						continue;
+					}
 					targets j[U];
 #pragma unroll
 					for( int u = 0; u < U; u++ ) j[u] = load_targets( v.col + r[u].off + ( e < len[u] ? e : 0 ) );
@@ -938,14 +985,14 @@ __global__ __launch_bounds__( 256 ) void k_window_passes( dview v )
 
 // One workgroup per tile, those with incoming synapses first; then (plastic models) the
 // workgroups of the passes of the window before.
-// REC: one step, from segment records (an instance of its own: in the others the registers of
-// its delivery cost 2 % -- Brunel 1e6 0.88 us per step, 0.90 with it inside).
-template <typename Model, bool FIXED, int BS, bool REC = false>
+// FORM: what the delivery reads (instances of their own: with the delivery from records in all of
+// them its registers cost 2 % -- Brunel 1e6 0.88 us per step, 0.90 with it inside). Records: one step.
+template <typename Model, bool FIXED, int BS, int FORM = IDS32>
 __global__ __launch_bounds__( BS ) void k_window( dview v, std::int32_t W )
 {
 	std::int32_t const b = blockIdx.x;
 	if( b < v.ntiles )
-		window_tile<Model, FIXED, BS, REC>( v, b < v.nact ? xcd_place( b, v.nact ) : b, REC ? 1 : W );
+		window_tile<Model, FIXED, BS, FORM>( v, b < v.nact ? xcd_place( b, v.nact ) : b, FORM == RECORDS ? 1 : W );
 	else if constexpr( is_plastic_v<Model> )
 		window_passes<Model, FIXED>( v, b - v.ntiles, std::int32_t( gridDim.x ) - v.ntiles, v.ntiles );
 }

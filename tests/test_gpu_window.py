@@ -154,3 +154,25 @@ def test_spikes_and_state_read_back(gpu, n):
         sizes.append(len(want))
     assert min(sizes) == 0 and max(sizes) == n
     d.close(), h.close()
+
+
+@pytest.mark.parametrize("model,layout,delay,launch", [
+    ("synth", ([66000], [(0, 0, 0.005)]), 3, (1024, 512)),  # ids past 16 bits, 5 targets per segment
+    ("vogels_abbott", ([700], [(0, 0, 0.1)]), 5, (64, 1024)),
+    ("synth", ([901], [(0, 0, 0.9)]), 4, (64, 512)),  # 8 per lane: 57 targets per segment
+    ("brunel_3pop", three_pop_layout(1500), 15, (640, 512)),
+    ("synth", ([300], [(0, 0, 1.0)]), 1, (256, 256)),  # step by step, too long for records
+    ("synth", ([257], [(0, 0, 1.0)]), 2, (64, 256)),
+])
+def test_halved_row_store_bit_exact(gpu, model, layout, delay, launch):
+    """Deliveries from the low halves of the target ids, 4 and 8 per lane: segments that begin and
+    end anywhere in a piece, the row store's last ones, tiles on both sides of id 65,536."""
+    h = O.CpuSnn(model, layout, DT, delay, seed=31, fixed_point=True)
+    d = Snn(model, Layout(*layout), DT, delay, seed=31, fixed_point=True)
+    d.set_launch(tile_w=launch[0], recv_block=launch[1])
+    for n in (7, 160, 33):
+        d.run(n)
+        h.run(n)
+        assert_state_equal(d.neurons(), h.neurons(), model)
+    assert d.stats()["events"] > 0
+    d.close(), h.close()
