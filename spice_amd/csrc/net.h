@@ -1191,12 +1191,13 @@ private:
 	// them, with 4 per lane and with 8, at this mean length of a segment: 2.6 (Vogels, 30,000
 	// neurons, delay 2) 3.9, 4.1, 4.3; 6 (brunel_3pop 1e6) 0.86, 0.85, 0.93; 18 (Vogels 1e9, delay
 	// 8) 5.8, 4.8, 5.3; 45 (brunel_3pop 1e9) 2.8, 2.5, 2.5; 50 (200,000 neurons) 3.4, 3.0, 3.2; 64
-	// (Brunel 1e10) 17.2, 14.9, 12.5. None if they took more than a fifth of the free memory; none for
+	// (Brunel 1e10) 17.2, 14.9, 12.5; beside weights, 26 (brunel_with_plasticity 6e8) 12.5, 11.6, 45
+	// (brunel_3pop_stdp 1e9, steps 2,000 on) 24.9, 24.3. None if they took more than a fifth of the free memory; none for
 	// the nets of a batch, whose kernel reads the row store.
 	void build_halves()
 	{
 		_v.col16 = nullptr;
-		if constexpr( input_classes_v<Model> > 0 )
+		if constexpr( input_classes_v<Model> > 0 || ( plastic && windowed ) )
 		{
 			if( _window == 0 || _v.rec_lg || _p.batched || _g.nnz == 0 ) return;
 			// (lanes per segment: see choose_window)
@@ -1222,17 +1223,16 @@ private:
 				SPICE_LAUNCH( k_halves<<<unsigned( std::min<std::size_t>( ( n / 8 + 255 ) / 256, 256 * 32 ) ), 256, 0, _s>>>( _g.col.data(), _g.nnz, _col16.data() ) );
 			}
 			_v.col16 = _col16.data();
-			_v.vec16 = mean >= 56.0 ? 8 : 4;
+			_v.vec16 = !plastic && mean >= 56.0 ? 8 : 4;
 			_v.wlanes = 0;
 			while( _v.wlanes < 5 && double( _v.vec16 << _v.wlanes ) < mean + ( mean < 20.0 ? 2.0 : 1.0 ) * std::sqrt( mean ) + ( _v.vec16 == 8 ? 4.0 : 0.0 ) ) _v.wlanes++;
 		}
 	}
 
 	// Segment records (window.h) of networks that run step by step, where segments are short: the
-	// smallest record that holds one 2.9 standard deviations longer than the mean. Not if the records took over twice
-	// the row store's memory, or more than a fifth of the free memory, or if over 1 % of the
-	// segments did not fit (rows of very different lengths); not for served jobs, which are
-	// admitted by their memory.
+	// smallest record that holds one 2.9 standard deviations longer than the mean. Not if the records
+	// took over twice the row store's memory, or more than a fifth of the free memory, or if over 1 %
+	// of the segments did not fit (rows of very different lengths); not for the nets of a batch.
 	void build_records()
 	{
 		_recs.release();
@@ -1422,7 +1422,7 @@ private:
 			constexpr bool FX = decltype( fx )::value;
 			constexpr int BS = decltype( b )::value;
 			constexpr bool cl = input_classes_v<Model> > 0;
-			f( form == RECORDS ? &k_window<Model, FX, BS, cl ? RECORDS : IDS32> : form == IDS16 ? &k_window<Model, FX, BS, cl ? IDS16 : IDS32> : form == IDS16X8 ? &k_window<Model, FX, BS, cl ? IDS16X8 : IDS32> : &k_window<Model, FX, BS>,
+			f( form == RECORDS ? &k_window<Model, FX, BS, cl ? RECORDS : IDS32> : form == IDS16 ? &k_window<Model, FX, BS, cl || plastic ? IDS16 : IDS32> : form == IDS16X8 ? &k_window<Model, FX, BS, cl ? IDS16X8 : IDS32> : &k_window<Model, FX, BS>,
 			   [&]( int w ) { return window_lds<Model, FX>::bytes( BS, _lc.tile_w, w ); }, BS );
 		};
 		auto by_block = [&]( auto fx ) {

@@ -79,7 +79,7 @@ __device__ inline targets load_targets( std::int32_t const * p )
 }
 
 // ---- what a delivery reads of a row's segment in a tile --------------------------------------
-enum { IDS32, IDS16, IDS16X8, RECORDS }; // the row store; its halves, 4 or 8 per lane (models with input classes); segment records
+enum { IDS32, IDS16, IDS16X8, RECORDS }; // the row store; its halves, 4 or 8 per lane; segment records (the last two: models with input classes)
 
 // The low halves of the target ids, which tell a target within a tile (of at most 65,536); n of them
 // are read at once: 4 from any place, 8 from a multiple of 8 (the store is padded by 8).
@@ -502,7 +502,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 				for( std::int32_t e = l * V;; e += G * V )
 				{
 					// (past a segment's end its first entries are read, at valid addresses, and ignored)
-					if constexpr( FORM == IDS16 || FORM == IDS16X8 )
+					if constexpr( L::classes > 0 && ( FORM == IDS16 || FORM == IDS16X8 ) )
 					{
 						halves<V> j[U];
 #pragma unroll
@@ -517,7 +517,15 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 					}
 					targets j[U];
 #pragma unroll
-					for( int u = 0; u < U; u++ ) j[u] = load_targets( v.col + r[u].off + ( e < len[u] ? e : 0 ) );
+					for( int u = 0; u < U; u++ )
+						if constexpr( FORM == IDS16 )
+						{
+							halves<V> const low = load_halves<V>( v.col16 + r[u].off + ( e < len[u] ? e : 0 ) );
+#pragma unroll
+							for( int x = 0; x < V; x++ ) j[u].id[x] = t0 + ( ( low.id[x] - t0 ) & 0xffff );
+						}
+						else
+							j[u] = load_targets( v.col + r[u].off + ( e < len[u] ? e : 0 ) );
 					synapses<S> sy[U];
 					if constexpr( plastic )
 					{
