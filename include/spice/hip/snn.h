@@ -108,7 +108,7 @@ public:
 		} );
 	}
 
-	// n steps without readback, replayed from a captured HIP graph (extension).
+	// n steps without readback, in windows or replayed from captured HIP graphs (extension).
 	void run( long_ n )
 	{
 		check( spice_hip_run( _net, n ) );

@@ -260,22 +260,20 @@ int spice_hip_step( spice_net * net, int32_t ** out_dspikes, uint32_t ** out_dco
  * Spike order is unspecified (atomic append), as in the reference. */
 int spice_hip_copy_spikes( spice_net * net, int32_t * out, uint64_t cap, uint64_t * out_count );
 
-/* Enqueues nsteps steps without spike readback, replaying a captured HIP graph of the
- * step sequence. Equivalent to nsteps calls of spice_hip_step. Asynchronous. */
+/* Enqueues nsteps steps without spike readback: in windows of up to the delay, one kernel each,
+ * or, step by step (a delay of one step, or plasticity of the general per-synapse contract),
+ * replaying captured HIP graphs. Equivalent to nsteps calls of spice_hip_step. Asynchronous (the
+ * host waits where very many launches would be queued). */
 int spice_hip_run( spice_net * net, int64_t nsteps );
 
 /* Enqueues nsteps steps without graph capture, each kernel launched with start and stop HIP
  * events attached to its dispatch (hipExtLaunchKernel: the kernel's own duration, without the
  * launch gap) on the net's stream, waits, and adds the summed per-kernel device times in
- * milliseconds to kernel_ms[0..2]. Two-kernel steps: kernel_ms[0] spike delivery (for plastic
- * models including the previous step's plasticity work, which runs in the same kernel),
- * kernel_ms[1] neuron update, kernel_ms[2] 0. Overlapped steps (models whose delivery may run
- * before the target's update, delay >= 2): kernel_ms[0] the first step's delivery, kernel_ms[1]
- * the last step's update, kernel_ms[2] the nsteps - 1 kernels that each run the update of a
- * step beside the delivery of the next. Fused steps (static models whose steps do not overlap,
- * launch shapes with one delivery workgroup per tile of at most four workgroup widths, every
- * tile receiving input): kernel_ms[0] = kernel_ms[1] = 0, kernel_ms[2] the nsteps kernels that
- * each deliver a step's input to a tile and update the tile's neurons. Same results as
+ * milliseconds to kernel_ms[0..2]. Windows of static models: kernel_ms[2] the kernels, kernel_ms[0] =
+ * kernel_ms[1] = 0. Windows of plastic models (each beside the plasticity of the window before):
+ * kernel_ms[0] the first kernel, kernel_ms[1] the last, kernel_ms[2] those between. Two-kernel
+ * steps: kernel_ms[0] spike delivery (for plastic models including the previous step's plasticity
+ * work, which runs in the same kernel), kernel_ms[1] neuron update, kernel_ms[2] 0. Same results as
  * spice_hip_run. Used for roofline figures. */
 int spice_hip_run_profiled( spice_net * net, int64_t nsteps, double * kernel_ms );
 
@@ -285,7 +283,7 @@ int spice_hip_synchronize( spice_net * net );
 /* ---- batches: many independent networks stepped together -------------------------------- */
 /* No counterpart in the reference (it steps one network per cuda::snn). A batch holds nnets
  * networks of one model (sizes, delays, seeds and parameters may differ; dt and flags are
- * shared) and steps all of them with one launch per step phase (a captured HIP graph).
+ * shared) and steps all of them with one launch per window (or step: a captured HIP graph).
  * Each network's results equal those of the same network stepped alone. */
 int spice_batch_create( int32_t model, int32_t nnets, const spice_net_desc * descs, float dt, uint32_t flags, spice_batch ** out_batch );
 int spice_batch_destroy( spice_batch * batch );
@@ -301,7 +299,7 @@ int spice_batch_net( spice_batch * batch, int32_t i, spice_net ** out_net );
 /* ---- launch shapes and the autotuner --------------------------------------------------- */
 /* No counterpart in the reference (its launch shapes are compile-time constants). tile_w:
  * targets per spike-delivery tile (multiple of 64, 64..1024; up to 8192 for models without
- * plasticity that run two kernels per step -- delay 1, or receive() reading target state without
+ * plasticity whose windows have one step -- delay 1, or receive() reading target state without
  * a split gate); flush_slots: synapses per
  * plasticity work item (a lazy flush's row slice, or an eager pass's row or target slice;
  * multiple of 64); flush_grid: plasticity workgroups (of 256 threads' worth);
@@ -320,7 +318,7 @@ typedef struct spice_launch
 int spice_hip_get_launch( spice_net * net, spice_launch * out );
 int spice_hip_set_launch( spice_net * net, const spice_launch * in );
 /* Times candidate launch shapes on a copy of the network (warmup steps first, then `steps`
- * graph-replayed steps per candidate, wall time per step: plasticity overlaps delivery, so
+ * steps per candidate, wall time per step: plasticity overlaps delivery, so
  * shapes are evaluated together; tile width first, then delivery parts, then the plasticity
  * shape; the three fastest are then timed again in turn, three times each, since the copy's
  * activity drifts between candidates),

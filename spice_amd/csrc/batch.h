@@ -1,9 +1,10 @@
 #pragma once
 // Batched stepping of many independent networks of one model (parameter sweeps, served
 // jobs). Every net keeps its own buffers, clock and statistics (it is an ordinary hip_net);
-// the batch adds device tables that map the workgroups of ONE launch per step phase to
-// (net, local tile), (net, local neuron block) and, for plastic models, (net, local flush
-// block), and replays captured HIP graphs of those launches (graphs.h). Per-net results are
+// the batch adds device tables that map the workgroups of ONE launch per window to (net, tile), for
+// plastic models (net, workgroup of the passes), and spike logs -- or, for nets on two-kernel
+// steps, of one launch per step phase; single steps replay captured HIP graphs of those launches
+// (graphs.h). Per-net results are
 // identical to stepping the nets one by one: the kernels run the same per-net bodies and all
 // randomness is keyed on (net seed, neuron, step). Nets may sit at different steps (served
 // jobs join a running mix): each net's clock slot is chosen from its own step parity.

@@ -54,11 +54,11 @@ namespace spice::hipx
 {
 constexpr int MAXA = 16;
 
-// Device clock. Four slots: the kernels of step T read slot T & 3 and the neuron-update
-// kernel writes step T + 1's clock into slot (T + 1) & 3, so the clock advances without
-// atomics or an extra kernel, the plasticity work of step T (which runs in step T + 1's
-// delivery kernel) still reads its own slot (ctl_prev), and a captured graph of a multiple of
-// 4 steps replays.
+// Device clock. Four slots: the kernels of step T (the window from T on) read slot T & 3, and the
+// window kernel or the neuron update writes the next one's, (T + W) & 3, so the clock advances
+// without atomics or an extra kernel (a window's length is never a multiple of 4), the plasticity
+// work of a two-kernel step, in the next delivery kernel, still reads its own slot (ctl_prev), and
+// a captured graph of a multiple of 4 steps replays.
 constexpr int CLOCK_SLOTS = 4;
 struct ctl_t
 {

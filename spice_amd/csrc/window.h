@@ -1,5 +1,5 @@
 #pragma once
-// The window kernel: one launch simulates a window of W <= delay steps of a static network.
+// The window kernel: one launch simulates a window of W <= delay steps of a network.
 //
 // A spike emitted at step T reaches its targets at T + D, so the arrivals of the steps
 // [T0, T0 + W), W <= D, are all known when the window starts, and a workgroup that owns a tile of
@@ -11,10 +11,12 @@
 // With W = 1 (delay 1, or a receive() that reads its target) the workgroup delivers and then
 // updates one step.
 //
-// What bounds it: the dependent loads of a delivery (with W = 1), the rate of scattered row
-// segments (larger windows). A row's segment inside a tile is walked by a group of 2^lg lanes of
-// WIN_VEC entries each (lg from the mean segment length), several segments per group in flight: no
-// per-event search, and an entry costs a quarter of a load and one LDS atomic.
+// What bounds it: small windows the chain of dependent loads and the launch (Vogels 1e8, one step:
+// 3.5 us in the kernel, 3 us around it), larger ones the lines that a CU can have in flight (Vogels
+// 1e9, delay 8: 27 of 36 us per window in the walk, 4,100 segments of 18 targets per tile), the largest the
+// memory (Brunel 1e10). A row's segment inside a tile is walked by a group of 2^lg lanes (lg from the
+// mean segment length), several segments per group in flight: no per-event search. What is read
+// of a segment, see below.
 //
 // Accumulators: models with input classes (model.h) count the inputs of each class, others add
 // the inputs up, in 64 bits (doubles, or fixed point). No 32-bit float atomics: ds_add_f32 takes
@@ -758,7 +760,7 @@ __device__ inline std::int32_t xcd_place( std::int32_t b, std::int32_t n )
 // read-modify-write; the traces at a and b are the per-step recurrence continued from the window's
 // start. One index space of work items, (row, part) then (target, part), taken round robin by the
 // waves of workgroups blk, blk + nblk, ...; statistics go to slots slot0 + blk. Bound by the rate
-// of random memory lines: the post pass's weights (profiles/random_line_probe.md).
+// of random memory lines, 43 to 53 G of 64 bytes a second on the whole card: the post pass's weights.
 template <typename Model, bool FIXED>
 __device__ inline void window_passes( dview const & v, std::int64_t blk, std::int64_t nblk, std::int64_t slot0 )
 {

@@ -223,13 +223,10 @@ class Snn:
     def run_profiled(self, nsteps):
         """Runs nsteps eagerly, each kernel launched with HIP events attached to its dispatch
         (its own duration, without the launch gap); returns summed device ms per kernel:
-        {"receive": ..., "update": ..., "step": ...}. Two-kernel steps: "receive" is the
-        delivery (with the previous step's plasticity work of plastic models), "update" the
-        neuron update, "step" 0. Overlapped steps: "receive" is the first delivery, "update"
-        the last update (with the passes of the step before it), "step" the nsteps - 1
-        overlapped kernels (update of step T, delivery of T + 1, plasticity work of T - 1).
-        Fused steps (static, delay-1 nets at shapes with one delivery workgroup per tile):
-        "receive" and "update" 0, "step" the nsteps kernels that each deliver and update."""
+        {"receive": ..., "update": ..., "step": ...}. Windows of static models: "step" is all of
+        them. Windows of plastic models: "receive" is the first kernel, "update" the last,
+        "step" those between. Two-kernel steps: "receive" is the delivery (with the previous
+        step's plasticity work of plastic models), "update" the neuron update, "step" 0."""
         ms = (_c.c_double * 3)(0.0, 0.0, 0.0)
         _lib.check(_lib.lib().spice_hip_run_profiled(self._h, int(nsteps), ms))
         return {"receive": ms[0], "update": ms[1], "step": ms[2]}
