@@ -7,12 +7,12 @@ dt = 0.1 ms, additive pair STDP on excitatory->excitatory synapses (model brunel
 Synthetic by construction: the random graph is generated on the device from a fixed seed and
 all state starts from the model's init.
 
-One "step" is one simulation time step of the whole network (spike delivery incl. lazy
-plasticity, neuron update, plasticity flush). The timed region replays captured HIP graphs
-of steps with all state resident in HBM; value = wall seconds / simulated (bio) seconds.
+One "step" is one simulation time step of the whole network (spike delivery, neuron update,
+plasticity). The timed region runs it in windows of up to the delay, one kernel each, with all
+state resident in HBM; value = wall seconds / simulated (bio) seconds.
 
-Printed: one JSON line with the metric, synapse events/s, a roofline object for the
-dominant kernel (algorithmic bytes per launch / mean kernel duration from HIP events attached
+Printed: one JSON line with the metric, synapse events/s, a roofline object for the window
+kernels (algorithmic bytes per step / mean kernel time per step from HIP events attached
 to each dispatch on the net's stream) and a cpu_baseline object (the single-threaded CPU checker, a restatement of
 the reference's cpu::snn, timed on this host on a bounded number of steps of the same net).
 """
@@ -77,10 +77,20 @@ def workload_layout(name):
     return [n], [(0, 0, p)]
 
 
+def window_steps(model, delay):
+    """Steps per kernel of a network's windows: up to the delay, at most 15 (plastic models: 10),
+    never a multiple of 4; one with a delay of one step. (Less where a very wide tile's
+    accumulators would not fit.)"""
+    from spice_amd.models import MODELS
+    w = min(delay, 10 if MODELS[model][2] else 15)
+    return max(1, w if w % 4 else w - 1)
+
+
 def algorithmic_bytes(model, n, st, steps):
-    """Algorithmic HBM bytes per launch of each kernel, from the device counters of the
-    profiled steps (per-neuron arrays that stay L2-resident -- spike history, traces' current
-    values -- are counted once per neuron in the update kernel, not per synapse):
+    """Algorithmic HBM bytes per launch of each kernel of two-kernel steps (launch shapes whose
+    tiles are split between workgroups), from the device counters of the profiled steps (per-neuron
+    arrays that stay L2-resident -- spike history, traces' current values -- are counted once per
+    neuron in the update kernel, not per synapse):
       receive: per delivered spike its id (4) and row offsets (16); per delivered event the
                target id (4) and, for models with per-synapse state, the weight read (4); per
                plastic synapse changed, the write-back of its state (4 for neuron-trace
@@ -98,8 +108,7 @@ def algorithmic_bytes(model, n, st, steps):
                neuron-trace, 12 per-synapse-trace) + per synapse written back its state write
                (eager passes write only synapses whose state the event changed; the lazy flush
                writes every one);
-      step   : the overlapped step kernel (update of step T, delivery of T + 1, plasticity work
-               of T - 1): one of each per launch.
+      step   : one of each.
     Target-neuron accumulation is counted as atomics, not bytes."""
     from spice_amd.models import MODELS
     _, nattrs, sattrs = MODELS[model]
@@ -115,13 +124,35 @@ def algorithmic_bytes(model, n, st, steps):
     recv = spk * 20 + ev * (8 if plastic else 4) + pev * (wb if plastic else 0)
     upd = n * (2 * s_n + 2 * acc_bytes + ((17 + 17) if traced else (25 if plastic else 0))) + spk * 4
     fl = (st["flush_slots"] * 4 + (st["flush_synapses"] + st["flush_written"]) * s_s) / steps if plastic else 0.0
-    # the plasticity work of step T - 1 runs inside the delivery kernel of step T (two-kernel
-    # step) or inside the overlapped kernel of step T
+    # the plasticity work of step T - 1 runs inside the delivery kernel of step T
     return {"receive": recv + fl, "update": upd, "step": recv + fl + upd}
 
 
+def window_bytes(model, n, st, steps, delay):
+    """Algorithmic HBM bytes per step of the window kernels, from the device counters of the
+    profiled steps:
+      delivery: per delivered spike its id (4) and row offsets (16); per delivered event the low
+                half of the target id (2) and, for plastic models, the weight read (4);
+      update  : per neuron and window its state read + write and, for plastic models, two history
+                words, the traces and the step flags read and written (34); 4 per emitted spike;
+      passes  : 4 per index word read (the target id of every plastic slot of the arriving rows, the
+                (source, offset) pair of every by-target entry of the spiking targets) + per synapse
+                brought up to date its weight read + per synapse changed its weight written.
+    Target-neuron accumulation is counted as atomics, not bytes."""
+    from spice_amd.models import MODELS
+    _, nattrs, sattrs = MODELS[model]
+    s_n = sum(np.dtype(t).itemsize for _, t in nattrs)
+    plastic = bool(sattrs)
+    spk = st["spikes"] / steps
+    ev = st["events"] / steps
+    recv = spk * 20 + ev * (6 if plastic else 2)
+    upd = n * (2 * s_n + (34 if plastic else 0)) / window_steps(model, delay) + spk * 4
+    fl = (st["flush_slots"] + st["flush_synapses"] + st["flush_written"]) * 4 / steps if plastic else 0.0
+    return recv + upd + fl
+
+
 def measured_traffic(workload, kernel):
-    """HBM bytes per launch of `kernel` on `workload` from the committed rocprofv3 PMC summary
+    """HBM bytes per step of `kernel` on `workload` from the committed rocprofv3 PMC summary
     (FETCH_SIZE and WRITE_SIZE runs, scaled by the copy calibration), or (None, None)."""
     path = os.path.join(ROOT, "profiles", "pmc_traffic.json")
     try:
@@ -130,19 +161,6 @@ def measured_traffic(workload, kernel):
         return int(t["fetch_bytes"] + t["write_bytes"]), "profiles/pmc_traffic.json"
     except (OSError, KeyError, ValueError):
         return None, None
-
-
-def measured_atomics(workload, kernel):
-    """Atomic operations per launch of `kernel` on `workload` from the committed rocprofv3 PMC
-    summary: LDS atomic lane operations (SQ_INSTS_LDS_ATOMIC_BANDWIDTH, counted in 64-byte units
-    of atomic data, x 16 for 4-byte operands) and L2 atomic requests (TCC_ATOMIC_sum), or None."""
-    path = os.path.join(ROOT, "profiles", "pmc_traffic.json")
-    try:
-        with open(path) as f:
-            t = json.load(f)[workload]["kernels"][kernel]
-        return {"lds_atomic_ops": int(t["lds_atomic_ops"]), "l2_atomic_requests": int(t["l2_atomic_requests"])}
-    except (OSError, KeyError, ValueError):
-        return None
 
 
 def sweep_nets(count, seed):
@@ -567,40 +585,22 @@ def main():
     st = net.stats()
     bio = args.steps * dt
     print(f"[bench] timed {args.steps} steps in {wall:.3f}s, stats {st}", file=sys.stderr, flush=True)
-    bytes_per = algorithmic_bytes(model, n, pst, args.profile_steps)
-    kern = max(ms, key=lambda k: ms[k])
-    # launches of each kernel in the profiled steps: two per step, or (overlapped steps) the
-    # first delivery, one overlapped kernel per step boundary and the last update, or (fused
-    # steps: no delivery kernel of its own) one step kernel per step
-    fused = ms["step"] > 0 and ms["receive"] == 0
-    overlapped = ms["step"] > 0 and not fused
-    launches = ({"receive": 1, "update": 1, "step": args.profile_steps - 1} if overlapped
-                else {"receive": args.profile_steps, "update": args.profile_steps,
-                      "step": args.profile_steps if fused else 1})
-    avg_ms = ms[kern] / launches[kern]
-    achieved = bytes_per[kern] / (avg_ms * 1e-3) / 1e9
-    kernel_names = {"receive": "k_receive_tiled", "update": "k_step_overlap" if overlapped else "k_update",
-                    "step": "k_step_fused" if fused else "k_step_overlap"}
-    traffic, traffic_src = measured_traffic(args.workload, kernel_names[kern])
+    # (windows of plastic networks: "receive" is the first kernel of the profiled steps, "update" the
+    # last, "step" those between)
+    windows = ms["step"] > 0
+    step_bytes = (window_bytes(model, n, pst, args.profile_steps, delay) if windows
+                  else algorithmic_bytes(model, n, pst, args.profile_steps)["step"])
+    step_ms = sum(ms.values()) / args.profile_steps
+    achieved = step_bytes / (step_ms * 1e-3) / 1e9
+    traffic, traffic_src = measured_traffic(args.workload, "k_window") if windows else (None, None)
     roofline = {
-        "bound": "hbm", "kernel": kernel_names[kern], "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
+        "bound": "hbm", "kernel": "k_window" if windows else "k_receive_tiled, k_update", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
         "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic, "traffic_source": traffic_src,
-        "bytes_per_launch": round(bytes_per[kern]), "avg_launch_us": round(avg_ms * 1e3, 3),
-        "kernel_us_per_step": {k: round(v / args.profile_steps * 1e3, 3) for k, v in ms.items()},
+        "steps_per_launch": window_steps(model, delay) if windows else 1, "bytes_per_step": round(step_bytes),
+        "avg_step_us": round(step_ms * 1e3, 3),
         # delivery accumulates every delivered event with one LDS atomic add per receive target
-        # (the kernels that deliver: the delivery kernels, or the overlapped step kernels)
-        "receive_lds_atomics_per_s": round(pst["events"] / ((ms["receive"] + ms["step"]) * 1e-3), 1),
+        "receive_lds_atomics_per_s": round(pst["events"] / args.profile_steps / (step_ms * 1e-3), 1),
     }
-    # the same throughput from the PMC counters of a rocprofv3 run of this workload: atomic
-    # operations counted per launch / this run's mean launch duration
-    counted = measured_atomics(args.workload, kernel_names[kern])
-    if counted is not None:
-        roofline["atomics_counted"] = {
-            "lds_atomic_ops_per_launch": counted["lds_atomic_ops"],
-            "lds_atomic_ops_per_s": round(counted["lds_atomic_ops"] / (avg_ms * 1e-3), 1),
-            "l2_atomic_requests_per_launch": counted["l2_atomic_requests"],
-            "l2_atomic_requests_per_s": round(counted["l2_atomic_requests"] / (avg_ms * 1e-3), 1),
-            "source": "profiles/pmc_traffic.json"}
 
     # The passes' traffic is random 64-byte lines, whose rate -- not the streaming peak -- bounds
     # the plastic step: the same kernel's line transfers per second next to the device's rate for
@@ -616,7 +616,7 @@ def main():
               "probe_read_lines_per_s": round(acc / (t_rd * 1e-6), 1),
               "probe_rmw_line_transfers_per_s": round(2 * acc / (t_rmw * 1e-6), 1)}
         if traffic:
-            rl["kernel_line_transfers_per_s"] = round(traffic / 64 / (avg_ms * 1e-3), 1)
+            rl["kernel_line_transfers_per_s"] = round(traffic / 64 / (step_ms * 1e-3), 1)
             rl["kernel_frac_of_rmw_probe"] = round(rl["kernel_line_transfers_per_s"] / rl["probe_rmw_line_transfers_per_s"], 4)
         roofline["random_lines"] = rl
 
