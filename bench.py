@@ -131,7 +131,7 @@ def algorithmic_bytes(model, n, st, steps):
 def window_bytes(model, n, st, steps, delay):
     """Algorithmic HBM bytes per step of the window kernels, from the device counters of the
     profiled steps:
-      delivery: per delivered spike its id (4) and row offsets (16); per delivered event the low
+      delivery: per delivered spike its id (4) and its row's place in a tile (8); per delivered event the low
                 half of the target id (2) and, for plastic models, the weight read (4);
       update  : per neuron and window its state read + write and, for plastic models, two history
                 words, the traces and the step flags read and written (34); 4 per emitted spike;
@@ -145,7 +145,7 @@ def window_bytes(model, n, st, steps, delay):
     plastic = bool(sattrs)
     spk = st["spikes"] / steps
     ev = st["events"] / steps
-    recv = spk * 20 + ev * (6 if plastic else 2)
+    recv = spk * 12 + ev * (6 if plastic else 2)
     upd = n * (2 * s_n + (34 if plastic else 0)) / window_steps(model, delay) + spk * 4
     fl = (st["flush_slots"] + st["flush_synapses"] + st["flush_written"]) * 4 / steps if plastic else 0.0
     return recv + upd + fl

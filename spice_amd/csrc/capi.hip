@@ -841,7 +841,7 @@ int spice_hip_autotune( spice_net * net, int64_t warmup, int64_t steps, spice_la
 					std::int64_t const tiles = ( N + tw - 1 ) / tw;
 					if( ( tw == start.tile_w && bs == start.recv_block ) || N * ( tiles + 1 ) * 8 > ( std::int64_t( 8 ) << 30 ) ||
 					    tw > n->max_tile_w() )
-						continue; // the start shape, pivots above 8 GB, or wider than the net's tiles
+						continue; // the start shape, a segment table above 8 GB, or wider than the net's tiles
 					launch_cfg x = start;
 					x.tile_w = tw;
 					x.recv_block = bs;

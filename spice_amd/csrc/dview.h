@@ -18,7 +18,8 @@
 //                        neuron i set iff i spiked at step t (H = 256 steps, plastic models)
 //   hasp     uint8[N]    row s has at least one plastic synapse
 //   pl_lo/hi int32[N]    first / one-past-last plastic slot of row s (offsets in the row)
-//   pivots   int64[N * (ntiles+1)]  per row and target tile: place in col of the tile's first target
+//   segs     uint64[N * ntiles]  per row and target tile: place in col and number of the row's targets
+//                        in the tile, 8 tiles of a row side by side (kernels.h, seg_at)
 //   tile_ids int32[ntiles] the tiles: first the nact ones that some row has targets in (at least
 //                        one), then the rest
 // lazy plasticity (per-synapse contract):
@@ -163,7 +164,7 @@ struct dview
 	ctl_t * ctl_prev; // the previous step's clock (its dt for the lazy flush of that step)
 	unsigned long long * bstats; // [nblocks_max * NSTAT]
 
-	std::int64_t * pivots; // [N][ntiles + 1]: place in col of row r's first target >= t * tile_w
+	std::uint64_t * segs; // the segment table: where row r's targets in tile t are (kernels.h, segment_of)
 	std::int32_t ntiles, tile_w;
 	std::int32_t * tile_ids; // [ntiles]: the tiles with incoming synapses (the delivery's), then the others
 	std::int32_t nact;

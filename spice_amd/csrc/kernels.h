@@ -528,19 +528,43 @@ constexpr int TILE_WIDE = 8192;
 // Delivery workgroups have 256 or 1024 threads (a launch shape): they stage that many spikes
 // per pass in LDS.
 
-// Per row r and tile t: place in col of the first target >= t * tile_w, for t = 0 .. ntiles (the
-// last entry is the row's end). One wave per row, binary searches. (Places, not offsets in the
-// row: a staged segment then costs one memory request, two neighbouring entries, and none for
-// where its row starts.)
-static inline __global__ __launch_bounds__( 256 ) void k_pivots( dview v )
+// The place of row r's entry of tile t in the segment table (and of its segment record): the entries
+// of 2^SEG_TILES tiles of a row lie side by side, in one line, then those of the next row. What a tile's
+// deliveries read of them thus stays within one part of the memory, whose page translations a CU
+// can hold, and neighbouring tiles share lines (us per step, with two places per row and tile, row
+// by row, before: Brunel 1e10 12.5, 11.9; brunel_with_plasticity 6e8 11.6, 11.5).
+constexpr int SEG_TILES = 3;
+__device__ inline std::int64_t seg_at( dview const & v, std::int64_t r, std::int32_t t )
+{
+	return ( ( std::int64_t( t >> SEG_TILES ) * v.N + r ) << SEG_TILES ) + ( t & ( ( 1 << SEG_TILES ) - 1 ) );
+}
+// Entries of the table for n rows and ntiles tiles.
+inline std::uint64_t seg_entries( std::int64_t n, std::int64_t ntiles ) { return std::uint64_t( n ) * std::uint64_t( ( ( ntiles - 1 ) >> SEG_TILES ) + 1 ) << SEG_TILES; }
+// The segment of row r in tile t: its place in col and its length (an entry has 40 and 24 bits of them).
+struct segment
+{
+	std::int64_t at;
+	std::int32_t len;
+};
+__device__ inline segment segment_of( dview const & v, std::int64_t r, std::int32_t t )
+{
+	std::uint64_t const e = v.segs[seg_at( v, r, t )];
+	return { std::int64_t( e & ( ( std::uint64_t( 1 ) << 40 ) - 1 ) ), std::int32_t( e >> 40 ) };
+}
+
+// The segment table. One wave per row, binary searches for 63 tiles at a time (the last lane's is
+// where the 63rd one ends).
+static inline __global__ __launch_bounds__( 256 ) void k_segments( dview v )
 {
 	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
 	if( r >= v.N ) return;
 	std::int64_t const lo = v.row_ptr[r];
 	std::int32_t const len = std::int32_t( v.row_ptr[r + 1] - lo );
 	std::int32_t const * c = v.col + lo;
-	for( int t = lane_id(); t <= v.ntiles; t += 64 )
+	int const lane = lane_id();
+	for( int t0 = 0; t0 < v.ntiles; t0 += 63 )
 	{
+		int const t = t0 + lane;
 		std::int64_t const x = std::int64_t( t ) * v.tile_w;
 		std::int32_t a = 0, b = len; // first index with c[index] >= x
 		while( a < b )
@@ -551,7 +575,8 @@ static inline __global__ __launch_bounds__( 256 ) void k_pivots( dview v )
 			else
 				b = m;
 		}
-		v.pivots[r * ( v.ntiles + 1 ) + t] = lo + a;
+		std::int32_t const next = std::int32_t( shfl_u32( std::uint32_t( a ), lane + 1 ) );
+		if( lane < 63 && t < v.ntiles ) v.segs[seg_at( v, r, t )] = std::uint64_t( lo + a ) | std::uint64_t( next - a ) << 40;
 	}
 }
 
@@ -560,9 +585,8 @@ static inline __global__ __launch_bounds__( 256 ) void k_tile_active( dview v, s
 {
 	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
 	if( r >= v.N ) return;
-	std::int64_t const * pv = v.pivots + r * ( v.ntiles + 1 );
 	for( int t = lane_id(); t < v.ntiles; t += 64 )
-		if( pv[t + 1] > pv[t] ) flag[t] = 1;
+		if( segment_of( v, r, t ).len > 0 ) flag[t] = 1;
 }
 
 // Attributes of the receiving neurons that the delivering workgroup copies into LDS: those
@@ -850,9 +874,9 @@ __device__ inline void receive_tile( dview const & v, std::int32_t work )
 			if( tid < cnt )
 			{
 				src = spk[c0 + tid];
-				std::int64_t const * pv = v.pivots + std::int64_t( src ) * ( v.ntiles + 1 ) + tile;
-				beg = pv[0];
-				len = std::int32_t( pv[1] - beg );
+				segment const s = segment_of( v, src, tile );
+				beg = s.at;
+				len = s.len;
 				if constexpr( deferred )
 				{
 					pend = catch_up && ( v.fl8[prev + src] & F8_ARRIVED );

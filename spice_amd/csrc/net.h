@@ -543,7 +543,7 @@ public:
 		     _fl_id.bytes() + _fl_synced.bytes() + _fl_pend.bytes() + _hasp.bytes() + _pl_lo.bytes() + _pl_hi.bytes() +
 		     _fl_count.bytes() + _xtr.bytes() + _ytr.bytes() + _fl8.bytes() + _sp8.bytes() + _po_id.bytes() + _po_count.bytes() +
 		     _tp_ptr.bytes() + _caught.bytes() + _tp_ent.bytes() + _ctl.bytes() + _bstats.bytes() +
-		     _pivots.bytes() + _recs.bytes() + _col16.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
+		     _segs.bytes() + _recs.bytes() + _col16.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
 		return b;
 	}
 
@@ -714,7 +714,7 @@ private:
 	launch_cfg _lc{};
 	std::shared_ptr<host_stage> _stage; // see stage_to_host
 	int _staged = 0;                    // calls that asked for it
-	dbuf<std::int64_t> _pivots;
+	dbuf<std::uint64_t> _segs;
 	dbuf<unsigned char> _recs; // segment records
 	dbuf<std::uint16_t> _col16;       // low halves of the row store
 	dbuf<std::int32_t> _tile_ids;
@@ -1052,11 +1052,11 @@ private:
 		if( retile )
 		{
 			std::int32_t const ntiles = std::int32_t( ( n + c.tile_w - 1 ) / c.tile_w );
-			_pivots.resize( std::size_t( n ) * ( ntiles + 1 ) );
+			_segs.resize( seg_entries( n, ntiles ) );
 			v.tile_w = c.tile_w;
 			v.ntiles = ntiles;
-			v.pivots = _pivots.data();
-			SPICE_LAUNCH( k_pivots<<<unsigned( ( n + 3 ) / 4 ), 256, 0, _s>>>( _v ) );
+			v.segs = _segs.data();
+			SPICE_LAUNCH( k_segments<<<unsigned( ( n + 3 ) / 4 ), 256, 0, _s>>>( _v ) );
 			find_active_tiles(); // (synchronizes)
 		}
 		double const mean_row = n > 0 ? double( _g.nnz ) / double( n ) : 0.0;
@@ -1107,7 +1107,7 @@ private:
 
 	// The delivery's tiles: those that some row has a target in (a population that no
 	// connection targets gets no delivery workgroups); at least one, so that every step has a
-	// delivery work item. Runs right after the pivots are built, before the views are copied.
+	// delivery work item. Runs right after the segment table is built, before the views are copied.
 	void find_active_tiles()
 	{
 		dview & v = _v;
@@ -1243,7 +1243,7 @@ private:
 			double const mean = double( _g.nnz ) / double( _g.n ) / _v.nact, need = mean + 2.9 * std::sqrt( mean );
 			int lg = 4;
 			while( lg < 8 && rec_capacity( lg ) < need ) lg++;
-			std::uint64_t const segs = std::uint64_t( _g.n ) * std::uint64_t( ( ( _v.ntiles - 1 ) >> REC_TILES ) + 1 ) << REC_TILES, bytes = segs << lg;
+			std::uint64_t const segs = seg_entries( _g.n, _v.ntiles ), bytes = segs << lg;
 			if( _v.wcap > 1 || _window == 0 || _p.batched || lg > 7 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
 			if( bytes > ( std::uint64_t( 1 ) << 30 ) )
 			{

@@ -124,15 +124,8 @@ static inline __global__ __launch_bounds__( 256 ) void k_halves( std::int32_t co
 // need no atomic, were slower to read (8.5 and 28.3).
 constexpr std::uint16_t REC_LONG = 0xffff;
 HYBRID constexpr int rec_capacity( int lg ) { return ( 1 << lg ) / 2 - 1; }
-// The place of row r's record of tile t: the records of 2^REC_TILES tiles of a row lie side by side,
-// then those of the next row. A tile's deliveries thus stay within one part of the memory, whose
-// page translations a CU can hold, and a line of small records still serves several tiles (synth
-// 1e9, 3.3 GB of records: 21.7 us per step with 8 tiles, 21.9 with 4, 23.3 with 32, 24.0 row by row).
-constexpr int REC_TILES = 3;
-__device__ inline std::int64_t rec_at( dview const & v, std::int64_t r, std::int32_t t )
-{
-	return ( ( std::int64_t( t >> REC_TILES ) * v.N + r ) << REC_TILES ) + ( t & ( ( 1 << REC_TILES ) - 1 ) );
-}
+// (A row's record of a tile lies where the segment table has their entry, see seg_at: synth 1e9, 3.3 GB
+// of records, 21.7 us per step with 8 tiles side by side, 21.9 with 4, 23.3 with 32, 24.0 row by row.)
 struct alignas( 16 ) rec_part // 16 bytes of a record
 {
 	std::uint16_t t[8];
@@ -145,7 +138,7 @@ template <int BS>
 __device__ inline int rec_group( int x, int gl, std::int32_t tile )
 {
 	int const ng = BS >> gl;
-	return ( x + ( ( tile & ( ( 1 << REC_TILES ) - 1 ) ) * ng >> REC_TILES ) ) & ( ng - 1 );
+	return ( x + ( ( tile & ( ( 1 << SEG_TILES ) - 1 ) ) * ng >> SEG_TILES ) ) & ( ng - 1 );
 }
 
 // Builds the records, one wave per row, a lane per tile; *longs counts the segments that do not fit.
@@ -153,14 +146,14 @@ static inline __global__ __launch_bounds__( 256 ) void k_records( dview v, unsig
 {
 	std::int64_t const r = uniform64( ( std::int64_t( blockIdx.x ) * blockDim.x + threadIdx.x ) >> 6 );
 	if( r >= v.N ) return;
-	std::int64_t const * pv = v.pivots + r * ( v.ntiles + 1 );
 	std::int64_t const nnz = v.row_ptr[v.N];
 	int const cap = rec_capacity( lg );
 	for( int t = lane_id(); t < v.ntiles; t += 64 )
 	{
-		std::int64_t const a = pv[t];
-		std::int32_t const len = std::int32_t( pv[t + 1] - a ), t0 = t * v.tile_w;
-		rec_part * const out = reinterpret_cast<rec_part *>( recs + ( rec_at( v, r, t ) << lg ) );
+		segment const s = segment_of( v, r, t );
+		std::int64_t const a = s.at;
+		std::int32_t const len = s.len, t0 = t * v.tile_w;
+		rec_part * const out = reinterpret_cast<rec_part *>( recs + ( seg_at( v, r, t ) << lg ) );
 		if( len > cap )
 		{
 			rec_part p{};
@@ -410,7 +403,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 				for( int u = 0; u < U; u++ )
 				{
 					r[u] = rec_part{};
-					if( c + u * ng < total ) r[u] = recs[( rec_at( v, src[u], tile ) << gl ) + l];
+					if( c + u * ng < total ) r[u] = recs[( seg_at( v, src[u], tile ) << gl ) + l];
 					at[u] = N::input_class( src[u], info ) * tws;
 				}
 				if( c == 0 ) __syncthreads(); // the accumulators are clear
@@ -428,7 +421,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 						if( ( x > 0 || l > 0 ) && e0 + x < len ) atomicAdd( acc + ( at[u] + r[u].t[x] ), 1u );
 					if( ok[u] && head == REC_LONG )
 					{
-						rec_part const whole = recs[rec_at( v, src[u], tile ) << gl];
+						rec_part const whole = recs[seg_at( v, src[u], tile ) << gl];
 						std::int32_t n;
 						std::int64_t off;
 						__builtin_memcpy( &n, &whole.t[2], 4 );
@@ -456,12 +449,8 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	{
 		win_seg * const mine = seg + wave * 64;
 		std::int32_t src, q = 0, src_n = 0, q_n = 0;
-		std::int64_t a, b;
-		auto fetch_seg = [&]() {
-			std::int64_t const * pv = v.pivots + std::int64_t( src ) * ( v.ntiles + 1 ) + tile;
-			a = pv[0];
-			b = pv[1];
-		};
+		segment sg;
+		auto fetch_seg = [&]() { sg = segment_of( v, src, tile ); };
 		src = fetch_id( k0 + mylane, q );
 		fetch_seg();
 		if( k0 + NW * per < total ) src_n = fetch_id( k0 + NW * per + mylane, q_n );
@@ -470,7 +459,8 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 		for( ; k0 < total; k0 += NW * per )
 		{
 			std::int32_t const cnt = ( total - k0 ) < per ? ( total - k0 ) : per;
-			std::int32_t const len = lane < cnt ? std::int32_t( b - a ) : 0;
+			std::int64_t const a = sg.at;
+			std::int32_t const len = lane < cnt ? sg.len : 0;
 			if constexpr( L::classes > 0 )
 				// in the place of the source: where the class's counters of the step start (for target 0)
 				// (IDS16X8 also: the piece that the segment begins in, its end from there on, its place there)
@@ -1125,9 +1115,9 @@ __global__ __launch_bounds__( TP_BLOCK ) void k_tp_tile( dview v, std::uint32_t 
 		std::int32_t len = 0;
 		if( r < v.N && v.hasp[r] )
 		{
-			std::int64_t const * pv = v.pivots + std::int64_t( r ) * ( v.ntiles + 1 ) + tile;
-			a = pv[0];
-			len = std::int32_t( pv[1] - a );
+			segment const s = segment_of( v, r, tile );
+			a = s.at;
+			len = s.len;
 			mine_in[lane] = std::int32_t( a - v.row_ptr[r] );
 		}
 		mine[lane] = rec{ len > 0 ? a : 0, r, len };
