@@ -1056,7 +1056,14 @@ private:
 			v.tile_w = c.tile_w;
 			v.ntiles = ntiles;
 			v.segs = _segs.data();
-			SPICE_LAUNCH( k_segments<<<unsigned( ( n + 3 ) / 4 ), 256, 0, _s>>>( _v ) );
+			if( _v.wcap > 1 && ntiles <= PASS_TILES && !_col16.size() && wants_halves( double( _g.nnz ) / double( n ) * double( c.tile_w ) / double( std::max<std::int64_t>( _g.targets, 1 ) ) ) &&
+			    allocate_halves() )
+			{
+				std::uint32_t const d = std::uint32_t( c.tile_w ) / 64, magic = d == 1 ? 0u : std::uint32_t( ( ( std::uint64_t( 1 ) << 32 ) + d - 1 ) / d );
+				SPICE_LAUNCH( k_segments_halves<<<unsigned( ( n + 3 ) / 4 ), 256, 16 * std::size_t( ntiles + 1 ), _s>>>( _v, _g.nnz, magic, _col16.data() ) );
+			}
+			else
+				SPICE_LAUNCH( k_segments<<<unsigned( ( n + 3 ) / 4 ), 256, 0, _s>>>( _v ) );
 			find_active_tiles(); // (synchronizes)
 		}
 		double const mean_row = n > 0 ? double( _g.nnz ) / double( n ) : 0.0;
@@ -1194,39 +1201,48 @@ private:
 	// (Brunel 1e10) 17.2, 14.9, 12.5; beside weights, 26 (brunel_with_plasticity 6e8) 12.5, 11.6, 45
 	// (brunel_3pop_stdp 1e9, steps 2,000 on) 24.9, 24.3. None if they took more than a fifth of the free memory; none for
 	// the nets of a batch, whose kernel reads the row store.
+	bool wants_halves( double mean ) const
+	{
+		return ( input_classes_v<Model> > 0 || ( plastic && windowed && !_lazy ) ) && !_p.batched && _g.nnz > 0 && mean >= 4.0;
+	}
+	bool allocate_halves()
+	{
+		std::size_t const n = std::size_t( _g.nnz ) + 8;
+		if( n > ( std::size_t( 1 ) << 29 ) )
+		{
+			std::size_t room = 0, all = 0;
+			SPICE_HIP( hipMemGetInfo( &room, &all ) );
+			if( 2 * n > room / 5 ) return false;
+		}
+		try
+		{
+			_col16.resize( n );
+		}
+		catch( std::bad_alloc const & )
+		{
+			return false;
+		}
+		return true;
+	}
 	void build_halves()
 	{
 		_v.col16 = nullptr;
-		if constexpr( input_classes_v<Model> > 0 || ( plastic && windowed ) )
+		double const mean = double( _g.nnz ) / double( _g.n ) / _v.nact;
+		if( _window == 0 || _v.rec_lg || !wants_halves( mean ) )
 		{
-			if( _window == 0 || _v.rec_lg || _p.batched || _g.nnz == 0 ) return;
-			// (lanes per segment: see choose_window)
-			double const mean = double( _g.nnz ) / double( _g.n ) / _v.nact;
-			if( mean < 4.0 ) return;
-			if( !_col16.size() )
-			{
-				std::size_t const n = std::size_t( _g.nnz ) + 8;
-				if( n > ( std::size_t( 1 ) << 29 ) )
-				{
-					std::size_t room = 0, all = 0;
-					SPICE_HIP( hipMemGetInfo( &room, &all ) );
-					if( 2 * n > room / 5 ) return;
-				}
-				try
-				{
-					_col16.resize( n );
-				}
-				catch( std::bad_alloc const & )
-				{
-					return;
-				}
-				SPICE_LAUNCH( k_halves<<<unsigned( std::min<std::size_t>( ( n / 8 + 255 ) / 256, 256 * 32 ) ), 256, 0, _s>>>( _g.col.data(), _g.nnz, _col16.data() ) );
-			}
-			_v.col16 = _col16.data();
-			_v.vec16 = !plastic && mean >= 56.0 ? 8 : 4;
-			_v.wlanes = 0;
-			while( _v.wlanes < 5 && double( _v.vec16 << _v.wlanes ) < mean + ( mean < 20.0 ? 2.0 : 1.0 ) * std::sqrt( mean ) + ( _v.vec16 == 8 ? 4.0 : 0.0 ) ) _v.wlanes++;
+			_col16.release();
+			return;
 		}
+		if( !_col16.size() )
+		{
+			if( !allocate_halves() ) return;
+			SPICE_LAUNCH( k_halves<<<unsigned( std::min<std::size_t>( ( std::size_t( _g.nnz ) / 8 + 256 ) / 256, 256 * 32 ) ), 256, 0, _s>>>( _g.col.data(), _g.nnz, _col16.data() ) );
+		}
+		_v.col16 = _col16.data();
+		_v.vec16 = !plastic && mean >= 56.0 ? 8 : 4;
+		// (lanes per segment: see choose_window)
+		_v.wlanes = 0;
+		while( _v.wlanes < 5 && double( _v.vec16 << _v.wlanes ) < mean + ( mean < 20.0 ? 2.0 : 1.0 ) * std::sqrt( mean ) + ( _v.vec16 == 8 ? 4.0 : 0.0 ) ) _v.wlanes++;
 	}
 
 	// Segment records (window.h) of networks that run step by step, where segments are short: the

@@ -163,6 +163,8 @@ def test_spikes_and_state_read_back(gpu, n):
     ("brunel_3pop", three_pop_layout(1500), 15, (640, 512)),
     ("synth", ([300], [(0, 0, 1.0)]), 1, (256, 256)),  # step by step, too long for records
     ("synth", ([257], [(0, 0, 1.0)]), 2, (64, 256)),
+    ("synth", ([40000], [(0, 0, 0.025)]), 3, (0, 0)),  # the tiles that it is built with: 209 of 192
+    ("vogels_abbott", ([20003], [(0, 0, 0.06)]), 6, (0, 0)),
     ("brunel_3pop_stdp", three_pop_layout(66000, 0.005), 15, (1024, 512)),  # beside the weights
     ("brunel_3pop_stdp", three_pop_layout(500), 3, (64, 256)),
 ])
