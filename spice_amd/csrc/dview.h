@@ -43,7 +43,7 @@
 //   po_id    int32[2][N] neurons that spiked in the window and have incoming plastic synapses
 //                        (their counters by k mod 4)
 // both:
-//   tp_ptr   int64[N+1], tp_ent {src, offset in src's row}[P]: the P plastic synapses by target
+//   tp_ptr   int64[N+1], tp_ent {src, place}[P]: the P plastic synapses by target
 // both:
 //   caught   int64       step whose plasticity work (and, eager, deferred events of the rows
 //                        arriving next) a synchronization already did
@@ -98,14 +98,11 @@ struct slog_t
 	std::uint64_t cap;
 };
 
-// One plastic synapse of the by-target index: its source row and its offset in that row
-// (offset first: read as one little-endian 64-bit word the source is the high half, so the
-// word orders entries by source).
-struct alignas( 8 ) tp_entry
-{
-	std::int32_t off;
-	std::int32_t src;
-};
+// One plastic synapse of the by-target index: its source row, and its place among the synapses (tp_form
+// TP_PLACE: 24 and 40 bits) or, in networks whose numbers do not fit those, its offset in that row
+// (TP_OFFSET: 32 and 32 bits), whose start costs one more gather.
+using tp_entry = std::uint64_t;
+enum { TP_OFFSET, TP_PLACE };
 
 // The spike counters of successive steps lie this many words apart: all tiles reserve their places
 // of all of a window's steps at about the same time, and atomics on one line wait for each other, 9
@@ -156,6 +153,7 @@ struct dview
 	std::uint32_t * po_count; // [4]
 	std::int64_t const * tp_ptr;
 	tp_entry const * tp_ent;
+	std::int32_t tp_form;
 	std::int64_t * caught;
 
 	ctl_t * ctl0;     // the clock slots

@@ -580,6 +580,17 @@ static inline __global__ __launch_bounds__( 256 ) void k_segments( dview v )
 	}
 }
 
+// Entry of the by-target index, its source and its synapse's place.
+__device__ inline tp_entry make_tp( dview const & v, std::int32_t src, std::int64_t place, std::int32_t off )
+{
+	return v.tp_form == TP_PLACE ? std::uint64_t( place ) | std::uint64_t( src ) << 40 : std::uint64_t( off ) | std::uint64_t( src ) << 32;
+}
+__device__ inline std::int32_t tp_src( dview const & v, tp_entry e ) { return std::int32_t( v.tp_form == TP_PLACE ? e >> 40 : e >> 32 ); }
+__device__ inline std::int64_t tp_place( dview const & v, tp_entry e )
+{
+	return v.tp_form == TP_PLACE ? std::int64_t( e & ( ( std::uint64_t( 1 ) << 40 ) - 1 ) ) : v.row_ptr[e >> 32] + std::int64_t( std::uint32_t( e ) );
+}
+
 // flag[t] = 1 for every tile t that some row has a target in. One wave per row.
 static inline __global__ __launch_bounds__( 256 ) void k_tile_active( dview v, std::uint8_t * flag )
 {
@@ -1532,7 +1543,7 @@ __device__ inline void stdp_block( dview const & v, std::int64_t T, std::int64_t
 				{
 					std::int64_t const k = base + lane + 64 * u;
 					ok[u] = k < end;
-					te[u] = ok[u] ? v.tp_ent[k] : tp_entry{ 0, 0 };
+					te[u] = ok[u] ? v.tp_ent[k] : 0;
 				}
 				// the source's flags, row start and trace: independent loads, issued together
 				std::int64_t e[UP];
@@ -1541,9 +1552,10 @@ __device__ inline void stdp_block( dview const & v, std::int64_t T, std::int64_t
 #pragma unroll
 				for( int u = 0; u < UP; u++ )
 				{
-					f8[u] = v.fl8[cur + te[u].src];
-					e[u] = v.row_ptr[te[u].src] + te[u].off;
-					xv[u] = v.xtr[cur + te[u].src];
+					std::int32_t const src = tp_src( v, te[u] );
+					f8[u] = v.fl8[cur + src];
+					e[u] = tp_place( v, te[u] );
+					xv[u] = v.xtr[cur + src];
 				}
 #pragma unroll
 				for( int u = 0; u < UP; u++ ) ok[u] = ok[u] && !( f8[u] & ( F8_ARRIVED | F8_ARRIVES_NEXT ) );

@@ -990,9 +990,17 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 #pragma unroll
 				for( int u = 0; u < U; u++ )
 				{
-					a8[u] = v.fl8[par + te[u].src];
-					e[u] = v.row_ptr[te[u].src] + te[u].off;
-					xv[u] = v.xtr[tr + te[u].src];
+					std::int32_t const src = tp_src( v, te[u] );
+					a8[u] = v.fl8[par + src];
+					e[u] = tp_place( v, te[u] );
+					xv[u] = v.xtr[tr + src];
+				}
+				typename S::tuple_t sy[U];
+				if constexpr( !has_inert_v<S> )
+				{
+					// (few sources arrived: their weights are read for nothing)
+#pragma unroll
+					for( int u = 0; u < U; u++ ) load_synapse<S>( sy[u], v.sa, e[u] );
 				}
 				for( int q = 0; q <= b; q++ )
 				{
@@ -1000,7 +1008,6 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 #pragma unroll
 					for( int u = 0; u < U; u++ ) xv[u] = fmaf( xv[u], dq, 0.0f ); // (no arrival in the window)
 				}
-				typename S::tuple_t sy[U];
 #pragma unroll
 				for( int u = 0; u < U; u++ )
 				{
@@ -1011,7 +1018,8 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 							ok[u] = false;
 							touched++;
 						}
-					if( ok[u] ) load_synapse<S>( sy[u], v.sa, e[u] );
+					if constexpr( has_inert_v<S> )
+						if( ok[u] ) load_synapse<S>( sy[u], v.sa, e[u] );
 				}
 #pragma unroll
 				for( int u = 0; u < U; u++ )
@@ -1204,7 +1212,7 @@ __global__ __launch_bounds__( TP_BLOCK ) void k_tp_tile( dview v, std::uint32_t 
 						if( e + x >= n[u] || !S::plastic( q[u].row, j[u].id[x], info ) ) continue;
 						std::uint32_t const at = atomicAdd( &cur[j[u].id[x] - t0], 1u );
 						if constexpr( !COUNT )
-							ent[first[j[u].id[x] - t0] + at] = tp_entry{ mine_in[( c + u * ng + g ) & 63] + e + x, q[u].row };
+							ent[first[j[u].id[x] - t0] + at] = make_tp( v, q[u].row, q[u].off + e + x, mine_in[( c + u * ng + g ) & 63] + e + x );
 					}
 			}
 		}
