@@ -98,11 +98,9 @@ struct slog_t
 	std::uint64_t cap;
 };
 
-// One plastic synapse of the by-target index: its source row, and its place among the synapses (tp_form
-// TP_PLACE: 24 and 40 bits) or, in networks whose numbers do not fit those, its offset in that row
-// (TP_OFFSET: 32 and 32 bits), whose start costs one more gather.
+// One plastic synapse of the by-target index: its source row (the upper 24 bits: a plastic network of
+// 2^24 neurons would need 2 TB for its segment table) and its place among the synapses (40 bits).
 using tp_entry = std::uint64_t;
-enum { TP_OFFSET, TP_PLACE };
 
 // The spike counters of successive steps lie this many words apart: all tiles reserve their places
 // of all of a window's steps at about the same time, and atomics on one line wait for each other, 9
@@ -153,7 +151,6 @@ struct dview
 	std::uint32_t * po_count; // [4]
 	std::int64_t const * tp_ptr;
 	tp_entry const * tp_ent;
-	std::int32_t tp_form;
 	std::int64_t * caught;
 
 	ctl_t * ctl0;     // the clock slots

@@ -581,15 +581,9 @@ static inline __global__ __launch_bounds__( 256 ) void k_segments( dview v )
 }
 
 // Entry of the by-target index, its source and its synapse's place.
-__device__ inline tp_entry make_tp( dview const & v, std::int32_t src, std::int64_t place, std::int32_t off )
-{
-	return v.tp_form == TP_PLACE ? std::uint64_t( place ) | std::uint64_t( src ) << 40 : std::uint64_t( off ) | std::uint64_t( src ) << 32;
-}
-__device__ inline std::int32_t tp_src( dview const & v, tp_entry e ) { return std::int32_t( v.tp_form == TP_PLACE ? e >> 40 : e >> 32 ); }
-__device__ inline std::int64_t tp_place( dview const & v, tp_entry e )
-{
-	return v.tp_form == TP_PLACE ? std::int64_t( e & ( ( std::uint64_t( 1 ) << 40 ) - 1 ) ) : v.row_ptr[e >> 32] + std::int64_t( std::uint32_t( e ) );
-}
+__device__ inline tp_entry make_tp( std::int32_t src, std::int64_t place ) { return std::uint64_t( place ) | std::uint64_t( src ) << 40; }
+__device__ inline std::int32_t tp_src( tp_entry e ) { return std::int32_t( e >> 40 ); }
+__device__ inline std::int64_t tp_place( tp_entry e ) { return std::int64_t( e & ( ( std::uint64_t( 1 ) << 40 ) - 1 ) ); }
 
 // flag[t] = 1 for every tile t that some row has a target in. One wave per row.
 static inline __global__ __launch_bounds__( 256 ) void k_tile_active( dview v, std::uint8_t * flag )
@@ -1545,16 +1539,16 @@ __device__ inline void stdp_block( dview const & v, std::int64_t T, std::int64_t
 					ok[u] = k < end;
 					te[u] = ok[u] ? v.tp_ent[k] : 0;
 				}
-				// the source's flags, row start and trace: independent loads, issued together
+				// the source's flags and trace: independent loads, issued together
 				std::int64_t e[UP];
 				float xv[UP];
 				std::uint8_t f8[UP];
 #pragma unroll
 				for( int u = 0; u < UP; u++ )
 				{
-					std::int32_t const src = tp_src( v, te[u] );
+					std::int32_t const src = tp_src( te[u] );
 					f8[u] = v.fl8[cur + src];
-					e[u] = tp_place( v, te[u] );
+					e[u] = tp_place( te[u] );
 					xv[u] = v.xtr[cur + src];
 				}
 #pragma unroll

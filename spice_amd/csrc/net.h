@@ -959,6 +959,7 @@ private:
 	void build_by_target()
 	{
 		std::int64_t const n = _g.n;
+		if( n > ( std::int64_t( 1 ) << 24 ) ) throw std::bad_alloc(); // (its segment table did not fit either)
 		dbuf<std::uint32_t> cnt( n );
 		SPICE_HIP( hipMemsetAsync( cnt.data(), 0, cnt.bytes(), _s ) ); // (tiles without inputs are not walked)
 		SPICE_LAUNCH( ( k_tp_tile<Model, true><<<unsigned( _v.nact ), TP_BLOCK, 0, _s>>>( _v, cnt.data(), nullptr ) ) );
@@ -969,7 +970,6 @@ private:
 		_tp_total = ptr[n];
 		_tp_ent.resize( std::size_t( std::max<std::int64_t>( _tp_total, 1 ) ) );
 		_v.tp_ent = _tp_ent.data();
-		_v.tp_form = n <= ( std::int64_t( 1 ) << 24 ) && _g.nnz <= ( std::int64_t( 1 ) << 40 ) ? TP_PLACE : TP_OFFSET;
 		if( _tp_total > 0 ) SPICE_LAUNCH( ( k_tp_tile<Model, false><<<unsigned( _v.nact ), TP_BLOCK, 0, _s>>>( _v, nullptr, _tp_ent.data() ) ) );
 		// targets with incoming plastic synapses (the mean in-degree sets the post-pass split)
 		_tp_targets = 0;

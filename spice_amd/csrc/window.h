@@ -983,16 +983,16 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 					ok[u] = x < end;
 					te[u] = v.tp_ent[ok[u] ? x : beg];
 				}
-				// the source's arrival, row start and trace: independent loads, issued together
+				// the source's arrival and trace: independent loads, issued together
 				std::int64_t e[U];
 				float xv[U];
 				std::uint8_t a8[U];
 #pragma unroll
 				for( int u = 0; u < U; u++ )
 				{
-					std::int32_t const src = tp_src( v, te[u] );
+					std::int32_t const src = tp_src( te[u] );
 					a8[u] = v.fl8[par + src];
-					e[u] = tp_place( v, te[u] );
+					e[u] = tp_place( te[u] );
 					xv[u] = v.xtr[tr + src];
 				}
 				typename S::tuple_t sy[U];
@@ -1156,7 +1156,6 @@ __global__ __launch_bounds__( TP_BLOCK ) void k_tp_tile( dview v, std::uint32_t 
 		std::int32_t len;
 	};
 	__shared__ rec segs[TP_BLOCK];
-	__shared__ std::int32_t in_row[TP_BLOCK]; // the segment's offset in its row
 	__shared__ std::uint32_t cur[TILE_MAX];
 	__shared__ std::int64_t first[COUNT ? 1 : TILE_MAX];
 	int const tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
@@ -1172,7 +1171,6 @@ __global__ __launch_bounds__( TP_BLOCK ) void k_tp_tile( dview v, std::uint32_t 
 	snn_info const info = info_of( v );
 	int const G = 1 << v.wlanes, g = lane >> v.wlanes, l = lane & ( G - 1 ), ng = 64 >> v.wlanes;
 	rec * const mine = segs + wave * 64;
-	std::int32_t * const mine_in = in_row + wave * 64;
 	for( std::int32_t r0 = wave * 64; r0 < v.N; r0 += TP_BLOCK )
 	{
 		std::int32_t const r = r0 + lane;
@@ -1183,7 +1181,6 @@ __global__ __launch_bounds__( TP_BLOCK ) void k_tp_tile( dview v, std::uint32_t 
 			segment const s = segment_of( v, r, tile );
 			a = s.at;
 			len = s.len;
-			mine_in[lane] = std::int32_t( a - v.row_ptr[r] );
 		}
 		mine[lane] = rec{ len > 0 ? a : 0, r, len };
 		wave_lds_fence();
@@ -1212,7 +1209,7 @@ __global__ __launch_bounds__( TP_BLOCK ) void k_tp_tile( dview v, std::uint32_t 
 						if( e + x >= n[u] || !S::plastic( q[u].row, j[u].id[x], info ) ) continue;
 						std::uint32_t const at = atomicAdd( &cur[j[u].id[x] - t0], 1u );
 						if constexpr( !COUNT )
-							ent[first[j[u].id[x] - t0] + at] = make_tp( v, q[u].row, q[u].off + e + x, mine_in[( c + u * ng + g ) & 63] + e + x );
+							ent[first[j[u].id[x] - t0] + at] = make_tp( q[u].row, q[u].off + e + x );
 					}
 			}
 		}
