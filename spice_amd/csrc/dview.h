@@ -36,6 +36,7 @@
 //   po_id    int32[2][N] neurons that spiked at T and have incoming plastic synapses
 // eager plasticity in windows (refractory endpoints), k = the window's number:
 //   xtr/ytr  f32[4][N]   traces before the window's first step, by k mod 4
+//   xpost    u32[2][N]   by k mod 2: what the post pass needs of a source in one gather
 //   fl8      u8[2][N]    by k mod 2: 1 + the step of the window at which the neuron's spike
 //                        arrived (0: none)
 //   sp8      u8[2][N]    by k mod 2: 1 + the step of the window at which the neuron spiked
@@ -101,6 +102,7 @@ struct slog_t
 // One plastic synapse of the by-target index: its source row (the upper 24 bits: a plastic network of
 // 2^24 neurons would need 2 TB for its segment table) and its place among the synapses (40 bits).
 using tp_entry = std::uint64_t;
+constexpr std::uint32_t X_ARRIVED = 0xffffffffu; // (a NaN that no arithmetic gives)
 
 // The spike counters of successive steps lie this many words apart: all tiles reserve their places
 // of all of a window's steps at about the same time, and atomics on one line wait for each other, 9
@@ -145,6 +147,7 @@ struct dview
 	std::uint32_t * fl_count; // [4]
 	float * xtr;
 	float * ytr;
+	std::uint32_t * xpost; // windows: [2][N] pre trace at the window's start, X_ARRIVED if the spike arrived in it
 	std::uint8_t * fl8;
 	std::uint8_t * sp8;
 	std::int32_t * po_id;

@@ -541,7 +541,7 @@ public:
 		for( int a = 0; a < MAXA; a++ ) b += _na[a].bytes() + _acc[a].bytes() + _sa[a].bytes();
 		b += _ring.bytes() + _counts.bytes() + _hring.bytes() + _last_spk.bytes() + _synced.bytes() + _pend.bytes() +
 		     _fl_id.bytes() + _fl_synced.bytes() + _fl_pend.bytes() + _hasp.bytes() + _pl_lo.bytes() + _pl_hi.bytes() +
-		     _fl_count.bytes() + _xtr.bytes() + _ytr.bytes() + _fl8.bytes() + _sp8.bytes() + _po_id.bytes() + _po_count.bytes() +
+		     _fl_count.bytes() + _xtr.bytes() + _ytr.bytes() + _fl8.bytes() + _xpost.bytes() + _sp8.bytes() + _po_id.bytes() + _po_count.bytes() +
 		     _tp_ptr.bytes() + _caught.bytes() + _tp_ent.bytes() + _ctl.bytes() + _bstats.bytes() +
 		     _segs.bytes() + _recs.bytes() + _col16.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
 		return b;
@@ -687,6 +687,7 @@ private:
 	dbuf<std::uint8_t> _hasp;
 	dbuf<std::int32_t> _pl_lo, _pl_hi;
 	dbuf<std::uint32_t> _fl_count;
+	dbuf<std::uint32_t> _xpost;                // eager windows: see dview
 	dbuf<float> _xtr, _ytr;                    // eager: traces, [2][N] by step parity or [4][N] by window
 	dbuf<std::uint8_t> _fl8, _sp8;             // eager: [2][N] step flags, or the windows' arrivals and spikes
 	dbuf<std::int32_t> _po_id;                 // eager: [2][N] spiking targets
@@ -788,6 +789,7 @@ private:
 				_xtr.resize( ( windowed ? 4 : 2 ) * n );
 				_ytr.resize( ( windowed ? 4 : 2 ) * n );
 				_fl8.resize( 2 * n );
+				if( windowed ) _xpost.resize( 2 * n );
 				if( windowed ) _sp8.resize( 2 * n );
 				_po_id.resize( 2 * n );
 				_po_count.resize( CLOCK_SLOTS );
@@ -836,6 +838,7 @@ private:
 		v.xtr = _xtr.data();
 		v.ytr = _ytr.data();
 		v.fl8 = _fl8.data();
+		v.xpost = _xpost.data();
 		v.sp8 = _sp8.data();
 		v.po_id = _po_id.data();
 		v.po_count = _po_count.data();

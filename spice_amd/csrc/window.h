@@ -621,7 +621,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 			// plastic models: the arrivals of this neuron's own spikes (of the steps from T0 - D), its
 			// traces, and the history words that the window's steps go to
 			std::uint32_t arrivals = 0;
-			float xt = 0.0f, yt = 0.0f;
+			float xt = 0.0f, yt = 0.0f, x0 = 0.0f;
 			unsigned long long h0 = 0, h1 = 0;
 			std::int64_t const hw0 = ( T0 & ( HISTORY - 1 ) ) >> 6, hw1 = ( ( T0 + W - 1 ) & ( HISTORY - 1 ) ) >> 6;
 			bool has_out = false, has_in = false;
@@ -635,6 +635,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 				if( hw1 != hw0 ) h1 = v.hring[hw1 * v.N + i];
 				xt = v.xtr[( clk.wseq & 3 ) * std::int64_t( v.N ) + i];
 				yt = v.ytr[( clk.wseq & 3 ) * std::int64_t( v.N ) + i];
+				x0 = xt;
 				has_out = v.hasp[i];
 				has_in = v.tp_ptr[i + 1] > v.tp_ptr[i];
 			}
@@ -706,6 +707,8 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 				v.xtr[nx] = xt;
 				v.ytr[nx] = yt;
 				v.fl8[par] = std::uint8_t( arrivals ? __builtin_ctz( arrivals ) + 1 : 0 );
+				std::uint32_t const x0b = __builtin_bit_cast( std::uint32_t, x0 );
+				v.xpost[par] = arrivals ? X_ARRIVED : x0b == X_ARRIVED ? 0x7fc00000u : x0b;
 				v.sp8[par] = std::uint8_t( spikes ? __builtin_ctz( spikes ) + 1 : 0 );
 				if( has_out && arrivals ) spikes |= 1u << W;
 				if( has_in && ( spikes & std::uint32_t( all ) ) ) spikes |= 2u << W;
@@ -983,17 +986,16 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 					ok[u] = x < end;
 					te[u] = v.tp_ent[ok[u] ? x : beg];
 				}
-				// the source's arrival and trace: independent loads, issued together
+				// the source's trace at the window's start, or that its spike arrived in the window
 				std::int64_t e[U];
 				float xv[U];
-				std::uint8_t a8[U];
 #pragma unroll
 				for( int u = 0; u < U; u++ )
 				{
-					std::int32_t const src = tp_src( te[u] );
-					a8[u] = v.fl8[par + src];
 					e[u] = tp_place( te[u] );
-					xv[u] = v.xtr[tr + src];
+					std::uint32_t const x = v.xpost[par + tp_src( te[u] )];
+					ok[u] = ok[u] && x != X_ARRIVED;
+					xv[u] = __builtin_bit_cast( float, x );
 				}
 				typename S::tuple_t sy[U];
 				if constexpr( !has_inert_v<S> )
@@ -1011,7 +1013,6 @@ __device__ inline void window_passes( dview const & v, std::int64_t blk, std::in
 #pragma unroll
 				for( int u = 0; u < U; u++ )
 				{
-					ok[u] = ok[u] && a8[u] == 0;
 					if constexpr( has_inert_v<S> )
 						if( ok[u] && S::inert( false, true, xv[u], 0.0f, dt_b ) ) // the event cannot change the synapse
 						{
