@@ -1743,35 +1743,52 @@ __global__ __launch_bounds__( 256 ) void k_sync_eager( dview v, std::int64_t now
 }
 
 // ---- by-target index of the plastic synapses (built by the tile kernels of window.h) ----------
-// ptr[0..n] = exclusive prefix sums of cnt[0..n-1]; one workgroup of 1024 threads, each
-// summing a contiguous slice (n is a neuron count: this runs once per network).
+// ptr[0..n] = exclusive prefix sums of cnt[0..n-1], ptr[n + 1] = how many of them are not 0; one
+// workgroup, 4,096 counts at a time (once per network).
 static inline __global__ __launch_bounds__( 1024 ) void k_tp_scan( std::uint32_t const * cnt, std::int64_t * ptr, std::int64_t n )
 {
-	__shared__ std::int64_t part[1024];
-	int const t = threadIdx.x;
-	std::int64_t const per = ( n + 1023 ) / 1024;
-	std::int64_t const a = t * per < n ? t * per : n, b = a + per < n ? a + per : n;
-	std::int64_t sum = 0;
-	for( std::int64_t i = a; i < b; i++ ) sum += cnt[i];
-	part[t] = sum;
+	__shared__ std::uint64_t wsum[16];
+	__shared__ unsigned long long used;
+	int const t = threadIdx.x, lane = lane_id(), wave = t >> 6;
+	if( t == 0 ) used = 0;
+	std::uint64_t run = 0; // before the pass
+	std::uint32_t mine = 0;
+	for( std::int64_t i0 = 0; i0 < n; i0 += 4096 )
+	{
+		std::int64_t const i = i0 + 4 * t;
+		std::uint32_t c[4];
+		std::uint64_t sum = 0;
+#pragma unroll
+		for( int x = 0; x < 4; x++ )
+		{
+			c[x] = i + x < n ? cnt[i + x] : 0u;
+			sum += c[x];
+			mine += c[x] > 0 ? 1u : 0u;
+		}
+		std::uint64_t const incl = wave_inclusive_scan( sum );
+		__syncthreads(); // the sums of the pass before are read
+		if( lane == 63 ) wsum[wave] = incl;
+		__syncthreads();
+		std::uint64_t at = run + incl - sum;
+		for( int w = 0; w < 16; w++ )
+		{
+			at += w < wave ? wsum[w] : 0;
+			run += wsum[w];
+		}
+#pragma unroll
+		for( int x = 0; x < 4; x++ )
+		{
+			if( i + x < n ) ptr[i + x] = std::int64_t( at );
+			at += c[x];
+		}
+	}
+	std::uint64_t const all = wave_inclusive_scan( mine );
+	if( lane == 63 && all ) atomicAdd( &used, (unsigned long long)( all ) );
 	__syncthreads();
 	if( t == 0 )
 	{
-		std::int64_t run = 0;
-		for( int k = 0; k < 1024; k++ )
-		{
-			std::int64_t const x = part[k];
-			part[k] = run;
-			run += x;
-		}
-		ptr[n] = run;
-	}
-	__syncthreads();
-	std::int64_t run = part[t];
-	for( std::int64_t i = a; i < b; i++ )
-	{
-		ptr[i] = run;
-		run += cnt[i];
+		ptr[n] = std::int64_t( run );
+		ptr[n + 1] = std::int64_t( used );
 	}
 }
 

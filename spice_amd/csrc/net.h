@@ -793,7 +793,7 @@ private:
 				if( windowed ) _sp8.resize( 2 * n );
 				_po_id.resize( 2 * n );
 				_po_count.resize( CLOCK_SLOTS );
-				_tp_ptr.resize( n + 1 );
+				_tp_ptr.resize( n + 2 ); // (then the number of targets that have any)
 				reset_eager( true );
 			}
 			if( _lazy )
@@ -967,16 +967,15 @@ private:
 		SPICE_HIP( hipMemsetAsync( cnt.data(), 0, cnt.bytes(), _s ) ); // (tiles without inputs are not walked)
 		SPICE_LAUNCH( ( k_tp_tile<Model, true><<<unsigned( _v.nact ), TP_BLOCK, 0, _s>>>( _v, cnt.data(), nullptr ) ) );
 		SPICE_LAUNCH( k_tp_scan<<<1, 1024, 0, _s>>>( cnt.data(), _tp_ptr.data(), n ) );
-		std::vector<std::int64_t> ptr( n + 1 );
-		SPICE_HIP( hipMemcpyAsync( ptr.data(), _tp_ptr.data(), ptr.size() * 8, hipMemcpyDeviceToHost, _s ) );
+		std::int64_t ends[2];
+		SPICE_HIP( hipMemcpyAsync( ends, _tp_ptr.data() + n, 16, hipMemcpyDeviceToHost, _s ) );
 		SPICE_HIP( hipStreamSynchronize( _s ) );
-		_tp_total = ptr[n];
+		_tp_total = ends[0];
 		_tp_ent.resize( std::size_t( std::max<std::int64_t>( _tp_total, 1 ) ) );
 		_v.tp_ent = _tp_ent.data();
 		if( _tp_total > 0 ) SPICE_LAUNCH( ( k_tp_tile<Model, false><<<unsigned( _v.nact ), TP_BLOCK, 0, _s>>>( _v, nullptr, _tp_ent.data() ) ) );
 		// targets with incoming plastic synapses (the mean in-degree sets the post-pass split)
-		_tp_targets = 0;
-		for( std::int64_t i = 0; i < n; i++ ) _tp_targets += ptr[i + 1] > ptr[i];
+		_tp_targets = ends[1];
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 		apply_launch( _lc ); // the views, and the post pass's split
 	}
@@ -1060,8 +1059,9 @@ private:
 			v.tile_w = c.tile_w;
 			v.ntiles = ntiles;
 			v.segs = _segs.data();
-			if( _v.wcap > 1 && ntiles <= PASS_TILES && !_col16.size() && wants_halves( double( _g.nnz ) / double( n ) * double( c.tile_w ) / double( std::max<std::int64_t>( _g.targets, 1 ) ) ) &&
-			    allocate_halves() )
+			double const mean = double( _g.nnz ) / double( n ) * double( c.tile_w ) / double( std::max<std::int64_t>( _g.targets, 1 ) );
+			bool const records = input_classes_v<Model> > 0 && _v.wcap == 1 && record_size( mean ) <= 7;
+			if( !records && ntiles <= PASS_TILES && !_col16.size() && wants_halves( mean ) && allocate_halves() )
 			{
 				std::uint32_t const d = std::uint32_t( c.tile_w ) / 64, magic = d == 1 ? 0u : std::uint32_t( ( ( std::uint64_t( 1 ) << 32 ) + d - 1 ) / d );
 				SPICE_LAUNCH( k_segments_halves<<<unsigned( ( n + 3 ) / 4 ), 256, 16 * std::size_t( ntiles + 1 ), _s>>>( _v, _g.nnz, magic, _col16.data() ) );
@@ -1249,9 +1249,16 @@ private:
 		while( _v.wlanes < 5 && double( _v.vec16 << _v.wlanes ) < mean + ( mean < 20.0 ? 2.0 : 1.0 ) * std::sqrt( mean ) + ( _v.vec16 == 8 ? 4.0 : 0.0 ) ) _v.wlanes++;
 	}
 
-	// Segment records (window.h) of networks that run step by step, where segments are short: the
-	// smallest record that holds one 2.9 standard deviations longer than the mean. Not if the records
-	// took over twice the row store's memory, or more than a fifth of the free memory, or if over 1 %
+	// log2 of the smallest record that holds a segment 2.9 standard deviations longer than the mean
+	// (8: none does)
+	static int record_size( double mean )
+	{
+		int lg = 4;
+		while( lg < 8 && rec_capacity( lg ) < mean + 2.9 * std::sqrt( mean ) ) lg++;
+		return lg;
+	}
+	// Segment records (window.h) of networks that run step by step, where segments are short. Not if the
+	// records took over twice the row store's memory, or more than a fifth of the free memory, or if over 1 %
 	// of the segments did not fit (rows of very different lengths); not for the nets of a batch.
 	void build_records()
 	{
@@ -1260,9 +1267,7 @@ private:
 		_v.rec_lg = 0;
 		if constexpr( input_classes_v<Model> > 0 )
 		{
-			double const mean = double( _g.nnz ) / double( _g.n ) / _v.nact, need = mean + 2.9 * std::sqrt( mean );
-			int lg = 4;
-			while( lg < 8 && rec_capacity( lg ) < need ) lg++;
+			int const lg = record_size( double( _g.nnz ) / double( _g.n ) / _v.nact );
 			std::uint64_t const segs = seg_entries( _g.n, _v.ntiles ), bytes = segs << lg;
 			if( _v.wcap > 1 || _window == 0 || _p.batched || lg > 7 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
 			if( bytes > ( std::uint64_t( 1 ) << 30 ) )
