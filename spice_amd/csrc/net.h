@@ -992,7 +992,7 @@ private:
 		c.tile_w = _lazy ? lazy_tile_w( n, cus ) : default_tile_w<Model>( n, _g.targets, _p.delay, cus );
 		if( _p.batched && windowed && !plastic && _v.wcap == 1 ) c.tile_w = std::max( c.tile_w, BATCH_TILE );
 		if constexpr( input_classes_v<Model> > 0 )
-			if( _v.wcap == 1 && !_p.batched && _g.targets > 0 && double( _g.nnz ) / double( n ) * REC_TILE / double( _g.targets ) <= 40.0 )
+			if( _v.wcap == 1 && !_p.batched && _g.targets > 0 && double( _g.nnz ) / double( n ) * REC_TILE / double( _g.targets ) <= 18.0 )
 				// Step by step, with segment records that fit: rather fewer and wider tiles, as all of
 				// them reserve their spikes' places on one address, 9 ns apart (us per step of Vogels
 				// nets of 22,361, 70,711 and 100,000 neurons: 6.6, 7.0 and 7.9 with a tile per CU, 5.8,
@@ -1060,7 +1060,7 @@ private:
 			v.ntiles = ntiles;
 			v.segs = _segs.data();
 			double const mean = double( _g.nnz ) / double( n ) * double( c.tile_w ) / double( std::max<std::int64_t>( _g.targets, 1 ) );
-			bool const records = input_classes_v<Model> > 0 && _v.wcap == 1 && record_size( mean ) <= 7;
+			bool const records = input_classes_v<Model> > 0 && _v.wcap == 1 && record_size( mean ) <= 6;
 			if( !records && ntiles <= PASS_TILES && !_col16.size() && wants_halves( mean ) && allocate_halves() )
 			{
 				std::uint32_t const d = std::uint32_t( c.tile_w ) / 64, magic = d == 1 ? 0u : std::uint32_t( ( ( std::uint64_t( 1 ) << 32 ) + d - 1 ) / d );
@@ -1257,8 +1257,9 @@ private:
 		while( lg < 8 && rec_capacity( lg ) < mean + 2.9 * std::sqrt( mean ) ) lg++;
 		return lg;
 	}
-	// Segment records (window.h) of networks that run step by step, where segments are short. Not if the
-	// records took over twice the row store's memory, or more than a fifth of the free memory, or if over 1 %
+	// Segment records (window.h) of networks that run step by step, where segments are short: 64 bytes
+	// hold one (with 128, brunel_3pop of 90,000 neurons at p = 0.08 took 8.2 us per step instead of 9.2,
+	// but 7.6 ms to build instead of 3.9). Not if the records took over twice the row store's memory, or more than a fifth of the free memory, or if over 1 %
 	// of the segments did not fit (rows of very different lengths); not for the nets of a batch.
 	void build_records()
 	{
@@ -1269,7 +1270,7 @@ private:
 		{
 			int const lg = record_size( double( _g.nnz ) / double( _g.n ) / _v.nact );
 			std::uint64_t const segs = seg_entries( _g.n, _v.ntiles ), bytes = segs << lg;
-			if( _v.wcap > 1 || _window == 0 || _p.batched || lg > 7 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
+			if( _v.wcap > 1 || _window == 0 || _p.batched || lg > 6 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
 			if( bytes > ( std::uint64_t( 1 ) << 30 ) )
 			{
 				std::size_t room = 0, all = 0;

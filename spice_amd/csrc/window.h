@@ -178,7 +178,7 @@ static inline __global__ __launch_bounds__( 256 ) void k_segments_halves( dview 
 // ---- segment records -------------------------------------------------------------------------
 // For models with input classes a delivery needs of a row's segment in a tile only the targets, and
 // those fit 16 bits inside a tile. Where segments are short and the network runs step by step, each
-// (row, tile) gets a record of 2^lg bytes, 16 to 128: the segment's length, then its targets less
+// (row, tile) gets a record of 2^lg bytes, 16 to 64: the segment's length, then its targets less
 // the tile's start. A segment then costs one aligned read instead of its bounds and, after them, an
 // unaligned piece of the row store; the chain of dependent accesses that bounds such a step loses
 // two links, as the arrivals' ids are read beside their count. A segment that does not fit has

@@ -55,7 +55,7 @@ def test_windows_bit_exact(gpu, model, layout, delay, launch):
 @pytest.mark.parametrize("model", ["vogels_abbott", "synth"])
 @pytest.mark.parametrize("p", [0.004, 0.02, 0.05, 0.1, 0.3])
 def test_segment_records_bit_exact(gpu, model, p):
-    """Delay 1: records of 16, 32, 64 and 128 bytes (segments of 1 to 26 targets, some longer than
+    """Delay 1: records of 16, 32 and 64 bytes (segments of 1 to 13 targets, some longer than
     their record) and segments too long for any; the tiles change on the way (Vogels: all neurons
     fire at step 139)."""
     lay = ([2500], [(0, 0, p)])
