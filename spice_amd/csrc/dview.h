@@ -11,9 +11,9 @@
 //                        point) / int32
 //   sa[a]    attribute a of every synapse         CSR order (plastic models only)
 //   ring     int32[rsize * N], counts uint32[rsize * COUNT_STRIDE] spike ids of the last steps (entry t mod
-//                        rsize; rsize >= D + 2 wcap: the last step of a window of W <= wcap steps
-//                        clears the entries of the wcap steps after it, while step T - D's may
-//                        still be read; never-written entries are empty)
+//                        rsize; rsize > D + 2 wcap (rules.h): a window of W <= wcap steps from T
+//                        clears the entries of the wcap steps after it, while those of steps T - D
+//                        and T - wcap - 1 may still be read; never-written entries are empty)
 //   hring    uint64[HWORDS * N]  spike-history ring: bit (t mod H) of word (t mod H)/64 of
 //                        neuron i set iff i spiked at step t (H = 256 steps, plastic models)
 //   hasp     uint8[N]    row s has at least one plastic synapse

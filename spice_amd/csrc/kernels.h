@@ -193,7 +193,7 @@ __device__ inline snn_info info_of( dview const & v )
 }
 __device__ inline float step_dt( dview const & v ) { return v.DT - v.ctl->c; }
 
-// Spike ring entry of step t (t >= -D): at least D + 2 wcap entries, so that the update of step T
+// Spike ring entry of step t (t >= -D): more than D + 2 wcap entries (or 4), so that the update of step T
 // clears the entries of the wcap steps after it (last read by deliveries of earlier steps) while
 // step T's delivery may still read the entry of step T - D.
 __device__ inline int ring_slot( dview const & v, std::int64_t t ) { return int( ( t + v.rsize ) % v.rsize ); }

@@ -8,6 +8,7 @@
 #include "graph.h"
 #include "graphs.h"
 #include "kernels.h"
+#include "rules.h"
 #include "window.h"
 
 #include <spice/models/model.h>
@@ -144,13 +145,6 @@ template <typename Model>
 int window_cap( int delay )
 {
 	return windowed_v<Model> && delay >= 2 ? std::max( 1, window_steps( std::min( delay, longest_window_v<Model> ) ) ) : 1;
-}
-// Entries of the spike ring: the delay and two windows; four at least, so that with a delay of
-// one step the entry of a step is its clock slot, known without reading the clock.
-template <typename Model>
-int ring_entries( int delay )
-{
-	return std::max( 4, delay + 2 * window_cap<Model>( delay ) );
 }
 
 constexpr int REC_TILE = 768; // widest tile that segment records alone are a reason for (default_launch)
@@ -768,7 +762,7 @@ private:
 			if constexpr( !factored || !is_factored_attr<S>( int( I ) ) ) _sa[I].resize( ( _g.nnz + COL_PAD ) * sizeof( A ) ); // (read in pieces like the row store)
 		} );
 		_v.wcap = window_cap<Model>( _p.delay );
-		_v.rsize = ring_entries<Model>( _p.delay );
+		_v.rsize = ring_entries( _p.delay, _v.wcap );
 		_ring.resize( std::size_t( _v.rsize ) * n );
 		_counts.resize( std::size_t( _v.rsize ) * COUNT_STRIDE );
 		SPICE_HIP( hipMemsetAsync( _counts.data(), 0, _counts.bytes(), _s ) );

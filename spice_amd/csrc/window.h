@@ -23,21 +23,13 @@
 // 193 cycles per wave instruction on gfx950 (three per lane, whatever the addresses), ds_add_f64
 // 21 and ds_add_u32 7 at random addresses, and was what a Vogels-Abbott delivery waited for.
 #include "kernels.h"
+#include "rules.h"
 
 #include <algorithm>
 
 namespace spice::hipx
 {
-constexpr int WINDOW_MAX = 15;              // longest window (steps)
 constexpr std::size_t LDS_PER_CU = 160 << 10;
-
-// The longest window of at most n steps: never a multiple of CLOCK_SLOTS, so that the clock a
-// window writes is not the slot its workgroups read.
-inline int window_steps( std::int64_t n )
-{
-	int const w = int( std::min<std::int64_t>( n, WINDOW_MAX ) );
-	return w % CLOCK_SLOTS == 0 ? w - 1 : w;
-}
 
 // One staged row segment of a chunk of spikes.
 struct alignas( 16 ) win_seg
@@ -743,8 +735,8 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	}
 	if( tile == 0 )
 	{
-		// the counters of the steps after the window (no window before them reads those entries),
-		// and the clock of the step after it
+		// the counters of the steps after the window (no workgroup of this launch reads those
+		// entries: ring_entries), and the clock of the step after it
 		if( tid < v.wcap ) v.counts[entry( W + tid ) * COUNT_STRIDE] = 0;
 		if( tid == 0 )
 		{

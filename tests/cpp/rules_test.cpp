@@ -1,0 +1,54 @@
+// Host-only checks of spice_amd/csrc/rules.h. Exits non-zero on the first failure.
+#include "rules.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <set>
+
+using namespace spice::hipx;
+
+#define CHECK( c, ... )                                                           \
+	do                                                                            \
+	{                                                                             \
+		if( !( c ) )                                                              \
+		{                                                                         \
+			std::printf( "FAIL %s:%d: %s -- ", __FILE__, __LINE__, #c );          \
+			std::printf( __VA_ARGS__ );                                           \
+			std::printf( "\n" );                                                  \
+			std::exit( 1 );                                                       \
+		}                                                                         \
+	} while( 0 )
+
+// No counter that a window, or the spike log beside it, reads is one that the window clears or adds
+// to: all delays, longest windows, and lengths of the window and of the one before it.
+static void ring()
+{
+	for( int delay = 1; delay <= 300; delay++ )
+		for( int longest = 1; longest <= WINDOW_MAX; longest++ )
+		{
+			int const cap = delay >= 2 ? std::max( 1, window_steps( std::min( delay, longest ) ) ) : 1;
+			int const R = ring_entries( delay, cap );
+			auto entry = [&]( int k ) { // as in the kernels: one wrap either way
+				CHECK( -R <= k && k < R, "delay %d cap %d entry %d", delay, cap, k );
+				return ( k + R ) % R;
+			};
+			for( int W = 1; W <= cap; W++ )
+				for( int n = 0; n <= cap; n++ )
+				{
+					std::set<int> read, cleared, added;
+					for( int q = 0; q < W; q++ ) read.insert( entry( q - delay ) ); // arrivals
+					if( n > 0 )
+						for( int q = -n - 1; q < 0; q++ ) read.insert( entry( q ) ); // spike log
+					for( int q = 0; q < W; q++ ) added.insert( entry( q ) );
+					for( int q = 0; q < cap; q++ ) cleared.insert( entry( W + q ) );
+					for( int e : read ) CHECK( !cleared.count( e ) && !added.count( e ), "delay %d cap %d W %d n %d entry %d", delay, cap, W, n, e );
+					for( int e : added ) CHECK( !cleared.count( e ), "delay %d cap %d W %d entry %d", delay, cap, W, e );
+				}
+		}
+}
+
+int main()
+{
+	ring();
+	std::printf( "ALL OK\n" );
+}

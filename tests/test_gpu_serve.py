@@ -160,3 +160,23 @@ def test_invalid_jobs_are_rejected_at_submit(gpu):
             sv.submit("brunel_3pop_stdp", Layout(*three_pop_layout(500)), DT, 10, delay=256)  # plastic delay limit
         with pytest.raises(ValueError):
             sv.submit("brunel_3pop", Layout(*three_pop_layout(500)), DT, 10, flags=2)  # unknown flag bit
+
+
+@pytest.mark.parametrize("model,delay", [("brunel_3pop", 15), ("brunel_3pop_stdp", 10)])
+def test_more_workgroups_than_fit_at_once(gpu, model, delay):
+    """40 jobs of 10,000 neurons in one group: 1,600 tiles of 256 neurons, of which at most 1,536 fit
+    on the card at once (windows of as many steps as the delay, the longest), so the workgroups that
+    write the spike logs start when tiles have ended. Every stream is the job's alone."""
+    lay, steps = Layout(*three_pop_layout(10000)), 100
+    with Server(budget_bytes=60e9, chunk_steps=64, keep_spikes=True) as sv:
+        ids = [sv.submit(model, lay, DT, steps, delay=delay, seed=301 + k, fixed_point=True) for k in range(40)]
+        recs = [sv.wait(i, timeout=120) for i in ids]
+        streams = [sv.spikes(i) for i in ids]
+    total = 0
+    for k, (rec, stream) in enumerate(zip(recs, streams)):
+        ref, st = _alone(model, lay, steps, delay, 301 + k, None)
+        for t in range(steps):
+            np.testing.assert_array_equal(np.sort(stream[t]), ref[t], err_msg=f"job {k} step {t}")
+        assert rec["digest"] == spike_digest(enumerate(ref)) and rec["spikes"] == st["spikes"], k
+        total += st["spikes"]
+    assert total > 40 * steps
