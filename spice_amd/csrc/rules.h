@@ -2,6 +2,8 @@
 // Sizes of a network's buffers and windows that follow from its numbers alone (no HIP in here).
 #include "dview.h"
 
+#include <spice/util/host_defines.h>
+
 #include <algorithm>
 #include <cstdint>
 
@@ -24,4 +26,20 @@ inline int window_steps( std::int64_t n )
 // least, so that with a delay of one step the entry of a step is its clock slot, known without
 // reading the clock.
 inline int ring_entries( int delay, int wcap ) { return std::max( 4, delay + 2 * wcap + 1 ); }
+
+// One staged row segment of a chunk of spikes (window.h). Rows may name a target many times, so a
+// segment may be longer than its tile is wide.
+struct alignas( 16 ) win_seg
+{
+	std::int64_t place; // first target id in the row store (0 for an empty segment), step of the window << 48
+	std::int32_t src;
+	std::int32_t len;
+
+	HYBRID static win_seg of( std::int64_t at, std::int32_t len, std::int32_t src, std::int32_t step = 0 )
+	{
+		return { ( len > 0 ? at : 0 ) | std::int64_t( step ) << 48, src, len };
+	}
+	HYBRID std::int64_t at() const { return place & ( ( std::int64_t( 1 ) << 48 ) - 1 ); }
+	HYBRID std::int32_t step() const { return std::int32_t( place >> 48 ); }
+};
 } // namespace spice::hipx

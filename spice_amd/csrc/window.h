@@ -31,14 +31,6 @@ namespace spice::hipx
 {
 constexpr std::size_t LDS_PER_CU = 160 << 10;
 
-// One staged row segment of a chunk of spikes.
-struct alignas( 16 ) win_seg
-{
-	std::int64_t off;  // first target id in the row store (0 for an empty segment)
-	std::int32_t src;
-	std::int32_t meta; // length | step of the window << 16
-};
-
 constexpr int WIN_VEC = 4;   // consecutive targets a lane reads at once (the row store is padded by as many)
 constexpr int WIN_TABLE = 64; // partial sums kept per input class
 
@@ -511,12 +503,14 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 			std::int64_t const a = sg.at;
 			std::int32_t const len = lane < cnt ? sg.len : 0;
 			if constexpr( L::classes > 0 )
-				// in the place of the source: where the class's counters of the step start (for target 0)
-				// (IDS16X8 also: the piece that the segment begins in, its end from there on, its place there)
-				mine[lane] = win_seg{ len > 0 ? a & ~std::int64_t( FORM == IDS16X8 ? 7 : 0 ) : 0, ( q * nacc + N::input_class( src, info ) ) * tws - ( FORM == IDS32 ? t0 : 0 ),
-				                      FORM == IDS16X8 && len > 0 ? ( len + ( int( a ) & 7 ) ) | ( int( a ) & 7 ) << 16 : len };
+			{
+				// in the place of the source: where the class's counters of the step start (for target 0).
+				// IDS16X8: from the piece that the segment begins in, its place there in the place of the step
+				std::int32_t const skip = FORM == IDS16X8 && len > 0 ? std::int32_t( a ) & 7 : 0;
+				mine[lane] = win_seg::of( a - skip, len + skip, ( q * nacc + N::input_class( src, info ) ) * tws - ( FORM == IDS32 ? t0 : 0 ), skip );
+			}
 			else
-				mine[lane] = win_seg{ len > 0 ? a : 0, src, len | ( q << 16 ) };
+				mine[lane] = win_seg::of( a, len, src, q );
 			ev += std::uint32_t( len );
 			wave_lds_fence();
 			if( k0 + NW * per < total )
@@ -531,13 +525,16 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 			for( std::int32_t c = 0; c < cnt; c += U * ng )
 			{
 				win_seg r[U];
-				std::int32_t len[U], most = 0;
+				constexpr bool steps = L::classes == 0 || FORM == IDS16X8; // the records hold steps (or skips)
+				std::int32_t len[U], step[U], most = 0;
 #pragma unroll
 				for( int u = 0; u < U; u++ )
 				{
 					std::int32_t const k = c + u * ng + g;
 					r[u] = mine[k & 63]; // (records from cnt on are empty)
-					len[u] = k < 64 ? ( r[u].meta & 0xffff ) : 0;
+					len[u] = k < 64 ? r[u].len : 0;
+					step[u] = steps ? r[u].step() : 0;
+					if constexpr( steps ) r[u].place = r[u].at();
 					most = len[u] > most ? len[u] : most;
 				}
 				for( std::int32_t e = l * V;; e += G * V )
@@ -547,12 +544,12 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 					{
 						halves<V> j[U];
 #pragma unroll
-						for( int u = 0; u < U; u++ ) j[u] = load_halves<V>( v.col16 + r[u].off + ( e < len[u] ? e : 0 ) );
+						for( int u = 0; u < U; u++ ) j[u] = load_halves<V>( v.col16 + r[u].place + ( e < len[u] ? e : 0 ) );
 #pragma unroll
 						for( int u = 0; u < U; u++ )
 #pragma unroll
 							for( int x = 0; x < V; x++ )
-								if( e + x < len[u] && ( V == WIN_VEC || e + x >= r[u].meta >> 16 ) ) atomicAdd( acc + ( r[u].src + ( ( j[u].id[x] - t0 ) & 0xffff ) ), 1u );
+								if( e + x < len[u] && ( V == WIN_VEC || e + x >= step[u] ) ) atomicAdd( acc + ( r[u].src + ( ( j[u].id[x] - t0 ) & 0xffff ) ), 1u );
 						if( e - l * V + G * V >= most ) break;
 						continue;
 					}
@@ -561,17 +558,17 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 					for( int u = 0; u < U; u++ )
 						if constexpr( FORM == IDS16 )
 						{
-							halves<V> const low = load_halves<V>( v.col16 + r[u].off + ( e < len[u] ? e : 0 ) );
+							halves<V> const low = load_halves<V>( v.col16 + r[u].place + ( e < len[u] ? e : 0 ) );
 #pragma unroll
 							for( int x = 0; x < V; x++ ) j[u].id[x] = t0 + ( ( low.id[x] - t0 ) & 0xffff );
 						}
 						else
-							j[u] = load_targets( v.col + r[u].off + ( e < len[u] ? e : 0 ) );
+							j[u] = load_targets( v.col + r[u].place + ( e < len[u] ? e : 0 ) );
 					synapses<S> sy[U];
 					if constexpr( plastic )
 					{
 #pragma unroll
-						for( int u = 0; u < U; u++ ) sy[u].load( v.sa, r[u].off + ( e < len[u] ? e : 0 ) );
+						for( int u = 0; u < U; u++ ) sy[u].load( v.sa, r[u].place + ( e < len[u] ? e : 0 ) );
 					}
 #pragma unroll
 					for( int u = 0; u < U; u++ )
@@ -583,11 +580,11 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 								atomicAdd( acc + ( r[u].src + j[u].id[x] ), 1u );
 							else
 							{
-								int const s = r[u].meta >> 16;
+								int const s = step[u];
 								tile_backend<FIXED> bak{ make_backend<FIXED>( v, std::uint32_t( r[u].src ), std::uint32_t( j[u].id[x] ), std::uint32_t( T0 + s ), util::TAG_RECEIVE ) };
 								win_iter<N, FIXED> dst{ &v, j[u].id[x], t0, tws, acc + s * ( nacc * tws ) };
 								if constexpr( plastic )
-									deliver_event<N>( r[u].src, dst, reg_iter<typename S::tuple_t>{ sy[u].s[x], std::uint32_t( r[u].off + e + x ) }, info, bak );
+									deliver_event<N>( r[u].src, dst, reg_iter<typename S::tuple_t>{ sy[u].s[x], std::uint32_t( r[u].place + e + x ) }, info, bak );
 								else
 									deliver_event<N>( r[u].src, dst, no_syn_iter{}, info, bak );
 							}

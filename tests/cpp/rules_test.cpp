@@ -47,8 +47,22 @@ static void ring()
 		}
 }
 
+// A staged segment gives back what it was made of, at any length that a row may have.
+static void staged_segments()
+{
+	for( std::int64_t at : { std::int64_t( 0 ), std::int64_t( 7 ), std::int64_t( 65536 ), ( std::int64_t( 1 ) << 40 ) - 1 } )
+		for( std::int32_t len : { 0, 1, 65528, 65535, 65536, 65537, 131072, 1 << 24, INT32_MAX - 7 } )
+			for( int step = 0; step < WINDOW_MAX; step++ )
+			{
+				win_seg const s = win_seg::of( at, len, 12345, step );
+				CHECK( s.at() == ( len > 0 ? at : 0 ) && s.len == len && s.src == 12345 && s.step() == step, "at %lld len %d step %d", (long long)( at ), len, step );
+			}
+	static_assert( sizeof( win_seg ) == 16, "" );
+}
+
 int main()
 {
 	ring();
+	staged_segments();
 	std::printf( "ALL OK\n" );
 }

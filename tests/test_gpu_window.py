@@ -180,3 +180,45 @@ def test_halved_row_store_bit_exact(gpu, model, layout, delay, launch):
         assert_state_equal(d.neurons(), h.neurons(), model)
     assert d.stats()["events"] > 0
     d.close(), h.close()
+
+
+def _repeated_rows(n, base, seed, first):
+    """Rows of `base` random targets from neuron `first` on; ten Poisson sources (of brunel_3pop) and two excitatory neurons
+    also name two targets of one tile 66,000 to 140,000 times in all."""
+    rng = np.random.default_rng(seed)
+    rows = [np.sort(first + rng.choice(n - first, base, replace=False)) for _ in range(n)]
+    sources = list(range(0, n // 5, max(1, n // 50)))[:10] + [n // 3, n // 2]
+    for k, s in enumerate(sources):
+        x = int(rng.integers(-(-first // 64), n // 64)) * 64
+        more = np.repeat([x + 3, x + 40], [65536 + 7 * k, 400 + 6500 * k])
+        rows[s] = np.sort(np.concatenate([rows[s], more]))
+    rp = np.zeros(n + 1, np.int64)
+    np.cumsum([r.size for r in rows], out=rp[1:])
+    return rp, np.concatenate(rows).astype(np.int32), (max(r.size for r in rows) + 31) // 32 * 32
+
+
+@pytest.mark.parametrize("model,n,base,delay", [
+    ("brunel_3pop", 512, 40, 15),   # low halves, 8 per lane
+    ("brunel_3pop", 1984, 40, 15),  # low halves, 4 per lane
+    ("brunel_3pop", 9984, 5, 6),    # the row store itself
+    ("brunel_3pop", 1984, 20, 1),   # records, and segments too long for any
+    ("brunel_3pop_stdp", 512, 40, 15),
+    ("brunel_3pop_stdp", 9984, 5, 1),
+    ("brunel_with_plasticity", 1984, 20, 9),
+])
+def test_targets_named_many_times(gpu, model, n, base, delay):
+    """More than 65,536 entries of a row in one tile, in windows of every length."""
+    # (brunel_with_plasticity: targets in its LIF half, as windows need)
+    rp, col, width = _repeated_rows(n, base, 91, n // 2 if model == "brunel_with_plasticity" else 0)
+    h = O.CpuSnn.from_csr(model, rp, col, width, DT, delay, seed=91, fixed_point=True)
+    d = Snn.from_csr(model, rp, col, width, DT, delay, seed=91, fixed_point=True)
+    for k in (130, 1, 7, 62):
+        d.run(k)
+        h.run(k)
+        assert_state_equal(d.neurons(), h.neurons(), model)
+    np.testing.assert_array_equal(np.sort(d.step(True)), np.sort(h.step(True)))
+    events = d.stats()["events"]
+    assert events > 65536, events
+    if model == "brunel_3pop_stdp":
+        np.testing.assert_array_equal(d.synapses(ell=False)["W"].view(np.uint32), h.synapses(ell=False)["W"].view(np.uint32))
+    d.close(), h.close()
