@@ -26,6 +26,7 @@
 // the per-step sequence of cuda::snn::step (spice/cuda/snn.d.cpp:233-289).
 #include "common.h"
 #include "dview.h"
+#include "rules.h"
 
 #include <spice/models/model.h>
 #include <spice/util/meta.h>
@@ -518,13 +519,11 @@ constexpr std::int64_t UPDATE_LARGE_N = 131072; // from this many neurons
 #ifndef SPICE_BATCH_RECV_BLOCK
 #define SPICE_BATCH_RECV_BLOCK 256
 #endif
-constexpr int TILE_MAX = 1024; // targets per tile (LDS accumulators)
-// Wide tiles (static models, two-kernel step only: a second instantiation of the delivery kernel,
+// Wide tiles (TILE_WIDE: static models, two-kernel step only: a second instantiation of the delivery kernel,
 // so the other kernels keep the smaller LDS footprint; up to 157 KB of LDS for two 8-byte
 // accumulators and 1,024-thread workgroups). A sparse network's rows have few targets in each
 // 1,024-neuron tile (the reference's synth network: ~1.6), and every delivery workgroup stages
 // all of the step's spikes: wider tiles stage each spike in fewer workgroups.
-constexpr int TILE_WIDE = 8192;
 // Delivery workgroups have 256 or 1024 threads (a launch shape): they stage that many spikes
 // per pass in LDS.
 
@@ -533,13 +532,10 @@ constexpr int TILE_WIDE = 8192;
 // deliveries read of them thus stays within one part of the memory, whose page translations a CU
 // can hold, and neighbouring tiles share lines (us per step, with two places per row and tile, row
 // by row, before: Brunel 1e10 12.5, 11.9; brunel_with_plasticity 6e8 11.6, 11.5).
-constexpr int SEG_TILES = 3;
 __device__ inline std::int64_t seg_at( dview const & v, std::int64_t r, std::int32_t t )
 {
 	return ( ( std::int64_t( t >> SEG_TILES ) * v.N + r ) << SEG_TILES ) + ( t & ( ( 1 << SEG_TILES ) - 1 ) );
 }
-// Entries of the table for n rows and ntiles tiles.
-inline std::uint64_t seg_entries( std::int64_t n, std::int64_t ntiles ) { return std::uint64_t( n ) * std::uint64_t( ( ( ntiles - 1 ) >> SEG_TILES ) + 1 ) << SEG_TILES; }
 // The segment of row r in tile t: its place in col and its length (an entry has 40 and 24 bits of them).
 struct segment
 {

@@ -150,25 +150,11 @@ int window_cap( int delay )
 constexpr int REC_TILE = 768; // widest tile that segment records alone are a reason for (default_launch)
 constexpr int BATCH_TILE = 192; // narrowest tile of a batch's nets that run step by step (hip_batch::batch_tile_w)
 
-// Targets per delivery tile of a new network. Window kernels: one tile per CU, as
-// every tile stages all of the window's arrivals and a wider one does it less often (synth 1e9:
-// 29 us per step with 251 tiles of 3,200, 50 with 391 of 2,048), but none wider than its kernel
-// takes; windows of several steps, whose accumulators take LDS per step, two per CU beyond that.
-// targets: the neurons that have inputs (csr_dev::targets). The other tiles cost little, except in
-// windows of static models, whose workgroups of 1,024 threads (default_launch) have a CU each
-// (Brunel, 100,000 and 40,000 neurons of which half have inputs, us per step: 3.4 and 1.9 with a
-// tile per CU of all, 4.7 and 2.2 with one per CU of those). Two-kernel plastic steps: about two
-// tiles per CU, of 256 at least.
-inline int lazy_tile_w( std::int64_t n, int cus ) { return int( std::clamp<std::int64_t>( ( ( n + 2 * cus - 1 ) / ( 2 * cus ) + 63 ) / 64 * 64, 256, TILE_MAX ) ); }
+// Targets per delivery tile of a new network (rules.h).
 template <typename Model>
 int default_tile_w( std::int64_t n, std::int64_t targets, int delay, int cus )
 {
-	if( !windowed_v<Model> ) return lazy_tile_w( n, cus );
-	bool const ahead = overlap_capable_v<Model> && delay >= 2;
-	std::int64_t const tiled = ahead && !is_plastic_v<Model> ? n : targets;
-	auto const per = [&]( std::int64_t tiles ) { return ( ( tiled + tiles - 1 ) / tiles + 63 ) / 64 * 64; };
-	std::int64_t const most = ahead || is_plastic_v<Model> ? TILE_MAX : 4 * 1024;
-	return int( std::clamp<std::int64_t>( per( ahead && per( cus ) > most ? 2 * cus : cus ), 64, most ) );
+	return windowed_v<Model> ? window_tile_w( n, targets, is_plastic_v<Model>, overlap_capable_v<Model> && delay >= 2, cus ) : lazy_tile_w( n, cus );
 }
 
 template <typename Model>

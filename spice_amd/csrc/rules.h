@@ -27,6 +27,40 @@ inline int window_steps( std::int64_t n )
 // reading the clock.
 inline int ring_entries( int delay, int wcap ) { return std::max( 4, delay + 2 * wcap + 1 ); }
 
+constexpr int TILE_MAX = 1024;  // targets per tile (LDS accumulators)
+constexpr int TILE_WIDE = 8192; // and of the wide tiles that static models may have step by step
+constexpr int SEG_TILES = 3;    // log2 of the tiles of a row that lie side by side in the segment table (kernels.h, seg_at)
+
+// Entries of the segment table for n rows and ntiles tiles.
+inline std::uint64_t seg_entries( std::int64_t n, std::int64_t ntiles ) { return std::uint64_t( n ) * std::uint64_t( ( ( ntiles - 1 ) >> SEG_TILES ) + 1 ) << SEG_TILES; }
+
+// Width of `tiles` tiles over n neurons, in 64s.
+inline std::int64_t tile_width( std::int64_t n, std::int64_t tiles ) { return ( ( n + tiles - 1 ) / tiles + 63 ) / 64 * 64; }
+
+// Targets per delivery tile of a new network of n neurons, `targets` of which have inputs
+// (csr_dev::targets). Two-kernel plastic steps: about two tiles per CU, of 256 at least.
+inline int lazy_tile_w( std::int64_t n, int cus ) { return int( std::clamp<std::int64_t>( tile_width( n, 2 * cus ), 256, TILE_MAX ) ); }
+// Windows (ahead: of several steps): one tile per CU, as
+// every tile stages all of the window's arrivals and a wider one does it less often (synth 1e9:
+// 29 us per step with 251 tiles of 3,200, 50 with 391 of 2,048), but none wider than its kernel
+// takes; windows of several steps, whose accumulators take LDS per step, two per CU beyond that.
+// The tiles without inputs cost little, except in
+// windows of static models, whose workgroups of 1,024 threads (default_launch) have a CU each
+// (Brunel, 100,000 and 40,000 neurons of which half have inputs, us per step: 3.4 and 1.9 with a
+// tile per CU of all, 4.7 and 2.2 with one per CU of those). Where few neurons have inputs, the tiles
+// are still those of all neurons, and the segment table has an entry for each of them and row:
+// four per CU at most, or two where fewer than half have inputs and the table would take over 512 MB.
+constexpr std::uint64_t TABLE_SMALL = std::uint64_t( 512 ) << 20;
+inline int window_tile_w( std::int64_t n, std::int64_t targets, bool plastic, bool ahead, int cus )
+{
+	std::int64_t const tiled = targets <= 0 || ( ahead && !plastic ) ? n : targets;
+	std::int64_t const most = ahead || plastic ? TILE_MAX : 4 * 1024;
+	std::int64_t w = tile_width( tiled, ahead && tile_width( tiled, cus ) > most ? 2 * cus : cus );
+	w = std::max( w, tile_width( n, 4 * cus ) );
+	if( 2 * targets < n && 8 * seg_entries( n, ( n + w - 1 ) / w ) > TABLE_SMALL ) w = std::max( w, tile_width( n, 2 * cus ) );
+	return int( std::clamp<std::int64_t>( w, 64, most ) );
+}
+
 // One staged row segment of a chunk of spikes (window.h). Rows may name a target many times, so a
 // segment may be longer than its tile is wide.
 struct alignas( 16 ) win_seg

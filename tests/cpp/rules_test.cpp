@@ -60,8 +60,35 @@ static void staged_segments()
 	static_assert( sizeof( win_seg ) == 16, "" );
 }
 
+// Tiles: however few neurons have inputs, at most four per CU (or as wide as its kernel takes), and a
+// segment table of at most 512 MB, or that of tiles for two per CU; where half of the neurons have
+// inputs or more, one per CU of those (windows of several steps: of all, or two).
+static void tiles()
+{
+	int const cus = 256;
+	for( double x = 1; x < 3e7; x = x * 1.07 + 1 )
+		for( double share : { 0.0, 1e-5, 1e-3, 0.01, 0.1, 0.3, 0.4999, 0.5, 0.8, 1.0 } )
+			for( int kind = 0; kind < 4; kind++ )
+			{
+				bool const plastic = kind & 1, ahead = kind & 2;
+				std::int64_t const n = std::int64_t( x ), targets = share == 0.5 ? n - n / 2 : std::int64_t( share * double( n ) );
+				int const w = window_tile_w( n, targets, plastic, ahead, cus ), most = plastic || ahead ? TILE_MAX : 4 * 1024;
+				std::int64_t const tiles = ( n + w - 1 ) / w;
+				CHECK( w >= 64 && w <= most && w % 64 == 0, "n %lld w %d", (long long)n, w );
+				CHECK( tiles <= 4 * cus || w == most, "n %lld targets %lld kind %d w %d", (long long)n, (long long)targets, kind, w );
+				std::int64_t const two = std::min<std::int64_t>( tile_width( n, 2 * cus ), most );
+				if( share < 0.5 ) CHECK( 8 * seg_entries( n, tiles ) <= std::max( TABLE_SMALL, 8 * seg_entries( n, ( n + two - 1 ) / two ) ), "n %lld targets %lld kind %d w %d", (long long)n, (long long)targets, kind, w );
+				else
+				{
+					std::int64_t const of = ahead && !plastic ? n : targets, one = tile_width( of, cus );
+					CHECK( w == std::clamp<std::int64_t>( ahead && one > most ? tile_width( of, 2 * cus ) : one, 64, most ), "n %lld targets %lld kind %d w %d", (long long)n, (long long)targets, kind, w );
+				}
+			}
+}
+
 int main()
 {
+	tiles();
 	ring();
 	staged_segments();
 	std::printf( "ALL OK\n" );

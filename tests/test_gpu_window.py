@@ -222,3 +222,26 @@ def test_targets_named_many_times(gpu, model, n, base, delay):
     if model == "brunel_3pop_stdp":
         np.testing.assert_array_equal(d.synapses(ell=False)["W"].view(np.uint32), h.synapses(ell=False)["W"].view(np.uint32))
     d.close(), h.close()
+
+
+@pytest.mark.parametrize("model,pops,p,delay", [
+    ("synth", [299000, 1000], 0.05, 1),
+    ("brunel_3pop_stdp", [150000, 50000, 1500, 500], 0.02, 15),
+    ("synth", [200000], 0.0, 1),  # no synapse at all
+])
+def test_few_targets(gpu, model, pops, p, delay):
+    """Many sources, few targets: the memory of the network is in proportion (the segment table has
+    an entry for every row and tile, tiles without inputs included)."""
+    import torch
+    layout = (pops, [(s, len(pops) - 1, p) for s in range(len(pops))])
+    free = torch.cuda.mem_get_info()[0]
+    d = Snn(model, Layout(*layout), DT, delay, seed=93, fixed_point=True)
+    taken = free - torch.cuda.mem_get_info()[0]
+    assert taken < 3 << 30, taken
+    h = O.CpuSnn(model, layout, DT, delay, seed=93, fixed_point=True)
+    for k in (25, 3):
+        d.run(k)
+        h.run(k)
+        assert_state_equal(d.neurons(), h.neurons(), model)
+    np.testing.assert_array_equal(np.sort(d.step(True)), np.sort(h.step(True)))
+    d.close(), h.close()
