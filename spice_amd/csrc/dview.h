@@ -19,7 +19,8 @@
 //   hasp     uint8[N]    row s has at least one plastic synapse
 //   pl_lo/hi int32[N]    first / one-past-last plastic slot of row s (offsets in the row)
 //   segs     uint64[N * ntiles]  per row and target tile: place in col and number of the row's targets
-//                        in the tile, 8 tiles of a row side by side (kernels.h, seg_at)
+//                        in the tile, 8 tiles of a row side by side (kernels.h, seg_at); or
+//   offs     uint32[N * (ntiles + 1)]  offsets of the tiles' first targets in the row
 //   tile_ids int32[ntiles] the tiles: first the nact ones that some row has targets in (at least
 //                        one), then the rest
 // lazy plasticity (per-synapse contract):
@@ -163,6 +164,7 @@ struct dview
 	unsigned long long * bstats; // [nblocks_max * NSTAT]
 
 	std::uint64_t * segs; // the segment table: where row r's targets in tile t are (kernels.h, segment_of)
+	std::uint32_t * offs; // in its place if it is nullptr: offsets in the row
 	std::int32_t ntiles, tile_w;
 	std::int32_t * tile_ids; // [ntiles]: the tiles with incoming synapses (the delivery's), then the others
 	std::int32_t nact;

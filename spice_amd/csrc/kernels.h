@@ -536,17 +536,35 @@ __device__ inline std::int64_t seg_at( dview const & v, std::int64_t r, std::int
 {
 	return ( ( std::int64_t( t >> SEG_TILES ) * v.N + r ) << SEG_TILES ) + ( t & ( ( 1 << SEG_TILES ) - 1 ) );
 }
-// The segment of row r in tile t: its place in col and its length (an entry has 40 and 24 bits of them).
+// The segment of row r in tile t: its place in col and its length (an entry has 40 and 24 bits of
+// them). Where rows may be longer than that, or the table would take too much of the memory
+// (rules.h), it has the offsets of the tiles' first targets in the row instead, ntiles + 1 of 4 bytes
+// per row. Read and unpacked apart, so that nothing waits for what is read ahead.
 struct segment
 {
 	std::int64_t at;
 	std::int32_t len;
 };
-__device__ inline segment segment_of( dview const & v, std::int64_t r, std::int32_t t )
+struct packed_segment
 {
-	std::uint64_t const e = v.segs[seg_at( v, r, t )];
-	return { std::int64_t( e & ( ( std::uint64_t( 1 ) << 40 ) - 1 ) ), std::int32_t( e >> 40 ) };
+	std::uint64_t entry; // or two offsets
+	std::int64_t row;    // (offsets: where the row starts)
+};
+__device__ inline packed_segment load_segment( dview const & v, std::int64_t r, std::int32_t t )
+{
+	if( v.segs ) return { v.segs[seg_at( v, r, t )], 0 };
+	packed_segment p;
+	__builtin_memcpy( &p.entry, v.offs + ( r * ( v.ntiles + 1 ) + t ), 8 ); // (4-byte alignment suffices)
+	p.row = v.row_ptr[r];
+	return p;
 }
+__device__ inline segment unpack_segment( dview const & v, packed_segment const & p )
+{
+	if( v.segs ) return { std::int64_t( p.entry & ( ( std::uint64_t( 1 ) << 40 ) - 1 ) ), std::int32_t( p.entry >> 40 ) };
+	std::uint32_t const a = std::uint32_t( p.entry ), b = std::uint32_t( p.entry >> 32 );
+	return { p.row + std::int64_t( a ), std::int32_t( b - a ) };
+}
+__device__ inline segment segment_of( dview const & v, std::int64_t r, std::int32_t t ) { return unpack_segment( v, load_segment( v, r, t ) ); }
 
 // The segment table. One wave per row, binary searches for 63 tiles at a time (the last lane's is
 // where the 63rd one ends).
@@ -572,8 +590,13 @@ static inline __global__ __launch_bounds__( 256 ) void k_segments( dview v )
 				b = m;
 		}
 		std::int32_t const next = std::int32_t( shfl_u32( std::uint32_t( a ), lane + 1 ) );
-		if( lane < 63 && t < v.ntiles ) v.segs[seg_at( v, r, t )] = std::uint64_t( lo + a ) | std::uint64_t( next - a ) << 40;
+		if( lane == 63 || t >= v.ntiles ) continue;
+		if( v.segs )
+			v.segs[seg_at( v, r, t )] = std::uint64_t( lo + a ) | std::uint64_t( next - a ) << 40;
+		else
+			v.offs[r * ( v.ntiles + 1 ) + t] = std::uint32_t( a );
 	}
+	if( !v.segs && lane == 0 ) v.offs[r * ( v.ntiles + 1 ) + v.ntiles] = std::uint32_t( len );
 }
 
 // Entry of the by-target index, its source and its synapse's place.

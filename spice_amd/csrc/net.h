@@ -523,7 +523,7 @@ public:
 		     _fl_id.bytes() + _fl_synced.bytes() + _fl_pend.bytes() + _hasp.bytes() + _pl_lo.bytes() + _pl_hi.bytes() +
 		     _fl_count.bytes() + _xtr.bytes() + _ytr.bytes() + _fl8.bytes() + _xpost.bytes() + _sp8.bytes() + _po_id.bytes() + _po_count.bytes() +
 		     _tp_ptr.bytes() + _caught.bytes() + _tp_ent.bytes() + _ctl.bytes() + _bstats.bytes() +
-		     _segs.bytes() + _recs.bytes() + _col16.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
+		     _segs.bytes() + _offs.bytes() + _recs.bytes() + _col16.bytes() + _slog_ctl.bytes() + _slog_ids.bytes() + _slog_off.bytes();
 		return b;
 	}
 
@@ -695,7 +695,8 @@ private:
 	launch_cfg _lc{};
 	std::shared_ptr<host_stage> _stage; // see stage_to_host
 	int _staged = 0;                    // calls that asked for it
-	dbuf<std::uint64_t> _segs;
+	dbuf<std::uint64_t> _segs;  // the segment table,
+	dbuf<std::uint32_t> _offs;  // or offsets in its place
 	dbuf<unsigned char> _recs; // segment records
 	dbuf<std::uint16_t> _col16;       // low halves of the row store
 	dbuf<std::int32_t> _tile_ids;
@@ -1035,13 +1036,12 @@ private:
 		if( retile )
 		{
 			std::int32_t const ntiles = std::int32_t( ( n + c.tile_w - 1 ) / c.tile_w );
-			_segs.resize( seg_entries( n, ntiles ) );
 			v.tile_w = c.tile_w;
 			v.ntiles = ntiles;
-			v.segs = _segs.data();
+			allocate_table();
 			double const mean = double( _g.nnz ) / double( n ) * double( c.tile_w ) / double( std::max<std::int64_t>( _g.targets, 1 ) );
 			bool const records = input_classes_v<Model> > 0 && _v.wcap == 1 && record_size( mean ) <= 6;
-			if( !records && ntiles <= PASS_TILES && !_col16.size() && wants_halves( mean ) && allocate_halves() )
+			if( !records && v.segs && ntiles <= PASS_TILES && !_col16.size() && wants_halves( mean ) && allocate_halves() )
 			{
 				std::uint32_t const d = std::uint32_t( c.tile_w ) / 64, magic = d == 1 ? 0u : std::uint32_t( ( ( std::uint64_t( 1 ) << 32 ) + d - 1 ) / d );
 				SPICE_LAUNCH( k_segments_halves<<<unsigned( ( n + 3 ) / 4 ), 256, 16 * std::size_t( ntiles + 1 ), _s>>>( _v, _g.nnz, magic, _col16.data() ) );
@@ -1094,6 +1094,37 @@ private:
 		}
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 		_graphs.clear(); // the captured launches hold the old shapes
+	}
+
+	// Whether `bytes` of optional memory fit beside what this net still needs (rules.h).
+	bool fits( std::uint64_t bytes ) const
+	{
+		if( bytes <= OPTIONAL_SMALL ) return true;
+		std::size_t room = 0, all = 0;
+		SPICE_HIP( hipMemGetInfo( &room, &all ) );
+		return optional_fits( bytes, room, eager && !_lazy && !_tp_ent.size() ? 8 * std::uint64_t( _g.nnz ) : 0 );
+	}
+
+	// The segment table of the view's tiles, or offsets in its place (kernels.h, segment_of).
+	void allocate_table()
+	{
+		_segs.release();
+		_offs.release();
+		_v.segs = nullptr;
+		_v.offs = nullptr;
+		std::uint64_t const entries = seg_entries( _g.n, _v.ntiles );
+		if( _g.width < ( std::int64_t( 1 ) << 24 ) && ( _p.batched ? 8 * entries <= TABLE_BATCHED : fits( 8 * entries ) ) )
+			try
+			{
+				_segs.resize( entries );
+				_v.segs = _segs.data();
+				return;
+			}
+			catch( std::bad_alloc const & )
+			{
+			}
+		_offs.resize( std::size_t( _g.n ) * std::size_t( _v.ntiles + 1 ) );
+		_v.offs = _offs.data();
 	}
 
 	// The delivery's tiles: those that some row has a target in (a population that no
@@ -1192,12 +1223,7 @@ private:
 	bool allocate_halves()
 	{
 		std::size_t const n = std::size_t( _g.nnz ) + 8;
-		if( n > ( std::size_t( 1 ) << 29 ) )
-		{
-			std::size_t room = 0, all = 0;
-			SPICE_HIP( hipMemGetInfo( &room, &all ) );
-			if( 2 * n > room / 5 ) return false;
-		}
+		if( !fits( 2 * n ) ) return false;
 		try
 		{
 			_col16.resize( n );
@@ -1223,7 +1249,7 @@ private:
 			SPICE_LAUNCH( k_halves<<<unsigned( std::min<std::size_t>( ( std::size_t( _g.nnz ) / 8 + 256 ) / 256, 256 * 32 ) ), 256, 0, _s>>>( _g.col.data(), _g.nnz, _col16.data() ) );
 		}
 		_v.col16 = _col16.data();
-		_v.vec16 = !plastic && mean >= 56.0 ? 8 : 4;
+		_v.vec16 = !plastic && mean >= 56.0 && _v.segs ? 8 : 4; // (8: lengths of 24 bits)
 		// (lanes per segment: see choose_window)
 		_v.wlanes = 0;
 		while( _v.wlanes < 5 && double( _v.vec16 << _v.wlanes ) < mean + ( mean < 20.0 ? 2.0 : 1.0 ) * std::sqrt( mean ) + ( _v.vec16 == 8 ? 4.0 : 0.0 ) ) _v.wlanes++;
@@ -1251,12 +1277,7 @@ private:
 			int const lg = record_size( double( _g.nnz ) / double( _g.n ) / _v.nact );
 			std::uint64_t const segs = seg_entries( _g.n, _v.ntiles ), bytes = segs << lg;
 			if( _v.wcap > 1 || _window == 0 || _p.batched || lg > 6 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
-			if( bytes > ( std::uint64_t( 1 ) << 30 ) )
-			{
-				std::size_t room = 0, all = 0;
-				SPICE_HIP( hipMemGetInfo( &room, &all ) );
-				if( bytes > room / 5 ) return;
-			}
+			if( !fits( bytes ) ) return;
 			try
 			{
 				_recs.resize( bytes );

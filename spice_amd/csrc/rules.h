@@ -34,6 +34,20 @@ constexpr int SEG_TILES = 3;    // log2 of the tiles of a row that lie side by s
 // Entries of the segment table for n rows and ntiles tiles.
 inline std::uint64_t seg_entries( std::int64_t n, std::int64_t ntiles ) { return std::uint64_t( n ) * std::uint64_t( ( ( ntiles - 1 ) >> SEG_TILES ) + 1 ) << SEG_TILES; }
 
+// Optional memory (bytes; faster forms of what a network can do without them): at most a fifth of
+// the free memory less what the network still has to allocate. Small amounts are not asked about.
+constexpr std::uint64_t OPTIONAL_SMALL = std::uint64_t( 64 ) << 20;
+inline bool optional_fits( std::uint64_t bytes, std::uint64_t free, std::uint64_t reserve ) { return free > reserve && bytes <= ( free - reserve ) / 5; }
+// The largest table of 8-byte entries of a served or batched net (whose memory is estimated before
+// it is built; larger ones have 4-byte offsets).
+constexpr std::uint64_t TABLE_BATCHED = std::uint64_t( 1 ) << 30;
+// The most that the table of such a net of n neurons in ntiles tiles or fewer takes.
+inline std::uint64_t batched_table_bytes( std::int64_t n, std::int64_t ntiles )
+{
+	std::uint64_t const bytes = 8 * seg_entries( n, ntiles );
+	return bytes <= TABLE_BATCHED ? bytes : std::max( TABLE_BATCHED, 4 * std::uint64_t( n ) * std::uint64_t( ntiles + 1 ) );
+}
+
 // Width of `tiles` tiles over n neurons, in 64s.
 inline std::int64_t tile_width( std::int64_t n, std::int64_t tiles ) { return ( ( n + tiles - 1 ) / tiles + 63 ) / 64 * 64; }
 

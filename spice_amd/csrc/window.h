@@ -73,6 +73,7 @@ __device__ inline void wave_lds_fence()
 
 // ---- what a delivery reads of a row's segment in a tile --------------------------------------
 enum { IDS32, IDS16, IDS16X8, RECORDS }; // the row store; its halves, 4 or 8 per lane; segment records (the last two: models with input classes)
+constexpr int SKIP_AT = 28; // IDS16X8: a staged segment's first place in its piece lies above its length (of 24 bits: build_halves)
 
 // The low halves of the target ids, which tell a target within a tile (of at most 65,536); n of them
 // are read at once: 4 from any place, 8 from a multiple of 8 (the store is padded by 8).
@@ -489,8 +490,8 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 	{
 		win_seg * const mine = seg + wave * 64;
 		std::int32_t src, q = 0, src_n = 0, q_n = 0;
-		segment sg;
-		auto fetch_seg = [&]() { sg = segment_of( v, src, tile ); };
+		packed_segment ps;
+		auto fetch_seg = [&]() { ps = load_segment( v, src, tile ); };
 		src = fetch_id( k0 + mylane, q );
 		fetch_seg();
 		if( k0 + NW * per < total ) src_n = fetch_id( k0 + NW * per + mylane, q_n );
@@ -499,14 +500,16 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 		for( ; k0 < total; k0 += NW * per )
 		{
 			std::int32_t const cnt = ( total - k0 ) < per ? ( total - k0 ) : per;
+			segment const sg = unpack_segment( v, ps );
 			std::int64_t const a = sg.at;
 			std::int32_t const len = lane < cnt ? sg.len : 0;
 			if constexpr( L::classes > 0 )
 			{
 				// in the place of the source: where the class's counters of the step start (for target 0).
-				// IDS16X8: from the piece that the segment begins in, its place there in the place of the step
+				// IDS16X8: from the piece that the segment begins in, its place there above the length
+				std::int32_t const at = ( q * nacc + N::input_class( src, info ) ) * tws - ( FORM == IDS32 ? t0 : 0 );
 				std::int32_t const skip = FORM == IDS16X8 && len > 0 ? std::int32_t( a ) & 7 : 0;
-				mine[lane] = win_seg::of( a - skip, len + skip, ( q * nacc + N::input_class( src, info ) ) * tws - ( FORM == IDS32 ? t0 : 0 ), skip );
+				mine[lane] = win_seg::of( a & ~std::int64_t( FORM == IDS16X8 ? 7 : 0 ), ( len + skip ) | skip << SKIP_AT, at );
 			}
 			else
 				mine[lane] = win_seg::of( a, len, src, q );
@@ -524,16 +527,15 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 			for( std::int32_t c = 0; c < cnt; c += U * ng )
 			{
 				win_seg r[U];
-				constexpr bool steps = L::classes == 0 || FORM == IDS16X8; // the records hold steps (or skips)
 				std::int32_t len[U], step[U], most = 0;
 #pragma unroll
 				for( int u = 0; u < U; u++ )
 				{
 					std::int32_t const k = c + u * ng + g;
 					r[u] = mine[k & 63]; // (records from cnt on are empty)
-					len[u] = k < 64 ? r[u].len : 0;
-					step[u] = steps ? r[u].step() : 0;
-					if constexpr( steps ) r[u].place = r[u].at();
+					len[u] = k < 64 ? ( FORM == IDS16X8 ? r[u].len & ( ( 1 << SKIP_AT ) - 1 ) : r[u].len ) : 0;
+					step[u] = FORM == IDS16X8 ? r[u].len >> SKIP_AT : L::classes == 0 ? r[u].step() : 0; // (or skip)
+					if constexpr( L::classes == 0 ) r[u].place = r[u].at();
 					most = len[u] > most ? len[u] : most;
 				}
 				for( std::int32_t e = l * V;; e += G * V )

@@ -86,8 +86,32 @@ static void tiles()
 			}
 }
 
+// Optional memory leaves what the network still needs, however much of it was taken before, and a
+// served net's table never takes more than its estimate, also once its tiles are wider.
+static void memory()
+{
+	std::uint64_t const G = std::uint64_t( 1 ) << 30;
+	for( std::uint64_t free : { 0 * G, 1 * G, 7 * G, 50 * G, 288 * G } )
+		for( std::uint64_t reserve : { 0 * G, 1 * G, 6 * G, 49 * G, 200 * G } )
+		{
+			std::uint64_t left = free;
+			for( int k = 0; k < 5; k++ )
+				for( std::uint64_t bytes = OPTIONAL_SMALL + 1; bytes < 2 * left; bytes = bytes * 3 / 2 )
+					if( optional_fits( bytes, left, reserve ) ) left -= bytes;
+			CHECK( left == free || left >= reserve, "free %llu reserve %llu", (unsigned long long)free, (unsigned long long)reserve );
+		}
+	for( std::int64_t n : { 100, 40000, 900000, 8000000 } )
+		for( std::int64_t tiles = 1; tiles < n / 64 + 2; tiles = tiles * 5 / 4 + 1 )
+			for( std::int64_t fewer = tiles; fewer > 0; fewer = fewer * 9 / 10 )
+			{
+				std::uint64_t const bytes = 8 * seg_entries( n, fewer ), taken = bytes <= TABLE_BATCHED ? bytes : 4 * std::uint64_t( n ) * std::uint64_t( fewer + 1 );
+				CHECK( taken <= batched_table_bytes( n, tiles ), "n %lld tiles %lld now %lld", (long long)n, (long long)tiles, (long long)fewer );
+			}
+}
+
 int main()
 {
+	memory();
 	tiles();
 	ring();
 	staged_segments();

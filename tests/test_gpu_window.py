@@ -245,3 +245,55 @@ def test_few_targets(gpu, model, pops, p, delay):
         assert_state_equal(d.neurons(), h.neurons(), model)
     np.testing.assert_array_equal(np.sort(d.step(True)), np.sort(h.step(True)))
     d.close(), h.close()
+
+
+@pytest.mark.parametrize("model,layout,delay,launch", [
+    ("brunel_3pop", three_pop_layout(1500), 15, (0, 0)),
+    ("brunel_3pop", three_pop_layout(5000, 0.3), 15, (1024, 1024)),  # 200 targets per segment
+    ("brunel_3pop", three_pop_layout(2100), 3, (192, 256)),
+    ("brunel", brunel_ref_layout(1500), 1, (0, 0)),
+    ("vogels_abbott", ([2500], [(0, 0, 0.02)]), 1, (0, 0)),      # records
+    ("synth", ([9000], [(0, 0, 0.01)]), 7, (64, 512)),           # more than 63 tiles
+    ("synth", ([3000], [(0, 0, 0.001)]), 1, (1024, 256)),
+    ("brunel_3pop_stdp", three_pop_layout(1500), 15, (0, 0)),
+    ("brunel_3pop_stdp", three_pop_layout(1500), 1, (128, 256)),
+    ("brunel_3pop_stdp_deferred", three_pop_layout(1500), 4, (0, 0)),
+    ("brunel_with_plasticity", brunel_ref_layout(1200), 9, (0, 0)),
+    ("brunel_with_plasticity", ([300, 900], [(0, 0, 0.05), (1, 0, 0.05), (1, 1, 0.05)]), 9, (0, 0)),  # per-synapse contract
+])
+def test_offsets_in_place_of_the_segment_table(gpu, model, layout, delay, launch):
+    """Networks declared wide enough for rows of 2^24 targets have 4-byte offsets of each tile's
+    targets instead of the segment table (as do those whose table would take too much memory)."""
+    h = O.CpuSnn(model, layout, DT, delay, seed=95, fixed_point=True)
+    rp, col = h.csr()
+    d = Snn.from_csr(model, rp, col, 1 << 24, DT, delay, seed=95, fixed_point=True)
+    for k, (tw, bs) in ((100, (0, 0)), (31, launch), (8, launch)):
+        d.set_launch(tile_w=tw, recv_block=bs)
+        d.run(k)
+        h.run(k)
+        assert_state_equal(d.neurons(), h.neurons(), model)
+    np.testing.assert_array_equal(np.sort(d.step(True)), np.sort(h.step(True)))
+    if model.startswith("brunel_3pop_stdp"):
+        np.testing.assert_array_equal(d.synapses(ell=False)["W"].view(np.uint32), h.synapses(ell=False)["W"].view(np.uint32))
+    d.close(), h.close()
+
+
+def test_row_of_more_than_2_24_targets(gpu):
+    n, delay = 320, 4
+    rows = [np.arange(k % 7, n, 7) for k in range(n)]
+    rows[5] = np.sort(np.concatenate([np.full((1 << 24) + 9, 100), rows[5]]))
+    rp = np.zeros(n + 1, np.int64)
+    np.cumsum([r.size for r in rows], out=rp[1:])
+    col, width = np.concatenate(rows).astype(np.int32), (rows[5].size + 31) // 32 * 32
+    h = O.CpuSnn.from_csr("brunel_3pop", rp, col, width, DT, delay, seed=6, fixed_point=True)
+    d = Snn.from_csr("brunel_3pop", rp, col, width, DT, delay, seed=6, fixed_point=True)
+    fired = 0
+    for k in range(60):
+        d.run(20)
+        h.run(20)
+        assert_state_equal(d.neurons(), h.neurons(), f"after {20 * k + 20} steps")
+        fired = d.stats()["events"] >> 24
+        if fired:
+            break
+    assert fired  # neuron 5, a Poisson source
+    d.close(), h.close()
