@@ -299,20 +299,20 @@ public:
 		*c = _clock.compensation();
 	}
 
-	// Moves the clock (conversion constructor / resume). Spikes in flight and the lazy
-	// plasticity bookkeeping are reset: synapse state is taken as current through step-1.
+	// Moves the clock (conversion constructor / resume). Spikes in flight and the
+	// plasticity bookkeeping are reset, after the plasticity of the steps before is done: synapse
+	// state is current through step-1.
 	void set_clock( std::int64_t step, float sum, float c ) override
 	{
 		if( step < 0 || step > INT_MAX - 2 ) throw std::invalid_argument( "invalid step index" );
+		sync_synapses();
 		if( factored && !_lazy )
 		{
 			// (the traces are synapse state: kept, as windows number them from 0 again)
-			sync_synapses();
 			std::int64_t const from = trace_slot() * _g.n;
 			if( from )
 				for( auto * b : { &_xtr, &_ytr } ) SPICE_HIP( hipMemcpy( b->data(), b->data() + from, std::size_t( _g.n ) * 4, hipMemcpyDeviceToDevice ) );
 		}
-		synchronize();
 		ctl_t ctl{ step, sum, c, std::int32_t( step % _v.rsize ), 0, 0, 0.0f, 0.0f };
 		SPICE_HIP( hipMemcpy( _ctl.data() + ( step & ( CLOCK_SLOTS - 1 ) ), &ctl, sizeof( ctl ), hipMemcpyHostToDevice ) );
 		SPICE_HIP( hipMemset( _counts.data(), 0, _counts.bytes() ) );

@@ -1,0 +1,57 @@
+"""What a network keeps when its clock, its statistics or its launch shapes are changed between
+runs."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from spice_amd import Batch, Layout, Snn
+from tests.helpers import assert_state_equal, brunel_ref_layout, three_pop_layout
+
+pytestmark = pytest.mark.gpu
+
+DT = 1e-4
+
+
+def _start(model, layout, delay, seed):
+    """A network that is active from the first step on."""
+    d = Snn(model, Layout(*layout), DT, delay, seed=seed, fixed_point=True)
+    rng = np.random.default_rng(seed)
+    n = sum(layout[0])
+    s = d.neurons()
+    s["V"] = rng.uniform(0.0, 0.025, n).astype(np.float32)
+    d.set_neurons(s)
+    if model == "brunel_with_plasticity":  # traces as after a long silence: events move the weights
+        z = d.synapses(ell=False)
+        rp, dst = d.csr()
+        src = np.repeat(np.arange(n), np.diff(rp))
+        plastic = (src >= n // 2) & (src < 9 * n // 10) & (dst < 9 * n // 10)
+        for k in ("Zpre", "Zpost"):
+            z[k] = np.where(plastic, np.float32(1e-4), np.float32(1.0))
+        d.set_synapses(z, ell=False)
+    return d
+
+
+PLASTIC = [
+    ("brunel_3pop_stdp", three_pop_layout(1500), 15),
+    ("brunel_3pop_stdp", three_pop_layout(1500), 1),
+    ("brunel_3pop_stdp_deferred", three_pop_layout(1500), 4),
+    ("brunel_with_plasticity", brunel_ref_layout(1200), 9),
+    ("brunel_with_plasticity", ([300, 900], [(0, 0, 0.05), (1, 0, 0.05), (1, 1, 0.05)]), 9),  # per-synapse contract
+]
+
+
+@pytest.mark.parametrize("model,layout,delay", PLASTIC)
+@pytest.mark.parametrize("step", [0, 77])
+def test_set_clock_keeps_the_plasticity_of_all_steps(gpu, model, layout, delay, step):
+    """The synapses after set_clock() are those of the steps run before it, the last window's too."""
+    a, b = _start(model, layout, delay, 3), _start(model, layout, delay, 3)
+    before = a.synapses(ell=False)
+    for net in (a, b):
+        net.run(27)
+    want = a.synapses(ell=False)
+    assert not np.array_equal(before["W"], want["W"])
+    b.set_clock(step, step * DT, 0.0)
+    got = b.synapses(ell=False)
+    for k in want:
+        np.testing.assert_array_equal(got[k].view(np.uint32), want[k].view(np.uint32), err_msg=k)
+    a.close(), b.close()
