@@ -332,11 +332,7 @@ public:
 
 	void get_stats( spice_stats * out ) override
 	{
-		// (windows of different lengths leave different amounts of plasticity due: count all of it)
-		if( windowed && !_lazy )
-			sync_synapses();
-		else
-			synchronize();
+		sync_counted();
 		std::vector<unsigned long long> b( _bstats.size() );
 		SPICE_HIP( hipMemcpyAsync( b.data(), _bstats.data(), _bstats.bytes(), hipMemcpyDeviceToHost, _s ) );
 		SPICE_HIP( hipStreamSynchronize( _s ) );
@@ -347,7 +343,7 @@ public:
 	}
 	void reset_stats() override
 	{
-		synchronize();
+		sync_counted();
 		SPICE_HIP( hipMemsetAsync( _bstats.data(), 0, _bstats.bytes(), _s ) );
 		synchronize();
 		_stats_step0 = _step;
@@ -1559,6 +1555,16 @@ private:
 	{
 		launch_receive_events<F>( v, e[0], e[1] );
 		launch_update<F>( v, e[2], e[3] );
+	}
+
+	// Before the counters are read or cleared: windows of different lengths leave different amounts of
+	// plasticity due, and all of it counts to the steps before.
+	void sync_counted()
+	{
+		if( windowed && !_lazy )
+			sync_synapses();
+		else
+			synchronize();
 	}
 
 	// Brings all plastic synapses up to date through the last completed step.

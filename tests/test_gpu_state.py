@@ -55,3 +55,14 @@ def test_set_clock_keeps_the_plasticity_of_all_steps(gpu, model, layout, delay, 
     for k in want:
         np.testing.assert_array_equal(got[k].view(np.uint32), want[k].view(np.uint32), err_msg=k)
     a.close(), b.close()
+
+
+@pytest.mark.parametrize("model,layout,delay", PLASTIC)
+def test_reset_stats_counts_from_here(gpu, model, layout, delay):
+    """What earlier steps left to do is not counted after reset_stats()."""
+    d = _start(model, layout, delay, 4)
+    d.run(27)
+    d.reset_stats()
+    st = d.stats()
+    assert all(v == 0 for v in st.values()), st
+    d.close()
