@@ -125,10 +125,8 @@ public:
 			while( _window > 1 && bytes( _window ) > LDS_PER_CU / 4 ) _window = window_steps( _window - 1 );
 			_lds = bytes( _window );
 			if( !_windows ) _window = 0;
-			if( _lds > ( 64 << 10 ) )
-				SPICE_HIP( hipFuncSetAttribute( _fixed ? reinterpret_cast<void const *>( &k_batch_window<Model, true, window_block> )
-				                                       : reinterpret_cast<void const *>( &k_batch_window<Model, false, window_block> ),
-				                                hipFuncAttributeMaxDynamicSharedMemorySize, int( _lds ) ) );
+			allow_lds( _fixed ? reinterpret_cast<void const *>( &k_batch_window<Model, true, window_block> ) : reinterpret_cast<void const *>( &k_batch_window<Model, false, window_block> ),
+			           _lds );
 		}
 		// all tables in one buffer and one copy
 		std::vector<unsigned char> all;

@@ -1170,16 +1170,13 @@ private:
 			with_window_kernel( IDS32, [&]( auto, auto bytes, int ) {
 				// the LDS of a CU, shared by the workgroups that a CU gets
 				std::size_t const per_cu = std::size_t( std::clamp( ( _v.ntiles + device_cu_count() - 1 ) / device_cu_count(), 1, 3 ) );
-				std::size_t const room = ( LDS_PER_CU - 4096 ) / per_cu;
+				std::size_t const room = LDS_DYNAMIC / per_cu;
 				int w = _v.wcap;
 				while( w > 1 && bytes( w ) > room ) w = window_steps( w - 1 );
 				_window = w;
 			} );
 			for( int form : { IDS32, IDS16, IDS16X8, RECORDS } )
-				with_window_kernel( form, [&]( auto kernel, auto bytes, int ) {
-					if( bytes( _window ) > ( 64 << 10 ) )
-						SPICE_HIP( hipFuncSetAttribute( reinterpret_cast<void const *>( kernel ), hipFuncAttributeMaxDynamicSharedMemorySize, int( bytes( _window ) ) ) );
-				} );
+				with_window_kernel( form, [&]( auto kernel, auto bytes, int ) { allow_lds( reinterpret_cast<void const *>( kernel ), bytes( _window ) ); } );
 		}
 	}
 

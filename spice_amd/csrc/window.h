@@ -29,6 +29,14 @@
 namespace spice::hipx
 {
 constexpr std::size_t LDS_PER_CU = 160 << 10;
+constexpr std::size_t LDS_DYNAMIC = LDS_PER_CU - 4096; // beside what the window kernels declare themselves
+
+// Lets `kernel` be launched with `bytes` of dynamic LDS. The limit belongs to the kernel, whichever
+// networks run it, so it is set to the same for all of them.
+inline void allow_lds( void const * kernel, std::size_t bytes )
+{
+	if( bytes > ( 64 << 10 ) ) SPICE_HIP( hipFuncSetAttribute( kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int( std::max( bytes, LDS_DYNAMIC ) ) ) );
+}
 
 constexpr int WIN_VEC = 4;   // consecutive targets a lane reads at once (the row store is padded by as many)
 constexpr int WIN_TABLE = 64; // partial sums kept per input class

@@ -66,3 +66,21 @@ def test_reset_stats_counts_from_here(gpu, model, layout, delay):
     st = d.stats()
     assert all(v == 0 for v in st.values()), st
     d.close()
+
+
+def test_a_smaller_network_leaves_a_larger_one_its_lds(gpu):
+    """Both run the same kernel, at 144 KB (tiles of 1,024, 15 steps) and 76 KB (of 512) of LDS, and
+    the larger one was made first."""
+    lay, delay = three_pop_layout(3000), 15
+    h = O.CpuSnn("brunel_3pop", lay, DT, delay, seed=8, fixed_point=True)
+    large, small = (Snn("brunel_3pop", Layout(*lay), DT, delay, seed=8, fixed_point=True) for _ in range(2))
+    large.set_launch(tile_w=1024, recv_block=1024)
+    large.run(30)
+    small.set_launch(tile_w=512, recv_block=1024)
+    small.run(30)
+    large.run(45)
+    h.run(75)
+    assert_state_equal(large.neurons(), h.neurons(), "the larger")
+    small.run(45)
+    assert_state_equal(small.neurons(), h.neurons(), "the smaller")
+    large.close(), small.close(), h.close()
