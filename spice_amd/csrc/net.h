@@ -200,6 +200,7 @@ public:
 	// ---- simulation ----
 	void step( std::int32_t ** dspk, std::uint32_t ** dcnt ) override
 	{
+		require_whole();
 		std::int64_t const t = _step;
 		if( t < _single_until )
 			launch_window( t, 1, nullptr, nullptr, true );
@@ -215,6 +216,7 @@ public:
 	void run( std::int64_t n ) override
 	{
 		if( n < 0 ) throw std::invalid_argument( "negative step count" );
+		require_whole();
 		while( n > 0 && _step < _single_until )
 		{
 			launch_window( _step, 1, nullptr, nullptr, true );
@@ -248,6 +250,7 @@ public:
 	void run_profiled( std::int64_t n, double * kernel_ms ) override
 	{
 		if( n < 0 ) throw std::invalid_argument( "negative step count" );
+		require_whole();
 		if( _window )
 			run_profiled_windows( n, kernel_ms );
 		else
@@ -629,6 +632,10 @@ public:
 			apply_launch( fresh ? launch_cfg{} : _lc );
 		}
 	}
+	void require_whole() const
+	{
+		if( !_whole ) throw std::runtime_error( "the network lost buffers when memory ran out: set its launch shapes, or make it anew" );
+	}
 	bool logged() const { return _slog_ctl.size() > 0; }
 	int num_receive_parts() const { return _v.rparts; }
 	int num_update_blocks() const { return _grid_update; }
@@ -686,6 +693,7 @@ private:
 	bool _ahead = false; // the delivery of a step may run before the updates of earlier steps
 	std::int64_t _single_until = 0; // steps run one by one before this step (see import_neuron_attr)
 	bool _lazy = false; // plasticity by the per-synapse contract
+	bool _whole = false; // all buffers are there (see shape)
 	int _window = 0;       // longest window of the window kernels that run the steps (0: none)
 	launch_queue _queue;
 	launch_cfg _lc{};
@@ -1025,10 +1033,33 @@ private:
 		if( c.flush_slots < 64 || c.flush_slots > ( 1 << 20 ) || c.flush_slots % 64 )
 			throw std::invalid_argument( "flush_slots must be a multiple of 64 in [64, 2^20]" );
 		if( c.flush_grid < 1 || c.flush_grid > 64 * cus ) throw std::invalid_argument( "flush_grid must be in [1, 64 x CUs]" );
+		if( !_lc.tile_w )
+		{
+			shape( c ); // (a new network: nothing to go back to)
+			return;
+		}
+		launch_cfg const before = _lc;
+		try
+		{
+			shape( c );
+		}
+		catch( ... )
+		{
+			shape( before ); // (its buffers fitted)
+			throw;
+		}
+	}
+
+	// The buffers, views and windows of launch shapes c. If an allocation fails on the way the network
+	// is not whole until a call succeeds, and is not stepped.
+	void shape( launch_cfg const & c )
+	{
+		int const cus = device_cu_count();
 		std::int64_t const n = _g.n;
 		dview & v = _v;
-		bool const retile = c.tile_w != v.tile_w;
+		bool const retile = c.tile_w != v.tile_w || !( v.segs || v.offs );
 		int const had_window = _window;
+		_whole = false;
 		if( retile )
 		{
 			std::int32_t const ntiles = std::int32_t( ( n + c.tile_w - 1 ) / c.tile_w );
@@ -1075,10 +1106,11 @@ private:
 				SPICE_HIP( hipStreamSynchronize( _s ) );
 				for( std::size_t i = 0; i < b.size(); i++ ) keep[i % NSTAT] += b[i];
 			}
-			_bstats.resize( slots );
-			SPICE_HIP( hipMemsetAsync( _bstats.data(), 0, _bstats.bytes(), _s ) );
-			SPICE_HIP( hipMemcpyAsync( _bstats.data(), keep.data(), NSTAT * 8, hipMemcpyHostToDevice, _s ) );
+			dbuf<unsigned long long> more( slots );
+			SPICE_HIP( hipMemsetAsync( more.data(), 0, more.bytes(), _s ) );
+			SPICE_HIP( hipMemcpyAsync( more.data(), keep.data(), NSTAT * 8, hipMemcpyHostToDevice, _s ) );
 			SPICE_HIP( hipStreamSynchronize( _s ) ); // `keep` is a host temporary
+			_bstats = std::move( more );
 			v.bstats = _bstats.data();
 		}
 		for( int p = 0; p < CLOCK_SLOTS; p++ )
@@ -1090,6 +1122,7 @@ private:
 		}
 		SPICE_HIP( hipStreamSynchronize( _s ) );
 		_graphs.clear(); // the captured launches hold the old shapes
+		_whole = true;
 	}
 
 	// Whether `bytes` of optional memory fit beside what this net still needs (rules.h).
@@ -1572,6 +1605,7 @@ private:
 		{
 			if( _step > 0 && _caught_host != _step - 1 )
 			{
+				require_whole();
 				// the last step's plasticity work, which the next delivery kernel would run, then
 				// (eager) its events of the rows arriving next or (lazy) every row's replay up to it;
 				// recorded in `caught` so the next delivery kernel skips the former

@@ -84,3 +84,27 @@ def test_a_smaller_network_leaves_a_larger_one_its_lds(gpu):
     small.run(45)
     assert_state_equal(small.neurons(), h.neurons(), "the smaller")
     large.close(), small.close(), h.close()
+
+
+def test_launch_shapes_that_do_not_fit_leave_the_old_ones(gpu):
+    """Tiles of 64 of 2.5 million neurons: 390 GB for the offsets of every row and tile. The network
+    goes on with the shapes, counters and results that it had."""
+    lay, delay = ([2500000], [(0, 0, 2e-6)]), 1
+    h = O.CpuSnn("synth", lay, DT, delay, seed=9, fixed_point=True)
+    d = Snn("synth", Layout(*lay), DT, delay, seed=9, fixed_point=True)
+    for net in (h, d):
+        net.run(9)
+    before, stats = d.launch(), d.stats()
+    with pytest.raises(MemoryError):
+        d.set_launch(tile_w=64)
+    assert d.launch() == before and d.stats() == stats
+    for net in (h, d):
+        net.run(6)
+    assert_state_equal(d.neurons(), h.neurons(), "after the refused shapes")
+    np.testing.assert_array_equal(np.sort(d.step(True)), np.sort(h.step(True)))
+    d.set_launch(tile_w=2048)
+    for net in (h, d):
+        net.run(6)
+        net.step()
+    assert_state_equal(d.neurons(), h.neurons(), "after other shapes")
+    d.close(), h.close()
