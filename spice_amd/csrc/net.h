@@ -616,17 +616,52 @@ public:
 			if( _lazy ) return;
 			bool const fresh = _step == 0;
 			sync_synapses();
+			// All memory first, beside the by-target index, or else in its place; if it does not fit
+			// there either, the index comes back and the net stays as it was.
+			constexpr int traces[2] = { int( S::pre_trace ), int( S::post_trace ) };
+			dbuf<char> kept[2];
+			auto take = [&] {
+				try
+				{
+					for( auto & b : kept ) b.resize( std::size_t( _g.nnz + COL_PAD ) * sizeof( float ) );
+					alloc_lazy();
+				}
+				catch( ... )
+				{
+					for( auto & b : kept ) b.release();
+					throw;
+				}
+			};
+			try
+			{
+				take();
+			}
+			catch( std::bad_alloc const & )
+			{
+				if( !_tp_ent.size() ) throw;
+				_whole = false;
+				_tp_ent.release();
+				try
+				{
+					take();
+				}
+				catch( ... )
+				{
+					build_by_target();
+					throw;
+				}
+			}
+			for( int k = 0; k < 2; k++ )
+			{
+				expand_trace( traces[k], reinterpret_cast<float *>( kept[k].data() ) );
+				_sa[traces[k]] = std::move( kept[k] );
+				_v.sa[traces[k]] = _sa[traces[k]].data();
+			}
+			_whole = false; // until the views are right
 			_tp_ent.release();
 			_tp_total = _tp_targets = 0;
-			for( int a : { int( S::pre_trace ), int( S::post_trace ) } )
-			{
-				_sa[a].resize( std::size_t( _g.nnz + COL_PAD ) * sizeof( float ) );
-				_v.sa[a] = _sa[a].data();
-				expand_trace( a, reinterpret_cast<float *>( _sa[a].data() ) );
-			}
 			_lazy = true;
 			_single_until = 0;
-			alloc_lazy();
 			reset_lazy( std::int32_t( _step - 1 ) );
 			SPICE_HIP( hipMemset( _fl_count.data(), 0, _fl_count.bytes() ) );
 			apply_launch( fresh ? launch_cfg{} : _lc );
@@ -923,7 +958,10 @@ private:
 				SPICE_HIP( hipMemcpyAsync( &b, bad.data(), 4, hipMemcpyDeviceToHost, _s ) );
 				SPICE_HIP( hipStreamSynchronize( _s ) );
 				if( b )
+				{
+					tmp.release();
 					make_lazy();
+				}
 				else if( is_factored_attr<S>( a ) )
 				{
 					SPICE_HIP( hipMemcpy( kept.data() + at, t.data(), t.bytes(), hipMemcpyDeviceToDevice ) );

@@ -108,3 +108,47 @@ def test_launch_shapes_that_do_not_fit_leave_the_old_ones(gpu):
         net.step()
     assert_state_equal(d.neurons(), h.neurons(), "after other shapes")
     d.close(), h.close()
+
+
+@pytest.mark.parametrize("room,fits", [(1300, False), (1800, True)])
+def test_traces_that_do_not_fit_leave_the_network_as_it_was(gpu, room, fits):
+    """Imported traces that differ between the synapses of a neuron make the network keep them per
+    synapse: 2 x 1,220 MB here, for an import that takes 1,220 MB itself, with `room` MB of memory free;
+    the by-target index, 780 MB, may make way (and the runtime finds about 200). If they do not fit the import raises MemoryError, and
+    the network goes on as one that was not asked; with memory again, it is imported."""
+    import torch
+    model, lay, delay = "brunel_with_plasticity", brunel_ref_layout(80000), 15
+    a, b = _start(model, lay, delay, 11), _start(model, lay, delay, 11)
+    for net in (a, b):
+        net.run(21)
+    z = b.synapses(ell=False)
+    assert z["W"].nbytes >> 20 in range(1200, 1230), z["W"].nbytes
+    z["Zpre"] = np.random.default_rng(12).uniform(1e-4, 2e-4, z["W"].size).astype(np.float32)
+    fill = []
+    try:
+        while torch.cuda.mem_get_info()[0] > (room << 20) + (16 << 30):
+            fill.append(torch.empty(16 << 30, dtype=torch.uint8, device="cuda"))
+        left = torch.cuda.mem_get_info()[0] - (room << 20)
+        fill.append(torch.empty(left >> 21 << 21, dtype=torch.uint8, device="cuda"))
+        if abs(torch.cuda.mem_get_info()[0] - (room << 20)) > 24 << 20:
+            pytest.skip("the card's memory is used by others as well")
+        if fits:
+            a.set_synapses(z, ell=False)
+        else:
+            with pytest.raises(MemoryError):
+                a.set_synapses(z, ell=False)
+            for net in (a, b):
+                net.run(40)
+            assert_state_equal(a.neurons(), b.neurons(), "after the refused import")
+    finally:
+        del fill[:]
+        torch.cuda.empty_cache()
+    if not fits:
+        a.set_synapses(z, ell=False)
+    b.set_synapses(z, ell=False)
+    for net in (a, b):
+        net.run(40)
+    assert_state_equal(a.neurons(), b.neurons(), "after the import")
+    x, y = a.synapses(ell=False), b.synapses(ell=False)
+    assert_state_equal(x, y, "after the import")
+    a.close(), b.close()
