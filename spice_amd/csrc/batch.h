@@ -66,6 +66,7 @@ public:
 	// kernels.
 	void build()
 	{
+		_built = false; // (until all of it is done: an allocation may fail on the way)
 		_windows = windowed;
 		if constexpr( factored_v<Model> )
 		{
@@ -153,6 +154,18 @@ public:
 		_grid_tiles = std::min( _ntiles, ( recv_block == 256 ? SPICE_BATCH_GRID_PER_CU : SPICE_BATCH_GRID_PER_CU / 4 ) * device_cu_count() );
 		for( auto * n : _nets ) n->synchronize();
 		SPICE_HIP( hipStreamSynchronize( _s ) );
+		_built = true;
+	}
+
+	// The tables are those of the nets as they are now.
+	void ready()
+	{
+		bool stale = !_built;
+		if constexpr( factored_v<Model> )
+			for( auto * n : _nets ) stale = stale || ( _windows && n->lazy() );
+		if( !stale ) return;
+		synchronize();
+		build();
 	}
 
 	// Delivery tile width of a net of n neurons (at `tile_w` now) in a batch of nnets. Many nets
@@ -186,16 +199,8 @@ public:
 	{
 		if( n < 0 ) throw std::invalid_argument( "negative step count" );
 		if( n == 0 ) return;
-		if constexpr( factored_v<Model> )
-		{
-			bool lazy = false;
-			for( auto * net : _nets ) lazy = lazy || net->lazy();
-			if( lazy && _windows )
-			{
-				synchronize();
-				build();
-			}
-		}
+		ready();
+		for( auto * net : _nets ) net->require_whole();
 		// (state imported into a net may ask for a few steps one by one)
 		std::int64_t single = 0;
 		for( auto * net : _nets ) single = std::max( single, net->single_steps_left() );
@@ -220,6 +225,7 @@ public:
 	void begin_spike_log( std::int64_t nsteps ) override
 	{
 		for( auto * net : _nets ) net->note_spike_log( nsteps ); // validates nsteps first
+		ready();
 		std::int32_t const n = std::int32_t( _nets.size() );
 		SPICE_LAUNCH( k_batch_log_window<<<unsigned( ( n + 255 ) / 256 ), 256, 0, _s>>>( _views[_step & ( CLOCK_SLOTS - 1 )], n, nsteps ) );
 	}
@@ -243,6 +249,7 @@ private:
 	step_graphs _graphs;
 	bool _fixed = false;
 	bool _windows = false; // steps run as windows
+	bool _built = false;   // build() went through
 	// windows of up to _window steps (0: two-kernel steps)
 	static constexpr int window_block = 256;
 	// tiles of all nets, per CU: 48 nets of 1e4 to 1e7 synapses take, at 4 / 8 / 16 / 64, 2.6 / 1.8 /

@@ -110,6 +110,17 @@ def test_launch_shapes_that_do_not_fit_leave_the_old_ones(gpu):
     d.close(), h.close()
 
 
+def _fill(fill, room):
+    """Takes the card's memory but `room` MB (the runtime may find some 200 more)."""
+    import torch
+    while torch.cuda.mem_get_info()[0] > (room << 20) + (16 << 30):
+        fill.append(torch.empty(16 << 30, dtype=torch.uint8, device="cuda"))
+    left = torch.cuda.mem_get_info()[0] - (room << 20)
+    fill.append(torch.empty(left >> 21 << 21, dtype=torch.uint8, device="cuda"))
+    if abs(torch.cuda.mem_get_info()[0] - (room << 20)) > 24 << 20:
+        pytest.skip("the card's memory is used by others as well")
+
+
 @pytest.mark.parametrize("room,fits", [(1300, False), (1800, True)])
 def test_traces_that_do_not_fit_leave_the_network_as_it_was(gpu, room, fits):
     """Imported traces that differ between the synapses of a neuron make the network keep them per
@@ -126,12 +137,7 @@ def test_traces_that_do_not_fit_leave_the_network_as_it_was(gpu, room, fits):
     z["Zpre"] = np.random.default_rng(12).uniform(1e-4, 2e-4, z["W"].size).astype(np.float32)
     fill = []
     try:
-        while torch.cuda.mem_get_info()[0] > (room << 20) + (16 << 30):
-            fill.append(torch.empty(16 << 30, dtype=torch.uint8, device="cuda"))
-        left = torch.cuda.mem_get_info()[0] - (room << 20)
-        fill.append(torch.empty(left >> 21 << 21, dtype=torch.uint8, device="cuda"))
-        if abs(torch.cuda.mem_get_info()[0] - (room << 20)) > 24 << 20:
-            pytest.skip("the card's memory is used by others as well")
+        _fill(fill, room)
         if fits:
             a.set_synapses(z, ell=False)
         else:
@@ -152,3 +158,35 @@ def test_traces_that_do_not_fit_leave_the_network_as_it_was(gpu, room, fits):
     x, y = a.synapses(ell=False), b.synapses(ell=False)
     assert_state_equal(x, y, "after the import")
     a.close(), b.close()
+
+
+def test_a_batch_whose_tables_could_not_be_made_makes_them_later(gpu):
+    """A member's imported traces take the whole batch to traces per synapse (2 x 305 MB for the other
+    member, whose index gives 195 back) at the next run: without the memory run() raises MemoryError,
+    each time; with memory again it goes on as a batch that always had it."""
+    import torch
+    lay = brunel_ref_layout(40000)
+    batches = [Batch("brunel_with_plasticity", [(Layout(*lay), 15, 21 + k) for k in range(2)], DT, fixed_point=True) for _ in range(2)]
+    z = batches[0].net(0).synapses(ell=False)
+    z["Zpre"] = np.random.default_rng(22).uniform(1e-4, 2e-4, z["W"].size).astype(np.float32)
+    for b in batches:
+        b.run(20)
+        b.net(0).set_synapses(z, ell=False)
+    fill = []
+    try:
+        _fill(fill, 100)
+        for _ in range(2):
+            with pytest.raises(MemoryError):
+                batches[0].run(33)
+    finally:
+        del fill[:]
+        torch.cuda.empty_cache()
+    for b in batches:
+        b.run(33)
+    for k in range(2):
+        x, y = (b.net(k) for b in batches)
+        assert x.clock() == y.clock()
+        assert_state_equal(x.neurons(), y.neurons(), f"net {k}")
+        assert_state_equal(x.synapses(ell=False), y.synapses(ell=False), f"net {k}")
+    for b in batches:
+        b.close()
