@@ -311,7 +311,8 @@ typedef struct spice_launch
 	int32_t flush_slots;
 	int32_t flush_grid;
 	int32_t recv_block; /* delivery workgroup size: 256, 512 or 1024 threads */
-	int32_t recv_parts; /* delivery workgroups per tile, 1..16 (the step's spikes split between them) */
+	int32_t recv_parts; /* delivery workgroups per tile, 1..16 (the step's spikes split between them);
+	                       no effect on windows of several steps or of plastic models */
 	int32_t reserved[3];
 } spice_launch;
 
@@ -319,7 +320,7 @@ int spice_hip_get_launch( spice_net * net, spice_launch * out );
 int spice_hip_set_launch( spice_net * net, const spice_launch * in );
 /* Times candidate launch shapes on a copy of the network (warmup steps first, then `steps`
  * steps per candidate, wall time per step: plasticity overlaps delivery, so
- * shapes are evaluated together; tile width first, then delivery parts, then the plasticity
+ * shapes are evaluated together; tile width first, then delivery parts (where they have an effect), then the plasticity
  * shape; the three fastest are then timed again in turn, three times each, since the copy's
  * activity drifts between candidates),
  * applies the fastest to the network and returns it with its step time (us). The network

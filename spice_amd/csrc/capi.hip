@@ -847,6 +847,7 @@ int spice_hip_autotune( spice_net * net, int64_t warmup, int64_t steps, spice_la
 					x.recv_block = bs;
 					trial( x );
 				}
+			if( n->splits_delivery() )
 			{
 				launch_cfg const base = cfg;
 				for( int parts : { 2, 3, 4, 6 } )

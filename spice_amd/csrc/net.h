@@ -126,6 +126,7 @@ struct net_iface
 	virtual net_iface * clone() const = 0;
 	virtual bool is_plastic() const = 0;
 	virtual int max_tile_w() const = 0; // widest tile_w set_launch accepts
+	virtual bool splits_delivery() const = 0; // whether the steps' kernels depend on recv_parts
 };
 
 inline int device_cu_count()
@@ -534,6 +535,8 @@ public:
 		apply_launch( c );
 	}
 	bool is_plastic() const override { return plastic; }
+	// (windows of several steps, and of plastic models, have one workgroup per tile whatever it says)
+	bool splits_delivery() const override { return !windowed || _lazy || ( !plastic && !_ahead ); }
 	// widest delivery tile: wide tiles for static models that run step by step
 	int max_tile_w() const override { return !plastic && !_ahead ? TILE_WIDE : TILE_MAX; }
 

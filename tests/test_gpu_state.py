@@ -190,3 +190,13 @@ def test_a_batch_whose_tables_could_not_be_made_makes_them_later(gpu):
         assert_state_equal(x.synapses(ell=False), y.synapses(ell=False), f"net {k}")
     for b in batches:
         b.close()
+
+
+@pytest.mark.parametrize("model,delay", [("brunel_3pop", 15), ("brunel_3pop_stdp", 15), ("brunel_3pop_stdp", 1)])
+def test_autotune_leaves_parts_that_have_no_effect(gpu, model, delay):
+    """Windows of several steps, and of plastic models, have one workgroup per tile: the parts of a
+    delivery are not varied (a time that differs by chance would be reported as theirs)."""
+    d = Snn(model, Layout(*three_pop_layout(2000)), DT, delay, seed=10, fixed_point=True)
+    cfg, us = d.autotune(warmup=50, steps=20)
+    assert cfg["recv_parts"] == 1 and d.launch()["recv_parts"] == 1 and us > 0
+    d.close()
