@@ -62,16 +62,22 @@ inline int lazy_tile_w( std::int64_t n, int cus ) { return int( std::clamp<std::
 // windows of static models, whose workgroups of 1,024 threads (default_launch) have a CU each
 // (Brunel, 100,000 and 40,000 neurons of which half have inputs, us per step: 3.4 and 1.9 with a
 // tile per CU of all, 4.7 and 2.2 with one per CU of those). Where few neurons have inputs, the tiles
-// are still those of all neurons, and the segment table has an entry for each of them and row:
-// four per CU at most, or two where fewer than half have inputs and the table would take over 512 MB.
-constexpr std::uint64_t TABLE_SMALL = std::uint64_t( 512 ) << 20;
+// are still those of all neurons, and the segment table has an entry for each of them and row: two per
+// CU at most, or four with plasticity, whose tiles are the better the narrower, where the table takes
+// at most 1 GB then (us per step, with up to two and up to four: brunel_3pop_stdp, 100,000 neurons of
+// which 20,000 have inputs, 2.7 and 2.4; synth, 10,000 of 100,000 and of 300,000, 9.5 and 10.3, 12.1
+// and 19.0).
+constexpr std::uint64_t TABLE_SMALL = std::uint64_t( 1 ) << 30;
 inline int window_tile_w( std::int64_t n, std::int64_t targets, bool plastic, bool ahead, int cus )
 {
 	std::int64_t const tiled = targets <= 0 || ( ahead && !plastic ) ? n : targets;
 	std::int64_t const most = ahead || plastic ? TILE_MAX : 4 * 1024;
 	std::int64_t w = tile_width( tiled, ahead && tile_width( tiled, cus ) > most ? 2 * cus : cus );
-	w = std::max( w, tile_width( n, 4 * cus ) );
-	if( 2 * targets < n && 8 * seg_entries( n, ( n + w - 1 ) / w ) > TABLE_SMALL ) w = std::max( w, tile_width( n, 2 * cus ) );
+	if( 2 * targets < n )
+	{
+		if( plastic ) w = std::max( w, tile_width( n, 4 * cus ) );
+		if( !plastic || 8 * seg_entries( n, ( n + w - 1 ) / w ) > TABLE_SMALL ) w = std::max( w, tile_width( n, 2 * cus ) );
+	}
 	return int( std::clamp<std::int64_t>( w, 64, most ) );
 }
 

@@ -60,8 +60,8 @@ static void staged_segments()
 	static_assert( sizeof( win_seg ) == 16, "" );
 }
 
-// Tiles: however few neurons have inputs, at most four per CU (or as wide as its kernel takes), and a
-// segment table of at most 512 MB, or that of tiles for two per CU; where half of the neurons have
+// Tiles: however few neurons have inputs, at most two per CU, or four with plasticity (or as wide as its
+// kernel takes), and a segment table of at most 1 GB, or that of tiles for two per CU; where half of the neurons have
 // inputs or more, one per CU of those (windows of several steps: of all, or two).
 static void tiles()
 {
@@ -75,7 +75,7 @@ static void tiles()
 				int const w = window_tile_w( n, targets, plastic, ahead, cus ), most = plastic || ahead ? TILE_MAX : 4 * 1024;
 				std::int64_t const tiles = ( n + w - 1 ) / w;
 				CHECK( w >= 64 && w <= most && w % 64 == 0, "n %lld w %d", (long long)n, w );
-				CHECK( tiles <= 4 * cus || w == most, "n %lld targets %lld kind %d w %d", (long long)n, (long long)targets, kind, w );
+				CHECK( tiles <= ( plastic ? 4 : 2 ) * cus || w == most, "n %lld targets %lld kind %d w %d", (long long)n, (long long)targets, kind, w );
 				std::int64_t const two = std::min<std::int64_t>( tile_width( n, 2 * cus ), most );
 				if( share < 0.5 ) CHECK( 8 * seg_entries( n, tiles ) <= std::max( TABLE_SMALL, 8 * seg_entries( n, ( n + two - 1 ) / two ) ), "n %lld targets %lld kind %d w %d", (long long)n, (long long)targets, kind, w );
 				else
