@@ -197,11 +197,11 @@ static __device__ void long_connection( conn const & cn, int c, std::int64_t r, 
 }
 
 // Targets of rows, NW waves per row. A connection's draws are split into one stretch per wave; up to
-// 256 KB of them per wave are drawn once and kept in LDS for the total and then the positions, longer
+// 2,048 of them per wave (8 KB) are drawn once and kept in LDS for the total and then the positions, longer
 // connections are drawn twice by the row's first wave. Bound by the vector ALU (Philox, the
-// logarithm): 1e9 targets 2.3 ms, and 4.6 with every draw made twice and a division each in its
+// logarithm; busy 92 to 96 % of the time): 1e9 targets 2.3 ms, and 4.6 with every draw made twice and a division each in its
 // logarithm and its position.
-constexpr int KB = 8; // Philox blocks per lane
+constexpr int LANE_BLOCKS = 8; // Philox blocks (of 4 draws) per lane
 template <int NW>
 static __global__ __launch_bounds__( NW == 16 ? 1024 : 256 ) void k_targets(
     conn const * conns, int nconns, std::int64_t n, std::int64_t width, std::uint64_t seed, std::int64_t const * row_ptr, std::int32_t * col )
@@ -212,13 +212,13 @@ static __global__ __launch_bounds__( NW == 16 ? 1024 : 256 ) void k_targets(
 		std::uint32_t f[4];
 	};
 	__shared__ log_entry table[1 << LOG_BITS];
-	__shared__ block4 draws[bs * KB];
+	__shared__ block4 draws[bs * LANE_BLOCKS];
 	__shared__ double tot[2][NW];
 	fill_log_table( table );
 	__syncthreads();
 	int const lane = lane_id(), wave = threadIdx.x >> 6;
 	int const w = NW == 1 ? 0 : wave; // wave of the row
-	block4 * const mine = draws + wave * ( 64 * KB ) + lane;
+	block4 * const mine = draws + wave * ( 64 * LANE_BLOCKS ) + lane;
 	int turn = 0;
 	constexpr std::int64_t per_block = bs / ( 64 * NW );
 	for( std::int64_t r = uniform64( blockIdx.x * per_block + ( NW == 1 ? wave : 0 ) ); r < n; r += gridDim.x * per_block )
@@ -244,7 +244,7 @@ static __global__ __launch_bounds__( NW == 16 ? 1024 : 256 ) void k_targets(
 				std::int32_t const first = conns[c].dst_first;
 				std::int32_t const R = ( conns[c].dst_last - first ) - std::int32_t( d );
 				std::int64_t const nblk = ( d + 1 + 3 ) / 4;
-				if( nblk <= 64 * KB * NW )
+				if( nblk <= 64 * LANE_BLOCKS * NW )
 				{
 					// this wave's blocks
 					std::int32_t const each = ( std::int32_t( nblk ) + NW - 1 ) / NW;
@@ -331,9 +331,9 @@ static void launch_targets( std::vector<conn> const & conns, conn const * dconns
 		unsigned const grid = unsigned( std::min<std::int64_t>( ( n + per - 1 ) / per, blocks * 256 / bs ) );
 		SPICE_LAUNCH( k_targets<NW><<<dim3( grid ), bs, 0, s>>>( dconns, int( conns.size() ), n, width, seed, row_ptr, col ) );
 	};
-	if( longest < 256.0 * KB - 4.0 ) // (a wave holds 256 KB draws, the last one of a connection sets the scale)
+	if( longest < 256.0 * LANE_BLOCKS - 4.0 ) // (a wave holds 256 x LANE_BLOCKS draws, the last one of a connection sets the scale)
 		go( std::integral_constant<int, 1>{} );
-	else if( longest < 1024.0 * KB - 4.0 )
+	else if( longest < 1024.0 * LANE_BLOCKS - 4.0 )
 		go( std::integral_constant<int, 4>{} );
 	else
 		go( std::integral_constant<int, 16>{} );
