@@ -539,7 +539,10 @@ __device__ inline std::int64_t seg_at( dview const & v, std::int64_t r, std::int
 // The segment of row r in tile t: its place in col and its length (an entry has 40 and 24 bits of
 // them). Where rows may be longer than that, or the table would take too much of the memory
 // (rules.h), it has the offsets of the tiles' first targets in the row instead, ntiles + 1 of 4 bytes
-// per row. Read and unpacked apart, so that nothing waits for what is read ahead.
+// per row. Read and unpacked apart, so that nothing waits for what is read ahead. Which of the two a
+// network has is known to the window kernels of a single net (TABLE or OFFSETS: a test on the way to
+// the entry costs a step of small plastic networks 2 %), and looked up by the others (ANY).
+enum { TABLE, OFFSETS, ANY };
 struct segment
 {
 	std::int64_t at;
@@ -550,21 +553,23 @@ struct packed_segment
 	std::uint64_t entry; // or two offsets
 	std::int64_t row;    // (offsets: where the row starts)
 };
+template <int KIND>
 __device__ inline packed_segment load_segment( dview const & v, std::int64_t r, std::int32_t t )
 {
-	if( v.segs ) return { v.segs[seg_at( v, r, t )], 0 };
+	if( KIND == TABLE || ( KIND == ANY && v.segs ) ) return { v.segs[seg_at( v, r, t )], 0 };
 	packed_segment p;
 	__builtin_memcpy( &p.entry, v.offs + ( r * ( v.ntiles + 1 ) + t ), 8 ); // (4-byte alignment suffices)
 	p.row = v.row_ptr[r];
 	return p;
 }
+template <int KIND>
 __device__ inline segment unpack_segment( dview const & v, packed_segment const & p )
 {
-	if( v.segs ) return { std::int64_t( p.entry & ( ( std::uint64_t( 1 ) << 40 ) - 1 ) ), std::int32_t( p.entry >> 40 ) };
+	if( KIND == TABLE || ( KIND == ANY && v.segs ) ) return { std::int64_t( p.entry & ( ( std::uint64_t( 1 ) << 40 ) - 1 ) ), std::int32_t( p.entry >> 40 ) };
 	std::uint32_t const a = std::uint32_t( p.entry ), b = std::uint32_t( p.entry >> 32 );
 	return { p.row + std::int64_t( a ), std::int32_t( b - a ) };
 }
-__device__ inline segment segment_of( dview const & v, std::int64_t r, std::int32_t t ) { return unpack_segment( v, load_segment( v, r, t ) ); }
+__device__ inline segment segment_of( dview const & v, std::int64_t r, std::int32_t t ) { return unpack_segment<ANY>( v, load_segment<ANY>( v, r, t ) ); }
 
 // The segment table. One wave per row, binary searches for 63 tiles at a time (the last lane's is
 // where the 63rd one ends).

@@ -1249,7 +1249,7 @@ private:
 				while( w > 1 && bytes( w ) > room ) w = window_steps( w - 1 );
 				_window = w;
 			} );
-			for( int form : { IDS32, IDS16, IDS16X8, RECORDS } )
+			for( int form : { IDS32, IDS16, IDS16X8, RECORDS, IDS32_OFFSETS } )
 				with_window_kernel( form, [&]( auto kernel, auto bytes, int ) { allow_lds( reinterpret_cast<void const *>( kernel ), bytes( _window ) ); } );
 		}
 	}
@@ -1305,7 +1305,7 @@ private:
 	{
 		_v.col16 = nullptr;
 		double const mean = double( _g.nnz ) / double( _g.n ) / _v.nact;
-		if( _window == 0 || _v.rec_lg || !wants_halves( mean ) )
+		if( _window == 0 || _v.rec_lg || _v.offs || !wants_halves( mean ) )
 		{
 			_col16.release();
 			return;
@@ -1316,7 +1316,7 @@ private:
 			SPICE_LAUNCH( k_halves<<<unsigned( std::min<std::size_t>( ( std::size_t( _g.nnz ) / 8 + 256 ) / 256, 256 * 32 ) ), 256, 0, _s>>>( _g.col.data(), _g.nnz, _col16.data() ) );
 		}
 		_v.col16 = _col16.data();
-		_v.vec16 = !plastic && mean >= 56.0 && _v.segs ? 8 : 4; // (8: lengths of 24 bits)
+		_v.vec16 = !plastic && mean >= 56.0 ? 8 : 4;
 		// (lanes per segment: see choose_window)
 		_v.wlanes = 0;
 		while( _v.wlanes < 5 && double( _v.vec16 << _v.wlanes ) < mean + ( mean < 20.0 ? 2.0 : 1.0 ) * std::sqrt( mean ) + ( _v.vec16 == 8 ? 4.0 : 0.0 ) ) _v.wlanes++;
@@ -1343,7 +1343,7 @@ private:
 		{
 			int const lg = record_size( double( _g.nnz ) / double( _g.n ) / _v.nact );
 			std::uint64_t const segs = seg_entries( _g.n, _v.ntiles ), bytes = segs << lg;
-			if( _v.wcap > 1 || _window == 0 || _p.batched || lg > 6 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
+			if( _v.wcap > 1 || _window == 0 || _p.batched || _v.offs || lg > 6 || _g.nnz == 0 || bytes > std::max<std::uint64_t>( 64 << 20, 8 * std::uint64_t( _g.nnz ) ) ) return;
 			if( !fits( bytes ) ) return;
 			try
 			{
@@ -1496,7 +1496,7 @@ private:
 			if( alone ) launch_passes( t, _s );
 			if( _slog_ctl.size() ) throw std::logic_error( "nets with a spike log are stepped by a batch" );
 			dview v = _vs[t & ( CLOCK_SLOTS - 1 )];
-			with_window_kernel( v.rec_lg ? RECORDS : !v.col16 ? IDS32 : v.vec16 == 8 ? IDS16X8 : IDS16, [&]( auto kernel, auto bytes, int bs ) {
+			with_window_kernel( v.offs ? IDS32_OFFSETS : v.rec_lg ? RECORDS : !v.col16 ? IDS32 : v.vec16 == 8 ? IDS16X8 : IDS16, [&]( auto kernel, auto bytes, int bs ) {
 				std::int32_t W = w;
 				void * args[] = { &v, &W };
 				void const * fn = reinterpret_cast<void const *>( kernel );
@@ -1516,7 +1516,7 @@ private:
 			constexpr bool FX = decltype( fx )::value;
 			constexpr int BS = decltype( b )::value;
 			constexpr bool cl = input_classes_v<Model> > 0;
-			f( form == RECORDS ? &k_window<Model, FX, BS, cl ? RECORDS : IDS32> : form == IDS16 ? &k_window<Model, FX, BS, cl || plastic ? IDS16 : IDS32> : form == IDS16X8 ? &k_window<Model, FX, BS, cl ? IDS16X8 : IDS32> : &k_window<Model, FX, BS>,
+			f( form == RECORDS ? &k_window<Model, FX, BS, cl ? RECORDS : IDS32> : form == IDS16 ? &k_window<Model, FX, BS, cl || plastic ? IDS16 : IDS32> : form == IDS16X8 ? &k_window<Model, FX, BS, cl ? IDS16X8 : IDS32> : form == IDS32_OFFSETS ? &k_window<Model, FX, BS, IDS32_OFFSETS> : &k_window<Model, FX, BS>,
 			   [&]( int w ) { return window_lds<Model, FX>::bytes( BS, _lc.tile_w, w ); }, BS );
 		};
 		auto by_block = [&]( auto fx ) {

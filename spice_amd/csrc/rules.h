@@ -82,18 +82,30 @@ inline int window_tile_w( std::int64_t n, std::int64_t targets, bool plastic, bo
 }
 
 // One staged row segment of a chunk of spikes (window.h). Rows may name a target many times, so a
-// segment may be longer than its tile is wide.
+// segment may be longer than its tile is wide. step: of the window, in the bits that the source (of a
+// plastic network: 24 bits) or the place leaves.
 struct alignas( 16 ) win_seg
 {
-	std::int64_t place; // first target id in the row store (0 for an empty segment), step of the window << 48
+	std::int64_t at; // first target id in the row store (0 for an empty segment)
 	std::int32_t src;
 	std::int32_t len;
 
-	HYBRID static win_seg of( std::int64_t at, std::int32_t len, std::int32_t src, std::int32_t step = 0 )
+	template <bool plastic>
+	HYBRID static win_seg of( std::int64_t at, std::int32_t len, std::int32_t src, std::int32_t step )
 	{
-		return { ( len > 0 ? at : 0 ) | std::int64_t( step ) << 48, src, len };
+		if( len <= 0 ) at = 0;
+		return plastic ? win_seg{ at, src | step << 24, len } : win_seg{ at | std::int64_t( step ) << 48, src, len };
 	}
-	HYBRID std::int64_t at() const { return place & ( ( std::int64_t( 1 ) << 48 ) - 1 ); }
-	HYBRID std::int32_t step() const { return std::int32_t( place >> 48 ); }
+	// Gives the step, and leaves place and source alone.
+	template <bool plastic>
+	HYBRID std::int32_t take_step()
+	{
+		std::int32_t const step = plastic ? src >> 24 : std::int32_t( at >> 48 );
+		if( plastic )
+			src &= ( 1 << 24 ) - 1;
+		else
+			at &= ( std::int64_t( 1 ) << 48 ) - 1;
+		return step;
+	}
 };
 } // namespace spice::hipx

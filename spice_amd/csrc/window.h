@@ -80,8 +80,10 @@ __device__ inline void wave_lds_fence()
 }
 
 // ---- what a delivery reads of a row's segment in a tile --------------------------------------
-enum { IDS32, IDS16, IDS16X8, RECORDS }; // the row store; its halves, 4 or 8 per lane; segment records (the last two: models with input classes)
-constexpr int SKIP_AT = 28; // IDS16X8: a staged segment's first place in its piece lies above its length (of 24 bits: build_halves)
+// the row store; its halves, 4 or 8 per lane; segment records (the last two: models with input classes);
+// the row store by offsets in place of the segment table, or by either
+enum { IDS32, IDS16, IDS16X8, RECORDS, IDS32_OFFSETS, IDS32_ANY };
+constexpr int SKIP_AT = 28; // IDS16X8: a staged segment's first place in its piece lies above its length (of 24 bits, as the segment table has)
 
 // The low halves of the target ids, which tell a target within a tile (of at most 65,536); n of them
 // are read at once: 4 from any place, 8 from a multiple of 8 (the store is padded by 8).
@@ -331,6 +333,8 @@ template <typename Model, bool FIXED, int BS, int FORM = IDS32>
 __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 {
 	constexpr bool REC = FORM == RECORDS;
+	constexpr bool READS32 = FORM == IDS32 || FORM == IDS32_OFFSETS || FORM == IDS32_ANY;
+	constexpr int KIND = FORM == IDS32_OFFSETS ? OFFSETS : FORM == IDS32_ANY ? ANY : TABLE;
 	using N = typename Model::neuron;
 	using S = typename Model::synapse;
 	using L = window_lds<Model, FIXED>;
@@ -499,7 +503,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 		win_seg * const mine = seg + wave * 64;
 		std::int32_t src, q = 0, src_n = 0, q_n = 0;
 		packed_segment ps;
-		auto fetch_seg = [&]() { ps = load_segment( v, src, tile ); };
+		auto fetch_seg = [&]() { ps = load_segment<KIND>( v, src, tile ); };
 		src = fetch_id( k0 + mylane, q );
 		fetch_seg();
 		if( k0 + NW * per < total ) src_n = fetch_id( k0 + NW * per + mylane, q_n );
@@ -508,19 +512,19 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 		for( ; k0 < total; k0 += NW * per )
 		{
 			std::int32_t const cnt = ( total - k0 ) < per ? ( total - k0 ) : per;
-			segment const sg = unpack_segment( v, ps );
+			segment const sg = unpack_segment<KIND>( v, ps );
 			std::int64_t const a = sg.at;
 			std::int32_t const len = lane < cnt ? sg.len : 0;
 			if constexpr( L::classes > 0 )
 			{
 				// in the place of the source: where the class's counters of the step start (for target 0).
 				// IDS16X8: from the piece that the segment begins in, its place there above the length
-				std::int32_t const at = ( q * nacc + N::input_class( src, info ) ) * tws - ( FORM == IDS32 ? t0 : 0 );
+				std::int32_t const at = ( q * nacc + N::input_class( src, info ) ) * tws - ( READS32 ? t0 : 0 );
 				std::int32_t const skip = FORM == IDS16X8 && len > 0 ? std::int32_t( a ) & 7 : 0;
-				mine[lane] = win_seg::of( a & ~std::int64_t( FORM == IDS16X8 ? 7 : 0 ), ( len + skip ) | skip << SKIP_AT, at );
+				mine[lane] = win_seg{ len > 0 ? a & ~std::int64_t( FORM == IDS16X8 ? 7 : 0 ) : 0, at, ( len + skip ) | skip << SKIP_AT };
 			}
 			else
-				mine[lane] = win_seg::of( a, len, src, q );
+				mine[lane] = win_seg::of<plastic>( a, len, src, q );
 			ev += std::uint32_t( len );
 			wave_lds_fence();
 			if( k0 + NW * per < total )
@@ -542,8 +546,8 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 					std::int32_t const k = c + u * ng + g;
 					r[u] = mine[k & 63]; // (records from cnt on are empty)
 					len[u] = k < 64 ? ( FORM == IDS16X8 ? r[u].len & ( ( 1 << SKIP_AT ) - 1 ) : r[u].len ) : 0;
-					step[u] = FORM == IDS16X8 ? r[u].len >> SKIP_AT : L::classes == 0 ? r[u].step() : 0; // (or skip)
-					if constexpr( L::classes == 0 ) r[u].place = r[u].at();
+					step[u] = FORM == IDS16X8 ? r[u].len >> SKIP_AT : 0; // (its skip)
+					if constexpr( L::classes == 0 ) step[u] = r[u].template take_step<plastic>();
 					most = len[u] > most ? len[u] : most;
 				}
 				for( std::int32_t e = l * V;; e += G * V )
@@ -553,7 +557,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 					{
 						halves<V> j[U];
 #pragma unroll
-						for( int u = 0; u < U; u++ ) j[u] = load_halves<V>( v.col16 + r[u].place + ( e < len[u] ? e : 0 ) );
+						for( int u = 0; u < U; u++ ) j[u] = load_halves<V>( v.col16 + r[u].at + ( e < len[u] ? e : 0 ) );
 #pragma unroll
 						for( int u = 0; u < U; u++ )
 #pragma unroll
@@ -567,17 +571,17 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 					for( int u = 0; u < U; u++ )
 						if constexpr( FORM == IDS16 )
 						{
-							halves<V> const low = load_halves<V>( v.col16 + r[u].place + ( e < len[u] ? e : 0 ) );
+							halves<V> const low = load_halves<V>( v.col16 + r[u].at + ( e < len[u] ? e : 0 ) );
 #pragma unroll
 							for( int x = 0; x < V; x++ ) j[u].id[x] = t0 + ( ( low.id[x] - t0 ) & 0xffff );
 						}
 						else
-							j[u] = load_targets( v.col + r[u].place + ( e < len[u] ? e : 0 ) );
+							j[u] = load_targets( v.col + r[u].at + ( e < len[u] ? e : 0 ) );
 					synapses<S> sy[U];
 					if constexpr( plastic )
 					{
 #pragma unroll
-						for( int u = 0; u < U; u++ ) sy[u].load( v.sa, r[u].place + ( e < len[u] ? e : 0 ) );
+						for( int u = 0; u < U; u++ ) sy[u].load( v.sa, r[u].at + ( e < len[u] ? e : 0 ) );
 					}
 #pragma unroll
 					for( int u = 0; u < U; u++ )
@@ -593,7 +597,7 @@ __device__ inline void window_tile( dview const & v, std::int32_t pos, int W )
 								tile_backend<FIXED> bak{ make_backend<FIXED>( v, std::uint32_t( r[u].src ), std::uint32_t( j[u].id[x] ), std::uint32_t( T0 + s ), util::TAG_RECEIVE ) };
 								win_iter<N, FIXED> dst{ &v, j[u].id[x], t0, tws, acc + s * ( nacc * tws ) };
 								if constexpr( plastic )
-									deliver_event<N>( r[u].src, dst, reg_iter<typename S::tuple_t>{ sy[u].s[x], std::uint32_t( r[u].place + e + x ) }, info, bak );
+									deliver_event<N>( r[u].src, dst, reg_iter<typename S::tuple_t>{ sy[u].s[x], std::uint32_t( r[u].at + e + x ) }, info, bak );
 								else
 									deliver_event<N>( r[u].src, dst, no_syn_iter{}, info, bak );
 							}
@@ -1255,7 +1259,7 @@ __global__ __launch_bounds__( BS ) void k_batch_window( dview const * views, std
 	std::int32_t const b = blockIdx.x;
 	if( b < ntiles )
 	{
-		window_tile<Model, FIXED, BS>( views[tile_net[b]], tile_pos[b], W );
+		window_tile<Model, FIXED, BS, IDS32_ANY>( views[tile_net[b]], tile_pos[b], W );
 		return;
 	}
 	std::int32_t const p = b - ntiles;

@@ -4,6 +4,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <set>
+#include <type_traits>
 
 using namespace spice::hipx;
 
@@ -54,8 +55,16 @@ static void staged_segments()
 		for( std::int32_t len : { 0, 1, 65528, 65535, 65536, 65537, 131072, 1 << 24, INT32_MAX - 7 } )
 			for( int step = 0; step < WINDOW_MAX; step++ )
 			{
-				win_seg const s = win_seg::of( at, len, 12345, step );
-				CHECK( s.at() == ( len > 0 ? at : 0 ) && s.len == len && s.src == 12345 && s.step() == step, "at %lld len %d step %d", (long long)( at ), len, step );
+				for( std::int32_t src : { 0, 12345, ( 1 << 24 ) - 1 } )
+				{
+					auto back = [&]( auto plastic ) {
+						constexpr bool P = decltype( plastic )::value;
+						win_seg s = win_seg::of<P>( at, len, src, step );
+						CHECK( s.take_step<P>() == step && s.at == ( len > 0 ? at : 0 ) && s.len == len && s.src == src, "at %lld len %d step %d src %d", (long long)( at ), len, step, src );
+					};
+					back( std::true_type{} );
+					back( std::false_type{} );
+				}
 			}
 	static_assert( sizeof( win_seg ) == 16, "" );
 }
