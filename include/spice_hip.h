@@ -321,7 +321,7 @@ int spice_hip_set_launch( spice_net * net, const spice_launch * in );
 /* Times candidate launch shapes on a copy of the network (warmup steps first, then `steps`
  * steps per candidate, wall time per step: plasticity overlaps delivery, so
  * shapes are evaluated together; tile width first, then delivery parts (where they have an effect), then the plasticity
- * shape; the three fastest are then timed again in turn, three times each, since the copy's
+ * shape; the three fastest, and the one it had, are then timed again in turn, three times each, since the copy's
  * activity drifts between candidates),
  * applies the fastest to the network and returns it with its step time (us). The network
  * itself does not advance. Results are cached per (model, neurons, edges, delay, flags) for

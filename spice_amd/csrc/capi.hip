@@ -882,17 +882,21 @@ int spice_hip_autotune( spice_net * net, int64_t warmup, int64_t steps, spice_la
 			// network's step time moves by 2x and more): the three fastest shapes are timed
 			// again, in turn, three times each, and the fastest in total is kept
 			std::sort( timed.begin(), timed.end(), []( auto const & a, auto const & b ) { return a.first < b.first; } );
+			// -- the shape that the network had among them, as a lucky time is no reason to leave it
 			std::vector<launch_cfg> top;
+			auto add = [&]( launch_cfg const & x ) {
+				for( launch_cfg const & y : top )
+					if( x.tile_w == y.tile_w && x.flush_slots == y.flush_slots && x.flush_grid == y.flush_grid && x.recv_block == y.recv_block &&
+					    x.recv_parts == y.recv_parts )
+						return;
+				top.push_back( x );
+			};
 			for( auto const & tx : timed )
 			{
-				launch_cfg const & x = tx.second;
-				bool seen = false;
-				for( launch_cfg const & y : top )
-					seen = seen || ( x.tile_w == y.tile_w && x.flush_slots == y.flush_slots && x.flush_grid == y.flush_grid &&
-					                 x.recv_block == y.recv_block && x.recv_parts == y.recv_parts );
-				if( !seen ) top.push_back( x );
+				add( tx.second );
 				if( top.size() == 3 ) break;
 			}
+			add( start );
 			if( top.size() > 1 )
 			{
 				std::vector<double> sum( top.size(), 0.0 );
