@@ -190,6 +190,7 @@ public:
 	~hip_batch() override
 	{
 		if( _s ) (void)hipStreamSynchronize( _s );
+		_owned.clear(); // (before the graphs, as in hip_net)
 		_graphs.clear();
 		_queue.clear();
 		if( _s && _own_stream ) (void)hipStreamDestroy( _s );

@@ -193,6 +193,16 @@ public:
 	~hip_net() override
 	{
 		if( _s ) (void)hipStreamSynchronize( _s );
+		// the large buffers first, so that the little that graphs hold stays among the freed memory that
+		// the runtime keeps at hand (Brunel, 10,000 neurons, delay 1, after a run: 0.54 ms, 2.7 with the
+		// graphs first)
+		_recs.release();
+		_col16.release();
+		_segs.release();
+		_offs.release();
+		_tp_ent.release();
+		for( auto & b : _sa ) b.release();
+		_g.col.release();
 		_graphs.clear();
 		_queue.clear();
 		if( _s && _p.own_stream ) (void)hipStreamDestroy( _s );
